@@ -1,10 +1,11 @@
 // DSMC collisions on the device (collisions/DSMC.java:167-430): Bird's no-time-counter scheme
 // per cell after the counting sort, with Boyd's weighting for two species, a constant or VHS
 // (SigmaPlus.SigmaBird463) cross-section and the elastic VHS/VSS scattering of ModelElastic.
-// One wave per cell.  The cell's particle list is the cell range of the sorted species, ordered
-// by particle id in LDS, so that the pair choice (an index into that list) and the cell's
-// Philox stream give the same collisions on every run.  The pairs of a cell are processed in
-// sequence, as in the reference, by the wave's first lane.
+// A cell's particle list is the cell range of the sorted species, ordered by particle id (one wave
+// per cell, dsmc_order), so that the pair choice (an index into that list) and the cell's Philox
+// stream give the same collisions on every run.  The pairs of a cell are processed in sequence, as
+// in the reference, by one lane; a wave runs 64 cells (dsmc_collide).
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
@@ -13,10 +14,10 @@
 
 namespace sf {
 
-constexpr int DSMC_MAXP = 2048;   // particles of one species in one cell held in LDS
-// Cells whose particle ranges are at most DSMC_SMALL long go through a copy of the kernel with
-// DSMC_SMALL-entry LDS lists (8 KB per one-wave workgroup instead of 32 KB), so that a CU holds
-// four times as many of the latency-bound cell loops; the rest through the DSMC_MAXP copy.
+constexpr int DSMC_MAXP = 2048;   // binned particles of one species in one cell
+// Ranges of at most DSMC_SMALL particles are ordered in the registers of one wave (8 keys a lane,
+// 16 registers), longer ones by a workgroup in LDS: twice the keys would double the wave's registers
+// and unrolled code for cells that few runs have.
 constexpr int DSMC_SMALL = 512;
 
 struct DsmcParams {
@@ -49,180 +50,301 @@ __device__ int dsmc_count(const MeshP& m, const PState& s, int a, int b, bool ed
     return n;
 }
 
-// Loads (id << 32 | slot) of the binned particles of [a, b) into key[0..n) and sorts key[0..pow2)
-// by id (bitonic, padded with all-ones).  One wave.
-__device__ void dsmc_load_sorted(const MeshP& m, const PState& s, int a, int b, unsigned long long* key, int& n) {
+// What the collision loop of a cell needs from dsmc_order: the number of candidate pairs (0: none)
+// and of binned particles of each species.
+struct DsmcCell {
+    int nsel, n1, n2;
+};
+
+// Slots of the binned particles of [a, b), ordered by id, into order[a ..), for ranges of at most
+// 64 E particles: a bitonic sort of (id << 32 | slot) in registers.  Element i of the list is
+// register i % E of lane i / E, so strides below E stay in a lane and the others are one 64-bit
+// shuffle; padding is all-ones.
+template <int E>
+__device__ __forceinline__ void order_in_registers(const MeshP& m, const PState& s, int a, int b,
+                                                   int32_t* __restrict__ order) {
+    constexpr int LE = E == 1 ? 0 : (E == 2 ? 1 : (E == 4 ? 2 : 3));
+    static_assert((1 << LE) == E, "E is 1, 2, 4 or 8");
     const int lane = threadIdx.x & 63;
-    int base = 0;
-    for (int p0 = a; p0 < b; p0 += 64) {
-        const int p = p0 + lane;
+    unsigned long long k[E];
+    int n = 0;
+#pragma unroll
+    for (int j = 0; j < E; j++) {
+        const int p = a + j * 64 + lane;
+        const bool in = p < b && dsmc_in_cell(m, s, p);
+        k[j] = in ? ((unsigned long long)(uint32_t)s.id[p] << 32) | (uint32_t)p : ~0ull;
+        n += __popcll(__ballot(in));
+    }
+#pragma unroll
+    for (int sz = 1; sz <= 6 + LE; sz++) {
+#pragma unroll
+        for (int st = sz - 1; st >= 0; st--) {
+            if (st >= LE) {
+                const int lx = 1 << (st - LE);
+                const bool up = sz == 6 + LE || (lane & (1 << (sz - LE))) == 0;
+                const bool keep_min = ((lane & lx) == 0) == up;
+#pragma unroll
+                for (int j = 0; j < E; j++) {
+                    const unsigned long long o = __shfl_xor(k[j], lx);
+                    k[j] = ((o < k[j]) == keep_min) ? o : k[j];
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < E; j++) {
+                    const int q = j ^ (1 << st);
+                    if (q < j) continue;
+                    const bool up = sz < LE ? (j & (1 << sz)) == 0
+                                            : (sz == 6 + LE || (lane & (1 << (sz - LE))) == 0);
+                    const unsigned long long x = k[j], y = k[q];
+                    const bool sw = (x > y) == up;
+                    k[j] = sw ? y : x;
+                    k[q] = sw ? x : y;
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < E; j++)
+        if (lane * E + j < n) order[a + lane * E + j] = (int32_t)(uint32_t)k[j];
+}
+
+__device__ __forceinline__ void order_small(const MeshP& m, const PState& s, int a, int b, int32_t* order) {
+    const int len = b - a;
+    if (len <= 64) order_in_registers<1>(m, s, a, b, order);
+    else if (len <= 128) order_in_registers<2>(m, s, a, b, order);
+    else if (len <= 256) order_in_registers<4>(m, s, a, b, order);
+    else order_in_registers<8>(m, s, a, b, order);
+}
+
+// The same for a longer range, by one workgroup of 256 threads in LDS (key[0 .. pow2), pow2 <=
+// DSMC_MAXP: only binned particles enter it, and dsmc_order refuses more).
+__device__ void order_in_lds(const MeshP& m, const PState& s, int a, int b, int32_t* order, unsigned long long* key,
+                             int* count) {
+    const int t = threadIdx.x, lane = t & 63;
+    if (t == 0) *count = 0;
+    __syncthreads();
+    for (int p0 = a; p0 < b; p0 += 256) {
+        const int p = p0 + t;
         const bool in = p < b && dsmc_in_cell(m, s, p);
         const unsigned long long mask = __ballot(in);
-        const int before = __popcll(mask & ((1ull << lane) - 1ull));
-        if (in) key[base + before] = ((unsigned long long)(uint32_t)s.id[p] << 32) | (uint32_t)p;
-        base += __popcll(mask);
+        int base = 0;
+        if (lane == 0) base = atomicAdd(count, __popcll(mask));
+        base = __shfl(base, 0);
+        if (in)
+            key[base + __popcll(mask & ((1ull << lane) - 1ull))] =
+                ((unsigned long long)(uint32_t)s.id[p] << 32) | (uint32_t)p;
     }
-    n = base;
+    __syncthreads();
+    const int n = *count;
     int np2 = 1;
     while (np2 < n) np2 <<= 1;
-    for (int k = n + lane; k < np2; k += 64) key[k] = ~0ull;
+    for (int k = n + t; k < np2; k += 256) key[k] = ~0ull;
     __syncthreads();
     for (int size = 2; size <= np2; size <<= 1) {
         for (int stride = size >> 1; stride > 0; stride >>= 1) {
-            for (int k = lane; k < np2; k += 64) {
-                const int partner = k ^ stride;
-                if (partner > k) {
-                    const bool up = (k & size) == 0;
-                    const unsigned long long x = key[k], y = key[partner];
-                    if ((x > y) == up) {
-                        key[k] = y;
-                        key[partner] = x;
-                    }
+            for (int q = t; q < np2 / 2; q += 256) {
+                const int k = 2 * q - (q & (stride - 1)), partner = k + stride;
+                const bool up = (k & size) == 0;
+                const unsigned long long x = key[k], y = key[partner];
+                if ((x > y) == up) {
+                    key[k] = y;
+                    key[partner] = x;
                 }
             }
             __syncthreads();
         }
     }
+    for (int k = t; k < n; k += 256) order[a + k] = (int32_t)(uint32_t)key[k];
+    __syncthreads();   // key and count are reused
 }
 
-// (held to 128 registers, four waves per SIMD: the small copy's cell loops then fill a CU four
-// deep at the cost of 172 bytes of spills, 6.4 -> 5.5 ms per pass on 5e7 particles)
-template <int CAP>
-__global__ void __launch_bounds__(64, 4) dsmc_kernel(MeshP m, PState sa, const int32_t* __restrict__ off_a, PState sb,
+// Pair count and particle order of every cell, one wave per cell.  The sort is what bounds it
+// (about 45 compare-exchange steps for the 380 particles of a cell of the 512 x 256 gas); it
+// stays in registers, so no LDS limits the waves in flight.  Cells with a range longer than
+// DSMC_SMALL go to the list big (big[0] counts it), whose order dsmc_order_big makes.
+// 5e7 particles in 512 x 256 cells, at least one candidate pair in each: a pass of a step (order
+// and collisions) takes 0.52 ms here, 0.02 in dsmc_order_big and 0.30 in dsmc_collide; it took 4.8 ms
+// as one kernel with a bitonic sort in LDS and the pair loop on one lane of the cell's wave.
+__global__ void __launch_bounds__(256) dsmc_order(MeshP m, PState sa, const int32_t* __restrict__ off_a, PState sb,
                                                   const int32_t* __restrict__ off_b, DsmcParams pp,
-                                                  double* __restrict__ sig_cr_max, double* __restrict__ rem,
-                                                  double* __restrict__ count_sum, double* __restrict__ real_sum,
-                                                  unsigned long long* __restrict__ ncol, int* __restrict__ overflow) {
-    __shared__ unsigned long long key_a[CAP], key_b[CAP];
-    const int lane = threadIdx.x;
-    const int ncells = m.nci * m.ncj;
-    for (int c = blockIdx.x; c < ncells; c += gridDim.x) {
-        const int ci = c % m.nci, cj = c / m.nci;
-        const bool edge = ci == m.nci - 1 || cj == m.ncj - 1;
-        const int a0 = off_a[c], a1 = off_a[c + 1];
-        int b0 = a0, b1 = a1;
-        if (!pp.same) {
-            b0 = off_b[c];
-            b1 = off_b[c + 1];
-        }
-        // each cell goes through exactly one of the two copies, by its range lengths
-        const bool small = a1 - a0 <= DSMC_SMALL && b1 - b0 <= DSMC_SMALL;
-        if (small != (CAP == DSMC_SMALL)) continue;
-        const double np1 = dsmc_count(m, sa, a0, a1, edge);
-        double np2 = np1;
-        if (!pp.same) np2 = dsmc_count(m, sb, b0, b1, edge);
-        // collideCell (DSMC.java:238-350): NTC pair count with Boyd's weights (eq. 5); evaluated
-        // without fused multiply-adds, so that its integer part is the reference's
-        const double scm0 = sig_cr_max[c];
-        double nsel_f;
-        {
-#pragma clang fp contract(off)
-            const double cell_volume = node_vol_at(m, ci + 0.5, cj + 0.5);
-            double Pab = pp.spwt_b / pp.spwt_a, Pba = pp.spwt_a / pp.spwt_b;
-            if (Pab > 1) Pab = 1;
-            if (Pba > 1) Pba = 1;
-            nsel_f = ((np1 * pp.spwt_a / cell_volume) * np2 * pp.delta_t * scm0) / (Pab + (pp.spwt_b / pp.spwt_a) * Pba);
-            if (!pp.same) nsel_f *= 2.0;
-            nsel_f += rem[c];
-        }
-        int nsel = (int)nsel_f;
-        if ((pp.same && (np1 < 2 || np2 < 2)) || np1 < 1 || np2 < 1) continue;
-        double new_rem = nsel_f - nsel;   // an exact subtraction
-        if (nsel > np1 * np2) {
-            nsel = (int)(np1 * np2);
-            new_rem = 0;
-        }
-        if (nsel == 0) {
-            if (lane == 0) rem[c] = new_rem;
-            continue;
-        }
-        if (np1 > CAP || np2 > CAP) {
-            if (lane == 0) atomicMax(overflow, (int)fmax(np1, np2));
-            continue;
-        }
-        int n1 = 0, n2 = 0;
-        dsmc_load_sorted(m, sa, a0, a1, key_a, n1);
-        unsigned long long* kb = key_a;
-        if (!pp.same) {
-            dsmc_load_sorted(m, sb, b0, b1, key_b, n2);
-            kb = key_b;
-        }
-        if (lane == 0) {
-            ParticleRng rng{pp.k0, pp.k1, (uint32_t)c, pp.step, pp.tag};
-            uint32_t k = 0;
-            double scm = 0, sums0 = 0, sums1 = 0;
-            const double rm1 = pp.mass_a / (pp.mass_a + pp.mass_b), rm2 = pp.mass_b / (pp.mass_a + pp.mass_b);
-            for (int q = 0; q < nsel; q++) {
-                const int p1 = (int)(rng.draw(k++) * np1);
-                int p2;
-                do {
-                    p2 = (int)(rng.draw(k++) * np2);
-                } while (pp.same && p1 == p2);
-                const int64_t ga = (int64_t)(uint32_t)key_a[p1];
-                const int64_t gb = (int64_t)(uint32_t)kb[p2];
-                const PState& Sb = pp.same ? sa : sb;
-                double va[3] = {sa.vx[ga], sa.vy[ga], sa.vz[ga]};
-                double vb[3] = {Sb.vx[gb], Sb.vy[gb], Sb.vz[gb]};
-                const double g0 = va[0] - vb[0], g1 = va[1] - vb[1], g2 = va[2] - vb[2];
-                const double cr = sqrt(g0 * g0 + g1 * g1 + g2 * g2);
-                const double sigma_cr = cr * dsmc_sigma(pp, cr);
-                if (sigma_cr > scm) scm = sigma_cr;
-                const double P = sigma_cr / scm0;
-                if (rng.draw(k++) < P) {
-                    // ModelElastic (DSMC.java:360-430), Bird's DSMC0 scattering
-                    double vc[3], vr[3];
-                    for (int d = 0; d < 3; d++) vc[d] = rm1 * va[d] + rm2 * vb[d];
-                    if (fabs(pp.vss_inv - 1.) < 1.e-4) {
-                        const double B = 2. * rng.draw(k++) - 1.0;
-                        const double A = sqrt(1. - B * B);
-                        vr[0] = B * cr;
-                        const double C = 2. * M_PI * rng.draw(k++);
-                        vr[1] = A * cos(C) * cr;
-                        vr[2] = A * sin(C) * cr;
-                    } else {
-                        const double B = 2. * (pow(rng.draw(k++), pp.vss_inv)) - 1.;
-                        const double A = sqrt(1. - B * B);
-                        const double C = 2. * M_PI * rng.draw(k++);
-                        const double OC = cos(C), SC = sin(C);
-                        const double D = sqrt(g1 * g1 + g2 * g2);
-                        if (D > 1.e-6) {
-                            vr[0] = B * g0 + A * SC * D;
-                            vr[1] = B * g1 + A * (cr * g2 * OC - g0 * g1 * SC) / D;
-                            vr[2] = B * g2 - A * (cr * g1 * OC + g0 * g2 * SC) / D;
-                        } else {
-                            vr[0] = B * g1;
-                            vr[1] = A * OC * g1;
-                            vr[2] = A * SC * g1;
-                        }
-                    }
-                    bool wa = true, wb = true;
-                    if (pp.spwt_a != pp.spwt_b) {   // Boyd's probabilities for unequal weights
-                        wa = rng.draw(k++) < pp.spwt_b / pp.spwt_a;
-                        wb = rng.draw(k++) < pp.spwt_a / pp.spwt_b;
-                    }
-                    if (wa) {
-                        sa.vx[ga] = (float)(vc[0] + vr[0] * rm2);
-                        sa.vy[ga] = (float)(vc[1] + vr[1] * rm2);
-                        sa.vz[ga] = (float)(vc[2] + vr[2] * rm2);
-                    }
-                    if (wb) {
-                        Sb.vx[gb] = (float)(vc[0] - vr[0] * rm1);
-                        Sb.vy[gb] = (float)(vc[1] - vr[1] * rm1);
-                        Sb.vz[gb] = (float)(vc[2] - vr[2] * rm1);
-                    }
-                    sums0 += 1.0;
-                    sums1 += 0.5 * (pp.spwt_a + pp.spwt_b);
-                }
-            }
-            rem[c] = new_rem;
-            if (scm > 0) sig_cr_max[c] = scm;
-            const size_t u = (size_t)cj * m.ni + ci;
-            count_sum[u] += sums0;
-            real_sum[u] += sums1;
-            if (sums0 > 0) atomicAdd(ncol, (unsigned long long)sums0);
-        }
-        __syncthreads();   // the LDS lists are reused by the next cell
+                                                  const double* __restrict__ sig_cr_max, double* __restrict__ rem,
+                                                  int32_t* __restrict__ order_a, int32_t* __restrict__ order_b,
+                                                  DsmcCell* __restrict__ cells, int* __restrict__ big,
+                                                  int* __restrict__ overflow) {
+    const int lane = threadIdx.x & 63;
+    const int c = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (c >= m.nci * m.ncj) return;
+    const int ci = c % m.nci, cj = c / m.nci;
+    const bool edge = ci == m.nci - 1 || cj == m.ncj - 1;
+    const int a0 = off_a[c], a1 = off_a[c + 1];
+    int b0 = a0, b1 = a1;
+    if (!pp.same) {
+        b0 = off_b[c];
+        b1 = off_b[c + 1];
     }
+    const double np1 = dsmc_count(m, sa, a0, a1, edge);
+    double np2 = np1;
+    if (!pp.same) np2 = dsmc_count(m, sb, b0, b1, edge);
+    // collideCell (DSMC.java:238-350): NTC pair count with Boyd's weights (eq. 5); evaluated
+    // without fused multiply-adds, so that its integer part is the reference's
+    const double scm0 = sig_cr_max[c];
+    double nsel_f;
+    {
+#pragma clang fp contract(off)
+        const double cell_volume = node_vol_at(m, ci + 0.5, cj + 0.5);
+        double Pab = pp.spwt_b / pp.spwt_a, Pba = pp.spwt_a / pp.spwt_b;
+        if (Pab > 1) Pab = 1;
+        if (Pba > 1) Pba = 1;
+        nsel_f = ((np1 * pp.spwt_a / cell_volume) * np2 * pp.delta_t * scm0) / (Pab + (pp.spwt_b / pp.spwt_a) * Pba);
+        if (!pp.same) nsel_f *= 2.0;
+        nsel_f += rem[c];
+    }
+    int nsel = (int)nsel_f;
+    const bool pairs = !((pp.same && (np1 < 2 || np2 < 2)) || np1 < 1 || np2 < 1);
+    double new_rem = nsel_f - nsel;   // an exact subtraction
+    if (nsel > np1 * np2) {
+        nsel = (int)(np1 * np2);
+        new_rem = 0;
+    }
+    const bool over = pairs && nsel != 0 && (np1 > DSMC_MAXP || np2 > DSMC_MAXP);
+    const bool go = pairs && nsel != 0 && !over;
+    if (lane == 0) {
+        if (pairs && !over) rem[c] = new_rem;
+        if (over) atomicMax(overflow, (int)fmax(np1, np2));
+        cells[c] = DsmcCell{go ? nsel : 0, (int)np1, (int)np2};
+    }
+    if (!go) return;
+    if (a1 - a0 > DSMC_SMALL || b1 - b0 > DSMC_SMALL) {
+        if (lane == 0) big[1 + atomicAdd(&big[0], 1)] = c;
+        return;
+    }
+    order_small(m, sa, a0, a1, order_a);
+    if (!pp.same) order_small(m, sb, b0, b1, order_b);
+}
+
+// A cell's range holds its binned particles and, in the last row and column, particles on the last
+// node line: those of a range may exceed DSMC_MAXP, the binned ones that enter the LDS list not.
+__global__ void __launch_bounds__(256) dsmc_order_big(MeshP m, PState sa, const int32_t* __restrict__ off_a, PState sb,
+                                                      const int32_t* __restrict__ off_b, int same,
+                                                      int32_t* __restrict__ order_a, int32_t* __restrict__ order_b,
+                                                      const int* __restrict__ big) {
+    __shared__ unsigned long long key[DSMC_MAXP];
+    __shared__ int count;
+    const int nbig = big[0];
+    for (int q = blockIdx.x; q < nbig; q += gridDim.x) {
+        const int c = big[1 + q];
+        order_in_lds(m, sa, off_a[c], off_a[c + 1], order_a, key, &count);
+        if (!same) order_in_lds(m, sb, off_b[c], off_b[c + 1], order_b, key, &count);
+    }
+}
+
+// The last Philox block a stream drew from: draws 2q and 2q + 1 are its two halves.
+struct PairedRng {
+    ParticleRng r;
+    uint32_t block;
+    double even, odd;
+    __device__ __forceinline__ double draw(uint32_t k) {
+        if ((k >> 1) != block) {
+            block = k >> 1;
+            const uint4 o = philox4x32_10(make_uint4(block, r.id, r.step, r.tag), r.k0, r.k1);
+            even = (double)((((uint64_t)o.y << 32) | o.x) >> 11) * 0x1.0p-53;
+            odd = (double)((((uint64_t)o.w << 32) | o.z) >> 11) * 0x1.0p-53;
+        }
+        return (k & 1) ? odd : even;
+    }
+};
+
+// The collision loop of every cell, one LANE per cell.  A cell's pairs are sequential (a particle
+// drawn twice must see its first collision's velocity, and a pair's draws follow the last one's),
+// but the cells are independent: 64 of them share a wave's instruction stream, where a loop on one
+// lane of a wave per cell spent the same instructions (Philox, pow, sin, cos) on one cell.
+__global__ void __launch_bounds__(64) dsmc_collide(MeshP m, PState sa, const int32_t* __restrict__ off_a, PState sb,
+                                                   const int32_t* __restrict__ off_b, DsmcParams pp,
+                                                   const int32_t* __restrict__ order_a,
+                                                   const int32_t* __restrict__ order_b,
+                                                   const DsmcCell* __restrict__ cells, double* __restrict__ sig_cr_max,
+                                                   double* __restrict__ count_sum, double* __restrict__ real_sum,
+                                                   unsigned long long* __restrict__ ncol) {
+    const int c = blockIdx.x * 64 + threadIdx.x;
+    double sums0 = 0, sums1 = 0;
+    if (c < m.nci * m.ncj && cells[c].nsel > 0) {
+        const DsmcCell cell = cells[c];
+        const int ci = c % m.nci, cj = c / m.nci;
+        const double np1 = cell.n1, np2 = cell.n2, scm0 = sig_cr_max[c];
+        const int32_t* la = order_a + off_a[c];
+        const int32_t* lb = pp.same ? la : order_b + off_b[c];
+        const PState& Sb = pp.same ? sa : sb;
+        PairedRng rng{{pp.k0, pp.k1, (uint32_t)c, pp.step, pp.tag}, 0xFFFFFFFFu, 0.0, 0.0};
+        uint32_t k = 0;
+        double scm = 0;
+        const double rm1 = pp.mass_a / (pp.mass_a + pp.mass_b), rm2 = pp.mass_b / (pp.mass_a + pp.mass_b);
+        for (int q = 0; q < cell.nsel; q++) {
+            const int p1 = (int)(rng.draw(k++) * np1);
+            int p2;
+            do {
+                p2 = (int)(rng.draw(k++) * np2);
+            } while (pp.same && p1 == p2);
+            const int64_t ga = la[p1], gb = lb[p2];
+            double va[3] = {sa.vx[ga], sa.vy[ga], sa.vz[ga]};
+            double vb[3] = {Sb.vx[gb], Sb.vy[gb], Sb.vz[gb]};
+            const double g0 = va[0] - vb[0], g1 = va[1] - vb[1], g2 = va[2] - vb[2];
+            const double cr = sqrt(g0 * g0 + g1 * g1 + g2 * g2);
+            const double sigma_cr = cr * dsmc_sigma(pp, cr);
+            if (sigma_cr > scm) scm = sigma_cr;
+            const double P = sigma_cr / scm0;
+            if (rng.draw(k++) < P) {
+                // ModelElastic (DSMC.java:360-430), Bird's DSMC0 scattering
+                double vc[3], vr[3];
+                for (int d = 0; d < 3; d++) vc[d] = rm1 * va[d] + rm2 * vb[d];
+                if (fabs(pp.vss_inv - 1.) < 1.e-4) {
+                    const double B = 2. * rng.draw(k++) - 1.0;
+                    const double A = sqrt(1. - B * B);
+                    vr[0] = B * cr;
+                    const double C = 2. * M_PI * rng.draw(k++);
+                    vr[1] = A * cos(C) * cr;
+                    vr[2] = A * sin(C) * cr;
+                } else {
+                    const double B = 2. * (pow(rng.draw(k++), pp.vss_inv)) - 1.;
+                    const double A = sqrt(1. - B * B);
+                    const double C = 2. * M_PI * rng.draw(k++);
+                    const double OC = cos(C), SC = sin(C);
+                    const double D = sqrt(g1 * g1 + g2 * g2);
+                    if (D > 1.e-6) {
+                        vr[0] = B * g0 + A * SC * D;
+                        vr[1] = B * g1 + A * (cr * g2 * OC - g0 * g1 * SC) / D;
+                        vr[2] = B * g2 - A * (cr * g1 * OC + g0 * g2 * SC) / D;
+                    } else {
+                        vr[0] = B * g1;
+                        vr[1] = A * OC * g1;
+                        vr[2] = A * SC * g1;
+                    }
+                }
+                bool wa = true, wb = true;
+                if (pp.spwt_a != pp.spwt_b) {   // Boyd's probabilities for unequal weights
+                    wa = rng.draw(k++) < pp.spwt_b / pp.spwt_a;
+                    wb = rng.draw(k++) < pp.spwt_a / pp.spwt_b;
+                }
+                if (wa) {
+                    sa.vx[ga] = (float)(vc[0] + vr[0] * rm2);
+                    sa.vy[ga] = (float)(vc[1] + vr[1] * rm2);
+                    sa.vz[ga] = (float)(vc[2] + vr[2] * rm2);
+                }
+                if (wb) {
+                    Sb.vx[gb] = (float)(vc[0] - vr[0] * rm1);
+                    Sb.vy[gb] = (float)(vc[1] - vr[1] * rm1);
+                    Sb.vz[gb] = (float)(vc[2] - vr[2] * rm1);
+                }
+                sums0 += 1.0;
+                sums1 += 0.5 * (pp.spwt_a + pp.spwt_b);
+            }
+        }
+        if (scm > 0) sig_cr_max[c] = scm;
+        const size_t u = (size_t)cj * m.ni + ci;
+        count_sum[u] += sums0;
+        real_sum[u] += sums1;
+    }
+    for (int o = 32; o > 0; o >>= 1) sums0 += __shfl_xor(sums0, o);
+    if (threadIdx.x == 0 && sums0 > 0) atomicAdd(ncol, (unsigned long long)sums0);
 }
 
 __global__ void dsmc_fields_kernel(int64_t nn, int which, const double* __restrict__ count_sum,
@@ -267,6 +389,8 @@ struct sf_dsmc {
     double* d_rem = nullptr;      // [ncells]
     double* d_count = nullptr;    // [nn] col-count-sum
     double* d_real = nullptr;     // [nn] col-real-sum
+    DsmcCell* d_cells = nullptr;  // [ncells] pair and particle counts of the running pass
+    int* d_big = nullptr;         // [1 + ncells] count and list of the cells that dsmc_order_big orders
     unsigned long long* d_ncol = nullptr;
     int* d_overflow = nullptr;
     int num_samples = 0;
@@ -325,6 +449,8 @@ int sf_dsmc_create(sf_ctx* ctx, const sf_dsmc_desc* desc, sf_dsmc** out) {
     if (e == hipSuccess) e = hipMalloc((void**)&d->d_rem, nc * 8);
     if (e == hipSuccess) e = hipMalloc((void**)&d->d_count, nn * 8);
     if (e == hipSuccess) e = hipMalloc((void**)&d->d_real, nn * 8);
+    if (e == hipSuccess) e = hipMalloc((void**)&d->d_cells, nc * sizeof(DsmcCell));
+    if (e == hipSuccess) e = hipMalloc((void**)&d->d_big, (nc + 1) * sizeof(int));
     if (e == hipSuccess) e = hipMalloc((void**)&d->d_ncol, 8);
     if (e == hipSuccess) e = hipMalloc((void**)&d->d_overflow, 4);
     if (e == hipSuccess) e = hipMemcpy(d->d_scm, scm.data(), nc * 8, hipMemcpyHostToDevice);
@@ -336,6 +462,8 @@ int sf_dsmc_create(sf_ctx* ctx, const sf_dsmc_desc* desc, sf_dsmc** out) {
         hipFree(d->d_rem);
         hipFree(d->d_count);
         hipFree(d->d_real);
+        hipFree(d->d_cells);
+        hipFree(d->d_big);
         hipFree(d->d_ncol);
         hipFree(d->d_overflow);
         delete d;
@@ -354,6 +482,8 @@ int sf_dsmc_destroy(sf_dsmc* d) {
     hipFree(d->d_rem);
     hipFree(d->d_count);
     hipFree(d->d_real);
+    hipFree(d->d_cells);
+    hipFree(d->d_big);
     hipFree(d->d_ncol);
     hipFree(d->d_overflow);
     release_stream(d->ctx, d->desc.seed, d->pp.tag);
@@ -382,14 +512,18 @@ int sf_dsmc_perform(sf_dsmc* d, int it, int64_t* collisions) {
     pp.step = (uint32_t)it;
     SF_HIP(ctx, hipMemsetAsync(d->d_ncol, 0, 8, ctx->stream));
     SF_HIP(ctx, hipMemsetAsync(d->d_overflow, 0, 4, ctx->stream));
+    SF_HIP(ctx, hipMemsetAsync(d->d_big, 0, 4, ctx->stream));
     const int ncells = ctx->mp.nci * ctx->mp.ncj;
-    const int grid = ncells < 65536 ? ncells : 65536;
-    hipLaunchKernelGGL(dsmc_kernel<DSMC_SMALL>, dim3(grid), dim3(64), 0, ctx->stream, ctx->mp, A->buf[A->cur],
-                       (const int32_t*)A->offsets, B->buf[B->cur], (const int32_t*)B->offsets, pp, d->d_scm, d->d_rem,
-                       d->d_count, d->d_real, d->d_ncol, d->d_overflow);
-    hipLaunchKernelGGL(dsmc_kernel<DSMC_MAXP>, dim3(grid), dim3(64), 0, ctx->stream, ctx->mp, A->buf[A->cur],
-                       (const int32_t*)A->offsets, B->buf[B->cur], (const int32_t*)B->offsets, pp, d->d_scm, d->d_rem,
-                       d->d_count, d->d_real, d->d_ncol, d->d_overflow);
+    // the species' key arrays hold nothing between pushes: the passes keep the cells' orders there
+    const PState sa = A->buf[A->cur], sb = B->buf[B->cur];
+    const int32_t *oa = A->offsets, *ob = B->offsets;
+    hipLaunchKernelGGL(dsmc_order, dim3((ncells + 3) / 4), dim3(256), 0, ctx->stream, ctx->mp, sa, oa, sb, ob, pp,
+                       (const double*)d->d_scm, d->d_rem, A->key, B->key, d->d_cells, d->d_big, d->d_overflow);
+    hipLaunchKernelGGL(dsmc_order_big, dim3(std::min(ncells, 1024)), dim3(256), 0, ctx->stream, ctx->mp, sa, oa, sb, ob,
+                       pp.same, A->key, B->key, (const int*)d->d_big);
+    hipLaunchKernelGGL(dsmc_collide, dim3((ncells + 63) / 64), dim3(64), 0, ctx->stream, ctx->mp, sa, oa, sb, ob, pp,
+                       (const int32_t*)A->key, (const int32_t*)B->key, (const DsmcCell*)d->d_cells, d->d_scm,
+                       d->d_count, d->d_real, d->d_ncol);
     SF_HIP(ctx, hipGetLastError());
     unsigned long long n = 0;
     int over = 0;

@@ -146,3 +146,59 @@ def test_dsmc_full_size_conservation():
         if dsmc is not None:
             dsmc.close()
         sim.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("two", [False, True])
+def test_cell_orders_at_their_size_limits(two):
+    """Cells of 1, 2, 63 .. 65, 127 .. 129, 255 .. 257, 511 .. 513, 1024 and 2048 particles, the
+    lengths at which the pass changes how it orders a cell, the same lengths in the last cell column
+    with five more particles on the last node line (not binned), and ids in random order: one pass
+    matches the oracle collision for collision.  Velocities within the FP32 rounding of at most
+    about ten collisions of one particle, 10 x 2^-24 of the largest, with a margin of ten."""
+    from starfish_amd.interactions import DsmcHip
+    from starfish_amd.plugin import Simulation
+    deck = _deck(two, 8e14)
+    m = deck.mesh
+    geo, _ = geometry(deck)
+    o = oracle_for(deck, geo)
+    counts = [1, 2, 63, 64, 65, 127, 128, 129, 255, 256, 257, 511, 512, 513, 1024, 2048]
+    sim = Simulation(deck, capacity=40000, track_ids=True)
+    dsmc = None
+    try:
+        for k, mat in enumerate(sim.materials):
+            rng = np.random.default_rng(3 + k)
+            lc = []
+            for q, n in enumerate(counts):
+                n = counts[-1 - q] if k else n
+                for ci in (3, m.ni - 2):
+                    lc.append(np.stack([ci + 0.999 * rng.random(n), q + 0.999 * rng.random(n)], 1))
+                lc.append(np.stack([np.full(5, m.ni - 1.0), q + 0.999 * rng.random(5)], 1))
+            lc = np.concatenate(lc).astype(np.float32).astype(np.float64)
+            n = len(lc)
+            v = (rng.normal(size=(n, 3)) * 350.0).astype(np.float32).astype(np.float64)
+            x, y = lc[:, 0] * m.dh[0], lc[:, 1] * m.dh[1]
+            ids = rng.permutation(n).astype(np.int32)
+            mat.add_particles(x, y, v[:, 0], v[:, 1], v[:, 2], ids=ids, rewind=False)
+            o.load_particles(k, np.stack([x, y, np.zeros(n)], 1), v, ids=ids, rewind=False)
+        dsmc = DsmcHip(sim, sim.materials[0], sim.materials[-1], sig_cr_max=2e-16, seed=5, tag=1, **N2)
+        ncell = (m.ni - 1) * (m.nj - 1)
+        st = {"sig_cr_max": np.full(ncell, 2e-16), "rem": np.zeros(ncell)}
+        acc = {"count_sum": np.zeros(sim.nn), "real_sum": np.zeros(sim.nn)}
+        pair = {"sigma_type": 1, "diam": N2["diam"], "ref_temp": N2["ref_temp"],
+                "visc_temp_index": N2["visc_temp_index"], "vss_alpha": (1.0, 1.0)}
+        ng = dsmc.perform(1)
+        no = o.dsmc_perform(0, len(sim.materials) - 1, pair, 5, 1, 1, 1, st, acc)
+        assert ng == no and ng > 1000
+        assert np.array_equal(dsmc.field("col-count-sum"), acc["count_sum"])
+        assert np.allclose(dsmc.sig_cr_max(), st["sig_cr_max"], rtol=1e-6)
+        for k, mat in enumerate(sim.materials):
+            gid, gv = _vel_by_id(mat.particles(ids=True))
+            op = o.particles(k)
+            oo = np.argsort(op["id"])
+            assert np.array_equal(gid, op["id"][oo])
+            assert np.abs(gv - op["vel"][oo]).max() / np.abs(op["vel"]).max() < 100 * 2.0 ** -24
+    finally:
+        if dsmc is not None:
+            dsmc.close()
+        sim.close()
