@@ -122,3 +122,48 @@ def test_mcc_full_size_rz_collision_count():
         if mcc is not None:
             mcc.close()
         sim.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,scale", [(1, 20.0), (3, 20.0), (1023, 1.0), (1025, 1e-2), (5003, 1e-3), (600001, 1e-4),
+                                     (6001, 100.0)])
+def test_mcc_queue_edges_match_oracle(n, scale):
+    """Particle counts around the pass's groups of 4, 256 and 1024 slots and its 2048 workgroups, at
+    densities from almost no particle passing the bound to every one: two passes collide exactly
+    the oracle's particles, with holes left by the push in between."""
+    from starfish_amd.interactions import MccHip
+    from starfish_amd.plugin import Simulation
+    deck = _deck("XY")
+    m = deck.mesh
+    geo, _ = geometry(deck)
+    o = oracle_for(deck, geo)
+    rng = np.random.default_rng(n)
+    lc0 = rng.uniform(0, m.ni - 1, n).astype(np.float32).astype(np.float64)
+    lc1 = rng.uniform(0, m.nj - 1, n).astype(np.float32).astype(np.float64)
+    v = (rng.normal(size=(n, 3)) * 800.0 + [300.0, 0, 0]).astype(np.float32).astype(np.float64)
+    x, y = m.x0[0] + lc0 * m.dh[0], m.x0[1] + lc1 * m.dh[1]
+    ids = np.arange(n, dtype=np.int32)
+    o.load_particles(0, np.stack([x, y, np.zeros(n)], 1), v, ids=ids, rewind=False)
+    tgt = _target(m)
+    tgt["den"] = tgt["den"] * scale
+    nn = m.ni * m.nj
+    acc = {"count_sum": np.zeros(nn), "real_sum": np.zeros(nn), "S": np.zeros(nn)}
+    sim = Simulation(deck, capacity=n + 16, track_ids=True)
+    mcc = None
+    try:
+        mat = sim.materials[0]
+        mat.add_particles(x, y, v[:, 0], v[:, 1], v[:, 2], ids=ids, rewind=False)
+        mcc = MccHip(sim, mat, "CEX", 5e-19, 131.0, seed=77, tag=3)
+        mcc.set_target(tgt["den"], tgt["u"], tgt["v"], tgt["w"], tgt["T"])
+        for it in (1, 2):
+            ng = mcc.perform(it, (it - 1) * deck.dt)
+            no = o.mcc_perform(0, tgt, 131.0 * AMU, 5e-19, 0, -1.0, 77, 3, it, 1, acc)
+            assert ng == no
+            assert np.array_equal(mcc.field("col-count-sum"), acc["count_sum"])
+            mat.update()
+            o.move()
+            o.round_state_fp32(0)
+    finally:
+        if mcc is not None:
+            mcc.close()
+        sim.close()
