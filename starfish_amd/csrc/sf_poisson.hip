@@ -39,14 +39,19 @@ constexpr int NK_RING = 8;
 // linear solves converge more slowly, and looser inner solves pay: on the 2048 x 1024 RZ deck warm
 // solves take 18.1, 17.6, 16.2 and 19.0 ms at eta = 2e-2, 5e-2, 1e-1 and 2e-1 (the 1024 x 512
 // deck: 0.63 ms at 5e-2, 0.66 at 1e-1, 0.70 at 2e-1).
-constexpr double ETA_COLD = 1e-3, ETA_WARM = 5e-2, ETA_WARM_LARGE = 1e-1;
+// With the multigrid preconditioner an iteration gains about a digit and a loose inner solve costs
+// little: cold solves of the 1024 x 512 RZ mesh take 9.8, 7.8, 6.7, 7.0 and 6.2 ms at eta = 1e-3, 1e-2,
+// 5e-2, 1e-1 and 2e-1, warm ones of 2048 x 1024 2.2, 2.3 and 2.1 ms at the last three and of 600 x 400
+// 0.94, 0.94 and 1.38 ms.
+constexpr double ETA_COLD = 1e-3, ETA_WARM = 5e-2, ETA_WARM_LARGE = 1e-1, ETA_MG = 1e-1;
+constexpr int MG_MAXLEV = 36;   // a mesh has at most 65536 = 2^16 nodes a side, halved one side at a time at worst
 struct NkState {
     double tol2;   // PCG tolerance (squared) of the current linear solve
     double r2;     // ||r||^2 of the Newton residual at the current linear solve's start (at stop: final)
     int k;         // PCG iteration within the current linear solve
     int newton;    // Newton updates so far
     int pcg;       // PCG iterations so far
-    int done;      // 0 running, 1 converged, 2 Newton iteration cap, 3 residual not finite
+    int done;      // 0 running, else the NK_ stop code
 };
 struct PoissonState {
     sf_poisson_desc desc{};
@@ -76,6 +81,18 @@ struct PoissonState {
     int last_pairs = 24;          // step pairs of the last device-driven solve (sizes its first batch)
     bool host_newton = false;     // SF_HOST_NEWTON: keep every solve on the host-driven loop
     bool warm_hint = false;       // the last solve converged (the next one likely starts warm)
+    // multigrid hierarchy (null without one): per level >= 1 at lev_off, the fields below; level 0
+    // has only the links E0, N0 and the constant part mfix of its diagonal beyond the links
+    int nlev = 0, lev_bottom = 0;         // levels 1 .. nlev - 1; from lev_bottom on in one workgroup
+    int lev_ni[MG_MAXLEV] = {}, lev_nj[MG_MAXLEV] = {};
+    int lev_si[MG_MAXLEV] = {}, lev_sj[MG_MAXLEV] = {};   // a level's node (i, j) is (i >> si, j >> sj) on the next
+    int64_t lev_off[MG_MAXLEV + 1] = {};
+    float *mgE0 = nullptr, *mgN0 = nullptr, *mfix = nullptr, *res2 = nullptr;
+    float *mgE = nullptr, *mgN = nullptr, *mgS = nullptr;   // links and their sum per node
+    float *mgm = nullptr, *mgd = nullptr;                   // diagonal beyond the links, diagonal
+    float *mgr = nullptr, *mge = nullptr;                   // right-hand side, correction
+    int nblk_mg = 0;
+    bool mg_hint = false;         // the last solve needed the multigrid preconditioner
     NkState* nk = nullptr;        // [NK_RING] device-driven Newton-PCG state ring
     double* nkc = nullptr;        // [NK_RING][2] (r.z, r.r) combined by pair i's nk_step_a
     NkState* host_nk = nullptr;   // pinned copy of the last state read
@@ -152,7 +169,8 @@ void poisson_free(PoissonState* p) {
     if (!p) return;
     void* ptrs[] = {p->cls, p->W,  p->bfix, p->src, p->fixval, p->x,  p->r,       p->y,    p->rr,
                     p->D,   p->P,  p->d,    p->res, p->z,      p->p0, p->p1,      p->q,    p->partial,
-                    p->pz,  p->ppq, p->scal, p->istate};
+                    p->pz,  p->ppq, p->scal, p->istate, p->mgE0, p->mgN0, p->mfix, p->res2, p->mgE, p->mgN,
+                    p->mgS, p->mgm, p->mgd, p->mgr, p->mge};
     for (void* q : ptrs)
         if (q) hipFree(q);
     if (p->host_scal) hipHostFree(p->host_scal);
@@ -552,6 +570,344 @@ __global__ void __launch_bounds__(TS::NT) pcg_update(MeshP m, const uint8_t* __r
 }
 
 // ------------------------------------------------------------------------------------------
+// Multigrid preconditioner.  The tile preconditioner does not couple the tiles, so where the
+// Boltzmann term is weak against the Laplacian its iteration count grows with the mesh (554
+// iterations per warm solve of the 2048 x 1024 RZ mesh, 2206 for the cold one of 1024 x 512).  M is
+// here one symmetric V-cycle from a zero guess:
+//   * levels: 2 x 2 aggregates of nodes, or 2 x 1 along the shorter spacing while the spacings differ
+//     by more than sqrt(2) (at a ratio of two, 7 iterations instead of 24).  A level keeps the diagonal
+//     part beyond its links (fixed neighbours and the Boltzmann term) as the sum over the aggregate,
+//     and a link between two aggregates as HALF the sum of the links it replaces along a halved
+//     direction: twice the distance, which is what the five-point operator of the doubled spacing has
+//     (the plain Galerkin sum took 20-25 iterations where this takes 6).  So every level is a
+//     five-point operator, and objects and faces need no interpolation rules: nodes that are not free
+//     have no links.
+//   * smoothing: red then black Gauss-Seidel before, black then red after the coarse correction;
+//     restriction sums, prolongation copies: M is symmetric.
+// After the first red half-sweep from zero a red value is r / d, and after the black one the
+// residual is zero on black nodes and sum c x_black on red ones; the second pass overwrites black
+// values before it reads them.  So neither pass stores its smoothed values: the down kernel leaves
+// only the restricted residual and the up kernel starts again from r / d plus the correction.  A
+// block computes the two rings of halo values it needs itself, which makes each level two kernels
+// without any exchange; the levels of at most MG_BOTTOM nodes in all run in one workgroup in LDS.
+// Measured: warm solves of the 2048 x 1024 RZ mesh 30.4 -> 2.2 ms (554 -> 8 iterations), the cold one of
+// 1024 x 512 57.6 -> 7.6 ms (2206 -> 69).  An iteration at 2048 x 1024 takes about 125 us: 18 + 34 + 23 in
+// the three kernels on the fine level (21 + 36 + 21 B a node), 5 in each of the two kernels of the
+// four middle levels, 14 in the bottom kernel, the rest between launches.
+// ------------------------------------------------------------------------------------------
+constexpr int MG_W = 64, MG_H = 16, MG_NT = 256;      // nodes of a block's tile, threads
+constexpr int MG_LW = MG_W + 4, MG_LH = MG_H + 4;     // with two rings of halo
+constexpr int MG_LN = MG_LW * MG_LH;
+constexpr int MG_BOTTOM = 6144, MG_PAD = 512;         // nodes of the bottom kernel's levels, most per row
+static_assert(MG_W * MG_H == 4 * MG_NT, "one thread per 2 x 2 aggregate");
+// A linear solve that takes more tile-preconditioned iterations than this goes on with the
+// multigrid.  At 1024 x 512 an iteration costs 20 us with the tiles and 70 us with the multigrid, which
+// needs 3 to 6: past 16 the switch pays however long the linear solve would have been.
+// The first linear solve of a cold solve shows it too (56 iterations at 1e-3 on the 1024 x 512 cylinder
+// deck, 184 on the RZ mesh; 13 at 256 x 128, where the tiles stay the better choice: 2.4 ms).
+constexpr int MG_SWITCH = 16;
+constexpr int64_t MG_MIN_NODES = 1024;   // below, a few tiles are the whole mesh
+
+struct MgLevel {
+    int ni, nj;                   // nodes of this level
+    const float *E, *N, *d, *r;   // links to the node right and above, diagonal, right-hand side
+    int si, sj, nI;               // shifts to the next level's nodes, its row length
+};
+struct MgTile {
+    float r[MG_LN], d[MG_LN], E[MG_LN], N[MG_LN], x[MG_LN];
+};
+__device__ __forceinline__ float mg_links(const MgTile& T, int l) {   // sum of link * neighbour value
+    return T.E[l] * T.x[l + 1] + T.E[l - 1] * T.x[l - 1] + T.N[l] * T.x[l + MG_LW] + T.N[l - MG_LW] * T.x[l - MG_LW];
+}
+// black values of the tile and its first ring from the red ones of tile and second ring
+__device__ __forceinline__ void mg_black(MgTile& T) {
+    for (int l = threadIdx.x; l < MG_LN; l += MG_NT) {
+        const int a = l % MG_LW, b = l / MG_LW;
+        if (((a + b) & 1) && a >= 1 && b >= 1 && a < MG_LW - 1 && b < MG_LH - 1) T.x[l] = (T.r[l] + mg_links(T, l)) / T.d[l];
+    }
+    __syncthreads();
+}
+
+// Restricted residual after red-black smoothing from zero.  UPDATE (finest level, a PCG
+// iteration): the step d += alpha p, r_out = r - alpha q is taken here; a block recomputes it on its
+// halo from the old residual, so r_out is another array than r.
+template <bool UPDATE>
+__global__ void __launch_bounds__(MG_NT) mg_down(MgLevel L, float* __restrict__ rc, const float* __restrict__ p,
+                                                 const float* __restrict__ q, float* __restrict__ dsol,
+                                                 float* __restrict__ r_out, const double* __restrict__ ppq, int nbq,
+                                                 const double* __restrict__ pz_cur, int nbz,
+                                                 const int* __restrict__ istate) {
+    if (istate[0]) return;
+    float alpha = 0.0f;
+    if (UPDATE) {
+        double pq[1], cur[2];
+        combine_partials<1>(ppq, nbq, pq);
+        combine_partials<2>(pz_cur, nbz, cur);
+        alpha = (float)(cur[0] / pq[0]);
+    }
+    __shared__ MgTile T;
+    const int ntx = (L.ni + MG_W - 1) / MG_W;
+    const int i0 = (blockIdx.x % ntx) * MG_W, j0 = (blockIdx.x / ntx) * MG_H;
+    for (int l = threadIdx.x; l < MG_LN; l += MG_NT) {
+        const int a = l % MG_LW, b = l / MG_LW;
+        const int i = i0 + a - 2, j = j0 + b - 2;
+        float rv = 0.0f, dv = 1.0f, ev = 0.0f, nv = 0.0f;
+        if (i >= 0 && j >= 0 && i < L.ni && j < L.nj) {
+            const size_t u = (size_t)j * L.ni + i;
+            rv = L.r[u];
+            dv = L.d[u];
+            ev = L.E[u];
+            nv = L.N[u];
+            if (UPDATE) {
+                rv -= alpha * q[u];
+                if (a >= 2 && b >= 2 && a < MG_LW - 2 && b < MG_LH - 2) {
+                    dsol[u] += alpha * p[u];
+                    r_out[u] = rv;
+                }
+            }
+        }
+        T.r[l] = rv;
+        T.d[l] = dv;
+        T.E[l] = ev;
+        T.N[l] = nv;
+        T.x[l] = ((a + b) & 1) ? 0.0f : rv / dv;
+    }
+    __syncthreads();
+    mg_black(T);
+    // Each thread has a 2 x 2 quad of nodes from an even corner: its lower left and upper right node
+    // are red.  They are one aggregate's on a level that halves both directions, two aggregates'
+    // (the only red node of each) on one that halves one.
+    const int qa = threadIdx.x % (MG_W / 2), qb = threadIdx.x / (MG_W / 2);
+    const int i = i0 + 2 * qa, j = j0 + 2 * qb;
+    const int l = (2 * qb + 2) * MG_LW + 2 * qa + 2;
+    float* const c0 = rc + (size_t)(j >> L.sj) * L.nI + (i >> L.si);
+    const bool both = L.si && L.sj;
+    if (i < L.ni && j < L.nj) *c0 = mg_links(T, l) + (both ? mg_links(T, l + MG_LW + 1) : 0.0f);
+    if (!both) {
+        // the other aggregate: right of or above the first; where its red node is outside the mesh
+        // and the aggregate is not, its residual is zero
+        const int I = (i + (L.si ? 0 : 1)) >> L.si, J = (j + (L.sj ? 0 : 1)) >> L.sj;
+        if ((L.si ? i : i + 1) < L.ni && (L.sj ? j : j + 1) < L.nj)
+            rc[(size_t)J * L.nI + I] = i + 1 < L.ni && j + 1 < L.nj ? mg_links(T, l + MG_LW + 1) : 0.0f;
+    }
+}
+
+// z = (red-black smoothed r) + coarse correction ec, smoothed black then red.  FINEST: also the
+// (r.z, r.r) partials of the next PCG iteration.
+template <bool FINEST>
+__global__ void __launch_bounds__(MG_NT) mg_up(MgLevel L, const float* __restrict__ ec, float* __restrict__ z,
+                                               double* __restrict__ pz_next, const int* __restrict__ istate) {
+    if (istate[0]) return;
+    __shared__ MgTile T;
+    const int ntx = (L.ni + MG_W - 1) / MG_W;
+    const int i0 = (blockIdx.x % ntx) * MG_W, j0 = (blockIdx.x / ntx) * MG_H;
+    for (int l = threadIdx.x; l < MG_LN; l += MG_NT) {
+        const int a = l % MG_LW, b = l / MG_LW;
+        const int i = i0 + a - 2, j = j0 + b - 2;
+        float rv = 0.0f, dv = 1.0f, ev = 0.0f, nv = 0.0f, xv = 0.0f;
+        if (i >= 0 && j >= 0 && i < L.ni && j < L.nj) {
+            const size_t u = (size_t)j * L.ni + i;
+            rv = L.r[u];
+            dv = L.d[u];
+            ev = L.E[u];
+            nv = L.N[u];
+            if (!((a + b) & 1)) xv = rv / dv + ec[(size_t)(j >> L.sj) * L.nI + (i >> L.si)];
+        }
+        T.r[l] = rv;
+        T.d[l] = dv;
+        T.E[l] = ev;
+        T.N[l] = nv;
+        T.x[l] = xv;
+    }
+    __syncthreads();
+    mg_black(T);
+    double v[2] = {0.0, 0.0};
+    for (int t = threadIdx.x; t < MG_W * MG_H; t += MG_NT) {
+        const int a = t % MG_W, b = t / MG_W;
+        const int i = i0 + a, j = j0 + b;
+        if (i >= L.ni || j >= L.nj) continue;
+        const int l = (b + 2) * MG_LW + a + 2;
+        // red values are read by nobody here: no update in place
+        const float zv = ((a + b) & 1) ? T.x[l] : (T.r[l] + mg_links(T, l)) / T.d[l];
+        z[(size_t)j * L.ni + i] = zv;
+        if (FINEST) {
+            v[0] += (double)T.r[l] * (double)zv;
+            v[1] += (double)T.r[l] * (double)T.r[l];
+        }
+    }
+    if (FINEST) block_partials<2>(v, pz_next);
+}
+
+// The coarsest levels (offsets off[0 .. n), the first of them off[0] = 0) in one workgroup: the same
+// cycle in LDS down to a single node, whose equation is solved.
+struct MgBottom {
+    int n, total;
+    int ni[MG_MAXLEV], nj[MG_MAXLEV], off[MG_MAXLEV], si[MG_MAXLEV], sj[MG_MAXLEV];
+};
+__global__ void __launch_bounds__(1024) mg_bottom(MgBottom B, const float* __restrict__ E, const float* __restrict__ N,
+                                                  const float* __restrict__ d, const float* __restrict__ r,
+                                                  float* __restrict__ e, const int* __restrict__ istate) {
+    if (istate[0]) return;
+    // (sd: 1/d.  MG_PAD zeros on either side: a node of a first or last row or column reads across its
+    // level's ends, always with a zero link, since a level's last column and row have none)
+    __shared__ float sE_[MG_BOTTOM + 2 * MG_PAD], sN_[MG_BOTTOM + 2 * MG_PAD], sx_[MG_BOTTOM + 2 * MG_PAD];
+    __shared__ float sd[MG_BOTTOM], sr[MG_BOTTOM];
+    float *const sE = sE_ + MG_PAD, *const sN = sN_ + MG_PAD, *const sx = sx_ + MG_PAD;
+    const int t = threadIdx.x;
+    for (int u = t - MG_PAD; u < B.total + MG_PAD; u += 1024) {
+        const bool in = u >= 0 && u < B.total;
+        sE[u] = in ? E[u] : 0.0f;
+        sN[u] = in ? N[u] : 0.0f;
+        sx[u] = 0.0f;
+        if (in) sd[u] = 1.0f / d[u];
+    }
+    for (int u = t; u < B.ni[0] * B.nj[0]; u += 1024) sr[u] = r[u];
+    __syncthreads();
+    auto links = [&](int k, int ni) -> float {   // node k = level offset + j ni + i
+        return sE[k] * sx[k + 1] + sN[k] * sx[k + ni] + sE[k - 1] * sx[k - 1] + sN[k - ni] * sx[k - ni];
+    };
+    // A level's three passes down and up, on nt threads with `sync` between the passes.  Nodes are
+    // numbered with rows of a power of two (2^lg >= ni): a division by ni for each node of each pass
+    // took longer than the rest of it.
+    auto log2up = [](int n) { return n > 1 ? 32 - __clz(n - 1) : 0; };
+    auto down = [&](int q, int nt, auto sync) {
+        const int ni = B.ni[q], nj = B.nj[q], o = B.off[q], lg = log2up(ni), mask = (1 << lg) - 1;
+        for (int u = t; u < nj << lg; u += nt) {
+            const int i = u & mask, j = u >> lg, k = o + j * ni + i;
+            if (i < ni && !((i + j) & 1)) sx[k] = sr[k] * sd[k];
+        }
+        sync();
+        for (int u = t; u < nj << lg; u += nt) {
+            const int i = u & mask, j = u >> lg, k = o + j * ni + i;
+            if (i < ni && ((i + j) & 1)) sx[k] = (sr[k] + links(k, ni)) * sd[k];
+        }
+        sync();
+        const int nI = B.ni[q + 1], nJ = B.nj[q + 1], O = B.off[q + 1], Lg = log2up(nI), Mask = (1 << Lg) - 1;
+        const int si = B.si[q], sj = B.sj[q];
+        for (int u = t; u < nJ << Lg; u += nt) {
+            const int I = u & Mask, J = u >> Lg, i = I << si, j = J << sj;
+            if (I >= nI) continue;
+            float s = 0.0f;   // over the aggregate's red nodes
+            for (int e = 0; e < 4; e++) {
+                const int x = i + (e & 1), y = j + (e >> 1);
+                if ((e & 1) <= si && (e >> 1) <= sj && x < ni && y < nj && !((x + y) & 1)) s += links(o + y * ni + x, ni);
+            }
+            sr[O + J * nI + I] = s;
+        }
+        sync();
+    };
+    auto up = [&](int q, int nt, auto sync) {
+        const int ni = B.ni[q], nj = B.nj[q], o = B.off[q], lg = log2up(ni), mask = (1 << lg) - 1;
+        const int nI = B.ni[q + 1], O = B.off[q + 1];
+        for (int u = t; u < nj << lg; u += nt) {
+            const int i = u & mask, j = u >> lg, k = o + j * ni + i;
+            if (i < ni && !((i + j) & 1)) sx[k] = sr[k] * sd[k] + sx[O + (j >> B.sj[q]) * nI + (i >> B.si[q])];
+        }
+        sync();
+        for (int color = 1; color >= 0; color--) {
+            for (int u = t; u < nj << lg; u += nt) {
+                const int i = u & mask, j = u >> lg, k = o + j * ni + i;
+                if (i < ni && ((i + j) & 1) == color) sx[k] = (sr[k] + links(k, ni)) * sd[k];
+            }
+            sync();
+        }
+    };
+    // levels of at most 64 nodes run on the first wave alone: its LDS operations are in order, so a
+    // compiler fence stands for the workgroup barrier (about 0.1 instead of 0.3 us a pass)
+    int small = 0;
+    while (B.ni[small] * B.nj[small] > 64) small++;
+    auto group = [] { __syncthreads(); };
+    auto wave = [] {
+        __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_wave_barrier();
+    };
+    for (int q = 0; q < small; q++) down(q, 1024, group);
+    if (t < 64) {
+        for (int q = small; q + 1 < B.n; q++) down(q, 64, wave);
+        const int o = B.off[B.n - 1];
+        if (t == 0) sx[o] = sr[o] * sd[o];   // 1 x 1
+        wave();
+        for (int q = B.n - 2; q >= small; q--) up(q, 64, wave);
+    }
+    __syncthreads();
+    for (int q = min(small, B.n - 1) - 1; q >= 0; q--) up(q, 1024, group);
+    for (int u = t; u < B.ni[0] * B.nj[0]; u += 1024) e[u] = sx[u];
+}
+
+// Diagonal of one level that halves one direction only.
+__global__ void __launch_bounds__(256) mg_mass_one(int ni, int nj, int si, int sj, int nI, int nJ, int64_t off,
+                                                   const double* __restrict__ P, const float* __restrict__ mfix,
+                                                   const float* __restrict__ mf, const float* __restrict__ S,
+                                                   float* __restrict__ m, float* __restrict__ d,
+                                                   int* __restrict__ istate) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        istate[0] = 0;
+        istate[1] = 0;
+    }
+    for (int64_t U = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; U < (int64_t)nI * nJ;
+         U += (int64_t)gridDim.x * blockDim.x) {
+        const int i0 = (int)(U % nI) << si, j0 = (int)(U / nI) << sj;
+        float v = 0.0f;
+        for (int j = j0; j < min(j0 + (1 << sj), nj); j++)
+            for (int i = i0; i < min(i0 + (1 << si), ni); i++) {
+                const size_t u = (size_t)j * ni + i;
+                v += P != nullptr ? (float)P[u] + mfix[u] : mf[u];
+            }
+        m[off + U] = v;
+        const float dd = v + S[off + U];
+        d[off + U] = dd > 0.0f ? dd : 1.0f;
+    }
+}
+
+// Diagonals of up to five levels from the finer level's m (l0 = 0: from P and the fixed links): a
+// block of 256 threads sums 32 x 32 nodes pairwise.  Also clears the PCG state word.
+struct MgMass {
+    int ni, nj, n;                       // the finer level's nodes, levels to write (1 .. 5)
+    int cni[5], cnj[5];
+    int64_t off[5];
+};
+__global__ void __launch_bounds__(256) mg_mass(MgMass A, const double* __restrict__ P, const float* __restrict__ mfix,
+                                               const float* __restrict__ mf, const float* __restrict__ S,
+                                               float* __restrict__ m, float* __restrict__ d, int* __restrict__ istate) {
+    __shared__ float sm[16 * 16];
+    const int t = threadIdx.x, a = t & 15, b = t >> 4;
+    if (blockIdx.x == 0 && t == 0) {
+        istate[0] = 0;
+        istate[1] = 0;
+    }
+    const int nbx = (A.ni + 31) / 32;
+    const int bx = blockIdx.x % nbx, by = blockIdx.x / nbx;
+    float v = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const int i = bx * 32 + 2 * a + (k & 1), j = by * 32 + 2 * b + (k >> 1);
+        if (i < A.ni && j < A.nj) {
+            const size_t u = (size_t)j * A.ni + i;
+            v += P != nullptr ? (float)P[u] + mfix[u] : mf[u];
+        }
+    }
+    int w = 16;
+    for (int q = 0; q < A.n; q++) {
+        // v: the value of thread (a, b) < (w, w) on level q
+        const int I = bx * w + a, J = by * w + b;
+        if (a < w && b < w && I < A.cni[q] && J < A.cnj[q]) {
+            const int64_t u = A.off[q] + (int64_t)J * A.cni[q] + I;
+            m[u] = v;
+            const float dd = v + S[u];
+            d[u] = dd > 0.0f ? dd : 1.0f;   // an aggregate without free nodes
+        }
+        if (q + 1 == A.n) break;
+        __syncthreads();
+        if (a < w && b < w) sm[b * 16 + a] = v;
+        __syncthreads();
+        w >>= 1;
+        v = a < w && b < w ? sm[2 * b * 16 + 2 * a] + sm[2 * b * 16 + 2 * a + 1] + sm[(2 * b + 1) * 16 + 2 * a] +
+                                 sm[(2 * b + 1) * 16 + 2 * a + 1]
+                           : 0.0f;
+    }
+}
+
+// ------------------------------------------------------------------------------------------
 // Device-driven Newton-PCG (warm solves).  The host queues pairs of kernels (nk_step_a,
 // nk_step_b) without reading anything back in between; each pair is one PCG iteration or one
 // Newton update, decided by every block from the same partial sums and the state the previous
@@ -573,10 +929,11 @@ struct NkParams {
     double eta2;          // squared forcing term (max(eta, 1e-5))^2
     double lim;           // Newton step limit (kTe)
     int max_it, nl_max;
+    int slow_k;           // a linear solve of that many iterations stops the loop (NK_SLOW)
 };
 
 enum { NK_PCG = 0, NK_UPDATE = 1, NK_STOP = 2 };
-enum { NK_CONVERGED = 1, NK_CAP = 2, NK_NOT_FINITE = 3, NK_COLD = 4 };
+enum { NK_CONVERGED = 1, NK_CAP = 2, NK_NOT_FINITE = 3, NK_COLD = 4, NK_SLOW = 5 };
 // ||r_ref||^2 as the host path uses it (1 when the reference residual vanishes)
 __device__ __forceinline__ double nk_ref2(const NkParams& np) {
     const double r = *np.ref2;
@@ -597,6 +954,7 @@ __device__ __forceinline__ int nk_decide(const NkState& S, const NkParams& np, c
         return NK_PCG;
     }
     if (!(cur[1] > S.tol2) || S.k >= np.max_it) return NK_UPDATE;
+    if (S.k >= np.slow_k) { code = NK_SLOW; return NK_STOP; }   // x holds the updates so far
     return NK_PCG;
 }
 
@@ -975,6 +1333,155 @@ static int reference_row_types(sf_ctx* ctx, std::vector<uint8_t>& rt) {
     return SF_OK;
 }
 
+// Levels of the multigrid: halved node counts down to 1 x 1, level 0 the mesh.  The bottom kernel
+// takes the levels from the first one from which all together fit its LDS.
+static void mg_levels(PoissonState* P, int ni, int nj, double ratio) {   // ratio: dx / dy
+    P->lev_ni[0] = ni;
+    P->lev_nj[0] = nj;
+    P->lev_off[0] = P->lev_off[1] = 0;
+    int n = 1;
+    while (P->lev_ni[n - 1] > 1 || P->lev_nj[n - 1] > 1) {
+        // both directions, or the one of the shorter spacing while it has nodes left to halve
+        const int fi = P->lev_ni[n - 1], fj = P->lev_nj[n - 1];
+        const int si = ratio > std::sqrt(2.0) && fj > 1 ? 0 : 1, sj = ratio < std::sqrt(0.5) && fi > 1 ? 0 : 1;
+        ratio *= (si ? 2.0 : 1.0) / (sj ? 2.0 : 1.0);
+        P->lev_si[n - 1] = si;
+        P->lev_sj[n - 1] = sj;
+        P->lev_ni[n] = si ? (fi + 1) / 2 : fi;
+        P->lev_nj[n] = sj ? (fj + 1) / 2 : fj;
+        P->lev_off[n + 1] = P->lev_off[n] + (int64_t)P->lev_ni[n] * P->lev_nj[n];
+        n++;
+    }
+    P->nlev = n;
+    P->lev_bottom = 1;
+    while (P->lev_off[n] - P->lev_off[P->lev_bottom] > MG_BOTTOM || P->lev_ni[P->lev_bottom] > MG_PAD) P->lev_bottom++;
+}
+
+// The links of every level and the constant part of the finest diagonal beyond its links.
+static int mg_setup(sf_ctx* ctx, PoissonState* P, const std::vector<uint8_t>& cls) {
+    const MeshP& m = ctx->mp;
+    const size_t nn = (size_t)m.ni * m.nj;
+    std::vector<float> E(nn, 0.f), N(nn, 0.f), mfix(nn, 0.f);
+    for (int j = 0; j < m.nj; j++)
+        for (int i = 0; i < m.ni; i++) {
+            const size_t u = (size_t)j * m.ni + i;
+            const uint8_t c = cls[u];
+            if (c == CLS_NOT_FREE) continue;
+            const Stencil st = stencil(m, i, j);
+            const double cc[4] = {st.cE, st.cW, st.cN, st.cS};
+            for (int d = 0; d < 4; d++)
+                if (((c >> (2 * d)) & 3) == NB_FIXED) mfix[u] += (float)cc[d];
+            if ((c & 3) == NB_FREE) E[u] = (float)st.cE;
+            if (((c >> 4) & 3) == NB_FREE) N[u] = (float)st.cN;
+        }
+    SF_HIP(ctx, hipMemcpy(P->mgE0, E.data(), nn * 4, hipMemcpyHostToDevice));
+    SF_HIP(ctx, hipMemcpy(P->mgN0, N.data(), nn * 4, hipMemcpyHostToDevice));
+    SF_HIP(ctx, hipMemcpy(P->mfix, mfix.data(), nn * 4, hipMemcpyHostToDevice));
+    std::vector<float> cE, cN, cS;
+    for (int l = 1; l < P->nlev; l++) {
+        const int ni = P->lev_ni[l - 1], nj = P->lev_nj[l - 1], nI = P->lev_ni[l], nJ = P->lev_nj[l];
+        const int si = P->lev_si[l - 1], sj = P->lev_sj[l - 1];
+        const float fx = si ? 0.5f : 1.0f, fy = sj ? 0.5f : 1.0f;
+        cE.assign((size_t)nI * nJ, 0.f);
+        cN.assign((size_t)nI * nJ, 0.f);
+        cS.assign((size_t)nI * nJ, 0.f);
+        for (int j = 0; j < nj; j++)
+            for (int i = 0; i < ni; i++) {
+                const size_t u = (size_t)j * ni + i, U = (size_t)(j >> sj) * nI + (i >> si);
+                if (!si || (i & 1)) cE[U] += fx * E[u];   // the links that cross into another aggregate
+                if (!sj || (j & 1)) cN[U] += fy * N[u];
+            }
+        for (int J = 0; J < nJ; J++)
+            for (int I = 0; I < nI; I++) {
+                const size_t U = (size_t)J * nI + I;
+                cS[U] = cE[U] + cN[U] + (I > 0 ? cE[U - 1] : 0.f) + (J > 0 ? cN[U - nI] : 0.f);
+            }
+        const size_t bytes = cE.size() * 4;
+        SF_HIP(ctx, hipMemcpy(P->mgE + P->lev_off[l], cE.data(), bytes, hipMemcpyHostToDevice));
+        SF_HIP(ctx, hipMemcpy(P->mgN + P->lev_off[l], cN.data(), bytes, hipMemcpyHostToDevice));
+        SF_HIP(ctx, hipMemcpy(P->mgS + P->lev_off[l], cS.data(), bytes, hipMemcpyHostToDevice));
+        E.swap(cE);
+        N.swap(cN);
+    }
+    return SF_OK;
+}
+
+// Diagonals of the levels for the current P (once per Newton step); clears the PCG state word.
+static void mg_diagonals(PoissonState* P, hipStream_t st) {
+    for (int l0 = 0; l0 + 1 < P->nlev;) {
+        const double* p = l0 == 0 ? (const double*)P->P : nullptr;
+        const float* mf = P->mgm + (l0 ? P->lev_off[l0] : 0);
+        int n = 0;
+        while (n < 5 && l0 + n + 1 < P->nlev && P->lev_si[l0 + n] && P->lev_sj[l0 + n]) n++;
+        if (n == 0) {
+            const int nI = P->lev_ni[l0 + 1], nJ = P->lev_nj[l0 + 1];
+            hipLaunchKernelGGL(mg_mass_one, dim3(grid_elem((int64_t)nI * nJ)), dim3(256), 0, st, P->lev_ni[l0],
+                               P->lev_nj[l0], P->lev_si[l0], P->lev_sj[l0], nI, nJ, P->lev_off[l0 + 1], p,
+                               (const float*)P->mfix, mf, (const float*)P->mgS, P->mgm, P->mgd, P->istate);
+            l0++;
+            continue;
+        }
+        MgMass A{};
+        A.ni = P->lev_ni[l0];
+        A.nj = P->lev_nj[l0];
+        A.n = n;
+        for (int q = 0; q < n; q++) {
+            A.cni[q] = P->lev_ni[l0 + 1 + q];
+            A.cnj[q] = P->lev_nj[l0 + 1 + q];
+            A.off[q] = P->lev_off[l0 + 1 + q];
+        }
+        hipLaunchKernelGGL(mg_mass, dim3(((A.ni + 31) / 32) * ((A.nj + 31) / 32)), dim3(256), 0, st, A, p,
+                           (const float*)P->mfix, mf, (const float*)P->mgS, P->mgm, P->mgd, P->istate);
+        l0 += n;
+    }
+}
+
+// z = M^-1 r and the (r.z, r.r) partials into pz_next.  k < 0: r is P->res; k >= 0: the PCG update of
+// iteration k (direction p) comes first, from the residual buffer k & 1 into the other one.
+static void mg_cycle(PoissonState* P, hipStream_t st, int k, const float* p, const double* pz_cur, int nbz,
+                     double* pz_next) {
+    float* const buf[2] = {P->res, P->res2};
+    auto level = [&](int l, const float* r) {
+        const int si = P->lev_si[l], sj = P->lev_sj[l], nI = P->lev_ni[l + 1];
+        if (l == 0) return MgLevel{P->lev_ni[0], P->lev_nj[0], P->mgE0, P->mgN0, P->D, r, si, sj, nI};
+        const int64_t o = P->lev_off[l];
+        return MgLevel{P->lev_ni[l], P->lev_nj[l], P->mgE + o, P->mgN + o, P->mgd + o, P->mgr + o, si, sj, nI};
+    };
+    auto tiles = [&](int l) { return dim3(((P->lev_ni[l] + MG_W - 1) / MG_W) * ((P->lev_nj[l] + MG_H - 1) / MG_H)); };
+    const int* is = P->istate;
+    if (k >= 0)
+        hipLaunchKernelGGL(mg_down<true>, tiles(0), dim3(MG_NT), 0, st, level(0, buf[k & 1]), P->mgr, p,
+                           (const float*)P->q, P->d, buf[(k + 1) & 1], (const double*)P->ppq, P->nblk_tile, pz_cur, nbz,
+                           is);
+    else
+        hipLaunchKernelGGL(mg_down<false>, tiles(0), dim3(MG_NT), 0, st, level(0, buf[0]), P->mgr,
+                           (const float*)nullptr, (const float*)nullptr, (float*)nullptr, (float*)nullptr,
+                           (const double*)nullptr, 0, (const double*)nullptr, 0, is);
+    const int lb = P->lev_bottom;
+    for (int l = 1; l < lb; l++)
+        hipLaunchKernelGGL(mg_down<false>, tiles(l), dim3(MG_NT), 0, st, level(l, nullptr), P->mgr + P->lev_off[l + 1],
+                           (const float*)nullptr, (const float*)nullptr, (float*)nullptr, (float*)nullptr,
+                           (const double*)nullptr, 0, (const double*)nullptr, 0, is);
+    MgBottom B{};
+    B.n = P->nlev - lb;
+    B.total = (int)(P->lev_off[P->nlev] - P->lev_off[lb]);
+    for (int q = 0; q < B.n; q++) {
+        B.ni[q] = P->lev_ni[lb + q];
+        B.nj[q] = P->lev_nj[lb + q];
+        B.off[q] = (int)(P->lev_off[lb + q] - P->lev_off[lb]);
+        B.si[q] = P->lev_si[lb + q];
+        B.sj[q] = P->lev_sj[lb + q];
+    }
+    const int64_t o = P->lev_off[lb];
+    hipLaunchKernelGGL(mg_bottom, dim3(1), dim3(1024), 0, st, B, (const float*)(P->mgE + o), (const float*)(P->mgN + o),
+                       (const float*)(P->mgd + o), (const float*)(P->mgr + o), P->mge + o, is);
+    for (int l = lb - 1; l >= 1; l--)
+        hipLaunchKernelGGL(mg_up<false>, tiles(l), dim3(MG_NT), 0, st, level(l, nullptr),
+                           (const float*)(P->mge + P->lev_off[l + 1]), P->mge + P->lev_off[l], (double*)nullptr, is);
+    hipLaunchKernelGGL(mg_up<true>, tiles(0), dim3(MG_NT), 0, st, level(0, buf[(k + 1) & 1]), (const float*)P->mge, P->z,
+                       pz_next, is);
+}
+
 int poisson_setup(sf_ctx* ctx, const sf_poisson_desc* dsc) {
     if (!ctx->mesh_ready) return sf_fail(ctx, SF_ERR_STATE, "mesh not set up");
     const MeshP& m = ctx->mp;
@@ -1063,6 +1570,8 @@ int poisson_setup(sf_ctx* ctx, const sf_poisson_desc* dsc) {
         const int nb_tile = P->wide_tiles ? tile_count<TileWide>(ni, nj) : tile_count<TileNarrow>(ni, nj);
         P->nblk_tile = nb_tile;
         P->nblk_elem = grid_elem((int64_t)nn);
+        P->nblk_mg = ((ni + MG_W - 1) / MG_W) * ((nj + MG_H - 1) / MG_H);
+        const int nb_pz = std::max(std::max(P->nblk_elem, nb_tile), P->nblk_mg);
         size_t npart = (size_t)std::max(nb_tile, P->nblk_elem) * 4 + 16;
         e = A((void**)&P->cls, nn);
         if (!e) e = A((void**)&P->W, nn * 8);
@@ -1082,7 +1591,15 @@ int poisson_setup(sf_ctx* ctx, const sf_poisson_desc* dsc) {
         if (!e) e = A((void**)&P->p1, nn * 4);
         if (!e) e = A((void**)&P->q, nn * 4);
         if (!e) e = A((void**)&P->partial, npart * 8);
-        if (!e) e = A((void**)&P->pz, (size_t)4 * std::max(P->nblk_elem, nb_tile) * 8);
+        if (!e) e = A((void**)&P->pz, (size_t)4 * nb_pz * 8);
+        if (!e && (int64_t)nn >= MG_MIN_NODES) {
+            mg_levels(P, ni, nj, m.dh[0] / m.dh[1]);
+            const size_t nc = (size_t)P->lev_off[P->nlev];
+            for (float** f : {&P->mgE0, &P->mgN0, &P->mfix, &P->res2})
+                if (!e) e = A((void**)f, nn * 4);
+            for (float** f : {&P->mgE, &P->mgN, &P->mgS, &P->mgm, &P->mgd, &P->mgr, &P->mge})
+                if (!e) e = A((void**)f, nc * 4);
+        }
         if (!e) e = A((void**)&P->ppq, (size_t)P->nblk_tile * 8);
         if (!e) e = A((void**)&P->scal, S_NSCAL * 8 * 2);
         if (!e) e = A((void**)&P->istate, 16);
@@ -1098,7 +1615,7 @@ int poisson_setup(sf_ctx* ctx, const sf_poisson_desc* dsc) {
         hipMemset(P->nk, 0, NK_RING * sizeof(NkState));
         hipMemset(P->nkc, 0, NK_RING * 2 * sizeof(double));
         P->host_newton = getenv("SF_HOST_NEWTON") != nullptr;
-        hipMemset(P->pz, 0, (size_t)4 * std::max(P->nblk_elem, nb_tile) * 8);
+        hipMemset(P->pz, 0, (size_t)4 * nb_pz * 8);
         hipMemset(P->ppq, 0, (size_t)P->nblk_tile * 8);
         hipMemset(P->y, 0, nn * 8);
         hipMemset(P->x, 0, nn * 8);
@@ -1118,6 +1635,11 @@ int poisson_setup(sf_ctx* ctx, const sf_poisson_desc* dsc) {
     SF_HIP(ctx, hipMemcpy(P->bfix, bfix.data(), nn * 8, hipMemcpyHostToDevice));
     SF_HIP(ctx, hipMemcpy(P->src, src.data(), nn * 4, hipMemcpyHostToDevice));
     SF_HIP(ctx, hipMemcpy(P->fixval, fixval.data(), nn * 8, hipMemcpyHostToDevice));
+    if (P->nlev > 1) {
+        rc = mg_setup(ctx, P, cls);
+        if (rc) return rc;
+    }
+    P->mg_hint = false;
     // phi starts with the Dirichlet values on fixed nodes (Node.bc_value)
     std::vector<double> phi(nn, 0.0);
     for (size_t u = 0; u < nn; u++) phi[u] = src[u] < 0 ? fixval[u] : 0.0;
@@ -1154,7 +1676,7 @@ int poisson_solve(sf_ctx* ctx, sf_solve_info* info) {
     const int max_it = D.max_it > 0 ? D.max_it : 5000;
     const int nl_max = D.linear ? 1 : (D.nl_max_it > 0 ? D.nl_max_it : 50);
     double* pz0 = P->pz;
-    double* pz1 = P->pz + 2 * std::max(ge, gt);   // partials of both parities, by block
+    double* pz1 = P->pz + 2 * std::max(std::max(ge, gt), P->nblk_mg);   // partials of both parities, by block
     double* ypart = P->partial + 2 * std::max(ge, gt);   // Newton step norm partials (not overwritten by residuals)
     // the reference's Newton stop ||y||_2 / N < nl_tol (N = all nodes), used when nl_tol > 0
     const double nl_tol = D.linear ? 0.0 : D.nl_tol;
@@ -1175,7 +1697,8 @@ int poisson_solve(sf_ctx* ctx, sf_solve_info* info) {
     const bool device_ok = !D.linear && !(nl_tol > 0) && !debug && !P->host_newton;
     auto device_newton = [&](double eta_d) -> int {
         const double ee = std::max(eta_d, 1e-5);
-        NkParams np{(const double*)(P->scal + S_R0), rel_tol * rel_tol, ee * ee, lim0, max_it, nl_max};
+        NkParams np{(const double*)(P->scal + S_R0), rel_tol * rel_tol, ee * ee, lim0, max_it, nl_max,
+                    P->nlev > 1 ? MG_SWITCH : max_it + 1};
         auto step_b = [&](int i, int init) {
             with_tile_shape(P->wide_tiles, [&](auto ts) {
                 using TS = decltype(ts);
@@ -1214,6 +1737,11 @@ int poisson_solve(sf_ctx* ctx, sf_solve_info* info) {
         }
         const NkState fin = *P->host_nk;
         if (fin.done == NK_COLD) return NK_COLD;
+        if (fin.done == NK_SLOW) {   // x holds the Newton updates so far; the host loop goes on from it
+            newton = fin.newton;
+            pcg_total = fin.pcg;
+            return NK_SLOW;
+        }
         P->last_pairs = fin.newton + fin.pcg + 1;
         ref = std::sqrt(P->host_scal[S_R0]);
         if (!(ref > 0)) ref = 1.0;
@@ -1231,10 +1759,17 @@ int poisson_solve(sf_ctx* ctx, sf_solve_info* info) {
     // the last solve converged and this one starts from its potential: go straight to the device
     // loop (it hands a cold start back untouched)
     bool device_done = false;
-    if (device_ok && P->warm_hint) {
+    // A solve goes on with the multigrid preconditioner once a linear solve has taken MG_SWITCH
+    // iterations; the next warm solve then starts with it, until it needs no more than one iteration
+    // per Newton step.
+    bool mg = P->mg_hint && P->warm_hint;
+    int mg_its = 0, mg_steps = 0;
+    bool warm = true;
+    if (device_ok && P->warm_hint && !mg) {
         const int code = device_newton(eta_warm);
         if (code < 0) return code;
-        device_done = code != NK_COLD;
+        device_done = code != NK_COLD && code != NK_SLOW;
+        mg = code == NK_SLOW;
     }
     if (!device_done) {
     rc = read_scalars(ctx, P);
@@ -1262,7 +1797,7 @@ int poisson_solve(sf_ctx* ctx, sf_solve_info* info) {
         finalize<1>(P, st, P->partial, ge, S_NORM2);
     };
     bool have_residual = false;   // the residual of the current x is already in host_scal
-    for (int it = 0; it <= nl_max; it++) {
+    for (int it = newton; it <= nl_max; it++) {   // (newton: updates that the device loop made)
         if (!have_residual) {
             launch_residual(nullptr);
             rc = read_scalars(ctx, P);
@@ -1278,11 +1813,19 @@ int poisson_solve(sf_ctx* ctx, sf_solve_info* info) {
         if (!eta_chosen) {
             eta = rel < 0.5 ? eta_warm : ETA_COLD;
             eta_chosen = true;
+            warm = rel < 0.5;
+            if (mg) eta = ETA_MG;
         }
-        if (it == 0 && rel < 0.5 && device_ok) {
+        if (it == 0 && rel < 0.5 && device_ok && !mg) {
             const int code = device_newton(eta);
             if (code < 0) return code;
-            if (code != NK_COLD) break;
+            if (code != NK_COLD && code != NK_SLOW) break;
+            if (code == NK_SLOW) {
+                mg = true;
+                eta = ETA_MG;
+                it = newton - 1;
+                continue;   // the residual of the updated x
+            }
         }
         newton++;
         // inexact Newton: solve J y = r to max(eta*||r||, 0.5*tol*ref) with FP32 PCG + FP64 refinement
@@ -1304,11 +1847,17 @@ int poisson_solve(sf_ctx* ctx, sf_solve_info* info) {
             // inner FP32 tolerance: a relative reduction FP32 can deliver
             double inner_tol = std::max(lin_target, 1e-5 * rr);
             const double tol2 = inner_tol * inner_tol;
-            with_tile_shape(P->wide_tiles, [&](auto ts) {
-                using TS = decltype(ts);
-                hipLaunchKernelGGL(pcg_precond<TS>, dim3(gt), dim3(TS::NT), 0, st, m, (const uint8_t*)P->cls,
-                                   (const float*)P->D, (const float*)P->res, P->z, pz0, P->istate);
-            });
+            if (mg) {
+                mg_diagonals(P, st);
+                mg_cycle(P, st, -1, nullptr, nullptr, 0, pz0);
+                mg_steps++;
+            } else {
+                with_tile_shape(P->wide_tiles, [&](auto ts) {
+                    using TS = decltype(ts);
+                    hipLaunchKernelGGL(pcg_precond<TS>, dim3(gt), dim3(TS::NT), 0, st, m, (const uint8_t*)P->cls,
+                                       (const float*)P->D, (const float*)P->res, P->z, pz0, P->istate);
+                });
+            }
             // When this linear solve is the Newton step's last (it aims at the step's own target),
             // the update and the next Newton residual are queued behind the first batch of PCG
             // iterations.  They run only if that batch converged (the kernels read istate), and
@@ -1319,12 +1868,25 @@ int poisson_solve(sf_ctx* ctx, sf_solve_info* info) {
             // iterations queued between host checks: one more than the last linear solve needed,
             // doubling while unconverged (a converged iteration turns the rest into no-ops)
             int k = 0, its = 0, batch = std::min(8, std::max(3, P->last_its + 1));
+            int before = 0;   // tile-preconditioned iterations before a switch to the multigrid
             bool first_batch = true, done_in_first = false;
             while (true) {
-                const int nb = std::min(batch, max_it - k);
+                const int nb = std::min(batch, max_it - before - k);
                 for (int b = 0; b < nb; b++, k++) {
                     double* cur = (k & 1) ? pz1 : pz0;
                     double* nxt = (k & 1) ? pz0 : pz1;
+                    if (mg) {
+                        with_tile_shape(P->wide_tiles, [&](auto ts) {
+                            using TS = decltype(ts);
+                            hipLaunchKernelGGL(pcg_spmv<TS>, dim3(gt), dim3(TS::NT), 0, st, m, (const uint8_t*)P->cls,
+                                               (const float*)P->D, (const float*)P->z, (const float*)pa, pb, P->q,
+                                               (const double*)cur, (const double*)nxt, P->nblk_mg, k, P->ppq, tol2,
+                                               P->istate);
+                        });
+                        mg_cycle(P, st, k, pb, cur, P->nblk_mg, nxt);
+                        std::swap(pa, pb);
+                        continue;
+                    }
                     with_tile_shape(P->wide_tiles, [&](auto ts) {
                         using TS = decltype(ts);
                         hipLaunchKernelGGL(pcg_spmv<TS>, dim3(gt), dim3(TS::NT), 0, st, m, (const uint8_t*)P->cls,
@@ -1354,12 +1916,26 @@ int poisson_solve(sf_ctx* ctx, sf_solve_info* info) {
                     done_in_first = first_batch;
                     break;
                 }
-                if (k >= max_it) { its = k; break; }
-                batch = std::min(2 * batch, 64);
+                if (before + k >= max_it) { its = k; break; }
+                batch = std::min(2 * batch, mg ? 8 : 64);
                 first_batch = false;
+                if (!mg && P->nlev > 1 && k >= MG_SWITCH) {
+                    // the same linear solve from its current residual and correction, conjugate
+                    // directions started anew
+                    mg = true;
+                    if (!D.linear) eta = ETA_MG;   // of the Newton steps after this one
+                    before = k;
+                    k = 0;
+                    batch = 4;
+                    mg_diagonals(P, st);
+                    mg_cycle(P, st, -1, nullptr, nullptr, 0, pz0);
+                    mg_steps++;
+                }
             }
+            if (mg) mg_its += its;
+            its += before;
             pcg_total += its;
-            P->last_its = its;
+            P->last_its = its - before;
             if (ahead && done_in_first && P->host_istate[0] == 1) {
                 stepped = true;
                 break;
@@ -1398,6 +1974,7 @@ int poisson_solve(sf_ctx* ctx, sf_solve_info* info) {
     }
     }   // !device_done
     P->warm_hint = converged;
+    if (mg && warm) P->mg_hint = mg_its > mg_steps;
     if (!device_done)   // (the device loop expanded phi with its last batch)
         hipLaunchKernelGGL(expand_phi, dim3(ge), dim3(256), 0, st, nn, (const int32_t*)P->src,
                            (const double*)P->fixval, (const double*)P->x, ctx->d_phi);

@@ -2,6 +2,7 @@
 finite-volume matrix (Solver.initCoefficients), E = -grad(phi) against the assembled Gi/Gj,
 and the Newton/PCG potential against a tight solve of the reference's discrete system."""
 import copy
+import math
 
 import numpy as np
 import pytest
@@ -254,5 +255,53 @@ def test_linear_potential_is_the_exact_solution_at_full_size(ni, nj):
               info.rel_residual, "ms %.2f" % info.ms, "err %.2e" % err, flush=True)
         assert rc == 0 and info.rel_residual <= 1e-8
         assert err < 2.4e-5
+    finally:
+        sim.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ni,nj,ratio", [(32, 32, 1.0), (65, 17, 1.0), (64, 18, 1.0), (67, 35, 1.0), (131, 129, 2.0),
+                                         (1025, 5, 1.0), (5, 1025, 1.0), (700, 401, 0.5), (1500, 900, 1.0),
+                                         (33, 257, 0.1), (301, 35, 6.0)])
+def test_multigrid_solves_a_thin_plasma(ni, nj, ratio):
+    """The closed form of the full-size test in a plasma whose Debye length is the whole domain, where
+    the tile preconditioner alone would need hundreds of iterations: a cold solve and one from phi* plus
+    a wide bump, which both hand over to the multigrid, and one that starts with it, at sizes around the 64 x 16-node tiles, with odd aggregates, meshes a few nodes
+    wide, cells of another aspect and levels on both sides of the bottom kernel's.  Bounds: the
+    Jacobian's smallest eigenvalue exceeds pi^2 / (4 Lx^2) and its largest is below 4 / dx^2 + 4 / dy^2,
+    so ||phi - phi*|| <= cond * rel_tol ||phi*||.  That the hierarchy works: a V-cycle gains a factor of 2
+    or more an iteration, so the last solve's linear solves to a tenth take at most 8 (a mesh of a few
+    tiles may stay on them)."""
+    import ctypes as C
+    from starfish_amd.plugin import Simulation, _dp
+    V, dx, kTe = -2.0, 1e-4, 2.0
+    dy = dx * ratio
+    Lx = (ni - 1) * dx
+    n0 = 8.85418782e-12 * kTe / (QE * Lx * Lx)
+    mesh = D.MeshSpec("XY", ni, nj, (0.0, 0.0), (dx, dy), {"LEFT": ("DIRICHLET", 0.0), "RIGHT": ("DIRICHLET", V)})
+    solver = D.SolverSpec("poisson_hip", "GS", False, n0, kTe, 0.0)
+    solver.rel_tol = 1e-10
+    deck = D.Deck(mesh, materials=[D.MaterialSpec("Xe+", "kinetic_hip", 131.0, 1.0, 1e4, 0.0)], solver=solver,
+                  num_it=1, dt=1e-8, seed=1)
+    n = ni * nj
+    X, Y = (np.arange(n) % ni) * dx, (np.arange(n) // ni) * dy
+    exact = V * X / Lx
+    cond = (4 / dx ** 2 + 4 / dy ** 2) / (math.pi ** 2 / (4 * Lx * Lx))
+    sim = Simulation(deck, capacity=16)
+    try:
+        sim.ctx.call("sf_rho_set", _dp(QE * n0 * np.exp(exact / kTe)))
+        info = sim.solver.last
+        bump = 0.05 * np.sin(np.pi * X / Lx) * np.cos(np.pi * Y / ((nj - 1) * dy))
+        for start in (np.zeros(n), exact + bump, exact + 0.5 * bump):
+            sim.ctx.call("sf_phi_set", _dp(start))
+            rc = sim.ctx.call("sf_poisson_solve", None, C.byref(info))
+            err = np.linalg.norm(sim.phi() - exact) / np.linalg.norm(exact)
+            print(ni, nj, "newton", info.newton_iterations, "pcg", info.pcg_iterations, "rel", info.rel_residual,
+                  "err %.2e" % err, flush=True)
+            assert rc == 0 and info.rel_residual <= 1e-10
+            assert err <= cond * 1e-10
+            assert info.newton_iterations < 12
+        if n > 4000:
+            assert info.pcg_iterations <= 8 * info.newton_iterations
     finally:
         sim.close()
