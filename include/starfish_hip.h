@@ -320,17 +320,18 @@ int sf_source_added(sf_ctx* ctx, int source, int64_t* count);
 
 /* ------------------------------------------------------------------------------------------
  * Timing of the last sf_push_deposit (device ms, with sf_set_timing(ctx, 1)): out4[0] the push
- * (push + deposit, in place), out4[1] cell scan (sort step) or macro-particle count (other steps),
- * out4[2] the scatter into cell order (exactly 0 on a step without a sort), out4[3] normalisation.
+ * (push + deposit, in place), out4[1] cell scan (sort step; other steps count macro-particles with
+ * the normalisation), out4[2] the scatter into cell order (exactly 0 on a step without a sort),
+ * out4[3] normalisation, samples and computeFields.
  * ------------------------------------------------------------------------------------------ */
 int sf_last_timings(sf_ctx* ctx, double* out4);
 /* Split of out4[0]: out3[0] the tiled kernel over the cell-sorted particles, out3[1] the kernel
- * over the particles appended since the last sort (injected ones), out3[2] how many slots that
- * second kernel covered. */
+ * over the particles appended since the last sort (injected ones) where it runs by itself (otherwise
+ * the slow-list kernel pushes them beside its own), out3[2] how many slots are appended ones. */
 int sf_last_push_timings(sf_ctx* ctx, double* out3);
-/* The XY tile kernel pushes in FP32 every particle whose cell is away from segments and mesh faces
- * and leaves the others to per-tile slow lists that a second kernel pushes with the full reference
- * loop: out2[0] that kernel's ms (with sf_set_timing), out2[1] how many particles the last push
+/* The tile kernel pushes every particle whose cell is away from segments and mesh faces and that moves
+ * less than two cells, and leaves the others to slow lists that a second kernel pushes with the full
+ * reference loop: out2[0] that kernel's ms (with sf_set_timing), out2[1] how many particles the last push
  * left to it.  The environment variable SF_NO_FAST_PUSH (at context creation) makes every step
  * run the full loop in the general tile kernel. */
 int sf_last_push_queue(sf_ctx* ctx, double* out2);

@@ -137,9 +137,10 @@ static void free_species(Species* sp) {
     dfree(sp->sums);
     dfree(sp->mpc_sum);
     dfree(sp->gas);
-    dfree(sp->flags);
-    dfree(sp->qcount);
-    dfree(sp->tile_nslow);
+    dfree(sp->ctrl);
+    if (sp->result) hipHostFree(sp->result);
+    dfree(sp->parts);
+    dfree(sp->nparts);
     dfree(sp->slow_items);
     dfree(sp->bnd_hits);
     dfree(sp->den);
@@ -147,7 +148,6 @@ static void free_species(Species* sp) {
     dfree(sp->offsets);
     dfree(sp->cursor);
     dfree(sp->blocksum);
-    dfree(sp->stats);
     delete sp;
 }
 
@@ -304,22 +304,26 @@ int sf_mesh_setup(sf_ctx* ctx, const sf_mesh_desc* mesh, const int* face_type, c
     ctx->nseg = nseg;
     ctx->nbnd = 0;
     TRY(dalloc(ctx, &ctx->d_hasseg, nn));
-    // Cells whose particles can take the push's fast path.  The fast path moves a particle by
-    // less than 0.99 cell per axis, so from cell (i, j) (lc in [i, i+1)) the new lc lies in
-    // (i - 0.99, i + 1.99): ProcessBoundary's bounding box (KineticMaterial.java:482-512) spans
-    // nodes [i-1, i+1] x [j-1, j+1], and the particle stays strictly inside the mesh when
-    // 1 <= i <= nci-2 and 1 <= j <= ncj-2 (no face is crossed).  Any other cell, or one whose
-    // box lists a DIRICHLET/SINK segment, is "slow": its particles run the full reference loop.
+    // Cells whose particles can take the push's fast path.  It moves a particle by less than 0.99
+    // cells per axis (k = 1) or 1.99 (k = 2), so from cell (i, j) (lc in [i, i+1)) the new lc lies in
+    // (i - k, i + 1 + k): ProcessBoundary's bounding box (KineticMaterial.java:482-512) spans nodes
+    // [i-k, i+k] x [j-k, j+k], and the particle stays strictly inside the mesh when k <= i <= nci-1-k
+    // and k <= j <= ncj-1-k (no face is crossed).  Any other cell, or one whose box lists a
+    // DIRICHLET/SINK segment, is slow for such moves; a cell that is slow for both runs the full
+    // reference loop.
     const int nci = ni - 1, ncj = nj - 1;
-    std::vector<uint8_t> cslow((size_t)nci * ncj, 1);
-    for (int j = 1; j <= ncj - 2; j++)
-        for (int i = 1; i <= nci - 2; i++) {
-            uint8_t any = 0;
-            for (int b = j - 1; b <= j + 1 && !any; b++)
-                for (int a = i - 1; a <= i + 1; a++)
-                    if (has[(size_t)b * ni + a]) { any = 1; break; }
-            cslow[(size_t)j * nci + i] = any;
-        }
+    std::vector<uint8_t> cslow((size_t)nci * ncj, 2);
+    for (int k = 1; k <= 2; k++)
+        for (int j = k; j <= ncj - 1 - k; j++)
+            for (int i = k; i <= nci - 1 - k; i++) {
+                uint8_t& flag = cslow[(size_t)j * nci + i];
+                if (flag != 3 - k) continue;   // (slow for one cell: slow for two)
+                uint8_t any = 0;
+                for (int b = j - k; b <= j + k && !any; b++)
+                    for (int a = i - k; a <= i + k; a++)
+                        if (has[(size_t)b * ni + a]) { any = 1; break; }
+                if (!any) flag = 2 - k;
+            }
     TRY(dalloc(ctx, &ctx->d_cellslow, cslow.size()));
     SF_HIP(ctx, hipMemcpy(ctx->d_cellslow, cslow.data(), cslow.size(), hipMemcpyHostToDevice));
     TRY(dalloc(ctx, &ctx->d_node_vol, nn));
@@ -387,12 +391,16 @@ int sf_species_create(sf_ctx* ctx, const sf_species_desc* desc, int* species) {
     if (!rc) rc = dalloc(ctx, &sp->sums, NCH * nn);
     if (!rc) rc = dalloc(ctx, &sp->mpc_sum, ncells);
     if (!rc) rc = dalloc(ctx, &sp->gas, NGAS * nn);
-    if (!rc) rc = dalloc(ctx, &sp->flags, 1);
     const size_t ntiles = (size_t)std::max(1, ctx->mp.ntx * ctx->mp.nty);
-    if (!rc) rc = dalloc(ctx, &sp->qcount, 2);
-    if (!rc) rc = dalloc(ctx, &sp->tile_nslow, ntiles);
-    // a tile of n slow particles makes ceil(n / 256) items: at most cap / 256 + tiles in all
-    if (!rc) rc = dalloc(ctx, &sp->slow_items, cap / 256 + ntiles + 1);
+    if (!rc) rc = dalloc(ctx, &sp->ctrl, 1);
+    if (!rc && hipHostMalloc((void**)&sp->result, sizeof(PushResult)) != hipSuccess)
+        rc = sf_fail(ctx, SF_ERR_OOM, "hipHostMalloc of %zu bytes failed", sizeof(PushResult));
+    // a tile of n particles makes ceil(n / part) parts, part >= 1024, and a part of n slow particles
+    // ceil(n / 256) items
+    const size_t nparts = cap / 1024 + ntiles + 1;
+    if (!rc) rc = dalloc(ctx, &sp->parts, nparts);
+    if (!rc) rc = dalloc(ctx, &sp->nparts, 1);
+    if (!rc) rc = dalloc(ctx, &sp->slow_items, cap / 256 + nparts);
     if (!rc && ctx->nbnd > 0) {
         rc = dalloc(ctx, &sp->bnd_hits, (size_t)ctx->nbnd);
         if (!rc) SF_HIP(ctx, hipMemset(sp->bnd_hits, 0, ctx->nbnd * sizeof(unsigned long long)));
@@ -402,7 +410,6 @@ int sf_species_create(sf_ctx* ctx, const sf_species_desc* desc, int* species) {
     if (!rc) rc = dalloc(ctx, &sp->offsets, ncells + 1);
     if (!rc) rc = dalloc(ctx, &sp->cursor, ncells);
     if (!rc) rc = dalloc(ctx, &sp->blocksum, ncells / 4096 + 2);
-    if (!rc) rc = dalloc(ctx, &sp->stats, (size_t)STAT_SLOTS * STAT_STRIDE);
     if (rc) {
         free_species(sp);
         return rc;
@@ -410,7 +417,7 @@ int sf_species_create(sf_ctx* ctx, const sf_species_desc* desc, int* species) {
     hipMemset(sp->acc, 0, NCH * nn * sizeof(unsigned long long));
     hipMemset(sp->sums, 0, NCH * nn * sizeof(double));
     hipMemset(sp->mpc_sum, 0, ncells * sizeof(long long));
-    hipMemset(sp->flags, 0, sizeof(int));
+    hipMemset(sp->ctrl, 0, sizeof(PushCtrl));
     // Material.init: the "t" field starts at init_vals.T, t1-t3 and the averages at zero
     // (Material.java:718-736, KineticMaterial.java:103-110)
     {

@@ -39,7 +39,7 @@ constexpr int TILE_CH = TILE_H + 2 * TILE_HALO;
 constexpr int TILE_CELLS = TILE_CW * TILE_CH;
 constexpr int NCH = 7;                          // deposit channels: n, nu, nv, nw, nuu, nvv, nww
 constexpr int NGAS = 10;                        // computeFields outputs kept on the device
-// bits of Species::flags, set by the push kernels
+// bits of PushCtrl::flags, set by the push kernels
 constexpr int PUSH_FLAG_FAST = 1;               // a velocity beyond the fixed-point fast range: exact slow quantisation
 constexpr int PUSH_FLAG_OVERFLOW = 2;           // a moment contribution beyond the int64 range: moments invalid
 constexpr int PUSH_THREADS = 256;
@@ -109,6 +109,19 @@ struct PushC {
     double vfast, vover;
 };
 
+// Status words of a push on the device, zero between pushes, and their totals in pinned host memory.
+struct PushCtrl {
+    long long stats[STAT_SLOTS * STAT_STRIDE];   // fixed-point mover sums, largest deviation
+    int flags;                                   // PUSH_FLAG_*
+    int qcount[2];                               // particles left to the reference loop, work items
+};
+struct PushResult {
+    long long sums[5];
+    double dmax;
+    int total;                                   // particles kept by a sort step
+    int flags, queued;
+};
+
 struct Species {
     sf_species_desc desc;
     double charge, mass, qm;
@@ -120,20 +133,22 @@ struct Species {
     int cur = 0;
     PState buf[2]{};
     int32_t* key = nullptr;        // new cell key per particle (-1 dead); the push's slow lists
-    int* qcount = nullptr;         // [2] particles the last push left to the reference loop, work items
-    int32_t* tile_nslow = nullptr; // [tiles] length of each push tile's slow list (kept in key)
-    int2* slow_items = nullptr;    // (tile, chunk) work items of the slow lists
+    PushCtrl* ctrl = nullptr;
+    PushResult* result = nullptr;  // pinned
+    bool ctrl_dirty = false;       // a push ended before it cleared ctrl
+    int4* slow_items = nullptr;    // work items of the slow lists (kept in key)
+    int2* parts = nullptr;         // work items of the tile push, made by every sort: (tile, first particle)
+    int* nparts = nullptr;
+    int part = 8192;               // particles per part at the last sort
     unsigned long long* acc = nullptr;   // [NCH][nn] int64 deposit accumulators
     double* sums = nullptr;        // [NCH][nn] running moment sums, physical units (FP64)
     long long* mpc_sum = nullptr;  // [ncells]
     double* gas = nullptr;         // [NGAS][nn] computeFields results (t, t1-t3, nd-ave, u/v/w-ave, p, mpc)
-    int* flags = nullptr;          // device status word of the push (SF_PUSH_FLAG_*)
     double* den = nullptr;         // [4][nn] nd, u, v, w
     int32_t* counts = nullptr;     // [ncells] histogram of new cells
     int32_t* offsets = nullptr;    // [ncells+1] exclusive scan (cell ranges of the sorted array)
     int32_t* cursor = nullptr;     // [ncells]
     int32_t* blocksum = nullptr;   // scan scratch
-    long long* stats = nullptr;    // [STAT_SLOTS][STAT_STRIDE] int64 fixed-point mover sums
     int id_counter = 0;
     int num_samples = 0;
     bool first_time = true;        // KineticMaterial.first_time: computeFields on the first update
@@ -199,7 +214,9 @@ struct sf_ctx {
     int32_t* d_nseg_idx = nullptr;
     sf::DevSeg* d_seg = nullptr;
     uint8_t* d_hasseg = nullptr;
-    uint8_t* d_cellslow = nullptr; // [ncells] 1: a particle of this cell may meet a segment or a mesh face
+    // [ncells] 0: no particle of this cell meets a segment or a mesh face in a move of less than two
+    // cells a direction, 1: in one of less than a cell, 2: neither
+    uint8_t* d_cellslow = nullptr;
     double* d_node_vol = nullptr;
     // fields
     double* d_phi = nullptr;

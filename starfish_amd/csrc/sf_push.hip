@@ -2,12 +2,14 @@
 //
 // One step of KineticMaterial.updateFields() (core/materials/KineticMaterial.java:117-197,
 // 1553-1595) runs as:
-//   push    (push_deposit_tile / push_deposit_tail): gather E, push, boundary processing and
-//           deposit of the 7 moment channels into LDS int64 accumulators of a 32x4-cell tile,
-//           LDS histogram of the new cells; the pushed state is written back to the
-//           particle's own slot (a dead particle becomes a hole, cell = -1).
+//   push    (push_tile_fast, then push_tile_slow for the particles it leaves and for those appended
+//           since the last sort): gather E, push, boundary processing and deposit of the 7 moment
+//           channels into LDS int64 accumulators of a 32x4-cell tile, LDS histogram of the new cells;
+//           the pushed state is written back to the particle's own slot (a dead particle becomes a
+//           hole, cell = -1).  push_deposit_tile_inplace runs the reference loop for every particle
+//           (SF_NO_FAST_PUSH).
 //   scan    (scan_*, sort steps): exclusive scan of the cell histogram -> cell ranges, cursors,
-//           mpc-sum.  On other steps the histogram only feeds mpc-sum (mpc_accumulate).
+//           mpc-sum.  On other steps the histogram only feeds mpc-sum (normalize_nodes).
 //   scatter (copy_scatter, sort steps): each pushed particle to its slot of its new cell
 //           (counting sort + compaction of the holes).
 //   normalise (normalize_nodes): int64 channels -> nd, u, v, w; running sums += channels.
@@ -491,33 +493,43 @@ __device__ __forceinline__ void push_one_global(const MeshP& m, const MeshD& md,
     s.cell[p] = key;
 }
 
+// The particles appended since the last sort, slots [p0, p1).
+template <bool HAS_B>
+__device__ __forceinline__ void push_tail(const MeshP& m, const MeshD& md, const PushC& pc, const PState& s, int64_t p0,
+                                          int64_t p1, int block, int nblocks, unsigned long long* __restrict__ acc,
+                                          int32_t* __restrict__ counts, int* flags, StatAcc& st) {
+    for (int64_t p = p0 + block * (int64_t)blockDim.x + threadIdx.x; p < p1; p += (int64_t)nblocks * blockDim.x) {
+        if (s.cell[p] < 0) continue;   // hole left by a dead particle
+        push_one_global<HAS_B>(m, md, pc, s, p, acc, counts, flags, st);
+    }
+}
 template <bool HAS_B>
 __global__ void __launch_bounds__(256) push_deposit_tail(MeshP m, MeshD md, PushC pc, PState s, int64_t p0,
                                                          int64_t p1, unsigned long long* __restrict__ acc,
                                                          int32_t* __restrict__ counts, long long* stats,
                                                          int* flags) {
     StatAcc st{0, 0, 0, 0, 0, 0.0};
-    for (int64_t p = p0 + blockIdx.x * (int64_t)blockDim.x + threadIdx.x; p < p1;
-         p += (int64_t)gridDim.x * blockDim.x) {
-        if (s.cell[p] < 0) continue;   // hole left by a dead particle
-        push_one_global<HAS_B>(m, md, pc, s, p, acc, counts, flags, st);
-    }
+    push_tail<HAS_B>(m, md, pc, s, p0, p1, blockIdx.x, gridDim.x, acc, counts, flags, st);
     stat_flush(st, stats);
 }
 
 // ----------------------------------------------------------------------------------------
-// fast tile kernel (XY, no magnetic field): the push of every particle whose cell is away from
-// segments and mesh faces, in FP32 relative to its cell; everything else goes to the queue.
+// fast tile kernel: the push of every particle whose cell is away from segments and mesh faces;
+// everything else goes to the queue.
 //
-// A particle of a cell without the slow flag that moves less than one cell in each direction
-// (and is not faster than the fixed-point fast range) is exactly the reference loop's first and
-// only sub-move: ProcessBoundary finds no segment in its bounding box and no face crossing, so
-// the particle lives and its new position is old + v dt.  In cell units that is
-// f' = f + v dt/dh with the new cell i + floor(f'), evaluated in FP32 (the stored precision).
+// A particle that moves less than 0.99 cells in each direction from a cell whose flag is at most 1, or
+// less than 1.99 from one whose flag is 0 (and is not faster than the fixed-point fast range) is
+// exactly the reference loop's first and only sub-move: ProcessBoundary finds no segment in its
+// bounding box and no face crossing, so the particle lives.  In XY without a magnetic field the new
+// position of a move below 0.99 is old + v dt in cell units, f' = f + v dt/dh with the new cell
+// i + floor(f'), evaluated in FP32 (the stored precision).  Longer moves, the RZ and ZR rotation and
+// Boris' rotation are evaluated in FP64, as push_particle does.  (In a stream whose fastest sixth
+// moves more than a cell a step, 2.8e6 of 1.9e7 particles, leaving those to push_tile_slow cost 0.39 ms
+// a step against 0.48 for all the others.)
 // The deposit adds the raw bit patterns fma(w, value, 1.5 2^52) of the fixed-point rounding into
 // LDS; every particle adds exactly one such pattern per channel to each corner of its new cell,
 // so the flush subtracts (particles of the four adjacent cells) x bits(1.5 2^52), counted by the
-// tile's cell histogram.  Integer sums modulo 2^64 keep this exact and order independent.
+// part's cell histogram.  Integer sums modulo 2^64 keep this exact and order independent.
 // ----------------------------------------------------------------------------------------
 struct FastC {
     float qmdt, cdx, cdy;          // q/m dt, dt/dx, dt/dy
@@ -525,12 +537,20 @@ struct FastC {
     double kn, kv, kvv, kst;       // fixed-point scales of the channels and of the mover sums
     double c0, c1, c2;             // reference velocity of the channels
     int ni, nj, nci, ncj, ntx;
+    double qm, qmdt64, dt;         // the FP64 push
+    double x0r, dhr, inv_dhr;      // origin and spacing of the radial direction
+    double inv_dha;                // 1 / spacing of the axial one
 };
 
+template <int DOM, bool HAS_B>
 struct FastLds {
     unsigned long long acc[NCH][TILE_NODES];
     int hist[TILE_CELLS];
     float2 ef[TILE_NODES];
+    float2 bf[HAS_B ? TILE_NODES : 1];
+    // radial weights (Ruyten): r+^2 - r-^2 of the window's radial cells, and its reciprocal
+    double r2[DOM == SF_DOMAIN_RZ ? TILE_CW : (DOM == SF_DOMAIN_ZR ? TILE_CH : 1)];
+    double rinv[DOM == SF_DOMAIN_RZ ? TILE_CW : (DOM == SF_DOMAIN_ZR ? TILE_CH : 1)];
     uint8_t slow[TILE_CELLS];
     int seg_start[TILE_H], seg_pre[TILE_H + 1];
     int nslow;
@@ -541,6 +561,15 @@ constexpr int SLOW_CHUNK = 256;     // slow-list particles per work item of push
 
 __device__ __forceinline__ unsigned long long qbits(double w, double v) {
     return (unsigned long long)__double_as_longlong(fma(w, v, QMAGIC));
+}
+
+// a / b from y, the rounded reciprocal of b: one correction step makes the quotient the correctly
+// rounded one, the value of the division itself (Markstein 1990), for operands away from the
+// exponent range's ends (positions in m).  A weight that rounds otherwise would show at nodes that
+// hold 1e-7 of a particle, where one quantum of the deposit is 1e-5 of the velocity.
+__device__ __forceinline__ double quotient(double a, double b, double y) {
+    const double q = a * y;
+    return fma(fma(-q, b, a), y, q);
 }
 
 // Row segments of a tile's particles: row r of the tile (cells ti0 .. ti0+TILE_W-1 of row
@@ -608,19 +637,56 @@ __device__ __forceinline__ void flush_tile(const unsigned long long (*lacc)[TILE
     }
 }
 
-__global__ void __launch_bounds__(PUSH_THREADS, 4) push_tile_fast_xy(FastC fc, const float2* __restrict__ ef,
-                                                                    const uint8_t* __restrict__ cellslow, PState s,
-                                                                    const int32_t* __restrict__ offsets,
-                                                                    unsigned long long* __restrict__ acc,
-                                                                    int32_t* __restrict__ counts,
-                                                                    long long* __restrict__ stats,
-                                                                    int32_t* __restrict__ slow_list,
-                                                                    int32_t* __restrict__ tile_nslow,
-                                                                    int2* __restrict__ slow_items,
-                                                                    int* __restrict__ qcount) {
-    __shared__ FastLds L;
+// Work of a workgroup: particles [k0, k0 + part) of tile `tile` (numbered across its row segments).
+// A tile of more than `part` particles is several parts, so a dense tile (a beam, a sheath, bunched
+// particles) does not keep one workgroup busy while the rest of the chip has run dry.
+__global__ void __launch_bounds__(256) tile_parts_kernel(int nci, int ncj, int ntx, int ntiles, int part,
+                                                         const int32_t* __restrict__ offsets,
+                                                         int2* __restrict__ parts, int* __restrict__ nparts) {
+    const int tile = blockIdx.x * 256 + threadIdx.x, lane = threadIdx.x & 63;
+    int n = 0;
+    if (tile < ntiles) {
+        const int ti0 = (tile % ntx) * TILE_W, tj0 = (tile / ntx) * TILE_H;
+        for (int r = 0; r < TILE_H && tj0 + r < ncj; r++)
+            n += offsets[(tj0 + r) * nci + min(ti0 + TILE_W, nci)] - offsets[(tj0 + r) * nci + ti0];
+    }
+    const int np = (n + part - 1) / part;
+    int pre = np;   // inclusive sum over the wave, one atomic for its parts
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(pre, o);
+        if (lane >= o) pre += y;
+    }
+    int base = 0;
+    if (lane == 63) base = atomicAdd(nparts, pre);
+    base = __shfl(base, 63) + pre - np;
+    for (int k = 0; k < np; k++) parts[base + k] = make_int2(tile, k * part);
+}
+
+// Bound by FP64 issue (half rate: about 65 FP64 operations a particle in XY, 200 in RZ), LDS atomics and
+// HBM at once, with four waves a SIMD to overlap them.  Measured a step: XY 2e7 particles (1024 x 512)
+// 0.43 ms uniform; bunched (one tile in ten has twice the mean, the fullest five times) 0.48 ms with
+// parts against 0.71 with one workgroup a tile.  RZ 1e8 (2048 x 1024) 2.4 ms against 4.2 for the general
+// tile kernel, which takes every particle through LDS for its stores and through the loop's
+// registers; ZR with B 1e6 (301 x 157) 50 against 74 us.
+template <int DOM, bool HAS_B>
+__global__ void __launch_bounds__(PUSH_THREADS, 4) push_tile_fast(FastC fc, const float2* __restrict__ ef,
+                                                                 const float2* __restrict__ bf,
+                                                                 const uint8_t* __restrict__ cellslow, PState s,
+                                                                 const int32_t* __restrict__ offsets,
+                                                                 const int2* __restrict__ parts,
+                                                                 const int* __restrict__ nparts, int part,
+                                                                 unsigned long long* __restrict__ acc,
+                                                                 int32_t* __restrict__ counts,
+                                                                 long long* __restrict__ stats,
+                                                                 int32_t* __restrict__ slow_list,
+                                                                 int4* __restrict__ slow_items,
+                                                                 int* __restrict__ qcount) {
+    constexpr bool F32 = DOM == SF_DOMAIN_XY && !HAS_B;   // the FP32 push
+    if ((int)blockIdx.x >= *nparts) return;
+    __shared__ FastLds<DOM, HAS_B> L;
     const int t = threadIdx.x;
-    const int tile = blockIdx.x;
+    const int2 work = parts[blockIdx.x];
+    const int tile = work.x;
     const int tx = tile % fc.ntx, ty = tile / fc.ntx;
     const int ti0 = tx * TILE_W, tj0 = ty * TILE_H;
     // the LDS window: nodes and cells from (ti0 - HALO, tj0 - HALO); node (a, b) of the window is
@@ -635,21 +701,31 @@ __global__ void __launch_bounds__(PUSH_THREADS, 4) push_tile_fast_xy(FastC fc, c
     for (int k = t; k < TILE_CELLS; k += PUSH_THREADS) {
         L.hist[k] = 0;
         const int i = w_i0 + k % TILE_CW, j = w_j0 + k / TILE_CW;
-        L.slow[k] = (i >= 0 && j >= 0 && i < fc.nci && j < fc.ncj) ? cellslow[(size_t)j * fc.nci + i] : 1;
+        L.slow[k] = (i >= 0 && j >= 0 && i < fc.nci && j < fc.ncj) ? cellslow[(size_t)j * fc.nci + i] : 2;
     }
     for (int k = t; k < TILE_NODES; k += PUSH_THREADS) {
         int i = w_i0 + k % TILE_NW, j = w_j0 + k / TILE_NW;
         i = min(max(i, 0), fc.ni - 1);
         j = min(max(j, 0), fc.nj - 1);
         L.ef[k] = ef[(size_t)j * fc.ni + i];
+        if (HAS_B) L.bf[k] = bf[(size_t)j * fc.ni + i];
+    }
+    if (DOM != SF_DOMAIN_XY) {
+        constexpr int n = DOM == SF_DOMAIN_RZ ? TILE_CW : TILE_CH;
+        if (t < n) {
+            const int i = (DOM == SF_DOMAIN_RZ ? w_i0 : w_j0) + t;
+            const double rp = fc.x0r + (i + 1) * fc.dhr, rm = fc.x0r + i * fc.dhr;
+            L.r2[t] = rp * rp - rm * rm;
+            L.rinv[t] = 1.0 / L.r2[t];
+        }
     }
     if (t == 0) tile_segments(offsets, fc.nci, fc.ncj, ti0, tj0, L.seg_start, L.seg_pre);
     __syncthreads();
-    // The tile's particles, numbered 0 .. total-1 across its row segments, are taken in windows of
-    // PUSH_THREADS; within a window thread t takes particle pt.  The waves run through the windows
-    // independently (no barrier): each loads its next window's particles before pushing the
-    // current ones and stores each pushed particle straight back to its slot.
-    const int total = L.seg_pre[TILE_H];
+    // The part's particles are taken in windows of PUSH_THREADS; within a window thread t takes
+    // particle pt.  The waves run through the windows independently (no barrier): each loads its
+    // next window's particles before pushing the current ones and stores each pushed particle
+    // straight back to its slot.
+    const int total = min(L.seg_pre[TILE_H], work.y + part);
     const int sg0 = L.seg_start[0], sg1 = L.seg_start[1], sg2 = L.seg_start[2], sg3 = L.seg_start[3];
     const int pr1 = L.seg_pre[1], pr2 = L.seg_pre[2], pr3 = L.seg_pre[3];
     // The slot and the loaded state are computed as values and assigned whole: selects or
@@ -681,8 +757,8 @@ __global__ void __launch_bounds__(PUSH_THREADS, 4) push_tile_fast_xy(FastC fc, c
     unsigned long long sp0 = 0, sp1 = 0, sp2 = 0, se = 0;
     double dmax = 0.0;
     PReg nxt;
-    load(nxt, pt);
-    for (int w0 = 0; w0 < total; w0 += PUSH_THREADS) {
+    load(nxt, work.y + pt);
+    for (int w0 = work.y; w0 < total; w0 += PUSH_THREADS) {
         const PReg cur = nxt;
         const bool ok = w0 + pt < total;
         load(nxt, w0 + PUSH_THREADS + pt);
@@ -693,68 +769,146 @@ __global__ void __launch_bounds__(PUSH_THREADS, 4) push_tile_fast_xy(FastC fc, c
             const int ci = cur.c & 0xFFFF, cj = (cur.c >> 16) & 0xFFFF;
             const int hi = ci - w_i0, hj = cj - w_j0;
             bool fast = (unsigned)hi < (unsigned)TILE_CW && (unsigned)hj < (unsigned)TILE_CH;
-            if (fast) fast = L.slow[hj * TILE_CW + hi] == 0;
+            int flag = 2;
+            if (fast) flag = L.slow[hj * TILE_CW + hi];
+            fast = flag < 2;
             if (fast) {
                 // Field2D.gather: bilinear in the cell (the slow flag keeps the cell off the last node line)
                 const int l = hj * TILE_NW + hi;
                 const float2 e00 = L.ef[l], e10 = L.ef[l + 1], e01 = L.ef[l + TILE_NW], e11 = L.ef[l + TILE_NW + 1];
-                const float gx = 1.0f - cur.fx, gy = 1.0f - cur.fy;
-                const float ex = gy * (gx * e00.x + cur.fx * e10.x) + cur.fy * (gx * e01.x + cur.fx * e11.x);
-                const float ey = gy * (gx * e00.y + cur.fx * e10.y) + cur.fy * (gx * e01.y + cur.fx * e11.y);
-                vxn = cur.vx + fc.qmdt * ex;
-                vyn = cur.vy + fc.qmdt * ey;
-                vzn = cur.vz;
-                const float dx = vxn * fc.cdx, dy = vyn * fc.cdy;
-                const double d0 = (double)vxn - fc.c0, d1 = (double)vyn - fc.c1, d2 = (double)vzn - fc.c2;
-                const double dev = fmax(fabs(d0), fmax(fabs(d1), fabs(d2)));
-                // |d| < 0.99 keeps f + d strictly inside (-1, 2) after FP32 rounding
-                fast = fabsf(dx) < 0.99f && fabsf(dy) < 0.99f && dev < fc.vfast;
-                if (fast) {
-                    const float xn = cur.fx + dx, yn = cur.fy + dy;
+                int nci = ci, ncj = cj;
+                bool longer = !F32;
+                if (F32) {
+                    const float gx = 1.0f - cur.fx, gy = 1.0f - cur.fy;
+                    const float ex = gy * (gx * e00.x + cur.fx * e10.x) + cur.fy * (gx * e01.x + cur.fx * e11.x);
+                    const float ey = gy * (gx * e00.y + cur.fx * e10.y) + cur.fy * (gx * e01.y + cur.fx * e11.y);
+                    vxn = cur.vx + fc.qmdt * ex;
+                    vyn = cur.vy + fc.qmdt * ey;
+                    vzn = cur.vz;
+                    const float dx = vxn * fc.cdx, dy = vyn * fc.cdy;
+                    // |d| < 0.99 keeps f + d strictly inside (-1, 2) after FP32 rounding
+                    longer = !(fabsf(dx) < 0.99f && fabsf(dy) < 0.99f);
+                    float xn, yn;
+                    {
+#pragma clang fp contract(off)
+                        xn = cur.fx + dx;   // the rounded move, as tested above
+                        yn = cur.fy + dy;
+                    }
                     const float flx = floorf(xn), fly = floorf(yn);
                     fxn = xn - flx;
                     fyn = yn - fly;
-                    int nci = ci + (int)flx, ncj = cj + (int)fly;
-                    // x' - floor(x') can round up to 1 for x' just below an integer: that position
-                    // is offset 0 of the next cell (the stored cell is floor(lc))
-                    if (fxn >= 1.0f) { fxn = 0.0f; nci++; }
-                    if (fyn >= 1.0f) { fyn = 0.0f; ncj++; }
+                    nci += (int)flx;
+                    ncj += (int)fly;
+                }
+                if (longer) {
+                    // push_particle's single sub-move in its order of operations; a cell without the
+                    // slow flag is off the axis, so R > 0
+                    const double di = cur.fx, dj = cur.fy;
+                    const double w00 = (1 - di) * (1 - dj), w10 = di * (1 - dj), w11 = di * dj, w01 = (1 - di) * dj;
+                    const double ex = w00 * e00.x + w10 * e10.x + w11 * e11.x + w01 * e01.x;
+                    const double ey = w00 * e00.y + w10 * e10.y + w11 * e11.y + w01 * e01.y;
+                    double v0 = cur.vx, v1 = cur.vy, v2 = cur.vz;
+                    bool electric = true;
+                    if (HAS_B) {
+                        const float2 b00 = L.bf[l], b10 = L.bf[l + 1], b01 = L.bf[l + TILE_NW], b11 = L.bf[l + TILE_NW + 1];
+                        const double bx = w00 * b00.x + w10 * b10.x + w11 * b11.x + w01 * b01.x;
+                        const double by = w00 * b00.y + w10 * b10.y + w11 * b11.y + w01 * b01.y;
+                        if (bx != 0 || by != 0) {
+                            boris_velocity(fc.qm, fc.dt, ex, ey, bx, by, v0, v1, v2);
+                            electric = false;
+                        }
+                    }
+                    if (electric) {
+                        v0 += fc.qmdt64 * ex;
+                        v1 += fc.qmdt64 * ey;
+                    }
+                    const double l0 = ci + di, l1 = cj + dj;
+                    double n0, n1;
+                    if (DOM == SF_DOMAIN_XY) {
+                        n0 = l0 + v0 * fc.dt * fc.inv_dhr;
+                        n1 = l1 + v1 * fc.dt * fc.inv_dha;
+                    } else {   // the rotation of the radial and azimuthal velocity (rotateToRZ, rotateToZR)
+                        const double vr = DOM == SF_DOMAIN_RZ ? v0 : v1, va = DOM == SF_DOMAIN_RZ ? v1 : v0;
+                        const double xr = fc.x0r + (DOM == SF_DOMAIN_RZ ? l0 : l1) * fc.dhr + vr * fc.dt;
+                        const double na = (DOM == SF_DOMAIN_RZ ? l1 : l0) + va * fc.dt * fc.inv_dha;
+                        const double A = v2 * fc.dt;
+                        const double R = sqrt(A * A + xr * xr);
+                        const double ir = 1.0 / R, c = quotient(xr, R, ir), sn_ = quotient(A, R, ir);
+                        const double nvr = c * vr + sn_ * v2;
+                        v2 = -sn_ * vr + c * v2;
+                        const double nr = (R - fc.x0r) * fc.inv_dhr;
+                        n0 = DOM == SF_DOMAIN_RZ ? nr : na;
+                        n1 = DOM == SF_DOMAIN_RZ ? na : nr;
+                        if (DOM == SF_DOMAIN_RZ) v0 = nvr;
+                        else v1 = nvr;
+                    }
+                    const double most = flag ? 0.99 : 1.99;
+                    fast = fabs(n0 - l0) < most && fabs(n1 - l1) < most;
+                    nci = (int)n0;
+                    ncj = (int)n1;
+                    {
+#pragma clang fp contract(off)
+                        fxn = (float)(n0 - nci);   // of the rounded coordinates, as cell_offsets
+                        fyn = (float)(n1 - ncj);
+                    }
+                    vxn = (float)v0;
+                    vyn = (float)v1;
+                    vzn = (float)v2;
+                }
+                // x' - floor(x') can round up to 1 for x' just below an integer: that position is
+                // offset 0 of the next cell (the stored cell is floor(lc))
+                if (fxn >= 1.0f) { fxn = 0.0f; nci++; }
+                if (fyn >= 1.0f) { fyn = 0.0f; ncj++; }
+                const double d0 = (double)vxn - fc.c0, d1 = (double)vyn - fc.c1, d2 = (double)vzn - fc.c2;
+                const double dev = fmax(fabs(d0), fmax(fabs(d1), fabs(d2)));
+                fast = fast && dev < fc.vfast;
+                if (fast) {
                     key = pack_cell(nci, ncj);
                     // mover sums (KineticMaterial.java:247-259, 406-413)
                     sn++;
                     sp0 += qbits(1.0, (double)vxn * fc.kst);
                     sp1 += qbits(1.0, (double)vyn * fc.kst);
                     sp2 += qbits(1.0, (double)vzn * fc.kst);
-                    se += qbits(1.0, (double)sqrtf(vxn * vxn + vyn * vyn + vzn * vzn) * fc.kst);
+                    if (F32) {
+                        se += qbits(1.0, (double)sqrtf(vxn * vxn + vyn * vyn + vzn * vzn) * fc.kst);
+                    } else {
+                        const double a0 = vxn, a1 = vyn, a2 = vzn;
+                        se += qbits(1.0, sqrt(a0 * a0 + a1 * a1 + a2 * a2) * fc.kst);
+                    }
                     dmax = fmax(dmax, dev);
-                    // deposit of the 7 channels from the stored FP32 state (Field2D.scatter)
-                    const double dfx = fxn, dfy = fyn;
-                    const double w00 = (1.0 - dfx) * (1.0 - dfy), w10 = dfx * (1.0 - dfy), w11 = dfx * dfy,
-                                 w01 = (1.0 - dfx) * dfy;
+                    // deposit of the 7 channels from the stored FP32 state (Field2D.scatter), with
+                    // Ruyten's radial weight in RZ and ZR
+                    double dfx = fxn, dfy = fyn;
+                    const int hn = nci - w_i0, hm = ncj - w_j0;
+                    const bool inside = (unsigned)hn < (unsigned)TILE_CW && (unsigned)hm < (unsigned)TILE_CH;
+                    if (DOM != SF_DOMAIN_XY) {
+                        const int i = DOM == SF_DOMAIN_RZ ? nci : ncj, h = DOM == SF_DOMAIN_RZ ? hn : hm;
+                        double& df = DOM == SF_DOMAIN_RZ ? dfx : dfy;
+                        const double rp = fc.x0r + (i + 1) * fc.dhr, rm = fc.x0r + i * fc.dhr,
+                                     r = fc.x0r + (i + df) * fc.dhr;
+                        const double num = 0.5 * (rp - r) * (2 * rp + 3 * rm - r);
+                        df = 1 - (inside ? quotient(num, L.r2[h], L.rinv[h]) : num / (rp * rp - rm * rm));
+                    }
                     const double val[NCH] = {fc.kn, d0 * fc.kv, d1 * fc.kv, d2 * fc.kv, d0 * d0 * fc.kvv,
                                              d1 * d1 * fc.kvv, d2 * d2 * fc.kvv};
-                    const int hn = nci - w_i0, hm = ncj - w_j0;
-                    if ((unsigned)hn < (unsigned)TILE_CW && (unsigned)hm < (unsigned)TILE_CH) {
+                    const double gfx = 1.0 - dfx, gfy = 1.0 - dfy;
+                    if (inside) {
                         atomicAdd(&L.hist[hm * TILE_CW + hn], 1);
-                        const int l0 = hm * TILE_NW + hn;
                         // lanes of one cell start at different corners (lane mod 4), so the
                         // same-address conflicts of an instruction drop about fourfold
-                        const int rot = t & 3;
-                        double wr[4];
-                        int offr[4];
-#pragma unroll
-                        for (int q = 0; q < 4; q++) {
-                            const int cq = (q + rot) & 3;
-                            wr[q] = cq == 0 ? w00 : (cq == 1 ? w10 : (cq == 2 ? w11 : w01));
-                            offr[q] = cq == 0 ? 0 : (cq == 1 ? 1 : (cq == 2 ? TILE_NW + 1 : TILE_NW));
-                        }
+                        const bool rx = t & 1, ry = t & 2;
+                        const double wx0 = rx ? dfx : gfx, wx1 = rx ? gfx : dfx, wy0 = ry ? dfy : gfy, wy1 = ry ? gfy : dfy;
+                        const int ox = rx ? -1 : 1, oy = ry ? -TILE_NW : TILE_NW;
+                        const int l0 = hm * TILE_NW + hn + (rx ? 1 : 0) + (ry ? TILE_NW : 0);
+                        const double wr[4] = {wx0 * wy0, wx1 * wy0, wx1 * wy1, wx0 * wy1};
+                        const int offr[4] = {0, ox, ox + oy, oy};
 #pragma unroll
                         for (int q = 0; q < 4; q++)
 #pragma unroll
                             for (int ch = 0; ch < NCH; ch++) atomicAdd(&L.acc[ch][l0 + offr[q]], qbits(wr[q], val[ch]));
                     } else {
                         atomicAdd(&counts[ncj * fc.nci + nci], 1);
-                        const double w4[4] = {w00, w10, w11, w01};
+                        const double w4[4] = {gfx * gfy, dfx * gfy, dfx * dfy, gfx * dfy};
                         const int ci4[4] = {0, 1, 1, 0}, cj4[4] = {0, 0, 1, 1};
 #pragma unroll
                         for (int c = 0; c < 4; c++) {
@@ -770,7 +924,7 @@ __global__ void __launch_bounds__(PUSH_THREADS, 4) push_tile_fast_xy(FastC fc, c
             }
             slow = !fast;
         }
-        // slow particles: the slot goes to the tile's slow list (stored in the tile's own slots
+        // slow particles: the slot goes to the part's slow list (stored in the part's own slots
         // of slow_list); push_tile_slow pushes and writes it
         {
             const unsigned long long mk = __ballot(slow);
@@ -781,7 +935,7 @@ __global__ void __launch_bounds__(PUSH_THREADS, 4) push_tile_fast_xy(FastC fc, c
                 if (lane == leader) base = atomicAdd(&L.nslow, __popcll(mk));
                 base = __shfl(base, leader);
                 if (slow)
-                    slow_list[tile_slot(L.seg_start, L.seg_pre, base + __popcll(mk & ((1ull << lane) - 1ull)))] =
+                    slow_list[tile_slot(L.seg_start, L.seg_pre, work.y + base + __popcll(mk & ((1ull << lane) - 1ull)))] =
                         (int32_t)cur.g;
             }
         }
@@ -798,12 +952,12 @@ __global__ void __launch_bounds__(PUSH_THREADS, 4) push_tile_fast_xy(FastC fc, c
     if (t == 0) {
         // the slow list goes to push_tile_slow as work items of SLOW_CHUNK particles
         const int n = L.nslow;
-        tile_nslow[tile] = n;
         if (n) {
             atomicAdd(&qcount[0], n);
             const int nch = (n + SLOW_CHUNK - 1) / SLOW_CHUNK;
             const int base = atomicAdd(&qcount[1], nch);
-            for (int c = 0; c < nch; c++) slow_items[base + c] = make_int2(tile, c);
+            for (int c = 0; c < nch; c++)
+                slow_items[base + c] = make_int4(tile, work.y + c * SLOW_CHUNK, min(SLOW_CHUNK, n - c * SLOW_CHUNK), 0);
         }
     }
     flush_tile(L.acc, L.hist, w_i0, w_j0, fc.ni, fc.nj, fc.nci, acc, counts, PUSH_THREADS);
@@ -812,37 +966,47 @@ __global__ void __launch_bounds__(PUSH_THREADS, 4) push_tile_fast_xy(FastC fc, c
     stat_flush(st, stats);
 }
 
-// The particles push_tile_fast_xy left to the reference loop (cells next to segments or mesh
+// The particles push_tile_fast left to the reference loop (cells next to segments or mesh
 // faces, moves of 0.99 cell or more, deviations beyond the fast quantisation range): the full
 // FP64 push with ProcessBoundary and the deposit into the tile's LDS window (raw patterns and
 // histogram as in the fast kernel), into global memory for particles that land outside it, or
-// with the exact quantisation past the fast range.  The work is a list of (tile, chunk) items of
-// SLOW_CHUNK particles each, taken by the workgroups in turn, so a tile with a long slow list
-// (a row of cells along a mesh face, or the cells around an object) is spread over many of them.
+// with the exact quantisation past the fast range.  The work is a list of items (tile, index of the
+// first list entry in the tile, length) of at most SLOW_CHUNK particles each, taken by the workgroups
+// in turn, so a tile with a long slow list (a row of cells along a mesh face, or the cells around an
+// object) is spread over many of them.  The last `ntail` workgroups push the particles appended since
+// the last sort instead: both are chains of dependent loads on few waves (about 20 us each for a few
+// hundred particles), so they run side by side.
 struct SlowLds {
     unsigned long long acc[NCH][TILE_NODES];
     int hist[TILE_CELLS];
     int seg_start[TILE_H], seg_pre[TILE_H + 1];
 };
 
+template <bool HAS_B>
 __global__ void __launch_bounds__(SLOW_CHUNK) push_tile_slow(MeshP m, MeshD md, PushC pc, PState s,
                                                              const int32_t* __restrict__ offsets,
                                                              const int32_t* __restrict__ slow_list,
-                                                             const int32_t* __restrict__ tile_nslow,
-                                                             const int2* __restrict__ slow_items,
+                                                             const int4* __restrict__ slow_items,
                                                              const int* __restrict__ qcount,
                                                              unsigned long long* __restrict__ acc,
                                                              int32_t* __restrict__ counts, long long* stats,
-                                                             int* flags) {
+                                                             int* flags, int ntail, int64_t p0, int64_t p1) {
     __shared__ SlowLds L;
     const int t = threadIdx.x;
+    const int nslow_blocks = (int)gridDim.x - ntail;
+    if ((int)blockIdx.x >= nslow_blocks) {
+        StatAcc st{0, 0, 0, 0, 0, 0.0};
+        push_tail<HAS_B>(m, md, pc, s, p0, p1, blockIdx.x - nslow_blocks, ntail, acc, counts, flags, st);
+        stat_flush(st, stats);
+        return;
+    }
     const int nitems = qcount[1];
     const size_t nn = (size_t)m.ni * m.nj;
     auto load_e = [&](int i, int j) -> float2 { return md.ef[(size_t)j * m.ni + i]; };
     auto hasseg = [&](int i, int j) -> int { return md.node_hasseg[(size_t)j * m.ni + i]; };
     StatAcc st{0, 0, 0, 0, 0, 0.0};
-    for (int it = blockIdx.x; it < nitems; it += gridDim.x) {
-        const int2 item = slow_items[it];
+    for (int it = blockIdx.x; it < nitems; it += nslow_blocks) {
+        const int4 item = slow_items[it];
         const int tile = item.x;
         const int tx = tile % m.ntx, ty = tile / m.ntx;
         const int ti0 = tx * TILE_W, tj0 = ty * TILE_H;
@@ -851,11 +1015,10 @@ __global__ void __launch_bounds__(SLOW_CHUNK) push_tile_slow(MeshP m, MeshD md, 
         for (int k = t; k < TILE_CELLS; k += SLOW_CHUNK) L.hist[k] = 0;
         if (t == 0) tile_segments(offsets, m.nci, m.ncj, ti0, tj0, L.seg_start, L.seg_pre);
         __syncthreads();
-        const int k = item.y * SLOW_CHUNK + t;
-        if (k < tile_nslow[tile]) {
-            const int64_t g = slow_list[tile_slot(L.seg_start, L.seg_pre, k)];
+        if (t < item.z) {
+            const int64_t g = slow_list[tile_slot(L.seg_start, L.seg_pre, item.y + t)];
             PIn q = load_particle(s, g);
-            const bool alive = push_particle<false>(m, md, pc, load_e, hasseg, q.lc0, q.lc1, q.v0, q.v1, q.v2);
+            const bool alive = push_particle<HAS_B>(m, md, pc, load_e, hasseg, q.lc0, q.lc1, q.v0, q.v1, q.v2);
             int32_t key = -1;
             if (alive) {
                 int ci, cj;
@@ -904,14 +1067,6 @@ __global__ void __launch_bounds__(SLOW_CHUNK) push_tile_slow(MeshP m, MeshD md, 
         __syncthreads();   // the next item reuses the LDS window
     }
     stat_flush(st, stats);
-}
-
-// cell counts of an in-place step only feed the macroparticle-per-cell samples
-__global__ void mpc_accumulate(int n, int32_t* __restrict__ counts, long long* __restrict__ mpc_sum) {
-    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < n; c += gridDim.x * blockDim.x) {
-        mpc_sum[c] += counts[c];
-        counts[c] = 0;
-    }
 }
 
 // ----------------------------------------------------------------------------------------
@@ -1099,15 +1254,56 @@ __global__ void __launch_bounds__(256) copy_scatter(MeshP m, PState s, PState d,
 // ----------------------------------------------------------------------------------------
 // The running sums are FP64 in physical units (mpw-weighted): each step adds its exact integer
 // totals, converted once, so they are deterministic and cannot wrap however long sampling runs.
-// fs_n, fs_v, fs_vv are spwt / 2^k of the density, velocity and second-moment channels.
+// inv_kw, inv_kv, inv_kvv are 1 / 2^k of the density, velocity and second-moment channels.
 // The channels hold W = sum w, D_k = sum w (v_k - c_k) and Q_k = sum w (v_k - c_k)^2 (unit
 // weight); the reference's sums are W, D_k + c_k W and Q_k + 2 c_k D_k + c_k^2 W, times mpw.
-__global__ void __launch_bounds__(256) normalize_nodes(int64_t nn, unsigned long long* __restrict__ acc,
+//
+// GAS (the first update and every tenth step): also KineticMaterial.computeFields(MeshData)
+// (core/materials/KineticMaterial.java:1606-1671) over the new running sums, in the reference's order
+// of operations: temperatures where count-sum > 0 (init_vals.T elsewhere), nd-ave = count-sum *
+// (1/num_samples) / nodeVol, u/v/w-ave = sum / count-sum (0 where the count is 0,
+// Field2D.divideByField), p = nd-ave K T, and mpc = mpc-sum * (1/num_samples) for the cells (row
+// j*ni + i of cell (i, j), 0 on the last node row and column).  gas: [NGAS][nn] t, t1, t2, t3,
+// nd-ave, u-ave, v-ave, w-ave, p, mpc.
+//
+// counts (steps without a sort; null otherwise): the cell counts of the push, added to mpc_sum and
+// cleared.  The node (i, j) and the cell (i, j) belong to one thread.
+//
+// The first workgroup also adds up the push's status words, leaves them in pinned host memory for the
+// call's one synchronisation and clears them for the next push.
+struct NormP {
+    double inv_kw, inv_kv, inv_kvv, c0, c1, c2, spwt, nd_back;
+    double f, init_T, inv_ns;      // computeFields: mass / k_B, temperature of empty nodes, 1 / samples
+};
+template <bool GAS>
+__global__ void __launch_bounds__(256) normalize_nodes(MeshP m, NormP np, unsigned long long* __restrict__ acc,
                                                        double* __restrict__ sums, const double* __restrict__ vol,
-                                                       double* __restrict__ den, double inv_kw, double inv_kv,
-                                                       double inv_kvv, double c0, double c1, double c2, double spwt,
-                                                       double nd_back, int samples) {
-    const double c[3] = {c0, c1, c2};
+                                                       double* __restrict__ den, int32_t* __restrict__ counts,
+                                                       long long* __restrict__ mpc_sum, double* __restrict__ gas,
+                                                       PushCtrl* __restrict__ ctrl, const int32_t* __restrict__ total,
+                                                       PushResult* __restrict__ result) {
+    if (blockIdx.x == 0 && threadIdx.x < STAT_SLOTS) {
+        long long* slot = ctrl->stats + threadIdx.x * STAT_STRIDE;
+        long long v[5];
+        double dmax = __longlong_as_double(slot[5]);
+#pragma unroll
+        for (int k = 0; k < 5; k++) v[k] = wave_sum_ll(slot[k]);
+        for (int o = 32; o > 0; o >>= 1) dmax = fmax(dmax, __shfl_xor(dmax, o));
+        for (int k = 0; k < 6; k++) slot[k] = 0;
+        if (threadIdx.x == 0) {
+            for (int k = 0; k < 5; k++) result->sums[k] = v[k];
+            result->dmax = dmax;
+            result->flags = ctrl->flags;
+            result->queued = ctrl->qcount[0];
+            result->total = total != nullptr ? *total : 0;
+            ctrl->flags = 0;
+            ctrl->qcount[0] = ctrl->qcount[1] = 0;
+            __threadfence_system();
+        }
+    }
+    static_assert(STAT_SLOTS == 64, "one slot a lane of the first wave");
+    const double c[3] = {np.c0, np.c1, np.c2};
+    const int64_t nn = (int64_t)m.ni * m.nj;
     for (int64_t u = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; u < nn; u += (int64_t)gridDim.x * blockDim.x) {
         long long a[NCH];
 #pragma unroll
@@ -1115,71 +1311,68 @@ __global__ void __launch_bounds__(256) normalize_nodes(int64_t nn, unsigned long
             a[ch] = (long long)acc[ch * nn + u];
             acc[ch * nn + u] = 0ull;
         }
-        const double W = (double)a[0] * inv_kw;
+        const double W = (double)a[0] * np.inv_kw;
         double D[3], Q[3];
 #pragma unroll
         for (int k = 0; k < 3; k++) {
-            D[k] = (double)a[1 + k] * inv_kv;
-            Q[k] = (double)a[4 + k] * inv_kvv;
+            D[k] = (double)a[1 + k] * np.inv_kv;
+            Q[k] = (double)a[4 + k] * np.inv_kvv;
         }
-        if (samples) {
-            sums[u] += W * spwt;
+        double sum[NCH];
+        sum[0] = sums[u] + W * np.spwt;
 #pragma unroll
-            for (int k = 0; k < 3; k++) {
-                sums[(1 + k) * nn + u] += (D[k] + c[k] * W) * spwt;
-                sums[(4 + k) * nn + u] += (Q[k] + 2.0 * c[k] * D[k] + c[k] * c[k] * W) * spwt;
-            }
+        for (int k = 0; k < 3; k++) {
+            sum[1 + k] = sums[(1 + k) * nn + u] + (D[k] + c[k] * W) * np.spwt;
+            sum[4 + k] = sums[(4 + k) * nn + u] + (Q[k] + 2.0 * c[k] * D[k] + c[k] * c[k] * W) * np.spwt;
         }
-        const double nd = W * spwt / vol[u];
+#pragma unroll
+        for (int ch = 0; ch < NCH; ch++) sums[ch * nn + u] = sum[ch];
+        const double nd = W * np.spwt / vol[u];
         double vel[3] = {0, 0, 0};
         if (a[0] != 0) {
 #pragma unroll
             for (int k = 0; k < 3; k++) vel[k] = D[k] / W + c[k];
         }
-        den[u] = nd + nd_back;
+        den[u] = nd + np.nd_back;
         den[nn + u] = vel[0];
         den[2 * nn + u] = vel[1];
         den[3 * nn + u] = vel[2];
-    }
-}
-
-// KineticMaterial.computeFields(MeshData) (core/materials/KineticMaterial.java:1606-1671) over
-// the running sums, in the reference's order of operations: temperatures where count-sum > 0
-// (init_vals.T elsewhere), nd-ave = count-sum * (1/num_samples) / nodeVol, u/v/w-ave = sum /
-// count-sum (0 where the count is 0, Field2D.divideByField), p = nd-ave K T, and mpc =
-// mpc-sum * (1/num_samples) for the cells (row j*ni + i of cell (i, j), 0 on the last node row
-// and column).  gas: [NGAS][nn] t, t1, t2, t3, nd-ave, u-ave, v-ave, w-ave, p, mpc.
-__global__ void __launch_bounds__(256) compute_fields_kernel(MeshP m, const double* __restrict__ sums,
-                                                             const long long* __restrict__ mpc_sum,
-                                                             const double* __restrict__ vol,
-                                                             double* __restrict__ gas, double f, double init_T,
-                                                             double inv_ns) {
-    const int64_t nn = (int64_t)m.ni * m.nj;
-    for (int64_t u = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; u < nn; u += (int64_t)gridDim.x * blockDim.x) {
-        const double count = sums[u];
-        double T = init_T, T1 = init_T, T2 = init_T, T3 = init_T;
-        if (count > 0) {
-            const double uu = sums[nn + u] / count, vv = sums[2 * nn + u] / count, ww = sums[3 * nn + u] / count;
-            const double uu2 = sums[4 * nn + u] / count - uu * uu;
-            const double vv2 = sums[5 * nn + u] / count - vv * vv;
-            const double ww2 = sums[6 * nn + u] / count - ww * ww;
-            T = (uu2 + vv2 + ww2) * f / 3.0;
-            T1 = uu2 * f;
-            T2 = vv2 * f;
-            T3 = ww2 * f;
+        if (!GAS && counts == nullptr) continue;
+        const int i = (int)(u % m.ni), j = (int)(u / m.ni);
+        long long mpc = 0;
+        if (i < m.nci && j < m.ncj) {
+            const size_t cell = (size_t)j * m.nci + i;
+            mpc = mpc_sum[cell];
+            if (counts != nullptr) {
+                mpc += counts[cell];
+                counts[cell] = 0;
+                mpc_sum[cell] = mpc;
+            }
         }
-        const double nd_ave = count * inv_ns / vol[u];
+        if (!GAS) continue;
+        const double count = sum[0];
+        double T = np.init_T, T1 = np.init_T, T2 = np.init_T, T3 = np.init_T;
+        if (count > 0) {
+            const double uu = sum[1] / count, vv = sum[2] / count, ww = sum[3] / count;
+            const double uu2 = sum[4] / count - uu * uu;
+            const double vv2 = sum[5] / count - vv * vv;
+            const double ww2 = sum[6] / count - ww * ww;
+            T = (uu2 + vv2 + ww2) * np.f / 3.0;
+            T1 = uu2 * np.f;
+            T2 = vv2 * np.f;
+            T3 = ww2 * np.f;
+        }
+        const double nd_ave = count * np.inv_ns / vol[u];
         gas[u] = T;
         gas[nn + u] = T1;
         gas[2 * nn + u] = T2;
         gas[3 * nn + u] = T3;
         gas[4 * nn + u] = nd_ave;
-        gas[5 * nn + u] = count != 0 ? sums[nn + u] / count : 0.0;
-        gas[6 * nn + u] = count != 0 ? sums[2 * nn + u] / count : 0.0;
-        gas[7 * nn + u] = count != 0 ? sums[3 * nn + u] / count : 0.0;
+        gas[5 * nn + u] = count != 0 ? sum[1] / count : 0.0;
+        gas[6 * nn + u] = count != 0 ? sum[2] / count : 0.0;
+        gas[7 * nn + u] = count != 0 ? sum[3] / count : 0.0;
         gas[8 * nn + u] = nd_ave * K_B * T;
-        const int i = (int)(u % m.ni), j = (int)(u / m.ni);
-        gas[9 * nn + u] = (i < m.nci && j < m.ncj) ? (double)mpc_sum[(size_t)j * m.nci + i] * inv_ns : 0.0;
+        gas[9 * nn + u] = i < m.nci && j < m.ncj ? (double)mpc * np.inv_ns : 0.0;
     }
 }
 
@@ -1549,11 +1742,11 @@ static int prepare_channel_scales(sf_ctx* ctx, Species* sp) {
     double c[3] = {0, 0, 0};
     for (int pass = 0; pass < 2; pass++) {
         PushC pc = make_pushc(ctx, sp);
-        SF_HIP(ctx, hipMemsetAsync(sp->stats, 0, sizeof(slots), ctx->stream));
         hipLaunchKernelGGL(velocity_range_kernel, dim3(grid_for(sp->np, 256, 2048)), dim3(256), 0, ctx->stream,
-                           sp->buf[sp->cur], sp->np, pc, sp->stats);
+                           sp->buf[sp->cur], sp->np, pc, sp->ctrl->stats);
         SF_HIP(ctx, hipGetLastError());
-        SF_HIP(ctx, hipMemcpyAsync(slots, sp->stats, sizeof(slots), hipMemcpyDeviceToHost, ctx->stream));
+        SF_HIP(ctx, hipMemcpyAsync(slots, sp->ctrl->stats, sizeof(slots), hipMemcpyDeviceToHost, ctx->stream));
+        SF_HIP(ctx, hipMemsetAsync(sp->ctrl->stats, 0, sizeof(slots), ctx->stream));
         SF_HIP(ctx, hipStreamSynchronize(ctx->stream));
         const double dmax = combine_stat_slots(slots, st);
         if (st[0] == 0) return SF_OK;
@@ -1569,6 +1762,26 @@ static int prepare_channel_scales(sf_ctx* ctx, Species* sp) {
     return SF_OK;
 }
 
+// Particles per part of a push tile: about eight parts per CU of a small species (never below 1024,
+// where the fixed cost of a part, its LDS window, outweighs the balance), at most 8192.
+static int part_size(const sf_ctx* ctx, int64_t np) {
+    const int64_t p = (np / (8 * (int64_t)std::max(1, ctx->ncu)) + 255) / 256 * 256;
+    return (int)std::min<int64_t>(8192, std::max<int64_t>(1024, p));
+}
+static int max_parts(const sf_ctx* ctx, const Species* sp) {
+    return ctx->mp.ntx * ctx->mp.nty + (int)(sp->nsorted / sp->part);
+}
+// The parts of the freshly sorted species' tiles.
+static int build_parts(sf_ctx* ctx, Species* sp, int64_t np) {
+    const MeshP& m = ctx->mp;
+    sp->part = part_size(ctx, np);
+    SF_HIP(ctx, hipMemsetAsync(sp->nparts, 0, sizeof(int), ctx->stream));
+    hipLaunchKernelGGL(tile_parts_kernel, dim3((m.ntx * m.nty + 255) / 256), dim3(256), 0, ctx->stream, m.nci, m.ncj,
+                       m.ntx, m.ntx * m.nty, sp->part, (const int32_t*)sp->offsets, sp->parts, sp->nparts);
+    SF_HIP(ctx, hipGetLastError());
+    return SF_OK;
+}
+
 static int run_scan(sf_ctx* ctx, Species* sp, bool samples) {
     const int ncells = ctx->mp.nci * ctx->mp.ncj;
     const int nb = (ncells + SCAN_TILE - 1) / SCAN_TILE;
@@ -1577,7 +1790,7 @@ static int run_scan(sf_ctx* ctx, Species* sp, bool samples) {
     hipLaunchKernelGGL(scan_write, dim3(nb), dim3(SCAN_THREADS), 0, ctx->stream, sp->counts, ncells, sp->blocksum,
                        sp->offsets, sp->cursor, samples ? sp->mpc_sum : (long long*)nullptr, nb);
     SF_HIP(ctx, hipGetLastError());
-    return SF_OK;
+    return build_parts(ctx, sp, sp->np);
 }
 
 static int read_total(sf_ctx* ctx, Species* sp, int64_t* total) {
@@ -1623,6 +1836,10 @@ int push_deposit(sf_ctx* ctx, Species* sp) {
     const MeshP& m = ctx->mp;
     MeshD md = ctx->meshd();
     md.bnd_hits = sp->bnd_hits;
+    // the push kernels find their status words zero: normalize_nodes clears them for the next push, and
+    // a push that ended early is made up for here
+    if (sp->ctrl_dirty) SF_HIP(ctx, hipMemsetAsync(sp->ctrl, 0, sizeof(PushCtrl), ctx->stream));
+    sp->ctrl_dirty = true;
     const int rc_scales = prepare_channel_scales(ctx, sp);
     if (rc_scales) return rc_scales;
     PushC pc = make_pushc(ctx, sp);
@@ -1634,18 +1851,17 @@ int push_deposit(sf_ctx* ctx, Species* sp) {
     const bool sort_step = (sp->since_sort + 1 >= sp->sort_interval) || sp->nsorted == 0 ||
                            (sp->np - sp->nsorted) > sp->np / 8;
     const int64_t np_before = sp->np, nsorted_before = sp->nsorted;
-    SF_HIP(ctx, hipMemsetAsync(sp->stats, 0, (size_t)STAT_SLOTS * STAT_STRIDE * sizeof(long long), ctx->stream));
-    SF_HIP(ctx, hipMemsetAsync(sp->flags, 0, sizeof(int), ctx->stream));
+    long long* const d_stats = sp->ctrl->stats;
+    int *const d_flags = &sp->ctrl->flags, *const d_qcount = sp->ctrl->qcount;
     if (ctx->timing) SF_HIP(ctx, hipEventRecord(ctx->ev[0], ctx->stream));
     const bool hb = md.bf != nullptr;
-    // XY without a magnetic field: the fast tile kernel, with the particles it leaves queued for
-    // the full reference loop; RZ / ZR / with B: the tile kernel that runs the loop itself
-    const bool fastk = m.domain == SF_DOMAIN_XY && !hb && !ctx->no_fast_push;
+    // the fast tile kernel, with the particles it leaves queued for the full reference loop; the tile
+    // kernel that runs the loop itself only on request (SF_NO_FAST_PUSH)
+    const bool fastk = !ctx->no_fast_push;
     const dim3 tg(tile_grid(ctx)), tb(PUSH_THREADS);
     const dim3 g_tail(grid_for(sp->np - sp->nsorted, 256, 4096)), b256(256);
     // Every step pushes in place (a dead particle becomes a hole, cell = -1).  A sort step then
     // moves the pushed particles into cell order by their new cell, compacting the holes.
-    SF_HIP(ctx, hipMemsetAsync(sp->qcount, 0, 2 * sizeof(int), ctx->stream));
     if (sp->nsorted > 0) {
         if (fastk) {
             FastC fc;
@@ -1665,40 +1881,65 @@ int push_deposit(sf_ctx* ctx, Species* sp) {
             fc.nci = m.nci;
             fc.ncj = m.ncj;
             fc.ntx = m.ntx;
-            hipLaunchKernelGGL(push_tile_fast_xy, tg, tb, 0, ctx->stream, fc, (const float2*)ctx->d_ef32,
-                               (const uint8_t*)ctx->d_cellslow, s, (const int32_t*)sp->offsets, sp->acc, sp->counts,
-                               sp->stats, sp->key, sp->tile_nslow, sp->slow_items, sp->qcount);
+            const int rd = m.domain == SF_DOMAIN_ZR ? 1 : 0;   // radial direction (x in XY)
+            fc.qm = pc.qm;
+            fc.qmdt64 = pc.qm_dt;
+            fc.dt = pc.dt;
+            fc.x0r = m.x0[rd];
+            fc.dhr = m.dh[rd];
+            fc.inv_dhr = m.inv_dh[rd];
+            fc.inv_dha = m.inv_dh[1 - rd];
+            auto launch = [&](auto kernel) {
+                hipLaunchKernelGGL(kernel, dim3(max_parts(ctx, sp)), tb, 0, ctx->stream, fc, (const float2*)ctx->d_ef32,
+                                   (const float2*)ctx->d_bf32, (const uint8_t*)ctx->d_cellslow, s,
+                                   (const int32_t*)sp->offsets, (const int2*)sp->parts, (const int*)sp->nparts,
+                                   sp->part, sp->acc, sp->counts, d_stats, sp->key, sp->slow_items, d_qcount);
+            };
+            if (m.domain == SF_DOMAIN_RZ) {
+                if (hb) launch(push_tile_fast<SF_DOMAIN_RZ, true>);
+                else launch(push_tile_fast<SF_DOMAIN_RZ, false>);
+            } else if (m.domain == SF_DOMAIN_ZR) {
+                if (hb) launch(push_tile_fast<SF_DOMAIN_ZR, true>);
+                else launch(push_tile_fast<SF_DOMAIN_ZR, false>);
+            } else {
+                if (hb) launch(push_tile_fast<SF_DOMAIN_XY, true>);
+                else launch(push_tile_fast<SF_DOMAIN_XY, false>);
+            }
         } else if (hb) {
             hipLaunchKernelGGL(push_deposit_tile_inplace_b, tg, tb, 0, ctx->stream, m, md, pc, s, sp->offsets,
-                               sp->acc, sp->counts, sp->stats, sp->flags);
+                               sp->acc, sp->counts, d_stats, d_flags);
         } else {
             hipLaunchKernelGGL(push_deposit_tile_inplace, tg, tb, 0, ctx->stream, m, md, pc, s, sp->offsets,
-                               sp->acc, sp->counts, sp->stats, sp->flags);
+                               sp->acc, sp->counts, d_stats, d_flags);
         }
     }
     if (ctx->timing) SF_HIP(ctx, hipEventRecord(ctx->ev[5], ctx->stream));
-    if (sp->nsorted > 0 && fastk)   // the item count is on the device; idle workgroups exit
-        hipLaunchKernelGGL(push_tile_slow, dim3(2048), dim3(SLOW_CHUNK), 0, ctx->stream, m, md, pc, s,
-                           (const int32_t*)sp->offsets, (const int32_t*)sp->key, (const int32_t*)sp->tile_nslow,
-                           (const int2*)sp->slow_items, (const int*)sp->qcount, sp->acc, sp->counts, sp->stats,
-                           sp->flags);
+    const bool merged = sp->nsorted > 0 && fastk;
+    const int ntail = sp->np > sp->nsorted ? (int)g_tail.x : 0;
+    if (merged) {   // the item count is on the device; idle workgroups exit
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(2048 + ntail), dim3(SLOW_CHUNK), 0, ctx->stream, m, md, pc, s,
+                               (const int32_t*)sp->offsets, (const int32_t*)sp->key, (const int4*)sp->slow_items,
+                               (const int*)d_qcount, sp->acc, sp->counts, d_stats, d_flags, ntail, sp->nsorted,
+                               sp->np);
+        };
+        if (hb) launch(push_tile_slow<true>);
+        else launch(push_tile_slow<false>);
+    }
     if (ctx->timing) SF_HIP(ctx, hipEventRecord(ctx->ev[6], ctx->stream));
-    if (sp->np > sp->nsorted) {
+    if (ntail && !merged) {
         if (hb)
             hipLaunchKernelGGL(push_deposit_tail<true>, g_tail, b256, 0, ctx->stream, m, md, pc, s, sp->nsorted,
-                               sp->np, sp->acc, sp->counts, sp->stats, sp->flags);
+                               sp->np, sp->acc, sp->counts, d_stats, d_flags);
         else
             hipLaunchKernelGGL(push_deposit_tail<false>, g_tail, b256, 0, ctx->stream, m, md, pc, s, sp->nsorted,
-                               sp->np, sp->acc, sp->counts, sp->stats, sp->flags);
+                               sp->np, sp->acc, sp->counts, d_stats, d_flags);
     }
     SF_HIP(ctx, hipGetLastError());
     if (ctx->timing) SF_HIP(ctx, hipEventRecord(ctx->ev[1], ctx->stream));
     if (sort_step) {
         int rc = run_scan(ctx, sp, true);
         if (rc) return rc;
-    } else {
-        hipLaunchKernelGGL(mpc_accumulate, dim3(grid_for(ncells, 256, 4096)), dim3(256), 0, ctx->stream, ncells,
-                           sp->counts, sp->mpc_sum);
     }
     if (ctx->timing) SF_HIP(ctx, hipEventRecord(ctx->ev[2], ctx->stream));
     if (sort_step && sp->np > 0) {
@@ -1712,35 +1953,32 @@ int push_deposit(sf_ctx* ctx, Species* sp) {
         SF_HIP(ctx, hipGetLastError());
     }
     if (ctx->timing) SF_HIP(ctx, hipEventRecord(ctx->ev[3], ctx->stream));
-    const double spwt = sp->desc.spwt;
-    hipLaunchKernelGGL(normalize_nodes, dim3(grid_for(nn, 256, 8192)), dim3(256), 0, ctx->stream, nn, sp->acc,
-                       sp->sums, (const double*)ctx->d_node_vol, sp->den, 1.0 / sp->kscale[0], 1.0 / sp->kscale[1],
-                       1.0 / sp->kscale[4], pc.c0, pc.c1, pc.c2, spwt, sp->desc.nd_back, 1);
-    SF_HIP(ctx, hipGetLastError());
-    if (ctx->timing) SF_HIP(ctx, hipEventRecord(ctx->ev[4], ctx->stream));
     // KineticMaterial.updateGasProperties (KineticMaterial.java:1553-1563): one more sample, and
     // computeFields on the first update and on steps that are multiples of 10
     sp->num_samples++;
     sp->pushes++;
     const int64_t step = ctx->it > 0 ? (int64_t)ctx->it : sp->pushes;
-    if (sp->first_time || step % 10 == 0) {
-        hipLaunchKernelGGL(compute_fields_kernel, dim3(grid_for(nn, 256, 8192)), dim3(256), 0, ctx->stream, m,
-                           (const double*)sp->sums, (const long long*)sp->mpc_sum, (const double*)ctx->d_node_vol,
-                           sp->gas, sp->mass / K_B, sp->desc.init_T, 1.0 / sp->num_samples);
-        SF_HIP(ctx, hipGetLastError());
-    }
+    NormP norm{1.0 / sp->kscale[0], 1.0 / sp->kscale[1], 1.0 / sp->kscale[4], pc.c0, pc.c1, pc.c2, sp->desc.spwt,
+               sp->desc.nd_back, sp->mass / K_B, sp->desc.init_T, 1.0 / sp->num_samples};
+    auto normalise = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(grid_for(nn, 256, 8192)), dim3(256), 0, ctx->stream, m, norm, sp->acc, sp->sums,
+                           (const double*)ctx->d_node_vol, sp->den, sort_step ? (int32_t*)nullptr : sp->counts,
+                           sp->mpc_sum, sp->gas, sp->ctrl,
+                           sort_step ? (const int32_t*)sp->offsets + ncells : (const int32_t*)nullptr, sp->result);
+    };
+    if (sp->first_time || step % 10 == 0) normalise(normalize_nodes<true>);
+    else normalise(normalize_nodes<false>);
+    SF_HIP(ctx, hipGetLastError());
+    if (ctx->timing) SF_HIP(ctx, hipEventRecord(ctx->ev[4], ctx->stream));
     sp->first_time = false;
     // mover sums (KineticMaterial.java:247-259); the count is the number of survivors
-    long long slots[STAT_SLOTS * STAT_STRIDE], st[5] = {0, 0, 0, 0, 0};
-    SF_HIP(ctx, hipMemcpyAsync(slots, sp->stats, sizeof(slots), hipMemcpyDeviceToHost, ctx->stream));
-    int64_t total = 0;
-    if (sort_step) SF_HIP(ctx, hipMemcpyAsync(&total, sp->offsets + ncells, sizeof(int32_t), hipMemcpyDeviceToHost,
-                                              ctx->stream));
-    int flags = 0, queued = 0;
-    SF_HIP(ctx, hipMemcpyAsync(&flags, sp->flags, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-    SF_HIP(ctx, hipMemcpyAsync(&queued, sp->qcount, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
     SF_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    const double dmax = combine_stat_slots(slots, st);
+    sp->ctrl_dirty = false;
+    const PushResult& res = *sp->result;
+    const long long* st = res.sums;
+    const int64_t total = res.total;
+    const int flags = res.flags, queued = res.queued;
+    const double dmax = res.dmax;
     const double inv_kst = 1.0 / sp->kstat;
     sp->stats_host[0] = (double)st[0] * sp->desc.spwt * sp->mass;
     sp->stats_host[1] = (double)st[1] * inv_kst * sp->desc.spwt * sp->mass;
