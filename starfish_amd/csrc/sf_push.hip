@@ -665,9 +665,19 @@ __global__ void __launch_bounds__(256) tile_parts_kernel(int nci, int ncj, int n
 // Bound by FP64 issue (half rate: about 65 FP64 operations a particle in XY, 200 in RZ), LDS atomics and
 // HBM at once, with four waves a SIMD to overlap them.  Measured a step: XY 2e7 particles (1024 x 512)
 // 0.43 ms uniform; bunched (one tile in ten has twice the mean, the fullest five times) 0.48 ms with
-// parts against 0.71 with one workgroup a tile.  RZ 1e8 (2048 x 1024) 2.4 ms against 4.2 for the general
+// parts against 0.71 with one workgroup a tile.  RZ 1e8 (2048 x 1024) 2.1 ms against 4.2 for the general
 // tile kernel, which takes every particle through LDS for its stores and through the loop's
 // registers; ZR with B 1e6 (301 x 157) 50 against 74 us.
+//
+// Which lane takes which particle decides the LDS conflicts: the particles of a sorted tile come
+// cell by cell, and lanes of one cell add to the same four nodes.  A part is cut into STRANDS equal
+// runs, lane t reads run t mod STRANDS, so a wave holds STRANDS places of the tile (about its four
+// rows) and still reads runs of 64 consecutive bytes.  Measured, ms a step: at 379 particles a cell
+// (513 x 257) 1.52 with a stride of 151 through windows of 256 particles, .95 with 2 strands, .81
+// with 4, 1.14 with 8 (32-byte runs); RZ at 48 a cell 2.45, 2.21, 2.05, 2.42; XY at 38 a cell,
+// bunched, .52, .52, .48, .55.
+constexpr int STRANDS = 4;   // runs of a part that a wave reads side by side
+
 template <int DOM, bool HAS_B>
 __global__ void __launch_bounds__(PUSH_THREADS, 4) push_tile_fast(FastC fc, const float2* __restrict__ ef,
                                                                  const float2* __restrict__ bf,
@@ -693,7 +703,7 @@ __global__ void __launch_bounds__(PUSH_THREADS, 4) push_tile_fast(FastC fc, cons
     // corner (0, 0) of window cell (a, b)
     const int w_i0 = ti0 - TILE_HALO, w_j0 = tj0 - TILE_HALO;
     const size_t nn = (size_t)fc.ni * fc.nj;
-    const int pt = (t * CHUNK_STRIDE) & (PUSH_THREADS - 1);
+    const int strand = t % STRANDS, pt = t / STRANDS;
     const unsigned long long MAGIC_BITS = (unsigned long long)__double_as_longlong(QMAGIC);
 
     for (int k = t; k < NCH * TILE_NODES; k += PUSH_THREADS) (&L.acc[0][0])[k] = 0ull;
@@ -721,10 +731,9 @@ __global__ void __launch_bounds__(PUSH_THREADS, 4) push_tile_fast(FastC fc, cons
     }
     if (t == 0) tile_segments(offsets, fc.nci, fc.ncj, ti0, tj0, L.seg_start, L.seg_pre);
     __syncthreads();
-    // The part's particles are taken in windows of PUSH_THREADS; within a window thread t takes
-    // particle pt.  The waves run through the windows independently (no barrier): each loads its
-    // next window's particles before pushing the current ones and stores each pushed particle
-    // straight back to its slot.
+    // The waves run through the part's runs independently (no barrier): each loads its next window's
+    // particles before pushing the current ones and stores each pushed particle straight back to
+    // its slot.
     const int total = min(L.seg_pre[TILE_H], work.y + part);
     const int sg0 = L.seg_start[0], sg1 = L.seg_start[1], sg2 = L.seg_start[2], sg3 = L.seg_start[3];
     const int pr1 = L.seg_pre[1], pr2 = L.seg_pre[2], pr3 = L.seg_pre[3];
@@ -737,8 +746,10 @@ __global__ void __launch_bounds__(PUSH_THREADS, 4) push_tile_fast(FastC fc, cons
         const int b = sg0 + ((k >= pr1 ? -1 : 0) & d1) + ((k >= pr2 ? -1 : 0) & d2) + ((k >= pr3 ? -1 : 0) & d3);
         return (int64_t)b + k;
     };
-    auto load = [&](PReg& r, int k) {
-        const bool in = k < total;
+    const int slen = (total - work.y + STRANDS - 1) / STRANDS, s0 = work.y + strand * slen;
+    auto load = [&](PReg& r, int q) {
+        const int k = s0 + q;
+        const bool in = q < slen && k < total;
         const int64_t g = in ? slot_of(k) : 0;
         int32_t c = -1;
         float fx = 0.f, fy = 0.f, vx = 0.f, vy = 0.f, vz = 0.f;
@@ -757,15 +768,14 @@ __global__ void __launch_bounds__(PUSH_THREADS, 4) push_tile_fast(FastC fc, cons
     unsigned long long sp0 = 0, sp1 = 0, sp2 = 0, se = 0;
     double dmax = 0.0;
     PReg nxt;
-    load(nxt, work.y + pt);
-    for (int w0 = work.y; w0 < total; w0 += PUSH_THREADS) {
+    load(nxt, pt);
+    for (int w0 = 0; w0 < slen; w0 += PUSH_THREADS / STRANDS) {
         const PReg cur = nxt;
-        const bool ok = w0 + pt < total;
-        load(nxt, w0 + PUSH_THREADS + pt);
+        load(nxt, w0 + PUSH_THREADS / STRANDS + pt);
         int32_t key = SLOT_KEEP;
         float fxn = 0.f, fyn = 0.f, vxn = 0.f, vyn = 0.f, vzn = 0.f;
         bool slow = false;
-        if (ok && cur.c >= 0) {
+        if (cur.c >= 0) {
             const int ci = cur.c & 0xFFFF, cj = (cur.c >> 16) & 0xFFFF;
             const int hi = ci - w_i0, hj = cj - w_j0;
             bool fast = (unsigned)hi < (unsigned)TILE_CW && (unsigned)hj < (unsigned)TILE_CH;
@@ -896,7 +906,7 @@ __global__ void __launch_bounds__(PUSH_THREADS, 4) push_tile_fast(FastC fc, cons
                         atomicAdd(&L.hist[hm * TILE_CW + hn], 1);
                         // lanes of one cell start at different corners (lane mod 4), so the
                         // same-address conflicts of an instruction drop about fourfold
-                        const bool rx = t & 1, ry = t & 2;
+                        const bool rx = pt & 1, ry = pt & 2;
                         const double wx0 = rx ? dfx : gfx, wx1 = rx ? gfx : dfx, wy0 = ry ? dfy : gfy, wy1 = ry ? gfy : dfy;
                         const int ox = rx ? -1 : 1, oy = ry ? -TILE_NW : TILE_NW;
                         const int l0 = hm * TILE_NW + hn + (rx ? 1 : 0) + (ry ? TILE_NW : 0);
