@@ -76,84 +76,121 @@ __device__ __forceinline__ bf16x8 zero8() {
 //   forward:       out[p][n] = sum_tap sum_k in[p + d(tap)][k] * w[tap][n][k]   (+ bias, ReLU)
 //   backward data: din[p][k'] = sum_tap sum_n' g[p - d(tap)][n'] * w[tap][n'][k'] with the weight
 //                  stored transposed as wt[tap][k'][n'] -> the same kernel with sgn = -1.
-// MODE 0: BF16 output with bias and optional ReLU; MODE 1: FP32 output (optionally accumulated);
-// MODE 2: the ReLU backward of the previous layer fused: BF16 output act > 0 ? din : 0, with act
-// that layer's BF16 activation.
-// Requirements (checked on the host): K multiple of 32, N multiple of 16, channel strides and
-// offsets multiples of 8 (16-byte operand loads).
+// What surrounds a convolution in the network happens in its own loads and stores, so no pass over
+// memory does only pooling, upsampling or a ReLU's backward:
+//   input    channels [0, kup) are the nearest 2x upsampling of `up` (half resolution), the others `in`
+//   FWD      BF16 output with bias and ReLU, and if `pool` is given its 2x2 mean at half resolution
+//   BWD_RELU the ReLU backward of the layer before (its BF16 activation `act`): act > 0 ? din : 0
+//   BWD_UP   channels [0, nup): the sum over each 2x2 block (the upsampling's backward) masked by
+//            `act` at half resolution, BF16; the others (the skip path) FP32 into `skip`
+//   BWD_POOL the 2x2 mean's backward plus the skip path: each of the four pixels of twice the
+//            resolution gets skip + din / 4, masked by its `act`, BF16
+// Before, the pooling and upsampling kernels of an Adam step at 1024 x 512, batch 4, took 650 of its 4900 us,
+// and the decoder's FP32 input gradients (800 MB at full resolution) were written and read whole.
+// Requirements: K a multiple of 32, N of TN, channel counts in memory multiples of 8 (16-byte operand
+// loads), kup a multiple of 32, nup a multiple of TN; H and W even with `up`, `pool` and BWD_UP (the
+// network's grid is a multiple of 4, so only its quarter resolution can be odd).
 // ------------------------------------------------------------------------------------------
-struct View {
-    uint16_t* p;
-    int cs;   // channel stride (elements per pixel)
-    int co;   // channel offset
-};
-struct FView {
-    float* p;
-    int cs, co;
+enum ConvMode { FWD, BWD_RELU, BWD_UP, BWD_POOL };
+struct ConvP {
+    const uint16_t* in;     // [B][H][W][in_cs]; channels from in_cs up are zero
+    const uint16_t* up;     // [B][H/2][W/2][kup]
+    const uint16_t* w;      // [tap][N][K]
+    const float* bias;
+    const uint16_t* act;
+    uint16_t *out, *pool;
+    float* skip;
+    int in_cs, kup, K, N, nup, H, W, B, sgn;
+    int nrt, gx, gy, nsp;   // row tiles of a workgroup, tiles along x and y, tiles of all images
 };
 
-// The operands are staged in LDS.  One workgroup: R rows of CONV_TP pixels x TN output channels
-// (TN = 64: waves 2 x 2 over pixels x channels; TN = 32: 4 x 1).  For each chunk of 32 input
-// channels the R + 2 input rows of CONV_TP + 2 pixels and the 9 x TN x 32 weights go to LDS once,
-// and every wave runs its 16 x 16 tiles of all R rows over the 9 taps from there: a weight fragment
-// is read once per tap for R x PT pixel tiles, an input fragment once for two channel tiles.  The
-// next chunk's operands are loaded into registers while the current one is multiplied.  The
-// weights are the MFMA's A operand (rows = output channels) and the pixels its B operand, so a
-// lane's result holds 4 consecutive channels of one pixel and leaves in one 8-byte (BF16) or
-// 16-byte (FP32) store.
-constexpr int CONV_TP = 128;
-template <int MODE, int TN, int R>
-__global__ void __launch_bounds__(256, 2) conv3x3_lds(const uint16_t* __restrict__ in, int in_cs, int in_co, int K,
-                                                   const uint16_t* __restrict__ w, const float* __restrict__ bias,
-                                                   int N, uint16_t* __restrict__ out, float* __restrict__ fout,
-                                                   int out_cs, int out_co, int H, int Wd, int relu, int sgn,
-                                                   int accumulate, const uint16_t* __restrict__ act, int act_cs,
-                                                   int act_co, int nrt) {
-    constexpr int WN = TN / 32;                 // waves along the channels (two 16-channel tiles each)
-    constexpr int WP = 4 / WN;                  // waves along the pixels
-    constexpr int PT = CONV_TP / 16 / WP;       // 16-pixel tiles per wave and row
+// lane's neighbour in its pair of lanes (2 q, 2 q + 1): the other pixel of a 2x2 block's row
+__device__ __forceinline__ float pair_lane(float v) {
+    int i;
+    memcpy(&i, &v, 4);
+    i = __builtin_amdgcn_update_dpp(0, i, 0xB1, 0xF, 0xF, true);   // quad_perm 1, 0, 3, 2
+    memcpy(&v, &i, 4);
+    return v;
+}
+// sum over a 2x2 block in the order of its pixels, in the even lane of the pair (r0, r1: its two rows)
+__device__ __forceinline__ float4 block_sum(const float4 r0, const float4 r1) {
+    return make_float4(0.f + r0.x + pair_lane(r0.x) + r1.x + pair_lane(r1.x),
+                       0.f + r0.y + pair_lane(r0.y) + r1.y + pair_lane(r1.y),
+                       0.f + r0.z + pair_lane(r0.z) + r1.z + pair_lane(r1.z),
+                       0.f + r0.w + pair_lane(r0.w) + r1.w + pair_lane(r1.w));
+}
+__device__ __forceinline__ float4 as_float4(const f32x4 v) { return make_float4(v[0], v[1], v[2], v[3]); }
+__device__ __forceinline__ float4 unpack_bf16x4(const uint2 u) {
+    return make_float4(bf2f((uint16_t)(u.x & 0xFFFFu)), bf2f((uint16_t)(u.x >> 16)), bf2f((uint16_t)(u.y & 0xFFFFu)),
+                       bf2f((uint16_t)(u.y >> 16)));
+}
+
+// The operands are staged in LDS.  One workgroup: CONV_R rows of CONV_TP pixels x CONV_TN output
+// channels, its four waves over the pixels.  For each chunk of 32 input channels the CONV_R + 2
+// input rows of CONV_TP + 2 pixels and the 9 x CONV_TN x 32 weights go to LDS once, and every wave
+// runs its 16 x 16 tiles of all rows over the 9 taps from there.  The next chunk's operands are
+// loaded into registers while the current one is multiplied.  The weights are the MFMA's A operand
+// (rows = output channels) and the pixels its B operand, so a lane's result holds 4 consecutive
+// channels of one pixel and leaves in one 8-byte (BF16) or 16-byte (FP32) store.
+//
+// The stages' latency bounds it, so many small workgroups do better than few that use their operands
+// more often: with 35 KB of LDS four run on a CU.  Measured against 128 pixels x 2 rows x 64 (or x 4
+// x 32) channels, two on a CU: Adam step (1024 x 512, batch 4) 3.97 against 4.12 ms; guess at
+// 301 x 157, where the large tiles leave most CUs idle, 140 against 227 us.
+//
+// The workgroups of an XCD (consecutive indices go round the eight) take a contiguous band of
+// tiles, and the channel tiles of one pixel tile follow each other, so the input rows that they
+// share, and the halo rows of neighbouring tiles, come from that XCD's L2.
+constexpr int CONV_TN = 32, CONV_R = 2, CONV_TP = 64;
+template <int MODE>
+__global__ void __launch_bounds__(256, 4) conv3x3_lds(const ConvP p) {
+    constexpr int TN = CONV_TN, R = CONV_R;
     constexpr int IW = CONV_TP + 2;             // staged pixels per row
     constexpr int NIN = (R + 2) * IW * 4;       // 16-byte groups of the input stage (8 channels each)
     constexpr int NWT = 9 * TN * 4;             // 16-byte groups of the weight stage
     constexpr int RIN = (NIN + 255) / 256, RWT = (NWT + 255) / 256;
+    static_assert(CONV_TP == 64 && TN == 32 && R == 2, "a wave has two rows of 16 pixels x 32 channels");
     __shared__ uint4 s_in[NIN];                 // [row][pixel][group]
     __shared__ uint4 s_w[NWT];                  // [tap][channel][group]
-    const int ntn = (N + TN - 1) / TN;
+    const int ntn = p.N / TN, per = (p.nsp + 7) / 8;
+    const int slot = blockIdx.x >> 3, sp = (blockIdx.x & 7) * per + slot / ntn;
+    if (slot / ntn >= per || sp >= p.nsp) return;
+    const int n0 = (slot % ntn) * TN;
     // the workgroup walks nrt tiles of R rows down its column; step it is chunk it % nkc of row
     // tile it / nkc, so the next tile's first chunk is loaded while the current tile is multiplied
-    const int x0 = blockIdx.x * CONV_TP, y_first = blockIdx.y * nrt * R;
-    const int nkc = K / 32;
-    const int steps = min(nrt, (H - y_first + R - 1) / R) * nkc;
-    const int b = blockIdx.z / ntn, n0 = (blockIdx.z % ntn) * TN;
+    const int x0 = (sp % p.gx) * CONV_TP, y_first = ((sp / p.gx) % p.gy) * p.nrt * R, b = sp / (p.gx * p.gy);
+    const int nkc = p.K / 32, H = p.H, Wd = p.W, N = p.N;
+    const int steps = min(p.nrt, (H - y_first + R - 1) / R) * nkc;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int wp = wave % WP, wn = wave / WP;
     const int prow = lane & 15, kq = lane >> 4;
     uint4 rin[RIN], rwt[RWT];
     auto fetch = [&](int it) __attribute__((always_inline)) {
         const int y0 = y_first + (it / nkc) * R, k0 = (it % nkc) * 32;
+        const bool from_up = k0 < p.kup;
+        const uint16_t* const src = from_up ? p.up : p.in;
+        const int sh = from_up ? 1 : 0, cs = from_up ? p.kup : p.in_cs, kc = from_up ? k0 : k0 - p.kup;
+        const int Hs = H >> sh, Ws = Wd >> sh;
 #pragma unroll
         for (int q = 0; q < RIN; q++) {
             const int e = threadIdx.x + 256 * q;
             const int g = e & 3, px = (e >> 2) % IW, r = (e >> 2) / IW;
             const int yy = y0 - 1 + r, xx = x0 - 1 + px;
-            const bool ok = e < NIN && yy >= 0 && yy < H && xx >= 0 && xx < Wd;
-            const size_t o = ok ? (((size_t)b * H + yy) * Wd + xx) * in_cs + in_co + k0 + g * 8 : 0;
-            rin[q] = sel4(ok, *reinterpret_cast<const uint4*>(in + o));
+            const bool ok = e < NIN && yy >= 0 && yy < H && xx >= 0 && xx < Wd && kc + g * 8 < cs;
+            const size_t o = ok ? (((size_t)b * Hs + (yy >> sh)) * Ws + (xx >> sh)) * cs + kc + g * 8 : 0;
+            rin[q] = sel4(ok, *reinterpret_cast<const uint4*>(src + o));
         }
 #pragma unroll
         for (int q = 0; q < RWT; q++) {
             const int e = threadIdx.x + 256 * q;
             const int g = e & 3, n = (e >> 2) % TN, tap = (e >> 2) / TN;
-            const bool ok = e < NWT && n0 + n < N;
-            const size_t o = ok ? ((size_t)tap * N + n0 + n) * K + k0 + g * 8 : 0;
-            rwt[q] = sel4(ok, *reinterpret_cast<const uint4*>(w + o));
+            const bool ok = e < NWT;
+            const size_t o = ok ? ((size_t)tap * N + n0 + n) * p.K + k0 + g * 8 : 0;
+            rwt[q] = sel4(ok, *reinterpret_cast<const uint4*>(p.w + o));
         }
     };
-    f32x4 acc[R][PT][2];
+    f32x4 acc[R][2];
 #pragma unroll
-    for (int r = 0; r < R; r++)
-#pragma unroll
-        for (int p = 0; p < PT; p++) acc[r][p][0] = acc[r][p][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int r = 0; r < R; r++) acc[r][0] = acc[r][1] = f32x4{0.f, 0.f, 0.f, 0.f};
     if (steps > 0) fetch(0);
     for (int it = 0; it < steps; it++) {
         __syncthreads();   // the previous chunk's fragments are read
@@ -165,75 +202,89 @@ __global__ void __launch_bounds__(256, 2) conv3x3_lds(const uint16_t* __restrict
             if (threadIdx.x + 256 * q < NWT) s_w[threadIdx.x + 256 * q] = rwt[q];
         __syncthreads();
         if (it + 1 < steps) fetch(it + 1);
-        // (taps not unrolled: the R x PT x 2 tiles of a tap are, and the accumulators stay in
-        // registers)
-#pragma unroll 1
+#pragma unroll
         for (int tap = 0; tap < 9; tap++) {
-            const int dy = sgn * (tap / 3 - 1), dx = sgn * (tap % 3 - 1);
+            const int dy = p.sgn * (tap / 3 - 1), dx = p.sgn * (tap % 3 - 1);
             bf16x8 bw[2];
 #pragma unroll
             for (int t = 0; t < 2; t++) {
-                const uint4 v = s_w[(tap * TN + wn * 32 + t * 16 + prow) * 4 + kq];
+                const uint4 v = s_w[(tap * TN + t * 16 + prow) * 4 + kq];
                 memcpy(&bw[t], &v, 16);
             }
 #pragma unroll
-            for (int r = 0; r < R; r++)
-#pragma unroll
-                for (int p = 0; p < PT; p++) {
-                    const int px = (wp * PT + p) * 16 + prow;
-                    const uint4 v = s_in[((r + 1 + dy) * IW + px + 1 + dx) * 4 + kq];
-                    bf16x8 a;
-                    memcpy(&a, &v, 16);
-                    acc[r][p][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bw[0], a, acc[r][p][0], 0, 0, 0);
-                    acc[r][p][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bw[1], a, acc[r][p][1], 0, 0, 0);
-                }
+            for (int r = 0; r < R; r++) {
+                const uint4 v = s_in[((r + 1 + dy) * IW + wave * 16 + prow + 1 + dx) * 4 + kq];
+                bf16x8 a;
+                memcpy(&a, &v, 16);
+                acc[r][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bw[0], a, acc[r][0], 0, 0, 0);
+                acc[r][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bw[1], a, acc[r][1], 0, 0, 0);
+            }
         }
         if (it % nkc != nkc - 1) continue;
         // the row tile's last chunk: store its outputs and clear the accumulators
-        const int y0 = y_first + (it / nkc) * R;
         // D layout: lane holds rows (lane/16)*4 + i (channels), column lane%16 (pixel)
+        const int y = y_first + (it / nkc) * R;   // rows y and y + 1 (y alone at the end of an odd image)
+        const int nrow = min(R, H - y);
+        const int xo = x0 + wave * 16 + prow;
+        if (xo < Wd) {   // (both lanes of a pair where W is even)
 #pragma unroll
-        for (int r = 0; r < R; r++) {
-            const int y = y0 + r;
-            if (y >= H) continue;
+            for (int t = 0; t < 2; t++) {
+                const int n = n0 + t * 16 + kq * 4;   // this lane's 4 channels n .. n + 3
+                const size_t px = ((size_t)b * H + y) * Wd + xo;
+                const float4 v0 = as_float4(acc[0][t]), v1 = as_float4(acc[1][t]);
+                if constexpr (MODE == FWD) {
+                    const float4 bs = *reinterpret_cast<const float4*>(p.bias + n);
+                    const uint2 u0 = pack_bf16x4(make_float4(fmaxf(v0.x + bs.x, 0.f), fmaxf(v0.y + bs.y, 0.f),
+                                                             fmaxf(v0.z + bs.z, 0.f), fmaxf(v0.w + bs.w, 0.f)));
+                    const uint2 u1 = pack_bf16x4(make_float4(fmaxf(v1.x + bs.x, 0.f), fmaxf(v1.y + bs.y, 0.f),
+                                                             fmaxf(v1.z + bs.z, 0.f), fmaxf(v1.w + bs.w, 0.f)));
+                    *reinterpret_cast<uint2*>(p.out + px * N + n) = u0;
+                    if (nrow > 1) *reinterpret_cast<uint2*>(p.out + (px + Wd) * N + n) = u1;
+                    if (p.pool) {
+                        const float4 s = block_sum(unpack_bf16x4(u0), unpack_bf16x4(u1));
+                        if (!(prow & 1))
+                            *reinterpret_cast<uint2*>(
+                                p.pool + (((size_t)b * (H / 2) + y / 2) * (Wd / 2) + xo / 2) * N + n) =
+                                pack_bf16x4(make_float4(0.25f * s.x, 0.25f * s.y, 0.25f * s.z, 0.25f * s.w));
+                    }
+                } else if constexpr (MODE == BWD_RELU) {
 #pragma unroll
-            for (int p = 0; p < PT; p++) {
-                const int xo = x0 + (wp * PT + p) * 16 + prow;
-                if (xo >= Wd) continue;
-#pragma unroll
-                for (int t = 0; t < 2; t++) {
-                    const int n = n0 + wn * 32 + t * 16 + kq * 4;   // this lane's 4 channels n .. n + 3
-                    if (n >= N) continue;
-                    const size_t o = (((size_t)b * H + y) * Wd + xo) * out_cs + out_co + n;
-                    const f32x4 v = acc[r][p][t];
-                    if (MODE == 0) {
-                        float e[4];
-#pragma unroll
-                        for (int i = 0; i < 4; i++) {
-                            e[i] = v[i] + bias[n + i];
-                            if (relu) e[i] = fmaxf(e[i], 0.f);
-                        }
-                        *reinterpret_cast<uint2*>(out + o) = make_uint2(pack_bf16x2(e[0], e[1]), pack_bf16x2(e[2], e[3]));
-                    } else if (MODE == 2) {
-                        const uint2 a = *reinterpret_cast<const uint2*>(
-                            act + (((size_t)b * H + y) * Wd + xo) * act_cs + act_co + n);
-                        *reinterpret_cast<uint2*>(out + o) = pack_bf16x4(relu_mask4(make_float4(v[0], v[1], v[2], v[3]), a));
+                    for (int k = 0; k < 2; k++) {
+                        if (k >= nrow) continue;
+                        const size_t o = (px + (size_t)k * Wd) * N + n;
+                        *reinterpret_cast<uint2*>(p.out + o) =
+                            pack_bf16x4(relu_mask4(k ? v1 : v0, *reinterpret_cast<const uint2*>(p.act + o)));
+                    }
+                } else if constexpr (MODE == BWD_UP) {
+                    if (n0 < p.nup) {
+                        const float4 s = block_sum(v0, v1);
+                        const size_t o = (((size_t)b * (H / 2) + y / 2) * (Wd / 2) + xo / 2) * p.nup + n;
+                        if (!(prow & 1))
+                            *reinterpret_cast<uint2*>(p.out + o) =
+                                pack_bf16x4(relu_mask4(s, *reinterpret_cast<const uint2*>(p.act + o)));
                     } else {
-                        float4* f = reinterpret_cast<float4*>(fout + o);
-                        if (accumulate) {
-                            const float4 g = *f;
-                            *f = make_float4(g.x + v[0], g.y + v[1], g.z + v[2], g.w + v[3]);
-                        } else {
-                            *f = make_float4(v[0], v[1], v[2], v[3]);
-                        }
+                        const size_t o = px * (N - p.nup) + n - p.nup;
+                        *reinterpret_cast<float4*>(p.skip + o) = v0;
+                        *reinterpret_cast<float4*>(p.skip + o + (size_t)Wd * (N - p.nup)) = v1;
+                    }
+                } else {
+#pragma unroll
+                    for (int k = 0; k < 8; k++) {   // pixel (k & 1, (k >> 1) & 1) of row y + (k >> 2)
+                        if ((k >> 2) >= nrow) continue;
+                        const float4 d = k >> 2 ? v1 : v0;
+                        const size_t o = ((((size_t)b * H + y + (k >> 2)) * 2 + ((k >> 1) & 1)) * (2 * Wd) + 2 * xo +
+                                          (k & 1)) * N + n;
+                        const float4 sk = *reinterpret_cast<const float4*>(p.skip + o);
+                        const float4 e = make_float4(sk.x + 0.25f * d.x, sk.y + 0.25f * d.y, sk.z + 0.25f * d.z,
+                                                     sk.w + 0.25f * d.w);
+                        *reinterpret_cast<uint2*>(p.out + o) =
+                            pack_bf16x4(relu_mask4(e, *reinterpret_cast<const uint2*>(p.act + o)));
                     }
                 }
             }
         }
 #pragma unroll
-        for (int r = 0; r < R; r++)
-#pragma unroll
-            for (int p = 0; p < PT; p++) acc[r][p][0] = acc[r][p][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int r = 0; r < R; r++) acc[r][0] = acc[r][1] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
 }
 
@@ -255,7 +306,10 @@ __global__ void __launch_bounds__(256, 2) conv3x3_lds(const uint16_t* __restrict
 // which is deterministic and avoids thousands of workgroups' atomics on the same addresses.
 // The kernel is held to 168 registers (three waves per SIMD: three workgroups per CU, as many as
 // its 46 KB of LDS allow); with 174 it ran two and took 243 instead of 141 us per launch.
-// Requirements: K and N multiples of 32, strides and offsets multiples of 8.
+// Input channels below kup are the nearest 2x upsampling of `up`, as in conv3x3_lds.  The channel
+// tile pairs of a run follow each other on one XCD, and an XCD takes neighbouring runs, so the rows
+// that they share are read from HBM once.
+// Requirements: K and N multiples of 32, kup too, channel counts in memory multiples of 8.
 constexpr int WG_PX = 64;           // pixels per chunk (two MFMA reduction steps)
 constexpr int WG_Q = WG_PX / 4 + 2; // four-pixel entries per staged row (with padding)
 constexpr int WG_PART = 9 * 32 * 32 + 32;   // floats of a workgroup's partial
@@ -264,20 +318,23 @@ __device__ __forceinline__ uint32_t bf_at(const uint4& v, int c) {
     const uint32_t w = c < 2 ? v.x : (c < 4 ? v.y : (c < 6 ? v.z : v.w));
     return (c & 1) ? (w >> 16) : (w & 0xFFFFu);
 }
-__global__ void __launch_bounds__(256, 3) conv3x3_wgrad_lds(const uint16_t* __restrict__ in, int in_cs, int in_co,
-                                                         int K, const uint16_t* __restrict__ g, int g_cs, int N,
-                                                         float* __restrict__ part, int H, int Wd, int B,
+__global__ void __launch_bounds__(256, 3) conv3x3_wgrad_lds(const uint16_t* __restrict__ in, int in_cs,
+                                                         const uint16_t* __restrict__ up, int kup, int K,
+                                                         const uint16_t* __restrict__ g, int N,
+                                                         float* __restrict__ part, int H, int Wd, int B, int nrun,
                                                          int chunks_per_block) {
     __shared__ uint2 s_in[3][3][32][WG_Q];   // [dx + 1][row % 3][input channel][pixel / 4]
     __shared__ uint2 s_g[32][WG_Q];          // [output channel][pixel / 4]
-    const int nkt = K / 32;
-    const int k0 = (blockIdx.y % nkt) * 32, n0 = (blockIdx.y / nkt) * 32;
+    const int nkt = K / 32, pairs = nkt * (N / 32), per = (nrun + 7) / 8;
+    const int slot_i = blockIdx.x >> 3, run = (blockIdx.x & 7) * per + slot_i / pairs, pair = slot_i % pairs;
+    if (slot_i / pairs >= per || run >= nrun) return;
+    const int k0 = (pair % nkt) * 32, n0 = (pair / nkt) * 32;
     const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
     const int ks = wave & 1, tk = wave >> 1;   // pixel half (reduction step), input-channel half
     const int prow = lane & 15, kq = lane >> 4;
     const int cpr = (Wd + WG_PX - 1) / WG_PX;
     const int nchunks = B * H * cpr;
-    const int c_begin = blockIdx.x * chunks_per_block;
+    const int c_begin = run * chunks_per_block;
     const int c_end = min(c_begin + chunks_per_block, nchunks);
     // chunk c: row y = c % H of column band (c / H) % cpr of image c / (H cpr)
     // staging items: waves 0..2 an input row each (row y - 1 + r; in a run's steady state only
@@ -289,8 +346,11 @@ __global__ void __launch_bounds__(256, 3) conv3x3_wgrad_lds(const uint16_t* __re
     const int r = wave, q = lane & 15, gq = lane >> 4;
     uint4 v[6];
     // (the same loads for both kinds of item, so that v stays in registers)
-    const uint16_t* const src = is_in ? in : g;
-    const int scs = is_in ? in_cs : g_cs, sco = is_in ? in_co + k0 + gq * 8 : n0 + gq * 8;
+    const bool from_up = is_in && k0 < kup;
+    const uint16_t* const src = from_up ? up : (is_in ? in : g);
+    const int sh = from_up ? 1 : 0, scs = from_up ? kup : (is_in ? in_cs : N);
+    const int sco = from_up ? k0 + gq * 8 : (is_in ? k0 - kup + gq * 8 : n0 + gq * 8);
+    const int Hs = H >> sh, Ws = Wd >> sh;
     const int sdx = is_in ? -1 : 0, sj = is_in ? 6 : 4;
     // rows of chunk c this thread stages: the run's first chunk and the first row of a band
     // stage all three input rows
@@ -302,8 +362,8 @@ __global__ void __launch_bounds__(256, 3) conv3x3_wgrad_lds(const uint16_t* __re
 #pragma unroll
         for (int j = 0; j < 6; j++) {
             const int xx = x0 + 4 * q + sdx + j;
-            const bool ok = j < sj && yy >= 0 && yy < H && xx >= 0 && xx < Wd;
-            const size_t o = ok ? (((size_t)b * H + yy) * Wd + xx) * scs + sco : 0;
+            const bool ok = j < sj && yy >= 0 && yy < H && xx >= 0 && xx < Wd && sco < scs;
+            const size_t o = ok ? (((size_t)b * Hs + (yy >> sh)) * Ws + (xx >> sh)) * scs + sco : 0;
             v[j] = sel4(ok, *reinterpret_cast<const uint4*>(src + o));
         }
     };
@@ -381,7 +441,7 @@ __global__ void __launch_bounds__(256, 3) conv3x3_wgrad_lds(const uint16_t* __re
     __syncthreads();
     if (ks == 1) return;
     // D rows (lane/16)*4+i = input channel, column lane%16 = output channel
-    float* const pb = part + ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * WG_PART;
+    float* const pb = part + ((size_t)pair * nrun + run) * WG_PART;
 #pragma unroll
     for (int tap = 0; tap < 9; tap++)
 #pragma unroll
@@ -412,6 +472,7 @@ __global__ void __launch_bounds__(256) wgrad_reduce(const float* __restrict__ pa
     float s = 0.f;
     if (e < WG_PART) {
         const float* p = part + (size_t)blockIdx.y * nblk * WG_PART + e;
+#pragma unroll 8
         for (int b = slice; b < nblk; b += 8) s += p[(size_t)b * WG_PART];
     }
     red[slice][el] = s;
@@ -421,98 +482,16 @@ __global__ void __launch_bounds__(256) wgrad_reduce(const float* __restrict__ pa
     for (int j = 1; j < 8; j++) s += red[j][el];
     if (e < 9 * 32 * 32) {
         const int tap = e / 1024, k = (e / 32) % 32, n = e % 32;
-        dw[((size_t)tap * N + n0 + n) * K + k0 + k] += s;
+        dw[((size_t)tap * N + n0 + n) * K + k0 + k] = s;
     } else if (k0 == 0) {
-        db[n0 + e - 9 * 32 * 32] += s;
+        db[n0 + e - 9 * 32 * 32] = s;
     }
 }
 
 
-
-// 2x2 average pooling (forward BF16, backward FP32 accumulate)
-// (8 channels per thread: C, strides and offsets multiples of 8)
-__global__ void avgpool_fwd(const uint16_t* __restrict__ in, int in_cs, int in_co, int C, int H, int Wd, int B,
-                            uint16_t* __restrict__ out, int out_cs, int out_co) {
-    const int Ho = H / 2, Wo = Wd / 2, G = C / 8;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < (int64_t)B * Ho * Wo * G;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const int c = 8 * (int)(i % G);
-        const int64_t q = i / G;
-        const int xo = (int)(q % Wo), yo = (int)((q / Wo) % Ho), b = (int)(q / ((int64_t)Wo * Ho));
-        float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        for (int a = 0; a < 2; a++)
-            for (int e = 0; e < 2; e++) {
-                const uint4 v = *reinterpret_cast<const uint4*>(
-                    in + (((size_t)b * H + 2 * yo + a) * Wd + 2 * xo + e) * in_cs + in_co + c);
-#pragma unroll
-                for (int k = 0; k < 8; k++) s[k] += bf2f((uint16_t)bf_at(v, k));
-            }
-        uint32_t o[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) o[k] = (uint32_t)f2bf(0.25f * s[2 * k]) | ((uint32_t)f2bf(0.25f * s[2 * k + 1]) << 16);
-        *reinterpret_cast<uint4*>(out + (((size_t)b * Ho + yo) * Wo + xo) * out_cs + out_co + c) =
-            make_uint4(o[0], o[1], o[2], o[3]);
-    }
-}
-// Backward of the 2x2 average pooling fused with the ReLU backward of the pooled activation: the
-// gradient of a full-resolution pixel is its skip-path gradient (the view gskip) plus a quarter of
-// its parent's (dout, [pixel][C]), masked by the activation (view act) and rounded to BF16 into
-// g [pixel][C].  4 channels per thread; C, strides and offsets multiples of 4.
-__global__ void avgpool_relu_bwd(const float* __restrict__ dout, int C, int H, int Wd, int B,
-                                 const float* __restrict__ gskip, int s_cs, int s_co, const uint16_t* __restrict__ act,
-                                 int a_cs, int a_co, uint16_t* __restrict__ g) {
-    const int Ho = H / 2, Wo = Wd / 2, G = C / 4;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < (int64_t)B * H * Wd * G;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const int c = 4 * (int)(i % G);
-        const int64_t q = i / G;
-        const int x = (int)(q % Wd), y = (int)((q / Wd) % H), b = (int)(q / ((int64_t)Wd * H));
-        const float4 d = *reinterpret_cast<const float4*>(dout + (((size_t)b * Ho + y / 2) * Wo + x / 2) * C + c);
-        const float4 sk = *reinterpret_cast<const float4*>(gskip + q * s_cs + s_co + c);
-        const uint2 a = *reinterpret_cast<const uint2*>(act + q * a_cs + a_co + c);
-        const float4 e = make_float4(sk.x + 0.25f * d.x, sk.y + 0.25f * d.y, sk.z + 0.25f * d.z, sk.w + 0.25f * d.w);
-        *reinterpret_cast<uint2*>(g + q * C + c) = pack_bf16x4(relu_mask4(e, a));
-    }
-}
-// nearest 2x upsampling (forward BF16 into a view, 8 channels per 16-byte access; backward FP32
-// sum of the four children).  Forward: C, strides and offset multiples of 8.
-__global__ void upsample_fwd(const uint16_t* __restrict__ in, int in_cs, int C, int Hi, int Wi, int B,
-                             uint16_t* __restrict__ out, int out_cs, int out_co) {
-    const int H = 2 * Hi, Wd = 2 * Wi, G = C / 8;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < (int64_t)B * H * Wd * G;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const int g = (int)(i % G);
-        const int64_t q = i / G;
-        const int x = (int)(q % Wd), y = (int)((q / Wd) % H), b = (int)(q / ((int64_t)Wd * H));
-        *reinterpret_cast<uint4*>(out + (((size_t)b * H + y) * Wd + x) * out_cs + out_co + 8 * g) =
-            *reinterpret_cast<const uint4*>(in + (((size_t)b * Hi + y / 2) * Wi + x / 2) * in_cs + 8 * g);
-    }
-}
-// Backward of the nearest 2x upsampling fused with the ReLU backward of the upsampled activation:
-// the sum of the four children's gradients (view dout, d_cs channels per pixel), masked by the
-// activation (act, [pixel][C] at the low resolution) and rounded to BF16 into g [pixel][C].  4
-// channels per thread; C and d_cs multiples of 4.
-__global__ void upsample_relu_bwd(const float* __restrict__ dout, int d_cs, int C, int Hi, int Wi, int B,
-                                  const uint16_t* __restrict__ act, uint16_t* __restrict__ g) {
-    const int H = 2 * Hi, Wd = 2 * Wi, G = C / 4;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < (int64_t)B * Hi * Wi * G;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const int c = 4 * (int)(i % G);
-        const int64_t q = i / G;
-        const int x = (int)(q % Wi), y = (int)((q / Wi) % Hi), b = (int)(q / ((int64_t)Wi * Hi));
-        float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
-        for (int a = 0; a < 2; a++)
-            for (int e = 0; e < 2; e++) {
-                const float4 v =
-                    *reinterpret_cast<const float4*>(dout + (((size_t)b * H + 2 * y + a) * Wd + 2 * x + e) * d_cs + c);
-                s = make_float4(s.x + v.x, s.y + v.y, s.z + v.z, s.w + v.w);
-            }
-        const uint2 av = *reinterpret_cast<const uint2*>(act + q * C + c);
-        *reinterpret_cast<uint2*>(g + q * C + c) = pack_bf16x4(relu_mask4(s, av));
-    }
-}
 // 1x1 head C -> 1 in FP32 on top of a base channel of the input: y = base + sum_c w[c] act[c] + b
 constexpr int HEAD_C = 32;   // channels into the 1x1 head
+constexpr int X0_C = 8;      // channels of the network's input in memory (4 used); c1a's others are zero
 __global__ void __launch_bounds__(256) head_fwd(const uint16_t* __restrict__ act, int64_t npix,
                                                 const float* __restrict__ w, const float* __restrict__ bias,
                                                 const uint16_t* __restrict__ base, int base_cs, int base_co,
@@ -600,61 +579,35 @@ __global__ void __launch_bounds__(256) head_bwd(const uint16_t* __restrict__ act
         atomicAdd(threadIdx.x < HEAD_C ? &dw[threadIdx.x] : db, v);
     }
 }
-// Adam (Kingma & Ba 2015) on FP32 master weights
-// The parameter tensors as one index space for the optimizer: segment k holds elements
-// [begin, begin + n) with its parameter, gradient and moment arrays.  One launch zeroes every
-// gradient and one runs Adam on every parameter (instead of one memset and one Adam launch per
-// tensor); each element finds its segment by binary search over the begins.
-struct AdamSeg {
-    float *p, *g, *m, *v;
-    int64_t begin, n;
-};
-constexpr int ADAM_MAXSEG = 32;
-__device__ __forceinline__ int adam_seg_of(const AdamSeg* s, int nseg, int64_t i) {
-    int lo = 0, hi = nseg - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (s[mid].begin <= i) lo = mid;
-        else hi = mid - 1;
-    }
-    return lo;
-}
-__global__ void __launch_bounds__(256) zero_grads(const AdamSeg* __restrict__ segs, int nseg, int64_t total) {
-    __shared__ AdamSeg s[ADAM_MAXSEG];
-    if (threadIdx.x < nseg) s[threadIdx.x] = segs[threadIdx.x];
-    __syncthreads();
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
-        const int k = adam_seg_of(s, nseg, i);
-        s[k].g[i - s[k].begin] = 0.f;
-    }
-}
-__global__ void __launch_bounds__(256) adam_segs(const AdamSeg* __restrict__ segs, int nseg, int64_t total, float lr,
-                                                 float b1, float b2, float eps, float c1, float c2) {
-    __shared__ AdamSeg s[ADAM_MAXSEG];
-    if (threadIdx.x < nseg) s[threadIdx.x] = segs[threadIdx.x];
-    __syncthreads();
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
-        const int k = adam_seg_of(s, nseg, i);
-        const int64_t j = i - s[k].begin;
-        const float gi = s[k].g[j];
-        const float mi = b1 * s[k].m[j] + (1 - b1) * gi;
-        const float vi = b2 * s[k].v[j] + (1 - b2) * gi * gi;
-        s[k].m[j] = mi;
-        s[k].v[j] = vi;
-        s[k].p[j] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+// Adam (Kingma & Ba 2015) on FP32 master weights: the parameters, their gradients and moments are
+// flat arrays of one order (that of sf_cnn_params), so one launch updates them all.
+__global__ void __launch_bounds__(256) adam(int64_t n, float* __restrict__ p, const float* __restrict__ g,
+                                            float* __restrict__ m, float* __restrict__ v, float lr, float b1, float b2,
+                                            float eps, float c1, float c2) {
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+        const float gi = g[i];
+        const float mi = b1 * m[i] + (1 - b1) * gi;
+        const float vi = b2 * v[i] + (1 - b2) * gi * gi;
+        m[i] = mi;
+        v[i] = vi;
+        p[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
     }
 }
 // master FP32 weights [tap][n][k] (k < Kreal used, padded to K) -> BF16 forward [tap][n][K] and
-// transposed backward [tap][k][n] copies
-__global__ void pack_weights(const float* __restrict__ wm, int N, int K, uint16_t* __restrict__ wf,
-                             uint16_t* __restrict__ wt) {
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < 9LL * N * K; i += (int64_t)gridDim.x * blockDim.x) {
-        int k = (int)(i % K);
-        int64_t q = i / K;
-        int n = (int)(q % N), tap = (int)(q / N);
-        uint16_t h = f2bf(wm[i]);
-        wf[i] = h;
-        wt[((size_t)tap * K + k) * N + n] = h;
+// transposed backward [tap][k][n] copies; blockIdx.y is the layer
+constexpr int NCONV = 10;
+struct PackP {
+    const float* wm[NCONV];
+    uint16_t *wf[NCONV], *wt[NCONV];
+    int N[NCONV], K[NCONV];
+};
+__global__ void __launch_bounds__(256) pack_weights(const PackP p) {
+    const int l = blockIdx.y, N = p.N[l], K = p.K[l];
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < 9 * N * K; i += gridDim.x * blockDim.x) {
+        const int k = i % K, q = i / K, n = q % N, tap = q / N;
+        const uint16_t h = f2bf(p.wm[l][i]);
+        p.wf[l][i] = h;
+        p.wt[l][((size_t)tap * K + k) * N + n] = h;
     }
 }
 
@@ -667,8 +620,7 @@ namespace sf {
 
 struct ConvL {
     int K = 0, N = 0, Kreal = 0;       // padded input channels, output channels, real inputs
-    float *wm = nullptr, *b = nullptr, *gw = nullptr, *gb = nullptr;
-    float *mw = nullptr, *vw = nullptr, *mb = nullptr, *vb = nullptr;
+    float *wm = nullptr, *b = nullptr, *gw = nullptr, *gb = nullptr;   // in the flat arrays
     uint16_t *wf = nullptr, *wt = nullptr;
     size_t nw() const { return (size_t)9 * N * K; }
 };
@@ -681,18 +633,21 @@ struct sf_cnn {
     int H = 0, W = 0;         // network grid (mesh padded to multiples of 4)
     int Bmax = 0;
     int C1 = sf::HEAD_C, C2 = 64, C3 = 128;
-    sf::ConvL c1a, c1b, c2a, c2b, c3a, c3b, c4a, c4b, c5a, c5b;
-    float *hw = nullptr, *hb = nullptr, *ghw = nullptr, *ghb = nullptr;
-    float *mhw = nullptr, *vhw = nullptr, *mhb = nullptr, *vhb = nullptr;
-    sf::AdamSeg* segs = nullptr;      // the optimizer's segment table (device)
-    // activations (BF16 NHWC)
-    uint16_t *x0 = nullptr, *e1a = nullptr, *u1 = nullptr, *p1 = nullptr, *e2a = nullptr, *u2 = nullptr,
+    sf::ConvL L[sf::NCONV];   // in the order of sf_cnn_params
+    // flat FP32 arrays of sf_cnn_params' order: parameters, gradients, Adam's moments
+    int64_t nparams = 0;
+    float *pm = nullptr, *pg = nullptr, *pmom = nullptr, *pvar = nullptr;
+    float *hw = nullptr, *hb = nullptr, *ghw = nullptr, *ghb = nullptr;   // the head's parts of pm and pg
+    float* loss = nullptr;            // follows the head's gradients: one fill clears all three
+    bool packed = false;              // the layers' BF16 copies hold pm
+    // activations (BF16 NHWC, no padding between pixels)
+    uint16_t *x0 = nullptr, *e1a = nullptr, *e1 = nullptr, *p1 = nullptr, *e2a = nullptr, *e2 = nullptr,
              *p2 = nullptr, *e3a = nullptr, *e3 = nullptr, *d2a = nullptr, *d2 = nullptr, *d1a = nullptr,
              *d1 = nullptr;
     uint16_t *gop = nullptr, *gop2 = nullptr;   // BF16 operand gradients [npix][channels] (backward)
     float* y = nullptr;
-    // FP32 gradients where two paths add
-    float *g_u1 = nullptr, *g_p1 = nullptr, *g_u2 = nullptr, *g_p2 = nullptr, *dy = nullptr, *loss = nullptr;
+    // FP32 gradients of the skip paths, which add to those of the pooled ones
+    float *g_s1 = nullptr, *g_s2 = nullptr, *dy = nullptr;
     // dataset
     std::vector<uint16_t*> s_in;      // [H][W][4] BF16: rho, mask, phi_b, 0
     std::vector<float*> s_t;          // [H][W] target phi / phi_ref
@@ -724,169 +679,130 @@ static int cnn_alloc(sf_cnn* c, T** p, size_t n) {
     return SF_OK;
 }
 
-static int conv_init(sf_cnn* c, ConvL& L, int Kreal, int N, std::mt19937_64& rng) {
-    L.Kreal = Kreal;
-    L.K = (Kreal + 31) / 32 * 32;
-    L.N = N;
-    size_t nw = L.nw();
-    int rc = 0;
-    rc |= cnn_alloc(c, &L.wm, nw);
-    rc |= cnn_alloc(c, &L.gw, nw);
-    rc |= cnn_alloc(c, &L.mw, nw);
-    rc |= cnn_alloc(c, &L.vw, nw);
-    rc |= cnn_alloc(c, &L.b, N);
-    rc |= cnn_alloc(c, &L.gb, N);
-    rc |= cnn_alloc(c, &L.mb, N);
-    rc |= cnn_alloc(c, &L.vb, N);
-    rc |= cnn_alloc(c, &L.wf, nw);
-    rc |= cnn_alloc(c, &L.wt, nw);
-    if (rc) return SF_ERR_OOM;
+// real input channels and output channels of the layers c1a, c1b, c2a, c2b, c3a, c3b, c4a, c4b, c5a, c5b
+enum { C1A, C1B, C2A, C2B, C3A, C3B, C4A, C4B, C5A, C5B };
+static int conv_init(sf_cnn* c, ConvL& L, std::mt19937_64& rng) {
+    const size_t nw = L.nw();
+    if (cnn_alloc(c, &L.wf, nw) || cnn_alloc(c, &L.wt, nw)) return SF_ERR_OOM;
     // He initialisation over the real fan-in; padded input channels stay zero
-    std::normal_distribution<double> nd(0.0, std::sqrt(2.0 / (9.0 * Kreal)));
+    std::normal_distribution<double> nd(0.0, std::sqrt(2.0 / (9.0 * L.Kreal)));
     std::vector<float> h(nw, 0.f);
     for (int tap = 0; tap < 9; tap++)
-        for (int n = 0; n < N; n++)
-            for (int k = 0; k < Kreal; k++) h[((size_t)tap * N + n) * L.K + k] = (float)nd(rng);
+        for (int n = 0; n < L.N; n++)
+            for (int k = 0; k < L.Kreal; k++) h[((size_t)tap * L.N + n) * L.K + k] = (float)nd(rng);
     if (hipMemcpy(L.wm, h.data(), nw * 4, hipMemcpyHostToDevice) != hipSuccess) return SF_ERR_HIP;
     return SF_OK;
 }
 
-static void conv_pack(sf_cnn* c, ConvL& L) {
-    hipLaunchKernelGGL(pack_weights, dim3(grid1(L.nw())), dim3(256), 0, c->ctx->stream, (const float*)L.wm, L.N, L.K,
-                       L.wf, L.wt);
+static void pack(sf_cnn* c) {
+    if (c->packed) return;
+    PackP p;
+    for (int l = 0; l < NCONV; l++) {
+        p.wm[l] = c->L[l].wm;
+        p.wf[l] = c->L[l].wf;
+        p.wt[l] = c->L[l].wt;
+        p.N[l] = c->L[l].N;
+        p.K[l] = c->L[l].K;
+    }
+    hipLaunchKernelGGL(pack_weights, dim3(64, NCONV), dim3(256), 0, c->ctx->stream, p);
+    c->packed = true;
 }
 
-// 3x3 convolution launch (conv3x3_lds): 64-channel workgroup tiles when N allows, else 32
 template <int MODE>
-static void conv_launch(sf_cnn* c, const uint16_t* in, int in_cs, int in_co, int K, const uint16_t* w,
-                        const float* bias, int N, uint16_t* out, float* fout, int out_cs, int out_co, int H, int W,
-                        int B, int relu, int sgn, int accumulate, const uint16_t* act = nullptr, int act_cs = 0,
-                        int act_co = 0) {
-    // rows per workgroup: 2 with 64-channel tiles, 4 with 32 (the same accumulator count)
-    const bool t64 = N % 64 == 0;
-    const int tn = t64 ? 64 : 32, rows = t64 ? 2 : 4;
+static void conv_launch(sf_cnn* c, ConvP p) {
+    const int rows = (p.H + CONV_R - 1) / CONV_R, ntn = p.N / CONV_TN;
+    p.gx = (p.W + CONV_TP - 1) / CONV_TP;
     // row tiles per workgroup: up to 4 while the launch keeps at least 1024 workgroups
-    const int64_t tiles = (int64_t)((W + CONV_TP - 1) / CONV_TP) * ((H + rows - 1) / rows) * B * ((N + tn - 1) / tn);
-    const int nrt = (int)std::max<int64_t>(1, std::min<int64_t>(4, tiles / 1024));
-    const dim3 g((W + CONV_TP - 1) / CONV_TP, (H + rows * nrt - 1) / (rows * nrt), B * ((N + tn - 1) / tn));
-    if (t64)
-        hipLaunchKernelGGL((conv3x3_lds<MODE, 64, 2>), g, dim3(256), 0, c->ctx->stream, in, in_cs, in_co, K, w, bias,
-                           N, out, fout, out_cs, out_co, H, W, relu, sgn, accumulate, act, act_cs, act_co, nrt);
-    else
-        hipLaunchKernelGGL((conv3x3_lds<MODE, 32, 4>), g, dim3(256), 0, c->ctx->stream, in, in_cs, in_co, K, w, bias,
-                           N, out, fout, out_cs, out_co, H, W, relu, sgn, accumulate, act, act_cs, act_co, nrt);
+    p.nrt = (int)std::max<int64_t>(1, std::min<int64_t>(4, (int64_t)p.gx * rows * p.B * ntn / 1024));
+    p.gy = (rows + p.nrt - 1) / p.nrt;
+    p.nsp = p.gx * p.gy * p.B;
+    hipLaunchKernelGGL(conv3x3_lds<MODE>, dim3((p.nsp + 7) / 8 * 8 * ntn), dim3(256), 0, c->ctx->stream, p);
 }
-// forward conv: in view (cs, co, K channels) -> out view, bias + ReLU
-static void conv_fwd(sf_cnn* c, const ConvL& L, const uint16_t* in, int in_cs, int in_co, uint16_t* out, int out_cs,
-                     int out_co, int H, int W, int B) {
-    conv_launch<0>(c, in, in_cs, in_co, L.K, (const uint16_t*)L.wf, (const float*)L.b, L.N, out, (float*)nullptr,
-                   out_cs, out_co, H, W, B, 1, 1, 0);
+// forward convolution of layer l: in [H][W][in_cs] (after the upsampling of up, kup channels) -> out
+// with bias and ReLU, and its 2x2 mean
+static void conv_fwd(sf_cnn* c, int l, const uint16_t* in, int in_cs, uint16_t* out, int H, int W, int B,
+                     uint16_t* pool = nullptr, const uint16_t* up = nullptr, int kup = 0) {
+    const ConvL& L = c->L[l];
+    ConvP p = {};
+    p.in = in, p.in_cs = in_cs, p.up = up, p.kup = kup, p.K = L.K, p.w = L.wf, p.bias = L.b, p.N = L.N;
+    p.out = out, p.pool = pool, p.H = H, p.W = W, p.B = B, p.sgn = 1;
+    conv_launch<FWD>(c, p);
 }
-// backward of one conv: g (BF16 [npix][N]) -> weight / bias gradients and, if din != null, the FP32
-// input gradient into the din view; if gout != null, the input gradient through the ReLU of the
-// layer that produced the input (activation view act) as BF16 [npix][K] into gout
-static void conv_bwd(sf_cnn* c, const ConvL& L, const uint16_t* in, int in_cs, int in_co, const uint16_t* g,
-                     float* din, int din_cs, int din_co, int H, int W, int B, uint16_t* gout = nullptr,
-                     const uint16_t* act = nullptr, int act_cs = 0, int act_co = 0) {
-    // weight gradient: about WG_BLOCKS workgroups over the (32 x 32 channel tile, pixel band)
-    // pairs, their partials summed in workgroup order
+// weight and bias gradients of layer l for the output gradient g: about WG_BLOCKS workgroups over
+// the (32 x 32 channel tile, pixel band) pairs, their partials summed in workgroup order
+static void conv_wgrad(sf_cnn* c, int l, const uint16_t* in, int in_cs, const uint16_t* g, int H, int W, int B,
+                       const uint16_t* up = nullptr, int kup = 0) {
+    const ConvL& L = c->L[l];
     const int nchunks = B * H * ((W + WG_PX - 1) / WG_PX);
     const int pairs = (L.K / 32) * (L.N / 32);
-    int bx = std::max(1, std::min(nchunks, (WG_BLOCKS + pairs - 1) / pairs));
-    const int cpb = (nchunks + bx - 1) / bx;
-    bx = (nchunks + cpb - 1) / cpb;
-    hipLaunchKernelGGL(conv3x3_wgrad_lds, dim3(bx, pairs), dim3(256), 0, c->ctx->stream, in, in_cs, in_co, L.K, g, L.N,
-                       L.N, c->wpart, H, W, B, cpb);
+    int nrun = std::max(1, std::min(nchunks, (WG_BLOCKS + pairs - 1) / pairs));
+    const int cpb = (nchunks + nrun - 1) / nrun;
+    nrun = (nchunks + cpb - 1) / cpb;
+    hipLaunchKernelGGL(conv3x3_wgrad_lds, dim3((nrun + 7) / 8 * 8 * pairs), dim3(256), 0, c->ctx->stream, in, in_cs, up,
+                       kup, L.K, g, L.N, c->wpart, H, W, B, nrun, cpb);
     hipLaunchKernelGGL(wgrad_reduce, dim3((WG_PART + 31) / 32, pairs), dim3(256), 0, c->ctx->stream,
-                       (const float*)c->wpart, bx, L.K, L.N, L.gw, L.gb);
-    if (din)
-        conv_launch<1>(c, g, L.N, 0, L.N, (const uint16_t*)L.wt, (const float*)nullptr, L.K, (uint16_t*)nullptr, din,
-                       din_cs, din_co, H, W, B, 0, -1, 0);
-    if (gout)
-        conv_launch<2>(c, g, L.N, 0, L.N, (const uint16_t*)L.wt, (const float*)nullptr, L.K, gout, (float*)nullptr,
-                       L.K, 0, H, W, B, 0, -1, 0, act, act_cs, act_co);
+                       (const float*)c->wpart, nrun, L.K, L.N, L.gw, L.gb);
+}
+// input gradient of layer l for the output gradient g -> out (see the modes of conv3x3_lds)
+template <int MODE>
+static void conv_bwd(sf_cnn* c, int l, const uint16_t* g, const uint16_t* act, uint16_t* out, int H, int W, int B,
+                     float* skip = nullptr, int nup = 0) {
+    const ConvL& L = c->L[l];
+    ConvP p = {};
+    p.in = g, p.in_cs = L.N, p.K = L.N, p.w = L.wt, p.N = L.K, p.act = act, p.out = out, p.skip = skip, p.nup = nup;
+    p.H = H, p.W = W, p.B = B, p.sgn = -1;
+    conv_launch<MODE>(c, p);
 }
 
 static void forward(sf_cnn* c, int B) {
     const int H = c->H, W = c->W, C1 = c->C1, C2 = c->C2, C3 = c->C3;
     const int H2 = H / 2, W2 = W / 2, H4 = H / 4, W4 = W / 4;
-    hipStream_t st = c->ctx->stream;
-    for (ConvL* L : {&c->c1a, &c->c1b, &c->c2a, &c->c2b, &c->c3a, &c->c3b, &c->c4a, &c->c4b, &c->c5a, &c->c5b})
-        conv_pack(c, *L);
-    conv_fwd(c, c->c1a, c->x0, 32, 0, c->e1a, C1, 0, H, W, B);
-    conv_fwd(c, c->c1b, c->e1a, C1, 0, c->u1, C2 + C1, C2, H, W, B);                  // e1 -> u1[C2:]
-    hipLaunchKernelGGL(avgpool_fwd, dim3(grid1((int64_t)B * H2 * W2 * C1 / 8)), dim3(256), 0, st, (const uint16_t*)c->u1,
-                       C2 + C1, C2, C1, H, W, B, c->p1, C1, 0);
-    conv_fwd(c, c->c2a, c->p1, C1, 0, c->e2a, C2, 0, H2, W2, B);
-    conv_fwd(c, c->c2b, c->e2a, C2, 0, c->u2, C3 + C2, C3, H2, W2, B);                // e2 -> u2[C3:]
-    hipLaunchKernelGGL(avgpool_fwd, dim3(grid1((int64_t)B * H4 * W4 * C2 / 8)), dim3(256), 0, st, (const uint16_t*)c->u2,
-                       C3 + C2, C3, C2, H2, W2, B, c->p2, C2, 0);
-    conv_fwd(c, c->c3a, c->p2, C2, 0, c->e3a, C3, 0, H4, W4, B);
-    conv_fwd(c, c->c3b, c->e3a, C3, 0, c->e3, C3, 0, H4, W4, B);
-    hipLaunchKernelGGL(upsample_fwd, dim3(grid1((int64_t)B * H2 * W2 * C3 / 8)), dim3(256), 0, st, (const uint16_t*)c->e3,
-                       C3, C3, H4, W4, B, c->u2, C3 + C2, 0);
-    conv_fwd(c, c->c4a, c->u2, C3 + C2, 0, c->d2a, C2, 0, H2, W2, B);
-    conv_fwd(c, c->c4b, c->d2a, C2, 0, c->d2, C2, 0, H2, W2, B);
-    hipLaunchKernelGGL(upsample_fwd, dim3(grid1((int64_t)B * H * W * C2 / 8)), dim3(256), 0, st, (const uint16_t*)c->d2, C2,
-                       C2, H2, W2, B, c->u1, C2 + C1, 0);
-    conv_fwd(c, c->c5a, c->u1, C2 + C1, 0, c->d1a, C1, 0, H, W, B);
-    conv_fwd(c, c->c5b, c->d1a, C1, 0, c->d1, C1, 0, H, W, B);
-    hipLaunchKernelGGL(head_fwd, dim3(grid1((int64_t)B * H * W)), dim3(256), 0, st, (const uint16_t*)c->d1,
-                       (int64_t)B * H * W, (const float*)c->hw, (const float*)c->hb, (const uint16_t*)c->x0, 32, 3, c->y);
+    pack(c);
+    conv_fwd(c, C1A, c->x0, X0_C, c->e1a, H, W, B);
+    conv_fwd(c, C1B, c->e1a, C1, c->e1, H, W, B, c->p1);
+    conv_fwd(c, C2A, c->p1, C1, c->e2a, H2, W2, B);
+    conv_fwd(c, C2B, c->e2a, C2, c->e2, H2, W2, B, c->p2);
+    conv_fwd(c, C3A, c->p2, C2, c->e3a, H4, W4, B);
+    conv_fwd(c, C3B, c->e3a, C3, c->e3, H4, W4, B);
+    conv_fwd(c, C4A, c->e2, C2, c->d2a, H2, W2, B, nullptr, c->e3, C3);
+    conv_fwd(c, C4B, c->d2a, C2, c->d2, H2, W2, B);
+    conv_fwd(c, C5A, c->e1, C1, c->d1a, H, W, B, nullptr, c->d2, C2);
+    conv_fwd(c, C5B, c->d1a, C1, c->d1, H, W, B);
+    hipLaunchKernelGGL(head_fwd, dim3(grid1((int64_t)B * H * W)), dim3(256), 0, c->ctx->stream, (const uint16_t*)c->d1,
+                       (int64_t)B * H * W, (const float*)c->hw, (const float*)c->hb, (const uint16_t*)c->x0, X0_C, 3,
+                       c->y);
 }
 
 // The BF16 operand gradients alternate between gop and gop2 (a layer's backward reads one and
 // writes the next into the other); every ReLU backward is fused into the kernel that produces the
-// gradient of the activation.  FP32 gradients remain only where two paths add: the inputs of the
-// decoder convolutions (upsampled part plus skip part) and the pooled activations.
+// gradient of the activation.  FP32 gradients remain only where two paths add: the skip inputs of
+// the decoder convolutions, which wait for the pooled activations' gradients.
 static void backward(sf_cnn* c, int B) {
     const int H = c->H, W = c->W, C1 = c->C1, C2 = c->C2, C3 = c->C3;
     const int H2 = H / 2, W2 = W / 2, H4 = H / 4, W4 = W / 4;
-    const int64_t n1 = (int64_t)B * H * W, n2 = (int64_t)B * H2 * W2, n4 = (int64_t)B * H4 * W4;
-    hipStream_t st = c->ctx->stream;
     uint16_t* ga = c->gop;
     uint16_t* gb = c->gop2;
-    hipLaunchKernelGGL(head_bwd, dim3(1024), dim3(256), 0, st, (const uint16_t*)c->d1, n1, (const float*)c->hw,
-                       (const float*)c->dy, c->ghw, c->ghb, ga);
-    conv_bwd(c, c->c5b, c->d1a, C1, 0, ga, nullptr, 0, 0, H, W, B, gb, c->d1a, C1, 0);
-    conv_bwd(c, c->c5a, c->u1, C2 + C1, 0, gb, c->g_u1, C2 + C1, 0, H, W, B);
-    hipLaunchKernelGGL(upsample_relu_bwd, dim3(grid1(n2 * C2 / 4)), dim3(256), 0, st, (const float*)c->g_u1, C2 + C1,
-                       C2, H2, W2, B, (const uint16_t*)c->d2, ga);
-    conv_bwd(c, c->c4b, c->d2a, C2, 0, ga, nullptr, 0, 0, H2, W2, B, gb, c->d2a, C2, 0);
-    conv_bwd(c, c->c4a, c->u2, C3 + C2, 0, gb, c->g_u2, C3 + C2, 0, H2, W2, B);
-    hipLaunchKernelGGL(upsample_relu_bwd, dim3(grid1(n4 * C3 / 4)), dim3(256), 0, st, (const float*)c->g_u2, C3 + C2,
-                       C3, H4, W4, B, (const uint16_t*)c->e3, ga);
-    conv_bwd(c, c->c3b, c->e3a, C3, 0, ga, nullptr, 0, 0, H4, W4, B, gb, c->e3a, C3, 0);
-    conv_bwd(c, c->c3a, c->p2, C2, 0, gb, c->g_p2, C2, 0, H4, W4, B);
-    hipLaunchKernelGGL(avgpool_relu_bwd, dim3(grid1(n2 * C2 / 4)), dim3(256), 0, st, (const float*)c->g_p2, C2, H2, W2,
-                       B, (const float*)c->g_u2, C3 + C2, C3, (const uint16_t*)c->u2, C3 + C2, C3, ga);
-    conv_bwd(c, c->c2b, c->e2a, C2, 0, ga, nullptr, 0, 0, H2, W2, B, gb, c->e2a, C2, 0);
-    conv_bwd(c, c->c2a, c->p1, C1, 0, gb, c->g_p1, C1, 0, H2, W2, B);
-    hipLaunchKernelGGL(avgpool_relu_bwd, dim3(grid1(n1 * C1 / 4)), dim3(256), 0, st, (const float*)c->g_p1, C1, H, W, B,
-                       (const float*)c->g_u1, C2 + C1, C2, (const uint16_t*)c->u1, C2 + C1, C2, ga);
-    conv_bwd(c, c->c1b, c->e1a, C1, 0, ga, nullptr, 0, 0, H, W, B, gb, c->e1a, C1, 0);
-    conv_bwd(c, c->c1a, c->x0, 32, 0, gb, nullptr, 0, 0, H, W, B);
-}
-
-static std::vector<std::pair<float*, size_t>> grads(sf_cnn* c) {
-    std::vector<std::pair<float*, size_t>> g;
-    for (ConvL* L : {&c->c1a, &c->c1b, &c->c2a, &c->c2b, &c->c3a, &c->c3b, &c->c4a, &c->c4b, &c->c5a, &c->c5b}) {
-        g.push_back({L->gw, L->nw()});
-        g.push_back({L->gb, (size_t)L->N});
-    }
-    g.push_back({c->ghw, (size_t)c->C1});
-    g.push_back({c->ghb, 1});
-    return g;
-}
-static std::vector<std::pair<float*, size_t>> params(sf_cnn* c) {
-    std::vector<std::pair<float*, size_t>> g;
-    for (ConvL* L : {&c->c1a, &c->c1b, &c->c2a, &c->c2b, &c->c3a, &c->c3b, &c->c4a, &c->c4b, &c->c5a, &c->c5b}) {
-        g.push_back({L->wm, L->nw()});
-        g.push_back({L->b, (size_t)L->N});
-    }
-    g.push_back({c->hw, (size_t)c->C1});
-    g.push_back({c->hb, 1});
-    return g;
+    hipLaunchKernelGGL(head_bwd, dim3(1024), dim3(256), 0, c->ctx->stream, (const uint16_t*)c->d1, (int64_t)B * H * W,
+                       (const float*)c->hw, (const float*)c->dy, c->ghw, c->ghb, ga);
+    conv_wgrad(c, C5B, c->d1a, C1, ga, H, W, B);
+    conv_bwd<BWD_RELU>(c, C5B, ga, c->d1a, gb, H, W, B);
+    conv_wgrad(c, C5A, c->e1, C1, gb, H, W, B, c->d2, C2);
+    conv_bwd<BWD_UP>(c, C5A, gb, c->d2, ga, H, W, B, c->g_s1, C2);
+    conv_wgrad(c, C4B, c->d2a, C2, ga, H2, W2, B);
+    conv_bwd<BWD_RELU>(c, C4B, ga, c->d2a, gb, H2, W2, B);
+    conv_wgrad(c, C4A, c->e2, C2, gb, H2, W2, B, c->e3, C3);
+    conv_bwd<BWD_UP>(c, C4A, gb, c->e3, ga, H2, W2, B, c->g_s2, C3);
+    conv_wgrad(c, C3B, c->e3a, C3, ga, H4, W4, B);
+    conv_bwd<BWD_RELU>(c, C3B, ga, c->e3a, gb, H4, W4, B);
+    conv_wgrad(c, C3A, c->p2, C2, gb, H4, W4, B);
+    conv_bwd<BWD_POOL>(c, C3A, gb, c->e2, ga, H4, W4, B, c->g_s2);
+    conv_wgrad(c, C2B, c->e2a, C2, ga, H2, W2, B);
+    conv_bwd<BWD_RELU>(c, C2B, ga, c->e2a, gb, H2, W2, B);
+    conv_wgrad(c, C2A, c->p1, C1, gb, H2, W2, B);
+    conv_bwd<BWD_POOL>(c, C2A, gb, c->e1, ga, H2, W2, B, c->g_s1);
+    conv_wgrad(c, C1B, c->e1a, C1, ga, H, W, B);
+    conv_bwd<BWD_RELU>(c, C1B, ga, c->e1a, gb, H, W, B);
+    conv_wgrad(c, C1A, c->x0, X0_C, gb, H, W, B);
 }
 
 // place sample s into batch slot b of x0 / target / mask
@@ -894,20 +810,22 @@ __global__ void assemble_batch(const uint16_t* __restrict__ sin, const float* __
                                const uint8_t* __restrict__ sm, int64_t npix, uint16_t* __restrict__ x0,
                                float* __restrict__ bt, uint8_t* __restrict__ bm) {
     for (int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; p < npix; p += (int64_t)gridDim.x * blockDim.x) {
-        for (int c = 0; c < 4; c++) x0[p * 32 + c] = sin[p * 4 + c];
-        for (int c = 4; c < 32; c++) x0[p * 32 + c] = 0;
+        const uint2 u = *reinterpret_cast<const uint2*>(sin + p * 4);
+        *reinterpret_cast<uint4*>(x0 + p * X0_C) = make_uint4(u.x, u.y, 0u, 0u);
         bt[p] = st[p];
         bm[p] = sm[p];
     }
 }
 // Snapshot of a context on the padded grid: input channels (rho / rho_ref, Dirichlet mask,
 // boundary phi / phi_ref, Boltzmann inversion (phi0 + kTe ln max(rho / (e n0), 1)) / phi_ref),
-// target phi / phi_ref and the free-node mask.  Pixels outside the mesh are zero.
+// target phi / phi_ref and the free-node mask.  Pixels outside the mesh are zero, and so are channels
+// from 4 up to the stride cs (a multiple of 4).
 __global__ void snapshot_kernel(int ni, int nj, int H, int W, const double* __restrict__ rho,
                                 const double* __restrict__ phi, const int32_t* __restrict__ src,
                                 const uint8_t* __restrict__ cls, const double* __restrict__ fixval, double inv_rho,
                                 double inv_phi, double inv_en0, double kTe, double phi0,
-                                uint16_t* __restrict__ sin, float* __restrict__ st, uint8_t* __restrict__ sm) {
+                                uint16_t* __restrict__ sin, int cs, float* __restrict__ st,
+                                uint8_t* __restrict__ sm) {
     for (int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; p < (int64_t)H * W; p += (int64_t)gridDim.x * blockDim.x) {
         int x = (int)(p % W), y = (int)(p / W);
         uint16_t r = 0, mk = 0, pb = 0, bz = 0;
@@ -923,10 +841,8 @@ __global__ void snapshot_kernel(int ni, int nj, int H, int W, const double* __re
             if (phi) t = (float)(phi[u] * inv_phi);
             m = cls[u] != 0xFF ? 1 : 0;
         }
-        sin[p * 4 + 0] = r;
-        sin[p * 4 + 1] = mk;
-        sin[p * 4 + 2] = pb;
-        sin[p * 4 + 3] = bz;
+        *reinterpret_cast<uint2*>(sin + p * cs) = make_uint2((uint32_t)r | (uint32_t)mk << 16, (uint32_t)pb | (uint32_t)bz << 16);
+        for (int k = 4; k < cs; k += 4) *reinterpret_cast<uint2*>(sin + p * cs + k) = make_uint2(0u, 0u);
         if (st) st[p] = t;
         if (sm) sm[p] = m;
     }
@@ -983,34 +899,41 @@ int sf_cnn_create(sf_ctx* ctx, int ni, int nj, int max_batch, uint64_t seed, sf_
     const int C1 = c->C1, C2 = c->C2, C3 = c->C3;
     const int64_t n1 = (int64_t)max_batch * c->H * c->W, n2 = n1 / 4, n4 = n1 / 16;
     int rc = 0;
-    rc |= conv_init(c, c->c1a, 4, C1, c->rng);
-    rc |= conv_init(c, c->c1b, C1, C1, c->rng);
-    rc |= conv_init(c, c->c2a, C1, C2, c->rng);
-    rc |= conv_init(c, c->c2b, C2, C2, c->rng);
-    rc |= conv_init(c, c->c3a, C2, C3, c->rng);
-    rc |= conv_init(c, c->c3b, C3, C3, c->rng);
-    rc |= conv_init(c, c->c4a, C3 + C2, C2, c->rng);
-    rc |= conv_init(c, c->c4b, C2, C2, c->rng);
-    rc |= conv_init(c, c->c5a, C2 + C1, C1, c->rng);
-    rc |= conv_init(c, c->c5b, C1, C1, c->rng);
+    const int kn[NCONV][2] = {{4, C1},  {C1, C1},      {C1, C2}, {C2, C2},      {C2, C3},
+                              {C3, C3}, {C3 + C2, C2}, {C2, C2}, {C2 + C1, C1}, {C1, C1}};
+    for (int l = 0; l < NCONV; l++) {
+        c->L[l].Kreal = kn[l][0];
+        c->L[l].K = (kn[l][0] + 31) / 32 * 32;
+        c->L[l].N = kn[l][1];
+        c->nparams += (int64_t)c->L[l].nw() + c->L[l].N;
+    }
+    c->nparams += C1 + 1;
+    rc |= cnn_alloc(c, &c->pm, c->nparams);
+    rc |= cnn_alloc(c, &c->pg, c->nparams + 1);
+    rc |= cnn_alloc(c, &c->pmom, c->nparams);
+    rc |= cnn_alloc(c, &c->pvar, c->nparams);
+    if (!rc) {
+        int64_t off = 0;
+        for (ConvL& L : c->L) {
+            L.wm = c->pm + off, L.gw = c->pg + off;
+            off += (int64_t)L.nw();
+            L.b = c->pm + off, L.gb = c->pg + off;
+            off += L.N;
+        }
+        c->hw = c->pm + off, c->ghw = c->pg + off;
+        c->hb = c->hw + C1, c->ghb = c->ghw + C1;
+        c->loss = c->ghb + 1;
+        for (ConvL& L : c->L) rc |= conv_init(c, L, c->rng);
+    }
     // (a launch has at most ceil(WG_BLOCKS / pairs) * pairs <= WG_BLOCKS + pairs - 1 workgroups;
     // the network's layers have at most 16 channel tile pairs)
     rc |= cnn_alloc(c, &c->wpart, (size_t)(WG_BLOCKS + 128) * WG_PART);
-    rc |= cnn_alloc(c, &c->hw, C1);
-    rc |= cnn_alloc(c, &c->hb, 1);
-    rc |= cnn_alloc(c, &c->ghw, C1);
-    rc |= cnn_alloc(c, &c->ghb, 1);
-    rc |= cnn_alloc(c, &c->mhw, C1);
-    rc |= cnn_alloc(c, &c->vhw, C1);
-    rc |= cnn_alloc(c, &c->mhb, 1);
-    rc |= cnn_alloc(c, &c->vhb, 1);
-    rc |= cnn_alloc(c, &c->segs, ADAM_MAXSEG);
-    rc |= cnn_alloc(c, &c->x0, n1 * 32);
+    rc |= cnn_alloc(c, &c->x0, n1 * X0_C);
     rc |= cnn_alloc(c, &c->e1a, n1 * C1);
-    rc |= cnn_alloc(c, &c->u1, n1 * (C2 + C1));
+    rc |= cnn_alloc(c, &c->e1, n1 * C1);
     rc |= cnn_alloc(c, &c->p1, n2 * C1);
     rc |= cnn_alloc(c, &c->e2a, n2 * C2);
-    rc |= cnn_alloc(c, &c->u2, n2 * (C3 + C2));
+    rc |= cnn_alloc(c, &c->e2, n2 * C2);
     rc |= cnn_alloc(c, &c->p2, n4 * C2);
     rc |= cnn_alloc(c, &c->e3a, n4 * C3);
     rc |= cnn_alloc(c, &c->e3, n4 * C3);
@@ -1018,15 +941,12 @@ int sf_cnn_create(sf_ctx* ctx, int ni, int nj, int max_batch, uint64_t seed, sf_
     rc |= cnn_alloc(c, &c->d2, n2 * C2);
     rc |= cnn_alloc(c, &c->d1a, n1 * C1);
     rc |= cnn_alloc(c, &c->d1, n1 * C1);
-    rc |= cnn_alloc(c, &c->gop, n1 * (C2 + C1));
+    rc |= cnn_alloc(c, &c->gop, n1 * C1);    // (n2 C2 and n4 C3 are smaller)
     rc |= cnn_alloc(c, &c->gop2, n1 * C1);
     rc |= cnn_alloc(c, &c->y, n1);
-    rc |= cnn_alloc(c, &c->g_u1, n1 * (C2 + C1));
-    rc |= cnn_alloc(c, &c->g_p1, n2 * C1);
-    rc |= cnn_alloc(c, &c->g_u2, n2 * (C3 + C2));
-    rc |= cnn_alloc(c, &c->g_p2, n4 * C2);
+    rc |= cnn_alloc(c, &c->g_s1, n1 * C1);
+    rc |= cnn_alloc(c, &c->g_s2, n2 * C2);
     rc |= cnn_alloc(c, &c->dy, n1);
-    rc |= cnn_alloc(c, &c->loss, 4);
     rc |= cnn_alloc(c, &c->bt, n1);
     rc |= cnn_alloc(c, &c->bmask, n1);
     rc |= cnn_alloc(c, &c->phi_save, (size_t)ni * nj);
@@ -1062,11 +982,7 @@ int sf_cnn_dims(const sf_cnn* c, int* H, int* W, int64_t* nparams) {
     if (!c) return SF_ERR_ARG;
     if (H) *H = c->H;
     if (W) *W = c->W;
-    if (nparams) {
-        int64_t n = 0;
-        for (auto& p : params(const_cast<sf_cnn*>(c))) n += (int64_t)p.second;
-        *nparams = n;
-    }
+    if (nparams) *nparams = c->nparams;
     return SF_OK;
 }
 
@@ -1129,13 +1045,18 @@ int sf_cnn_snapshot(sf_cnn* c, sf_ctx* src_ctx) {
     hipLaunchKernelGGL(snapshot_kernel, dim3(grid1(np)), dim3(256), 0, ctx->stream, c->ni, c->nj, c->H, c->W,
                        (const double*)src_ctx->d_rho, (const double*)src_ctx->d_phi, poisson_src(src_ctx),
                        poisson_cls(src_ctx), poisson_fixval(src_ctx), 1.0 / c->rho_ref, 1.0 / c->phi_ref,
-                       feat_inv_en0(src_ctx), feat_kTe(src_ctx), poisson_desc(src_ctx)->phi0, sin, st, sm);
+                       feat_inv_en0(src_ctx), feat_kTe(src_ctx), poisson_desc(src_ctx)->phi0, sin, 4, st, sm);
     SF_HIP(ctx, hipGetLastError());
     SF_HIP(ctx, hipStreamSynchronize(ctx->stream));
     c->s_in.push_back(sin);
     c->s_t.push_back(st);
     c->s_m.push_back(sm);
     return SF_OK;
+}
+
+// clears what the kernels of a step add to: the head's gradients and the loss
+static hipError_t clear_sums(sf_cnn* c) {
+    return hipMemsetAsync(c->ghw, 0, (c->C1 + 2) * sizeof(float), c->ctx->stream);
 }
 
 // Adam training on random mini-batches of the snapshots; returns the mean loss of the last
@@ -1151,35 +1072,16 @@ int sf_cnn_train(sf_cnn* c, int steps, int batch, double lr, double* loss_out) {
     std::uniform_int_distribution<int> pick(0, (int)c->s_in.size() - 1);
     double tail = 0;
     int ntail = 0;
-    auto P = params(c);
-    auto G = grads(c);
-    std::vector<std::pair<float*, float*>> mv;
-    for (ConvL* L : {&c->c1a, &c->c1b, &c->c2a, &c->c2b, &c->c3a, &c->c3b, &c->c4a, &c->c4b, &c->c5a, &c->c5b}) {
-        mv.push_back({L->mw, L->vw});
-        mv.push_back({L->mb, L->vb});
-    }
-    mv.push_back({c->mhw, c->vhw});
-    mv.push_back({c->mhb, c->vhb});
-    std::vector<AdamSeg> segs;
-    int64_t total = 0;
-    for (size_t q = 0; q < P.size(); q++) {
-        segs.push_back(AdamSeg{P[q].first, G[q].first, mv[q].first, mv[q].second, total, (int64_t)P[q].second});
-        total += (int64_t)P[q].second;
-    }
-    if (segs.size() > (size_t)ADAM_MAXSEG) return sf_fail(ctx, SF_ERR_STATE, "sf_cnn_train: too many tensors");
-    SF_HIP(ctx, hipMemcpy(c->segs, segs.data(), segs.size() * sizeof(AdamSeg), hipMemcpyHostToDevice));
-    const int nseg = (int)segs.size();
     for (int s = 0; s < steps; s++) {
         int64_t counted = 0;
         for (int b = 0; b < batch; b++) {
             int k = pick(c->rng);
             hipLaunchKernelGGL(assemble_batch, dim3(grid1(np)), dim3(256), 0, st, (const uint16_t*)c->s_in[k],
-                               (const float*)c->s_t[k], (const uint8_t*)c->s_m[k], np, c->x0 + b * np * 32,
+                               (const float*)c->s_t[k], (const uint8_t*)c->s_m[k], np, c->x0 + b * np * X0_C,
                                c->bt + b * np, c->bmask + b * np);
             counted += np;
         }
-        hipLaunchKernelGGL(zero_grads, dim3(grid1(total)), dim3(256), 0, st, (const AdamSeg*)c->segs, nseg, total);
-        SF_HIP(ctx, hipMemsetAsync(c->loss, 0, 4, st));
+        SF_HIP(ctx, clear_sums(c));
         forward(c, batch);
         hipLaunchKernelGGL(mse_loss, dim3(std::min(grid1((int64_t)batch * np), 256)), dim3(256), 0, st, (const float*)c->y,
                            (const float*)c->bt, (const uint8_t*)c->bmask, (int64_t)batch * np, 1.0f / (float)counted,
@@ -1188,8 +1090,9 @@ int sf_cnn_train(sf_cnn* c, int steps, int batch, double lr, double* loss_out) {
         c->adam_t++;
         const float b1 = 0.9f, b2 = 0.999f;
         const float c1 = 1.f - powf(b1, (float)c->adam_t), c2 = 1.f - powf(b2, (float)c->adam_t);
-        hipLaunchKernelGGL(adam_segs, dim3(grid1(total)), dim3(256), 0, st, (const AdamSeg*)c->segs, nseg, total,
-                           (float)lr, b1, b2, 1e-8f, c1, c2);
+        hipLaunchKernelGGL(adam, dim3(grid1(c->nparams)), dim3(256), 0, st, c->nparams, c->pm, (const float*)c->pg,
+                           c->pmom, c->pvar, (float)lr, b1, b2, 1e-8f, c1, c2);
+        c->packed = false;
         SF_HIP(ctx, hipGetLastError());
         if (s >= steps - std::max(1, steps / 10)) {
             float l = 0;
@@ -1215,9 +1118,7 @@ int sf_cnn_loss_and_grads(sf_cnn* c, int sample, double* loss_out, float* y_out,
     const int64_t np = (int64_t)c->H * c->W;
     hipLaunchKernelGGL(assemble_batch, dim3(grid1(np)), dim3(256), 0, st, (const uint16_t*)c->s_in[sample],
                        (const float*)c->s_t[sample], (const uint8_t*)c->s_m[sample], np, c->x0, c->bt, c->bmask);
-    auto G = grads(c);
-    for (auto& g : G) SF_HIP(ctx, hipMemsetAsync(g.first, 0, g.second * 4, st));
-    SF_HIP(ctx, hipMemsetAsync(c->loss, 0, 4, st));
+    SF_HIP(ctx, clear_sums(c));
     forward(c, 1);
     hipLaunchKernelGGL(mse_loss, dim3(std::min(grid1(np), 256)), dim3(256), 0, st, (const float*)c->y, (const float*)c->bt,
                        (const uint8_t*)c->bmask, np, 1.0f / (float)np, c->dy, c->loss);
@@ -1228,12 +1129,8 @@ int sf_cnn_loss_and_grads(sf_cnn* c, int sample, double* loss_out, float* y_out,
     SF_HIP(ctx, hipStreamSynchronize(st));
     if (loss_out) *loss_out = l;
     if (y_out) SF_HIP(ctx, hipMemcpy(y_out, c->y, np * 4, hipMemcpyDeviceToHost));
-    int64_t off = 0;
-    for (auto& g : G) {
-        if (grads_out) SF_HIP(ctx, hipMemcpy(grads_out + off, g.first, g.second * 4, hipMemcpyDeviceToHost));
-        off += (int64_t)g.second;
-    }
-    if (n_out) *n_out = off;
+    if (grads_out) SF_HIP(ctx, hipMemcpy(grads_out, c->pg, c->nparams * 4, hipMemcpyDeviceToHost));
+    if (n_out) *n_out = c->nparams;
     return SF_OK;
 }
 
@@ -1245,36 +1142,45 @@ int sf_cnn_activation(sf_cnn* c, int which, float* out, int64_t* count) {
     sf_ctx* ctx = c->ctx;
     const int64_t n1 = (int64_t)c->H * c->W, n2 = n1 / 4, n4 = n1 / 16;
     const int C1 = c->C1, C2 = c->C2, C3 = c->C3;
-    const uint16_t* src = nullptr;
-    int64_t n = 0;
+    // the tensor's channels [0, ca) are `a` (upsampled from half the width where up), [ca, ca + cb) are `b`
+    const uint16_t *a = nullptr, *b = nullptr;
+    int ca = 0, cb = 0, pad = 0, w = c->W;
+    bool up = false;
+    int64_t npix = n1;
     switch (which) {
-        case 0: src = c->x0; n = n1 * 32; break;
-        case 1: src = c->e1a; n = n1 * C1; break;
-        case 2: src = c->u1; n = n1 * (C2 + C1); break;
-        case 3: src = c->p1; n = n2 * C1; break;
-        case 4: src = c->e2a; n = n2 * C2; break;
-        case 5: src = c->u2; n = n2 * (C3 + C2); break;
-        case 6: src = c->p2; n = n4 * C2; break;
-        case 7: src = c->e3a; n = n4 * C3; break;
-        case 8: src = c->e3; n = n4 * C3; break;
-        case 9: src = c->d2a; n = n2 * C2; break;
-        case 10: src = c->d2; n = n2 * C2; break;
-        case 11: src = c->d1a; n = n1 * C1; break;
-        case 12: src = c->d1; n = n1 * C1; break;
-        case 13: n = n1; break;
+        case 0: a = c->x0; ca = X0_C; pad = 32 - X0_C; break;
+        case 1: a = c->e1a; ca = C1; break;
+        case 2: a = c->d2; ca = C2; up = true; b = c->e1; cb = C1; break;
+        case 3: a = c->p1; ca = C1; npix = n2; break;
+        case 4: a = c->e2a; ca = C2; npix = n2; break;
+        case 5: a = c->e3; ca = C3; up = true; b = c->e2; cb = C2; npix = n2; w = c->W / 2; break;
+        case 6: a = c->p2; ca = C2; npix = n4; break;
+        case 7: a = c->e3a; ca = C3; npix = n4; break;
+        case 8: a = c->e3; ca = C3; npix = n4; break;
+        case 9: a = c->d2a; ca = C2; npix = n2; break;
+        case 10: a = c->d2; ca = C2; npix = n2; break;
+        case 11: a = c->d1a; ca = C1; break;
+        case 12: a = c->d1; ca = C1; break;
+        case 13: ca = 1; break;
         default: return sf_fail(ctx, SF_ERR_ARG, "sf_cnn_activation: unknown tensor %d", which);
     }
-    if (count) *count = n;
+    const int C = ca + cb + pad;
+    if (count) *count = npix * C;
     if (!out) return SF_OK;
     SF_HIP(ctx, hipSetDevice(ctx->device));
     SF_HIP(ctx, hipStreamSynchronize(ctx->stream));
     if (which == 13) {
-        SF_HIP(ctx, hipMemcpy(out, c->y, n * 4, hipMemcpyDeviceToHost));
+        SF_HIP(ctx, hipMemcpy(out, c->y, npix * 4, hipMemcpyDeviceToHost));
         return SF_OK;
     }
-    std::vector<uint16_t> h(n);
-    SF_HIP(ctx, hipMemcpy(h.data(), src, n * 2, hipMemcpyDeviceToHost));
-    for (int64_t i = 0; i < n; i++) out[i] = bf2f(h[i]);
+    std::vector<uint16_t> ha((up ? npix / 4 : npix) * ca), hb(npix * cb);
+    SF_HIP(ctx, hipMemcpy(ha.data(), a, ha.size() * 2, hipMemcpyDeviceToHost));
+    if (cb) SF_HIP(ctx, hipMemcpy(hb.data(), b, hb.size() * 2, hipMemcpyDeviceToHost));
+    for (int64_t q = 0; q < npix; q++) {
+        const int64_t qa = up ? (q / w / 2) * (w / 2) + q % w / 2 : q;
+        for (int k = 0; k < C; k++)
+            out[q * C + k] = k < ca ? bf2f(ha[qa * ca + k]) : (k < ca + cb ? bf2f(hb[q * cb + k - ca]) : 0.f);
+    }
     return SF_OK;
 }
 
@@ -1285,15 +1191,12 @@ int sf_cnn_params(sf_cnn* c, int get, float* buf, int64_t* n_out) {
     sf_ctx* ctx = c->ctx;
     SF_HIP(ctx, hipSetDevice(ctx->device));
     SF_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    int64_t off = 0;
-    for (auto& p : params(c)) {
-        if (buf) {
-            if (get) SF_HIP(ctx, hipMemcpy(buf + off, p.first, p.second * 4, hipMemcpyDeviceToHost));
-            else SF_HIP(ctx, hipMemcpy(p.first, buf + off, p.second * 4, hipMemcpyHostToDevice));
-        }
-        off += (int64_t)p.second;
+    if (buf && get) SF_HIP(ctx, hipMemcpy(buf, c->pm, c->nparams * 4, hipMemcpyDeviceToHost));
+    if (buf && !get) {
+        c->packed = false;
+        SF_HIP(ctx, hipMemcpy(c->pm, buf, c->nparams * 4, hipMemcpyHostToDevice));
     }
-    if (n_out) *n_out = off;
+    if (n_out) *n_out = c->nparams;
     return SF_OK;
 }
 
@@ -1349,13 +1252,10 @@ int sf_cnn_predict(sf_cnn* c, sf_ctx* target) {
     SF_HIP(ctx, hipSetDevice(ctx->device));
     SF_HIP(ctx, hipStreamSynchronize(target->stream));
     const int64_t np = (int64_t)c->H * c->W;
-    uint16_t* sin = c->gop;   // scratch [np][4]
     hipLaunchKernelGGL(snapshot_kernel, dim3(grid1(np)), dim3(256), 0, ctx->stream, c->ni, c->nj, c->H, c->W,
                        (const double*)target->d_rho, (const double*)nullptr, poisson_src(target), poisson_cls(target),
                        poisson_fixval(target), 1.0 / c->rho_ref, 1.0 / c->phi_ref, feat_inv_en0(target),
-                       feat_kTe(target), poisson_desc(target)->phi0, sin, (float*)nullptr, (uint8_t*)nullptr);
-    hipLaunchKernelGGL(assemble_batch, dim3(grid1(np)), dim3(256), 0, ctx->stream, (const uint16_t*)sin,
-                       (const float*)c->bt, (const uint8_t*)c->bmask, np, c->x0, c->bt, c->bmask);
+                       feat_kTe(target), poisson_desc(target)->phi0, c->x0, X0_C, (float*)nullptr, (uint8_t*)nullptr);
     forward(c, 1);
     hipLaunchKernelGGL(guess_to_phi, dim3(grid1((int64_t)c->ni * c->nj)), dim3(256), 0, ctx->stream, c->ni, c->nj,
                        c->W, (const float*)c->y, c->phi_ref, target->d_phi);

@@ -184,3 +184,46 @@ def test_training_reduces_the_loss(ctx):
         assert np.isfinite(last) and last < initial / 10
     finally:
         net.close()
+
+
+@pytest.mark.gpu
+def test_large_and_small_grids_agree(ctx):
+    """On a 256 x 256 grid every workgroup of a convolution (forward, and the three backward forms) has
+    one tile; on a 2048 x 1024 one it walks several, and the tiles are spread differently over the
+    XCDs.  The same patch on both, with a loss that counts only the patch's middle: activations there
+    are the same bits (an output's sum has one order in every place, and the middle is further from the patch's edge than the 44 pixels that the network
+    reaches), and the gradients are those of the same terms.  The loss divides by the pixels, so the
+    operand gradients differ by exactly 2^5, and the weight gradients by that and by the order of
+    their FP32 sums over the pixels (1e-5 in norm)."""
+    from starfish_amd.learned import LearnedGuess
+    import cnn_oracle as N
+    flat = N.init_params(seed=11).astype(np.float32)
+    x4, t, m = _synthetic_sample(np.random.default_rng(11), 256, 256)
+    m[:] = 0
+    m[96:160, 96:160] = 1
+    got = []
+    for ni, nj, x0, y0 in ((256, 256, 0, 0), (2048, 1024, 640, 384)):
+        net = LearnedGuess(ctx, ni=ni, nj=nj, max_batch=1)
+        try:
+            net.set_params(flat)
+            gx, gt, gm = np.zeros((nj, ni, 4)), np.zeros((nj, ni)), np.zeros((nj, ni), np.uint8)
+            s = (slice(y0, y0 + 256), slice(x0, x0 + 256))
+            gx[s], gt[s], gm[s] = x4, t, m
+            net.add_sample(gx, gt, gm)
+            _, y, g = net.loss_and_grads(0)
+            acts = []
+            for name, c, r in (("p1", 32, 2), ("p2", 64, 4), ("e3", 128, 4), ("u2", 192, 2), ("u1", 96, 1), ("d1", 32, 1)):
+                a = net.activation(N.DEVICE_TENSORS.index(name)).reshape(nj // r, ni // r, c)
+                acts.append(a[(y0 + 96) // r:(y0 + 160) // r, (x0 + 96) // r:(x0 + 160) // r].copy())
+            got.append((acts, y[y0 + 96:y0 + 160, x0 + 96:x0 + 160].copy(), g.astype(np.float64) * (ni * nj / 65536)))
+        finally:
+            net.close()
+    for a, b in zip(got[0][0], got[1][0]):
+        assert np.array_equal(a, b)
+    assert np.array_equal(got[0][1], got[1][1])
+    off = 0
+    for name, k, n in N.LAYERS:
+        for cnt in (9 * n * k, n):
+            assert _rel(got[1][2][off:off + cnt], got[0][2][off:off + cnt]) < 1e-5, name
+            off += cnt
+    assert _rel(got[1][2][off:], got[0][2][off:]) < 1e-5
