@@ -59,6 +59,10 @@ __device__ __forceinline__ bf16x8 load8(const uint16_t* p) {
     memcpy(&r, &v, 16);
     return r;
 }
+__device__ __forceinline__ uint32_t bf_at(const uint4& v, int c) {
+    const uint32_t w = c < 2 ? v.x : (c < 4 ? v.y : (c < 6 ? v.z : v.w));
+    return (c & 1) ? (w >> 16) : (w & 0xFFFFu);
+}
 // u where ok, else zero: a select on the values (a select between the addresses of two locals
 // would keep them in scratch memory)
 __device__ __forceinline__ uint4 sel4(bool ok, const uint4 u) {
@@ -100,7 +104,7 @@ struct ConvP {
     const uint16_t* act;
     uint16_t *out, *pool;
     float* skip;
-    int in_cs, kup, K, N, nup, H, W, B, sgn;
+    int in_cs, kup, K, N, nup, H, W, B;
     int nrt, gx, gy, nsp;   // row tiles of a workgroup, tiles along x and y, tiles of all images
 };
 
@@ -127,16 +131,18 @@ __device__ __forceinline__ float4 unpack_bf16x4(const uint2 u) {
 
 // The operands are staged in LDS.  One workgroup: CONV_R rows of CONV_TP pixels x CONV_TN output
 // channels, its four waves over the pixels.  For each chunk of 32 input channels the CONV_R + 2
-// input rows of CONV_TP + 2 pixels and the 9 x CONV_TN x 32 weights go to LDS once, and every wave
-// runs its 16 x 16 tiles of all rows over the 9 taps from there.  The next chunk's operands are
-// loaded into registers while the current one is multiplied.  The weights are the MFMA's A operand
+// input rows of CONV_TP + 2 pixels and the 9 x CONV_TN x 32 weights go to LDS once (the weights once
+// in all where there is one chunk), and every wave runs its 16 x 16 tiles of all rows over the 9
+// taps from there, its 12 input fragments read once.  The next chunk's operands are loaded into
+// registers while the current one is multiplied.  The weights are the MFMA's A operand
 // (rows = output channels) and the pixels its B operand, so a lane's result holds 4 consecutive
 // channels of one pixel and leaves in one 8-byte (BF16) or 16-byte (FP32) store.
 //
 // The stages' latency bounds it, so many small workgroups do better than few that use their operands
 // more often: with 35 KB of LDS four run on a CU.  Measured against 128 pixels x 2 rows x 64 (or x 4
 // x 32) channels, two on a CU: Adam step (1024 x 512, batch 4) 3.97 against 4.12 ms; guess at
-// 301 x 157, where the large tiles leave most CUs idle, 140 against 227 us.
+// 301 x 157, where the large tiles leave most CUs idle, 140 against 227 us.  Four rows a tile, which
+// halve the LDS reads of a product, gain nothing (3.11 ms a step either way).
 //
 // The workgroups of an XCD (consecutive indices go round the eight) take a contiguous band of
 // tiles, and the channel tiles of one pixel tile follow each other, so the input rows that they
@@ -144,7 +150,7 @@ __device__ __forceinline__ float4 unpack_bf16x4(const uint2 u) {
 constexpr int CONV_TN = 32, CONV_R = 2, CONV_TP = 64;
 template <int MODE>
 __global__ void __launch_bounds__(256, 4) conv3x3_lds(const ConvP p) {
-    constexpr int TN = CONV_TN, R = CONV_R;
+    constexpr int TN = CONV_TN, R = CONV_R, SGN = MODE == FWD ? 1 : -1;
     constexpr int IW = CONV_TP + 2;             // staged pixels per row
     constexpr int NIN = (R + 2) * IW * 4;       // 16-byte groups of the input stage (8 channels each)
     constexpr int NWT = 9 * TN * 4;             // 16-byte groups of the weight stage
@@ -179,6 +185,7 @@ __global__ void __launch_bounds__(256, 4) conv3x3_lds(const ConvP p) {
             const size_t o = ok ? (((size_t)b * Hs + (yy >> sh)) * Ws + (xx >> sh)) * cs + kc + g * 8 : 0;
             rin[q] = sel4(ok, *reinterpret_cast<const uint4*>(src + o));
         }
+        if (nkc == 1 && it > 0) return;   // (the weights stay)
 #pragma unroll
         for (int q = 0; q < RWT; q++) {
             const int e = threadIdx.x + 256 * q;
@@ -197,14 +204,22 @@ __global__ void __launch_bounds__(256, 4) conv3x3_lds(const ConvP p) {
 #pragma unroll
         for (int q = 0; q < RIN; q++)
             if (threadIdx.x + 256 * q < NIN) s_in[threadIdx.x + 256 * q] = rin[q];
+        if (nkc > 1 || it == 0)
 #pragma unroll
-        for (int q = 0; q < RWT; q++)
-            if (threadIdx.x + 256 * q < NWT) s_w[threadIdx.x + 256 * q] = rwt[q];
+            for (int q = 0; q < RWT; q++)
+                if (threadIdx.x + 256 * q < NWT) s_w[threadIdx.x + 256 * q] = rwt[q];
         __syncthreads();
         if (it + 1 < steps) fetch(it + 1);
+        bf16x8 a[R + 2][3];
+#pragma unroll
+        for (int r = 0; r < R + 2; r++)
+#pragma unroll
+            for (int q = 0; q < 3; q++) {
+                const uint4 v = s_in[(r * IW + wave * 16 + prow + q) * 4 + kq];
+                memcpy(&a[r][q], &v, 16);
+            }
 #pragma unroll
         for (int tap = 0; tap < 9; tap++) {
-            const int dy = p.sgn * (tap / 3 - 1), dx = p.sgn * (tap % 3 - 1);
             bf16x8 bw[2];
 #pragma unroll
             for (int t = 0; t < 2; t++) {
@@ -212,20 +227,18 @@ __global__ void __launch_bounds__(256, 4) conv3x3_lds(const ConvP p) {
                 memcpy(&bw[t], &v, 16);
             }
 #pragma unroll
-            for (int r = 0; r < R; r++) {
-                const uint4 v = s_in[((r + 1 + dy) * IW + wave * 16 + prow + 1 + dx) * 4 + kq];
-                bf16x8 a;
-                memcpy(&a, &v, 16);
-                acc[r][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bw[0], a, acc[r][0], 0, 0, 0);
-                acc[r][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bw[1], a, acc[r][1], 0, 0, 0);
-            }
+            for (int r = 0; r < R; r++)
+#pragma unroll
+                for (int t = 0; t < 2; t++)
+                    acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        bw[t], a[r + 1 + SGN * (tap / 3 - 1)][1 + SGN * (tap % 3 - 1)], acc[r][t], 0, 0, 0);
         }
         if (it % nkc != nkc - 1) continue;
         // the row tile's last chunk: store its outputs and clear the accumulators
         // D layout: lane holds rows (lane/16)*4 + i (channels), column lane%16 (pixel)
+        const int xo = x0 + wave * 16 + prow;
         const int y = y_first + (it / nkc) * R;   // rows y and y + 1 (y alone at the end of an odd image)
         const int nrow = min(R, H - y);
-        const int xo = x0 + wave * 16 + prow;
         if (xo < Wd) {   // (both lanes of a pair where W is even)
 #pragma unroll
             for (int t = 0; t < 2; t++) {
@@ -248,13 +261,11 @@ __global__ void __launch_bounds__(256, 4) conv3x3_lds(const ConvP p) {
                                 pack_bf16x4(make_float4(0.25f * s.x, 0.25f * s.y, 0.25f * s.z, 0.25f * s.w));
                     }
                 } else if constexpr (MODE == BWD_RELU) {
-#pragma unroll
-                    for (int k = 0; k < 2; k++) {
-                        if (k >= nrow) continue;
-                        const size_t o = (px + (size_t)k * Wd) * N + n;
-                        *reinterpret_cast<uint2*>(p.out + o) =
-                            pack_bf16x4(relu_mask4(k ? v1 : v0, *reinterpret_cast<const uint2*>(p.act + o)));
-                    }
+                    const size_t o0 = px * N + n, o1 = (px + (nrow > 1 ? Wd : 0)) * N + n;
+                    const uint2 a0 = *reinterpret_cast<const uint2*>(p.act + o0);
+                    const uint2 a1 = *reinterpret_cast<const uint2*>(p.act + o1);
+                    *reinterpret_cast<uint2*>(p.out + o0) = pack_bf16x4(relu_mask4(v0, a0));
+                    if (nrow > 1) *reinterpret_cast<uint2*>(p.out + o1) = pack_bf16x4(relu_mask4(v1, a1));
                 } else if constexpr (MODE == BWD_UP) {
                     if (n0 < p.nup) {
                         const float4 s = block_sum(v0, v1);
@@ -269,16 +280,24 @@ __global__ void __launch_bounds__(256, 4) conv3x3_lds(const ConvP p) {
                     }
                 } else {
 #pragma unroll
-                    for (int k = 0; k < 8; k++) {   // pixel (k & 1, (k >> 1) & 1) of row y + (k >> 2)
-                        if ((k >> 2) >= nrow) continue;
-                        const float4 d = k >> 2 ? v1 : v0;
-                        const size_t o = ((((size_t)b * H + y + (k >> 2)) * 2 + ((k >> 1) & 1)) * (2 * Wd) + 2 * xo +
-                                          (k & 1)) * N + n;
-                        const float4 sk = *reinterpret_cast<const float4*>(p.skip + o);
-                        const float4 e = make_float4(sk.x + 0.25f * d.x, sk.y + 0.25f * d.y, sk.z + 0.25f * d.z,
-                                                     sk.w + 0.25f * d.w);
-                        *reinterpret_cast<uint2*>(p.out + o) =
-                            pack_bf16x4(relu_mask4(e, *reinterpret_cast<const uint2*>(p.act + o)));
+                    for (int r = 0; r < 2; r++) {
+                        // the four pixels (k & 1, k >> 1) of row y + r; all loads before the first use
+                        const float4 d = r ? v1 : v0;
+                        const size_t o = (((size_t)b * H + y + (nrow > 1 ? r : 0)) * 4 * Wd + 2 * xo) * N + n;
+                        const int ok[4] = {0, N, 2 * Wd * N, (2 * Wd + 1) * N};
+                        float4 sk[4];
+                        uint2 av[4];
+#pragma unroll
+                        for (int k = 0; k < 4; k++) {
+                            sk[k] = *reinterpret_cast<const float4*>(p.skip + o + ok[k]);
+                            av[k] = *reinterpret_cast<const uint2*>(p.act + o + ok[k]);
+                        }
+#pragma unroll
+                        for (int k = 0; k < 4; k++) {
+                            const float4 e = make_float4(sk[k].x + 0.25f * d.x, sk[k].y + 0.25f * d.y,
+                                                         sk[k].z + 0.25f * d.z, sk[k].w + 0.25f * d.w);
+                            if (r < nrow) *reinterpret_cast<uint2*>(p.out + o + ok[k]) = pack_bf16x4(relu_mask4(e, av[k]));
+                        }
                     }
                 }
             }
@@ -290,41 +309,57 @@ __global__ void __launch_bounds__(256, 4) conv3x3_lds(const ConvP p) {
 
 // Weight gradient with the operands staged in LDS.  One workgroup: 32 input x 32 output channels
 // for all 9 taps over a run of chunks, a chunk being 64 pixels of one row; the chunks of a run go
-// down the rows of a 64-pixel column band, so the three input rows a chunk needs (y - 1, y, y + 1)
-// stay in a ring of three LDS rows and each chunk stages one new input row (three at the start of
-// a run or a band) and its gradient row.  Rows are staged transposed to [channel][pixel], each in
-// three copies shifted by one pixel (dx = -1, 0, 1), so an operand fragment (8 consecutive pixels
-// of one channel) is one 16-byte LDS read; a row holds 16 four-pixel entries plus 2 of padding, so
-// the 16 channels of a fragment read start on distinct banks.  Wave w takes the pixels
-// 32 (w & 1) .. + 31 of every chunk (one MFMA reduction step) and input channels 16 (w >> 1) .. + 15
-// against all 32 output channels: 9 input and 2 gradient fragments per 18 MFMAs.  The next
-// chunk's rows are loaded into registers while the current one is multiplied.  The waves of the
-// first input-channel tile also sum the gradient over the pixels (the bias gradient) with one
-// more MFMA per output tile against an all-ones operand.  At the end the two pixel halves are
-// added through LDS and the workgroup stores its sums as a partial (WG_PART floats: [tap][k][n],
-// then the 32 bias sums); wgrad_reduce adds the partials of a channel tile pair in a fixed order,
-// which is deterministic and avoids thousands of workgroups' atomics on the same addresses.
-// The kernel is held to 168 registers (three waves per SIMD: three workgroups per CU, as many as
-// its 46 KB of LDS allow); with 174 it ran two and took 243 instead of 141 us per launch.
+// down the rows of a 64-pixel column band.  Two chunks (rows y, y + 1) are multiplied between two
+// barriers: they need the input rows y - 1 .. y + 2 out of a ring of six in LDS, where the rows
+// y + 3 and y + 4 of the next two, loaded into registers meanwhile, are stored after the products.
+// Rows stay as they are in memory, [pixel][channel]: the fragments (8 pixels of one channel a lane)
+// come from the transposing LDS read, and a tap's shift along x is an offset of whole pixels.  A
+// pixel's two 16-channel halves are swapped in every second group of 8 pixels, so the 8 pixels that
+// 32 lanes read fall on distinct banks.  An input fragment serves the taps of both rows.
+// Wave w takes the pixels 32 (w & 1) .. + 31 of every chunk (one MFMA reduction step) and input
+// channels 16 (w >> 1) .. + 15 against all 32 output channels: 12 input and 4 gradient fragments
+// for 36 MFMAs.  The waves of the first input-channel tile also sum the gradient over the pixels
+// (the bias gradient) with one more MFMA per output tile against an all-ones operand.  At the end
+// the two pixel halves are added through LDS and the workgroup stores its sums as a partial
+// (WG_PART floats: [tap][k][n], then the 32 bias sums); wgrad_reduce adds the partials of a channel
+// tile pair in a fixed order, which is deterministic and avoids thousands of workgroups' atomics on
+// the same addresses.
 // Input channels below kup are the nearest 2x upsampling of `up`, as in conv3x3_lds.  The channel
 // tile pairs of a run follow each other on one XCD, and an XCD takes neighbouring runs, so the rows
 // that they share are read from HBM once.
+// Bound by the LDS reads and the MFMAs alike (512 and 576 cycles for two chunks), the first and last
+// layers by HBM.  Measured at 1024 x 512, batch 4: 780 us for the ten layers of a step, against 1480
+// with rows transposed by two of the four waves as they were stored, three shifted copies of each,
+// and two barriers a chunk; the largest (96 x 32 channels at full resolution) 153 us, 760 TFLOP/s.
+// 158 registers: three workgroups a CU.
 // Requirements: K and N multiples of 32, kup too, channel counts in memory multiples of 8.
 constexpr int WG_PX = 64;           // pixels per chunk (two MFMA reduction steps)
-constexpr int WG_Q = WG_PX / 4 + 2; // four-pixel entries per staged row (with padding)
+constexpr int WG_IW = WG_PX + 2;    // staged pixels per input row
+constexpr int WG_RING = 6;          // staged input rows
 constexpr int WG_PART = 9 * 32 * 32 + 32;   // floats of a workgroup's partial
 constexpr int WG_BLOCKS = 768;              // target workgroups of a weight-gradient launch (3 per CU)
-__device__ __forceinline__ uint32_t bf_at(const uint4& v, int c) {
-    const uint32_t w = c < 2 ? v.x : (c < 4 ? v.y : (c < 6 ? v.z : v.w));
-    return (c & 1) ? (w >> 16) : (w & 0xFFFFu);
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+// this lane's place for an 8-byte piece of pixel px of a staged row: 16-channel half h, quarter of it c
+__device__ __forceinline__ int wg_at(int px, int h, int c) { return px * 64 + ((h ^ (px >> 3)) & 1) * 32 + c * 8; }
+// 8 pixels x 16 channels of a staged row: the transposing reads at lo (its first four pixels) and hi
+__device__ __forceinline__ bf16x8 wg_frag(const char* lo, const char* hi) {
+    typedef __attribute__((address_space(3))) s16x4 lds4;
+    const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4*)lo);
+    const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4*)hi);
+    bf16x8 r;
+    memcpy(&r, &a, 8);
+    memcpy((char*)&r + 8, &b, 8);
+    return r;
 }
 __global__ void __launch_bounds__(256, 3) conv3x3_wgrad_lds(const uint16_t* __restrict__ in, int in_cs,
                                                          const uint16_t* __restrict__ up, int kup, int K,
                                                          const uint16_t* __restrict__ g, int N,
                                                          float* __restrict__ part, int H, int Wd, int B, int nrun,
                                                          int chunks_per_block) {
-    __shared__ uint2 s_in[3][3][32][WG_Q];   // [dx + 1][row % 3][input channel][pixel / 4]
-    __shared__ uint2 s_g[32][WG_Q];          // [output channel][pixel / 4]
+    constexpr int ROW_IN = WG_IW * 64, ROW_G = WG_PX * 64;   // bytes of a staged row
+    __shared__ uint4 lds[(WG_RING * ROW_IN + 4 * ROW_G) / 16];
+    char* const s_in = reinterpret_cast<char*>(lds);         // [row % 6][pixel][channel]
+    char* const s_g = s_in + WG_RING * ROW_IN;               // [interval & 1][row][pixel][channel]
     const int nkt = K / 32, pairs = nkt * (N / 32), per = (nrun + 7) / 8;
     const int slot_i = blockIdx.x >> 3, run = (blockIdx.x & 7) * per + slot_i / pairs, pair = slot_i % pairs;
     if (slot_i / pairs >= per || run >= nrun) return;
@@ -334,39 +369,59 @@ __global__ void __launch_bounds__(256, 3) conv3x3_wgrad_lds(const uint16_t* __re
     const int prow = lane & 15, kq = lane >> 4;
     const int cpr = (Wd + WG_PX - 1) / WG_PX;
     const int nchunks = B * H * cpr;
+    // chunk c: row c % H of column band (c / H) % cpr of image c / (H cpr)
     const int c_begin = run * chunks_per_block;
     const int c_end = min(c_begin + chunks_per_block, nchunks);
-    // chunk c: row y = c % H of column band (c / H) % cpr of image c / (H cpr)
-    // staging items: waves 0..2 an input row each (row y - 1 + r; in a run's steady state only
-    // r = 2, the new row y + 1), wave 3 the gradient row y; a thread's item is the pixel quad q
-    // (pixels 4q - 1 .. 4q + 4 of 8 channels for the input, 4q .. 4q + 3 for the gradient) of
-    // channel group gq.  The quad is the fastest index, so the 16 lanes of an LDS write phase cover
-    // all banks.
-    const bool is_in = wave < 3;
-    const int r = wave, q = lane & 15, gq = lane >> 4;
-    uint4 v[6];
-    // (the same loads for both kinds of item, so that v stays in registers)
-    const bool from_up = is_in && k0 < kup;
-    const uint16_t* const src = from_up ? up : (is_in ? in : g);
-    const int sh = from_up ? 1 : 0, scs = from_up ? kup : (is_in ? in_cs : N);
-    const int sco = from_up ? k0 + gq * 8 : (is_in ? k0 - kup + gq * 8 : n0 + gq * 8);
+    const bool from_up = k0 < kup;
+    const uint16_t* const src = from_up ? up : in;
+    const int sh = from_up ? 1 : 0, scs = from_up ? kup : in_cs, sco = (from_up ? k0 : k0 - kup) + (t & 3) * 8;
     const int Hs = H >> sh, Ws = Wd >> sh;
-    const int sdx = is_in ? -1 : 0, sj = is_in ? 6 : 4;
-    // rows of chunk c this thread stages: the run's first chunk and the first row of a band
-    // stage all three input rows
-    auto stages = [&](int c) { return !is_in || r == 2 || c == c_begin || c % H == 0; };
-    auto fetch = [&](int c) {
-        const int y = c % H, band = c / H;
-        const int b = band / cpr, x0 = (band % cpr) * WG_PX;
-        const int yy = is_in ? y - 1 + r : y;
+    // staging: thread t takes the 8 channels 8 (t & 3) .. + 7 of one pixel a time, 264 pieces an input
+    // row and 256 a gradient row
+    uint4 vin[3], vg[2];
+    auto fetch_in = [&](int b, int x0, int y) __attribute__((always_inline)) {   // input rows y and y + 1
 #pragma unroll
-        for (int j = 0; j < 6; j++) {
-            const int xx = x0 + 4 * q + sdx + j;
-            const bool ok = j < sj && yy >= 0 && yy < H && xx >= 0 && xx < Wd && sco < scs;
+        for (int q = 0; q < 3; q++) {
+            const int e = t + 256 * q, r = e >= 4 * WG_IW ? 1 : 0, px = (e - r * 4 * WG_IW) >> 2;
+            const int yy = y + r, xx = x0 - 1 + px;
+            const bool ok = e < 8 * WG_IW && yy >= 0 && yy < H && xx >= 0 && xx < Wd && sco < scs;
             const size_t o = ok ? (((size_t)b * Hs + (yy >> sh)) * Ws + (xx >> sh)) * scs + sco : 0;
-            v[j] = sel4(ok, *reinterpret_cast<const uint4*>(src + o));
+            vin[q] = sel4(ok, *reinterpret_cast<const uint4*>(src + o));
         }
     };
+    auto store_in = [&](int y) __attribute__((always_inline)) {
+#pragma unroll
+        for (int q = 0; q < 3; q++) {
+            const int e = t + 256 * q, r = e >= 4 * WG_IW ? 1 : 0, px = (e - r * 4 * WG_IW) >> 2;
+            if (e < 8 * WG_IW)
+                *reinterpret_cast<uint4*>(s_in + ((y + r + WG_RING) % WG_RING) * ROW_IN +
+                                          wg_at(px, (t >> 1) & 1, (t & 1) * 2)) = vin[q];
+        }
+    };
+    auto fetch_g = [&](int b, int x0, int y, int nr) __attribute__((always_inline)) {   // gradient rows y and y + 1
+#pragma unroll
+        for (int r = 0; r < 2; r++) {
+            const int xx = x0 + (t >> 2);
+            const bool ok = r < nr && xx < Wd;   // (a second row outside of the run counts as zero)
+            const size_t o = ok ? (((size_t)b * H + y + r) * Wd + xx) * N + n0 + (t & 3) * 8 : 0;
+            vg[r] = sel4(ok, *reinterpret_cast<const uint4*>(g + o));
+        }
+    };
+    auto store_g = [&](int half) __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < 2; r++)
+            *reinterpret_cast<uint4*>(s_g + (half * 2 + r) * ROW_G + wg_at(t >> 2, (t >> 1) & 1, (t & 1) * 2)) = vg[r];
+    };
+    // fragment pieces: pixel 8 kq + 4 i + prow / 4 (+ the tap's shift), channels 4 (prow & 3) .. + 3 of a half
+    int at_in[3][2], at_g[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const int px = ks * 32 + kq * 8 + i * 4 + (prow >> 2);
+#pragma unroll
+        for (int dx = 0; dx < 3; dx++) at_in[dx][i] = wg_at(px + dx, tk, prow & 3);
+#pragma unroll
+        for (int n = 0; n < 2; n++) at_g[n][i] = wg_at(px, n, prow & 3);
+    }
     f32x4 acc[9][2];
 #pragma unroll
     for (int tap = 0; tap < 9; tap++) acc[tap][0] = acc[tap][1] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -378,54 +433,67 @@ __global__ void __launch_bounds__(256, 3) conv3x3_wgrad_lds(const uint16_t* __re
         const uint4 u = make_uint4(o2, o2, o2, o2);
         memcpy(&ones, &u, 16);
     }
-    if (c_begin < c_end && stages(c_begin)) fetch(c_begin);
-    for (int c = c_begin; c < c_end; c++) {
-        const int y = c % H;
-        __syncthreads();   // the previous chunk's fragments are read
-        if (stages(c)) {
-            if (is_in) {
-                const int slot = (y - 1 + r + 3) % 3;
+    // the products of rows y and y + 1: every tap's sum takes the rows in order
+    auto multiply = [&](int y, int half) __attribute__((always_inline)) {
+        bf16x8 bg[2][2];
 #pragma unroll
-                for (int d = 0; d < 3; d++)   // copy d holds pixels 4q + d - 1 + i: v[d + i]
+        for (int s = 0; s < 2; s++)
 #pragma unroll
-                    for (int ch = 0; ch < 8; ch++)
-                        s_in[d][slot][gq * 8 + ch][q] = make_uint2(bf_at(v[d], ch) | (bf_at(v[d + 1], ch) << 16),
-                                                                   bf_at(v[d + 2], ch) | (bf_at(v[d + 3], ch) << 16));
-            } else {
+            for (int n = 0; n < 2; n++) {
+                const char* const row = s_g + (half * 2 + s) * ROW_G;
+                bg[s][n] = wg_frag(row + at_g[n][0], row + at_g[n][1]);
+                if (do_bias) accb[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, bg[s][n], accb[n], 0, 0, 0);
+            }
 #pragma unroll
-                for (int ch = 0; ch < 8; ch++)
-                    s_g[gq * 8 + ch][q] = make_uint2(bf_at(v[0], ch) | (bf_at(v[1], ch) << 16),
-                                                     bf_at(v[2], ch) | (bf_at(v[3], ch) << 16));
+        for (int rr = 0; rr < 4; rr++) {   // input row y - 1 + rr: tap row rr - s of row y + s
+            const char* const row = s_in + ((y + rr + WG_RING - 1) % WG_RING) * ROW_IN;
+#pragma unroll
+            for (int dx = 0; dx < 3; dx++) {
+                const bf16x8 a = wg_frag(row + at_in[dx][0], row + at_in[dx][1]);
+#pragma unroll
+                for (int s = 0; s < 2; s++)
+                    if (rr - s >= 0 && rr - s < 3)
+#pragma unroll
+                        for (int n = 0; n < 2; n++) {
+                            f32x4& d = acc[(rr - s) * 3 + dx][n];
+                            d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bg[s][n], d, 0, 0, 0);
+                        }
             }
         }
-        __syncthreads();
-        if (c + 1 < c_end && stages(c + 1)) fetch(c + 1);
-        bf16x8 bg[2];
-#pragma unroll
-        for (int n = 0; n < 2; n++) {
-            const uint2 lo = s_g[n * 16 + prow][8 * ks + 2 * kq], hi = s_g[n * 16 + prow][8 * ks + 2 * kq + 1];
-            const uint4 u = make_uint4(lo.x, lo.y, hi.x, hi.y);
-            memcpy(&bg[n], &u, 16);
-            if (do_bias) accb[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, bg[n], accb[n], 0, 0, 0);
+    };
+    bool fresh = true;   // the run's first rows, or a band's
+    for (int c = c_begin, half = 0; c < c_end; half ^= 1) {
+        const int y = c % H, band = c / H, b = band / cpr, x0 = (band % cpr) * WG_PX;
+        auto rows = [&](int q) { return c + q + 1 < c_end && y + q + 1 < H ? 2 : 1; };
+        if (fresh) {
+            __syncthreads();   // the previous band's fragments are read
+            fetch_in(b, x0, y - 1);
+            fetch_g(b, x0, y, rows(0));
+            store_in(y - 1);
+            fetch_in(b, x0, y + 1);
+            store_g(half);
+            store_in(y + 1);
+            __syncthreads();
         }
-#pragma unroll
-        for (int tap = 0; tap < 9; tap++) {
-            const int dy = tap / 3, dx = tap % 3;   // copy indices (offset + 1)
-            const int slot = (y - 1 + dy + 3) % 3;
-            const uint2 lo = s_in[dx][slot][tk * 16 + prow][8 * ks + 2 * kq];
-            const uint2 hi = s_in[dx][slot][tk * 16 + prow][8 * ks + 2 * kq + 1];
-            const uint4 u = make_uint4(lo.x, lo.y, hi.x, hi.y);
-            bf16x8 a;
-            memcpy(&a, &u, 16);
-            acc[tap][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bg[0], acc[tap][0], 0, 0, 0);
-            acc[tap][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bg[1], acc[tap][1], 0, 0, 0);
+        const bool more = c + 2 < c_end && y + 2 < H;
+        if (more) {
+            fetch_in(b, x0, y + 3);
+            fetch_g(b, x0, y + 2, rows(2));
         }
+        multiply(y, half);
+        if (more) {   // (these rows' places were last read before the barrier before this)
+            store_in(y + 3);
+            store_g(half ^ 1);
+            __syncthreads();
+        }
+        fresh = !more;
+        c += rows(0);
     }
-    // the second pixel half's sums go through LDS (the input stage, 9 x 2 x 4 floats per lane and
-    // wave, then the bias sums) to the first half's waves, which add them and store the partial
+    // the second pixel half's sums go through LDS (9 x 2 x 4 floats per lane and wave, then the bias
+    // sums) to the first half's waves, which add them and store the partial
     __syncthreads();
-    float* const red = reinterpret_cast<float*>(&s_in[0][0][0][0]);   // 2 x 80 x 64 floats
-    static_assert(sizeof(s_in) >= 2 * 80 * 64 * sizeof(float), "reduction space");
+    float* const red = reinterpret_cast<float*>(lds);   // 2 x 80 x 64 floats
+    static_assert(sizeof(lds) >= 2 * 80 * 64 * sizeof(float), "reduction space");
     if (ks == 1) {
 #pragma unroll
         for (int tap = 0; tap < 9; tap++)
@@ -664,6 +732,10 @@ struct sf_cnn {
 
 namespace sf {
 
+// row tiles that a workgroup of a large launch walks: 1 takes 3.17 ms a step (1024 x 512, batch 4), 2 3.10, 4 and 8
+// 3.04, 16 3.09
+constexpr int CONV_NRT = 4;
+
 static int grid1(int64_t n) {
     int64_t b = (n + 255) / 256;
     return (int)std::max<int64_t>(1, std::min<int64_t>(b, 16384));
@@ -681,7 +753,8 @@ static int cnn_alloc(sf_cnn* c, T** p, size_t n) {
 
 // real input channels and output channels of the layers c1a, c1b, c2a, c2b, c3a, c3b, c4a, c4b, c5a, c5b
 enum { C1A, C1B, C2A, C2B, C3A, C3B, C4A, C4B, C5A, C5B };
-static int conv_init(sf_cnn* c, ConvL& L, std::mt19937_64& rng) {
+// (not inlined: within sf_cnn_create the generator's loop compiles to twice the time, 32 against 18 ms a network)
+__attribute__((noinline)) static int conv_init(sf_cnn* c, ConvL& L, std::mt19937_64& rng) {
     const size_t nw = L.nw();
     if (cnn_alloc(c, &L.wf, nw) || cnn_alloc(c, &L.wt, nw)) return SF_ERR_OOM;
     // He initialisation over the real fan-in; padded input channels stay zero
@@ -712,8 +785,8 @@ template <int MODE>
 static void conv_launch(sf_cnn* c, ConvP p) {
     const int rows = (p.H + CONV_R - 1) / CONV_R, ntn = p.N / CONV_TN;
     p.gx = (p.W + CONV_TP - 1) / CONV_TP;
-    // row tiles per workgroup: up to 4 while the launch keeps at least 1024 workgroups
-    p.nrt = (int)std::max<int64_t>(1, std::min<int64_t>(4, (int64_t)p.gx * rows * p.B * ntn / 1024));
+    // row tiles per workgroup: up to CONV_NRT while the launch keeps at least 1024 workgroups
+    p.nrt = (int)std::max<int64_t>(1, std::min<int64_t>(CONV_NRT, (int64_t)p.gx * rows * p.B * ntn / 1024));
     p.gy = (rows + p.nrt - 1) / p.nrt;
     p.nsp = p.gx * p.gy * p.B;
     hipLaunchKernelGGL(conv3x3_lds<MODE>, dim3((p.nsp + 7) / 8 * 8 * ntn), dim3(256), 0, c->ctx->stream, p);
@@ -725,7 +798,7 @@ static void conv_fwd(sf_cnn* c, int l, const uint16_t* in, int in_cs, uint16_t* 
     const ConvL& L = c->L[l];
     ConvP p = {};
     p.in = in, p.in_cs = in_cs, p.up = up, p.kup = kup, p.K = L.K, p.w = L.wf, p.bias = L.b, p.N = L.N;
-    p.out = out, p.pool = pool, p.H = H, p.W = W, p.B = B, p.sgn = 1;
+    p.out = out, p.pool = pool, p.H = H, p.W = W, p.B = B;
     conv_launch<FWD>(c, p);
 }
 // weight and bias gradients of layer l for the output gradient g: about WG_BLOCKS workgroups over
@@ -750,7 +823,7 @@ static void conv_bwd(sf_cnn* c, int l, const uint16_t* g, const uint16_t* act, u
     const ConvL& L = c->L[l];
     ConvP p = {};
     p.in = g, p.in_cs = L.N, p.K = L.N, p.w = L.wt, p.N = L.K, p.act = act, p.out = out, p.skip = skip, p.nup = nup;
-    p.H = H, p.W = W, p.B = B, p.sgn = -1;
+    p.H = H, p.W = W, p.B = B;
     conv_launch<MODE>(c, p);
 }
 
