@@ -179,6 +179,9 @@ int sf_ctx_destroy(sf_ctx* ctx) {
     for (Species* sp : ctx->species) free_species(sp);
     if (ctx->poisson) poisson_free(ctx->poisson);
     free_mesh(ctx);
+    if (ctx->stage) hipHostFree(ctx->stage);
+    if (ctx->inject_host) hipHostFree(ctx->inject_host);
+    dfree(ctx->inject_acc);
     for (auto& ev : ctx->ev) hipEventDestroy(ev);
     hipStreamDestroy(ctx->stream);
     delete ctx;

@@ -43,6 +43,7 @@ constexpr int NGAS = 10;                        // computeFields outputs kept on
 constexpr int PUSH_FLAG_FAST = 1;               // a velocity beyond the fixed-point fast range: exact slow quantisation
 constexpr int PUSH_FLAG_OVERFLOW = 2;           // a moment contribution beyond the int64 range: moments invalid
 constexpr int PUSH_THREADS = 256;
+constexpr int STAGE_MAX = 16384;                // particles of a batch added through the context's staging
 constexpr int CHUNK = 256;                      // particles staged in LDS per round
 constexpr int CHUNK_STRIDE = 151;               // odd stride of the lane->particle permutation
 // Mover sums are added into STAT_SLOTS copies (by workgroup index) of STAT_STRIDE int64 each, one
@@ -227,6 +228,12 @@ struct sf_ctx {
     float2* d_bf32 = nullptr;   // magnetic field, FP32 like E; allocated only while nonzero
     std::vector<sf::Species*> species;
     std::vector<sf::HostSource> sources;
+    // staging of small particle batches, allocated at the first one and kept: five columns of STAGE_MAX
+    // doubles and STAGE_MAX ids in pinned host memory, which the kernel reads; the accepted count of a
+    // device injection [sum, finished workgroups] and its pinned copy
+    double* stage = nullptr;
+    unsigned long long* inject_acc = nullptr;
+    unsigned long long* inject_host = nullptr;
     uint32_t inject_step = 0;      // batches sampled on the device (counter of their Philox streams)
     int it = 0;                    // TimeModule step (Starfish.getIt()); 0 = not set by the host
     int source_calls = 0;          // sf_sources_sample* calls: the sources' step while `it` is not set
