@@ -424,32 +424,34 @@ struct TileRows {
     uint8_t c[TS::RPT];
     bool in[TS::RPT];
 };
+// row s of the thread from its node's class c and diagonal Dv (unused where the node is not free)
+template <class TS>
+__device__ __forceinline__ void tile_row(const MeshP& m, int s, bool in, uint8_t c, float Dv, int i0, int j0,
+                                         TileRows<TS>& T) {
+    const int li = threadIdx.x % TS::W, lj = threadIdx.x / TS::W + TS::RSTEP * s;
+    const bool free = in && c != CLS_NOT_FREE;
+    T.in[s] = in;
+    T.c[s] = free ? c : CLS_NOT_FREE;
+    T.Dv[s] = free ? Dv : 1.0f;
+    T.cE[s] = T.cW[s] = T.cN[s] = T.cS[s] = 0.0f;
+    if (free) {
+        const Stencil st = stencil(m, i0 + li, j0 + lj);
+        // only free neighbours inside the tile couple
+        T.cE[s] = (nbc(c, 0) == NB_FREE && li + 1 < TS::W) ? (float)st.cE : 0.0f;
+        T.cW[s] = (nbc(c, 1) == NB_FREE && li > 0) ? (float)st.cW : 0.0f;
+        T.cN[s] = (nbc(c, 2) == NB_FREE && lj + 1 < TS::H) ? (float)st.cN : 0.0f;
+        T.cS[s] = (nbc(c, 3) == NB_FREE && lj > 0) ? (float)st.cS : 0.0f;
+    }
+}
 template <class TS>
 __device__ __forceinline__ void tile_rows(const MeshP& m, const uint8_t* __restrict__ cls, const float* __restrict__ D,
                                           int i0, int j0, TileRows<TS>& T) {
-    const int li = threadIdx.x % TS::W;
 #pragma unroll
     for (int s = 0; s < TS::RPT; s++) {
-        const int lj = threadIdx.x / TS::W + TS::RSTEP * s;
-        const int i = i0 + li, j = j0 + lj;
-        T.in[s] = i < m.ni && j < m.nj;
-        T.c[s] = CLS_NOT_FREE;
-        T.Dv[s] = 1.0f;
-        T.cE[s] = T.cW[s] = T.cN[s] = T.cS[s] = 0.0f;
-        if (T.in[s]) {
-            const size_t u = (size_t)j * m.ni + i;
-            const uint8_t c = cls[u];
-            T.c[s] = c;
-            if (c != CLS_NOT_FREE) {
-                const Stencil st = stencil(m, i, j);
-                T.Dv[s] = D[u];
-                // only free neighbours inside the tile couple
-                T.cE[s] = (nbc(c, 0) == NB_FREE && li + 1 < TS::W) ? (float)st.cE : 0.0f;
-                T.cW[s] = (nbc(c, 1) == NB_FREE && li > 0) ? (float)st.cW : 0.0f;
-                T.cN[s] = (nbc(c, 2) == NB_FREE && lj + 1 < TS::H) ? (float)st.cN : 0.0f;
-                T.cS[s] = (nbc(c, 3) == NB_FREE && lj > 0) ? (float)st.cS : 0.0f;
-            }
-        }
+        const int i = i0 + threadIdx.x % TS::W, j = j0 + threadIdx.x / TS::W + TS::RSTEP * s;
+        const bool in = i < m.ni && j < m.nj;
+        const size_t u = in ? (size_t)j * m.ni + i : 0;
+        tile_row<TS>(m, s, in, cls[u], D[u], i0, j0, T);
     }
 }
 // z = M^-1 r on the tile: rs holds r (0 at nodes that are not free or outside the mesh),
@@ -457,8 +459,12 @@ __device__ __forceinline__ void tile_rows(const MeshP& m, const uint8_t* __restr
 template <class TS>
 __device__ __forceinline__ void tile_sgs(const TileRows<TS>& T, int i0, int j0, const float* rs, float* zs) {
     const int li = threadIdx.x % TS::W;
+    float inv[TS::RPT];
 #pragma unroll
-    for (int s = 0; s < TS::RPT; s++) zs[(threadIdx.x / TS::W + TS::RSTEP * s) * TS::W + li] = 0.0f;
+    for (int s = 0; s < TS::RPT; s++) {
+        zs[(threadIdx.x / TS::W + TS::RSTEP * s) * TS::W + li] = 0.0f;
+        inv[s] = 1.0f / T.Dv[s];
+    }
     __syncthreads();
 #pragma unroll
     for (int h = 0; h < 2 * SGS_SWEEPS + 1; h++) {
@@ -468,12 +474,14 @@ __device__ __forceinline__ void tile_sgs(const TileRows<TS>& T, int i0, int j0, 
             const int lj = threadIdx.x / TS::W + TS::RSTEP * s;
             if (((i0 + li + j0 + lj) & 1) != color || T.c[s] == CLS_NOT_FREE || !T.in[s]) continue;
             const int l = lj * TS::W + li;
+            // (a node without a neighbour adds 0 times its own value: no branch around the read)
             float acc = rs[l];
-            if (T.cE[s] != 0.0f) acc += T.cE[s] * zs[l + 1];
-            if (T.cW[s] != 0.0f) acc += T.cW[s] * zs[l - 1];
-            if (T.cN[s] != 0.0f) acc += T.cN[s] * zs[l + TS::W];
-            if (T.cS[s] != 0.0f) acc += T.cS[s] * zs[l - TS::W];
-            zs[l] = acc / T.Dv[s];
+            acc += T.cE[s] * zs[l + (li + 1 < TS::W ? 1 : 0)];
+            acc += T.cW[s] * zs[l - (li > 0 ? 1 : 0)];
+            acc += T.cN[s] * zs[l + (lj + 1 < TS::H ? TS::W : 0)];
+            acc += T.cS[s] * zs[l - (lj > 0 ? TS::W : 0)];
+            const float z = acc * inv[s];   // acc / Dv, corrected by its remainder
+            zs[l] = fmaf(fmaf(-T.Dv[s], z, acc), inv[s], z);
         }
         __syncthreads();
     }
@@ -968,6 +976,35 @@ __global__ void __launch_bounds__(TS::NT) nk_step_a(MeshP m, const uint8_t* __re
                                                  double* __restrict__ ppq, const NkState* __restrict__ state,
                                                  double* __restrict__ nkc, NkParams np, int i) {
     const NkState S = state[(i - 1) % NK_RING];
+    // Bound by latency: a pair is a chain of trips to memory and barriers.  What does not depend on the
+    // decision is loaded before the state is even looked at: the direction's operands here (unused in a
+    // Newton update), the rows of nk_step_b there.  A warm solve of 5 Newton steps and 11 iterations at
+    // 1024 x 512 takes 0.363 ms with that, 0.412 without; 5 and 5 at 81 x 41 0.210 and 0.237.
+    const int nbx = (m.ni + TS::W - 1) / TS::W;
+    const int bx = blockIdx.x % nbx, by = blockIdx.x / nbx;
+    const int i0 = bx * TS::W - 1, j0 = by * TS::H - 1;
+    constexpr int NP = ((TS::H + 2) * (TS::W + 2) + TS::NT - 1) / TS::NT;
+    const float* pold = (i - 1) & 1 ? p_odd : p_even;
+    float zl[NP], pl[NP];
+#pragma unroll
+    for (int k = 0; k < NP; k++) {
+        const int t = threadIdx.x + k * TS::NT;
+        const int ii = i0 + t % (TS::W + 2), jj = j0 + t / (TS::W + 2);
+        const bool in = t < (TS::H + 2) * (TS::W + 2) && ii >= 0 && jj >= 0 && ii < m.ni && jj < m.nj;
+        const size_t u = in ? (size_t)jj * m.ni + ii : 0;
+        zl[k] = z[u];
+        pl[k] = pold[u];
+        if (!in) zl[k] = pl[k] = 0.0f;
+    }
+    uint8_t cl[TS::RPT];
+    float Dl[TS::RPT];
+#pragma unroll
+    for (int s = 0; s < TS::RPT; s++) {
+        const int ii = bx * TS::W + threadIdx.x % TS::W, jj = by * TS::H + threadIdx.x / TS::W + TS::RSTEP * s;
+        const size_t u = ii < m.ni && jj < m.nj ? (size_t)jj * m.ni + ii : 0;
+        cl[s] = cls[u];
+        Dl[s] = D[u];
+    }
     if (S.done) return;
     double cur[2];
     combine_partials<2>((i - 1) & 1 ? pz_odd : pz_even, nbz, cur);
@@ -980,8 +1017,6 @@ __global__ void __launch_bounds__(TS::NT) nk_step_a(MeshP m, const uint8_t* __re
     int code;
     const int act = nk_decide(S, np, cur, code);
     if (act == NK_STOP) return;
-    const int nbx = (m.ni + TS::W - 1) / TS::W;
-    const int bx = blockIdx.x % nbx, by = blockIdx.x / nbx;
     if (act == NK_UPDATE) {
         // x += limited d on the tile's free nodes
         const int li = threadIdx.x % TS::W;
@@ -1001,33 +1036,29 @@ __global__ void __launch_bounds__(TS::NT) nk_step_a(MeshP m, const uint8_t* __re
     }
     float beta = 0.0f;
     if (S.k > 0) beta = (float)(cur[0] / nkc[2 * ((i - 1) % NK_RING)]);   // r.z of pair i-2's partials
-    const float* pold = (i - 1) & 1 ? p_odd : p_even;
     float* pnew = i & 1 ? p_odd : p_even;
     __shared__ float ps[(TS::H + 2) * (TS::W + 2)];
-    const int i0 = bx * TS::W - 1, j0 = by * TS::H - 1;
-    for (int t = threadIdx.x; t < (TS::H + 2) * (TS::W + 2); t += blockDim.x) {
-        const int ii = i0 + t % (TS::W + 2), jj = j0 + t / (TS::W + 2);
-        float v = 0.0f;
-        if (ii >= 0 && jj >= 0 && ii < m.ni && jj < m.nj) {
-            const size_t u = (size_t)jj * m.ni + ii;
-            v = S.k == 0 ? z[u] : z[u] + beta * pold[u];
-        }
-        ps[t] = v;
+#pragma unroll
+    for (int k = 0; k < NP; k++) {
+        const int t = threadIdx.x + k * TS::NT;
+        if (t < (TS::H + 2) * (TS::W + 2)) ps[t] = S.k == 0 ? zl[k] : zl[k] + beta * pl[k];
     }
     __syncthreads();
     const int li = threadIdx.x % TS::W;
     double acc = 0;
-    for (int lj = threadIdx.x / TS::W; lj < TS::H; lj += TS::RSTEP) {
+#pragma unroll
+    for (int s = 0; s < TS::RPT; s++) {
+        const int lj = threadIdx.x / TS::W + TS::RSTEP * s;
         const int ii = i0 + 1 + li, jj = j0 + 1 + lj;
         if (ii >= m.ni || jj >= m.nj) continue;
         const size_t u = (size_t)jj * m.ni + ii;
-        const uint8_t c = cls[u];
+        const uint8_t c = cl[s];
         const int l = (lj + 1) * (TS::W + 2) + (li + 1);
         const float pv = ps[l];
         float qv = 0.0f;
         if (c != CLS_NOT_FREE) {
             const Stencil st = stencil(m, ii, jj);
-            qv = D[u] * pv;
+            qv = Dl[s] * pv;
             if (nbc(c, 0) == NB_FREE) qv -= (float)st.cE * ps[l + 1];
             if (nbc(c, 1) == NB_FREE) qv -= (float)st.cW * ps[l - 1];
             if (nbc(c, 2) == NB_FREE) qv -= (float)st.cN * ps[l + TS::W + 2];
@@ -1058,12 +1089,30 @@ __global__ void __launch_bounds__(TS::NT, TS::MINW) nk_step_b(MeshP m, const uin
     NkState S{0.0, 0.0, 0, 0, 0, 0};
     int act = NK_UPDATE;   // init: compute the residual
     double cur[2] = {0.0, 0.0};
+    const int nbx = (m.ni + TS::W - 1) / TS::W;
+    const int i0 = (blockIdx.x % nbx) * TS::W, j0 = (blockIdx.x / nbx) * TS::H;
+    const int li = threadIdx.x % TS::W;
+    const float* p = i & 1 ? p_odd : p_even;
+    uint8_t cl[TS::RPT];
+    float Dl[TS::RPT], pl[TS::RPT], ql[TS::RPT], dl[TS::RPT], sl[TS::RPT];
     if (!init) {
         S = state[(i - 1) % NK_RING];
-        if (!S.done) {   // the totals nk_step_a of this pair combined
-            cur[0] = nkc[2 * (i % NK_RING)];
-            cur[1] = nkc[2 * (i % NK_RING) + 1];
-        }
+        // the totals nk_step_a of this pair combined (older ones once the solve is done: not used)
+        cur[0] = nkc[2 * (i % NK_RING)];
+        cur[1] = nkc[2 * (i % NK_RING) + 1];
+    }
+#pragma unroll
+    for (int s4 = 0; s4 < TS::RPT; s4++) {   // (see nk_step_a)
+        const int ii = i0 + li, jj = j0 + threadIdx.x / TS::W + TS::RSTEP * s4;
+        const size_t u = ii < m.ni && jj < m.nj ? (size_t)jj * m.ni + ii : 0;
+        cl[s4] = cls[u];
+        Dl[s4] = D[u];
+        pl[s4] = p[u];
+        ql[s4] = q[u];
+        dl[s4] = d[u];
+        sl[s4] = res[u];
+    }
+    if (!init) {
         int code;
         act = nk_decide(S, np, cur, code);
         if (act == NK_STOP) {
@@ -1084,11 +1133,7 @@ __global__ void __launch_bounds__(TS::NT, TS::MINW) nk_step_b(MeshP m, const uin
         combine_partials<1>(ppq, nbq, pq);
         alpha = (float)(cur[0] / pq[0]);
     }
-    const float* p = i & 1 ? p_odd : p_even;
     __shared__ float rs[TS::H * TS::W], zs[TS::H * TS::W];
-    const int nbx = (m.ni + TS::W - 1) / TS::W;
-    const int i0 = (blockIdx.x % nbx) * TS::W, j0 = (blockIdx.x / nbx) * TS::H;
-    const int li = threadIdx.x % TS::W;
     double rr64[TS::RPT] = {};
     float rv[TS::RPT];
     if (act == NK_UPDATE) {
@@ -1100,7 +1145,7 @@ __global__ void __launch_bounds__(TS::NT, TS::MINW) nk_step_b(MeshP m, const uin
             rv[s4] = 0.0f;
             if (ii < m.ni && jj < m.nj) {
                 const size_t u = (size_t)jj * m.ni + ii;
-                const uint8_t c = cls[u];
+                const uint8_t c = cl[s4];
                 d[u] = 0.0f;
                 if (c == CLS_NOT_FREE) {
                     r[u] = 0;
@@ -1116,7 +1161,8 @@ __global__ void __launch_bounds__(TS::NT, TS::MINW) nk_step_b(MeshP m, const uin
                     const double ru = Wu * rho[u] * inv_eps + bfix[u] - Lx - Wu * bx;
                     r[u] = ru;
                     P[u] = Wu * bp;
-                    D[u] = (float)(diagL + Wu * bp);
+                    Dl[s4] = (float)(diagL + Wu * bp);
+                    D[u] = Dl[s4];
                     rv[s4] = (float)ru;
                     res[u] = rv[s4];
                     rr64[s4] = ru;
@@ -1124,10 +1170,11 @@ __global__ void __launch_bounds__(TS::NT, TS::MINW) nk_step_b(MeshP m, const uin
             }
             rs[lj * TS::W + li] = rv[s4];
         }
-        __syncthreads();   // the tile's D values, read by tile_rows below
     }
     TileRows<TS> T;
-    tile_rows<TS>(m, cls, D, i0, j0, T);
+#pragma unroll
+    for (int s4 = 0; s4 < TS::RPT; s4++)
+        tile_row<TS>(m, s4, i0 + li < m.ni && j0 + threadIdx.x / TS::W + TS::RSTEP * s4 < m.nj, cl[s4], Dl[s4], i0, j0, T);
     if (act == NK_PCG) {
 #pragma unroll
         for (int s4 = 0; s4 < TS::RPT; s4++) {
@@ -1135,9 +1182,8 @@ __global__ void __launch_bounds__(TS::NT, TS::MINW) nk_step_b(MeshP m, const uin
             rv[s4] = 0.0f;
             if (T.in[s4]) {
                 const size_t u = (size_t)(j0 + lj) * m.ni + i0 + li;
-                const float pv = p[u], qv = q[u];
-                d[u] = d[u] + alpha * pv;
-                rv[s4] = res[u] - alpha * qv;
+                d[u] = dl[s4] + alpha * pl[s4];
+                rv[s4] = sl[s4] - alpha * ql[s4];
                 res[u] = rv[s4];
                 if (T.c[s4] == CLS_NOT_FREE) rv[s4] = 0.0f;
             }
