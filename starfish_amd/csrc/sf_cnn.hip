@@ -753,12 +753,35 @@ static int cnn_alloc(sf_cnn* c, T** p, size_t n) {
 
 // real input channels and output channels of the layers c1a, c1b, c2a, c2b, c3a, c3b, c4a, c4b, c5a, c5b
 enum { C1A, C1B, C2A, C2B, C3A, C3B, C4A, C4B, C5A, C5B };
-// (not inlined: within sf_cnn_create the generator's loop compiles to twice the time, 32 against 18 ms a network)
-__attribute__((noinline)) static int conv_init(sf_cnn* c, ConvL& L, std::mt19937_64& rng) {
+// Normal deviates by Marsaglia's polar method, the sequence of std::normal_distribution<double> on this
+// generator (compared over 2e7 draws), without the long double logarithms that each of its draws can
+// cost: a network's 480 000 take 7 ms instead of 20 to 35.
+struct PolarNormal {
+    double sigma, kept = 0.0;
+    bool have = false;
+    static double unit(std::mt19937_64& r) {
+        const double u = (double)r() * 0x1p-64;
+        return u < 1.0 ? u : 1.0 - 0x1p-53;
+    }
+    double operator()(std::mt19937_64& r) {
+        have = !have;
+        if (!have) return kept * sigma;
+        double x, y, s;
+        do {
+            x = 2.0 * unit(r) - 1.0;
+            y = 2.0 * unit(r) - 1.0;
+            s = x * x + y * y;
+        } while (s > 1.0 || s == 0.0);
+        const double f = std::sqrt(-2.0 * std::log(s) / s);
+        kept = x * f;
+        return y * f * sigma;
+    }
+};
+static int conv_init(sf_cnn* c, ConvL& L, std::mt19937_64& rng) {
     const size_t nw = L.nw();
     if (cnn_alloc(c, &L.wf, nw) || cnn_alloc(c, &L.wt, nw)) return SF_ERR_OOM;
     // He initialisation over the real fan-in; padded input channels stay zero
-    std::normal_distribution<double> nd(0.0, std::sqrt(2.0 / (9.0 * L.Kreal)));
+    PolarNormal nd{std::sqrt(2.0 / (9.0 * L.Kreal))};
     std::vector<float> h(nw, 0.f);
     for (int tap = 0; tap < 9; tap++)
         for (int n = 0; n < L.N; n++)
@@ -1028,7 +1051,7 @@ int sf_cnn_create(sf_ctx* ctx, int ni, int nj, int max_batch, uint64_t seed, sf_
         delete c;
         return SF_ERR_OOM;
     }
-    std::normal_distribution<double> nd(0.0, std::sqrt(1.0 / C1));
+    PolarNormal nd{std::sqrt(1.0 / C1)};
     std::vector<float> h(C1);
     for (auto& v : h) v = (float)nd(c->rng);
     SF_HIP(ctx, hipMemcpy(c->hw, h.data(), C1 * 4, hipMemcpyHostToDevice));
