@@ -79,6 +79,19 @@ void release_stream(sf_ctx* ctx, uint64_t seed, uint32_t stream_tag) {
 
 }  // namespace sf
 
+namespace sf {
+// [nn] doubles for a field computed on the context's stream and read at once, allocated at the first
+// read and kept with the mesh (an allocation and a free, which waits for the device, took 60 us of each)
+int field_workspace(sf_ctx* ctx, double** out) {
+    if (!ctx->field_out) {
+        const int rc = dalloc(ctx, &ctx->field_out, (size_t)ctx->mp.ni * ctx->mp.nj);
+        if (rc) return rc;
+    }
+    *out = ctx->field_out;
+    return SF_OK;
+}
+}  // namespace sf
+
 extern "C" {
 
 const char* sf_version(void) { return "starfish_hip 0.1 (gfx950)"; }

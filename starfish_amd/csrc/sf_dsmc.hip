@@ -550,7 +550,8 @@ int sf_dsmc_field(sf_dsmc* d, int which, double* out) {
     }
     const int64_t nn = (int64_t)ctx->mp.ni * ctx->mp.nj;
     double* d_out = nullptr;
-    SF_HIP(ctx, hipMalloc((void**)&d_out, nn * 8));
+    const int rc = field_workspace(ctx, &d_out);
+    if (rc) return rc;
     const double inv_samples = d->num_samples > 0 ? 1.0 / d->num_samples : 0.0;
     // fc_nu = real_sum / (num_samples * frequency * dt) (DSMC.java:186-188)
     const double inv_time = 1.0 / (d->num_samples * d->desc.frequency * ctx->dt);
@@ -558,9 +559,8 @@ int sf_dsmc_field(sf_dsmc* d, int which, double* out) {
                        dim3(256), 0, ctx->stream, nn, which, (const double*)d->d_count, (const double*)d->d_real,
                        inv_samples, inv_time, d_out);
     hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = hipMemcpyAsync(out, d_out, nn * 8, hipMemcpyDeviceToHost, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-    if (e == hipSuccess) e = hipMemcpy(out, d_out, nn * 8, hipMemcpyDeviceToHost);
-    hipFree(d_out);
     if (e != hipSuccess) return sf_fail(ctx, SF_ERR_HIP, "sf_dsmc_field: %s", hipGetErrorString(e));
     return SF_OK;
 }

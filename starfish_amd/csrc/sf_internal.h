@@ -234,6 +234,7 @@ struct sf_ctx {
     double* stage = nullptr;
     unsigned long long* inject_acc = nullptr;
     unsigned long long* inject_host = nullptr;
+    double* field_out = nullptr;   // [nn] workspace of the collision fields' reads (field_workspace)
     uint32_t inject_step = 0;      // batches sampled on the device (counter of their Philox streams)
     int it = 0;                    // TimeModule step (Starfish.getIt()); 0 = not set by the host
     int source_calls = 0;          // sf_sources_sample* calls: the sources' step while `it` is not set
@@ -284,6 +285,7 @@ void release_stream(sf_ctx* ctx, uint64_t seed, uint32_t stream_tag);
 int species_alloc_buffers(sf_ctx* ctx, Species* sp);
 int push_deposit(sf_ctx* ctx, Species* sp);
 int sort_species(sf_ctx* ctx, Species* sp);
+int field_workspace(sf_ctx* ctx, double** out);
 int add_particles_device(sf_ctx* ctx, Species* sp, int64_t n, const double* x, const double* y, const double* u,
                          const double* v, const double* w, const int* ids, int mode);
 int noalloc_scratch_init(sf_ctx* ctx);

@@ -394,7 +394,8 @@ int sf_mcc_field(sf_mcc* c, int which, double* out) {
     const int64_t nn = (int64_t)ctx->mp.ni * ctx->mp.nj;
     Species* sp = ctx->species[c->desc.source_species];
     double* d_out = nullptr;
-    SF_HIP(ctx, hipMalloc((void**)&d_out, nn * sizeof(double)));
+    const int rc = field_workspace(ctx, &d_out);
+    if (rc) return rc;
     // the reference divides by the sampling time without a guard (MCC.java:152-153)
     const double inv_samples = c->num_samples > 0 ? 1.0 / c->num_samples : 0.0;
     const double inv_time = 1.0 / (c->time_last - c->time_start);
@@ -402,9 +403,8 @@ int sf_mcc_field(sf_mcc* c, int which, double* out) {
                        (const unsigned long long*)c->d_count, (const double*)c->d_S, (const double*)ctx->d_node_vol,
                        sp->desc.spwt, inv_samples, inv_time, d_out);
     hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = hipMemcpyAsync(out, d_out, nn * sizeof(double), hipMemcpyDeviceToHost, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-    if (e == hipSuccess) e = hipMemcpy(out, d_out, nn * sizeof(double), hipMemcpyDeviceToHost);
-    hipFree(d_out);
     if (e != hipSuccess) return sf_fail(ctx, SF_ERR_HIP, "sf_mcc_field: %s", hipGetErrorString(e));
     return SF_OK;
 }
