@@ -26,7 +26,7 @@ PEAK_HBM_GBS = 8000.0
 BYTES_PUSH = 48.0          # read + write of the 24 B particle state per particle pushed
 BYTES_SCATTER = 48.0       # sort step: read the 24 B pushed state (its cell is the key), write it sorted
 BYTES_STATE = 48.0         # read + write of the 24 B particle state (minimal push + deposit)
-TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "pmc_traffic_push_tile_fast_xy_c2.txt")
+TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "pmc_traffic_push_tile_fast_c2.txt")
 
 
 def measured_bytes_per_particle(kernel):
@@ -522,17 +522,17 @@ def main():
         return nbytes * k[1] / (k[0] * 1e-3) / 1e9 if k[0] > 0 else 0.0
 
     per_launch = k_push[1] / max(1, k_push[2])
-    bpp = measured_bytes_per_particle("push_tile_fast_xy")
+    bpp = measured_bytes_per_particle("push_tile_fast")
     achieved = rate(k_push, BYTES_PUSH)
     roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": PEAK_HBM_GBS, "unit": "GB/s",
                 "frac": round(achieved / PEAK_HBM_GBS, 4),
                 "traffic": round(bpp * per_launch) if bpp else None,
                 "traffic_bytes_per_particle": round(bpp, 2) if bpp else None,
-                "kernel": "push_tile_fast_xy", "bytes_per_particle": BYTES_PUSH,
+                "kernel": "push_tile_fast", "bytes_per_particle": BYTES_PUSH,
                 "particles_per_launch": round(per_launch),
                 "algorithmic_bytes_per_launch": round(BYTES_PUSH * per_launch),
                 "ms_per_launch": round(k_push[0] / max(1, k_push[2]), 4), "launches": k_push[2],
-                "per_kernel_GBs": {"push_tile_fast_xy": round(achieved, 1),
+                "per_kernel_GBs": {"push_tile_fast": round(achieved, 1),
                                    "push_tile_slow": round(rate(k_queue, BYTES_PUSH), 1),
                                    "copy_scatter": round(rate(k_scatter, BYTES_SCATTER), 1)},
                 "slow_particles_per_step": round(k_queue[1] / max(1, k_queue[2])),
