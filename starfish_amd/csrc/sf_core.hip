@@ -179,6 +179,7 @@ static void free_mesh(sf_ctx* c) {
     dfree(c->d_efj);
     dfree(c->d_ef32);
     dfree(c->d_bf32);
+    dfree(c->field_out);
 }
 
 int sf_ctx_destroy(sf_ctx* ctx) {
