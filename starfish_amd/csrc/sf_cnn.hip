@@ -108,6 +108,22 @@ struct ConvP {
     int nrt, gx, gy, nsp;   // row tiles of a workgroup, tiles along x and y, tiles of all images
 };
 
+// 16 bytes a lane from a uniform base (through which no lane reaches below its tensor) and a lane's own byte
+// offset; zeros where the offset is NOWHERE, which lies beyond the range of the resource.  The address
+// arithmetic of a stage is then a few scalar operations and one offset a lane kept for all of them (with
+// the addresses worked out per load, some 200 vector instructions a chunk of 36 MFMAs: 3.06 ms an Adam
+// step at 1024 x 512, batch 4, now 2.82; the weight gradients 780 us of it, now 640).
+constexpr uint32_t NOWHERE = 0x80000000u;
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t uniform_base(const uint16_t* p) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)p, (short)0, 0x7FFFFFFF, 0x00020000);
+}
+__device__ __forceinline__ uint4 load16(__amdgpu_buffer_rsrc_t base, uint32_t off) {
+    const auto v = __builtin_amdgcn_raw_buffer_load_b128(base, off, 0, 0);
+    uint4 r;
+    memcpy(&r, &v, 16);
+    return r;
+}
+
 // lane's neighbour in its pair of lanes (2 q, 2 q + 1): the other pixel of a 2x2 block's row
 __device__ __forceinline__ float pair_lane(float v) {
     int i;
@@ -170,30 +186,46 @@ __global__ void __launch_bounds__(256, 4) conv3x3_lds(const ConvP p) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int prow = lane & 15, kq = lane >> 4;
     uint4 rin[RIN], rwt[RWT];
+    // a lane's byte offsets: its pixels and channel group from pixel (x0 - 1, y0 - 1) of `in`, from the
+    // pixel of `up` that holds it, and its weights from those of channel n0
+    uint32_t oin[RIN], oup[MODE == FWD ? RIN : 1], owt[RWT];
+#pragma unroll
+    for (int q = 0; q < RIN; q++) {
+        const int e = threadIdx.x + 256 * q, g = e & 3, px = (e >> 2) % IW, r = (e >> 2) / IW, xx = x0 - 1 + px;
+        const bool ok = e < NIN && xx >= 0 && xx < Wd;
+        oin[q] = ok && g * 8 < p.in_cs ? (uint32_t)(2 * ((r * Wd + px) * p.in_cs + g * 8)) : NOWHERE;
+        if constexpr (MODE == FWD)   // (x0 and y0 are even: pixel x0 - 1 is the odd one of its pair)
+            oup[q] = ok ? (uint32_t)(2 * ((((r + 1) >> 1) * (Wd >> 1) + ((px + 1) >> 1)) * p.kup + g * 8)) : NOWHERE;
+    }
+#pragma unroll
+    for (int q = 0; q < RWT; q++) {
+        const int e = threadIdx.x + 256 * q, g = e & 3, n = (e >> 2) % TN, tap = (e >> 2) / TN;
+        owt[q] = e < NWT ? (uint32_t)(2 * ((tap * N + n) * p.K + g * 8)) : NOWHERE;
+    }
     auto fetch = [&](int it) __attribute__((always_inline)) {
         const int y0 = y_first + (it / nkc) * R, k0 = (it % nkc) * 32;
-        const bool from_up = k0 < p.kup;
-        const uint16_t* const src = from_up ? p.up : p.in;
-        const int sh = from_up ? 1 : 0, cs = from_up ? p.kup : p.in_cs, kc = from_up ? k0 : k0 - p.kup;
-        const int Hs = H >> sh, Ws = Wd >> sh;
+        const bool from_up = MODE == FWD && k0 < p.kup;
+        const int Hs = H >> 1, Ws = Wd >> 1;
+        const uint16_t* const src =
+            from_up ? p.up + (((int64_t)b * Hs + (y0 >> 1) - 1) * Ws + (x0 >> 1) - 1) * p.kup + k0
+                    : p.in + (((int64_t)b * H + y0 - 1) * Wd + x0 - 1) * p.in_cs + k0 - p.kup;
+        const __amdgpu_buffer_rsrc_t base = uniform_base(src);
+        const uint32_t up_mask = from_up ? ~0u : 0u;
+        const bool edge = y0 == 0 || y0 + R >= H;   // some of the rows y0 - 1 .. y0 + R are outside
 #pragma unroll
         for (int q = 0; q < RIN; q++) {
-            const int e = threadIdx.x + 256 * q;
-            const int g = e & 3, px = (e >> 2) % IW, r = (e >> 2) / IW;
-            const int yy = y0 - 1 + r, xx = x0 - 1 + px;
-            const bool ok = e < NIN && yy >= 0 && yy < H && xx >= 0 && xx < Wd && kc + g * 8 < cs;
-            const size_t o = ok ? (((size_t)b * Hs + (yy >> sh)) * Ws + (xx >> sh)) * cs + kc + g * 8 : 0;
-            rin[q] = sel4(ok, *reinterpret_cast<const uint4*>(src + o));
+            uint32_t o = oin[q];
+            if constexpr (MODE == FWD) o ^= (o ^ oup[q]) & up_mask;   // (a select would be one of addresses, in scratch)
+            if (edge) {
+                const int yy = y0 - 1 + (int)((threadIdx.x + 256 * q) >> 2) / IW;
+                if (yy < 0 || yy >= H) o = NOWHERE;
+            }
+            rin[q] = load16(base, o);
         }
         if (nkc == 1 && it > 0) return;   // (the weights stay)
+        const __amdgpu_buffer_rsrc_t wbase = uniform_base(p.w + (int64_t)n0 * p.K + k0);
 #pragma unroll
-        for (int q = 0; q < RWT; q++) {
-            const int e = threadIdx.x + 256 * q;
-            const int g = e & 3, n = (e >> 2) % TN, tap = (e >> 2) / TN;
-            const bool ok = e < NWT;
-            const size_t o = ok ? ((size_t)tap * N + n0 + n) * p.K + k0 + g * 8 : 0;
-            rwt[q] = sel4(ok, *reinterpret_cast<const uint4*>(p.w + o));
-        }
+        for (int q = 0; q < RWT; q++) rwt[q] = load16(wbase, owt[q]);
     };
     f32x4 acc[R][2];
 #pragma unroll
@@ -328,10 +360,10 @@ __global__ void __launch_bounds__(256, 4) conv3x3_lds(const ConvP p) {
 // tile pairs of a run follow each other on one XCD, and an XCD takes neighbouring runs, so the rows
 // that they share are read from HBM once.
 // Bound by the LDS reads and the MFMAs alike (512 and 576 cycles for two chunks), the first and last
-// layers by HBM.  Measured at 1024 x 512, batch 4: 780 us for the ten layers of a step, against 1480
+// layers by HBM.  Measured at 1024 x 512, batch 4: 640 us for the ten layers of a step, against 1480
 // with rows transposed by two of the four waves as they were stored, three shifted copies of each,
-// and two barriers a chunk; the largest (96 x 32 channels at full resolution) 153 us, 760 TFLOP/s.
-// 158 registers: three workgroups a CU.
+// and two barriers a chunk; the largest (96 x 32 channels at full resolution) 125 us, 930 TFLOP/s.
+// 162 registers: three workgroups a CU.
 // Requirements: K and N multiples of 32, kup too, channel counts in memory multiples of 8.
 constexpr int WG_PX = 64;           // pixels per chunk (two MFMA reduction steps)
 constexpr int WG_IW = WG_PX + 2;    // staged pixels per input row
@@ -373,20 +405,35 @@ __global__ void __launch_bounds__(256, 3) conv3x3_wgrad_lds(const uint16_t* __re
     const int c_begin = run * chunks_per_block;
     const int c_end = min(c_begin + chunks_per_block, nchunks);
     const bool from_up = k0 < kup;
-    const uint16_t* const src = from_up ? up : in;
-    const int sh = from_up ? 1 : 0, scs = from_up ? kup : in_cs, sco = (from_up ? k0 : k0 - kup) + (t & 3) * 8;
+    const uint16_t* const src = (from_up ? up : in) + (from_up ? k0 : k0 - kup);
+    const int sh = from_up ? 1 : 0, scs = from_up ? kup : in_cs;
     const int Hs = H >> sh, Ws = Wd >> sh;
     // staging: thread t takes the 8 channels 8 (t & 3) .. + 7 of one pixel a time, 264 pieces an input
-    // row and 256 a gradient row
+    // row and 256 a gradient row.  Its byte offsets from a band's first pixel are kept for the band: its
+    // pixels of an input row, and its pixel of a gradient row.
     uint4 vin[3], vg[2];
-    auto fetch_in = [&](int b, int x0, int y) __attribute__((always_inline)) {   // input rows y and y + 1
+    uint32_t oin[3], og = NOWHERE;
+    auto band_offsets = [&](int x0) __attribute__((always_inline)) {
 #pragma unroll
         for (int q = 0; q < 3; q++) {
-            const int e = t + 256 * q, r = e >= 4 * WG_IW ? 1 : 0, px = (e - r * 4 * WG_IW) >> 2;
-            const int yy = y + r, xx = x0 - 1 + px;
-            const bool ok = e < 8 * WG_IW && yy >= 0 && yy < H && xx >= 0 && xx < Wd && sco < scs;
-            const size_t o = ok ? (((size_t)b * Hs + (yy >> sh)) * Ws + (xx >> sh)) * scs + sco : 0;
-            vin[q] = sel4(ok, *reinterpret_cast<const uint4*>(src + o));
+            const int e = t + 256 * q, r = e >= 4 * WG_IW ? 1 : 0, px = (e - r * 4 * WG_IW) >> 2, xx = x0 - 1 + px;
+            // (from the pixel before x0, or from the one of `up` that holds it: x0 is even)
+            oin[q] = e < 8 * WG_IW && xx >= 0 && xx < Wd && (t & 3) * 8 < scs
+                         ? (uint32_t)(2 * (((px + sh) >> sh) * scs + (t & 3) * 8)) : NOWHERE;
+        }
+        og = x0 + (t >> 2) < Wd ? (uint32_t)(2 * ((t >> 2) * N + (t & 3) * 8)) : NOWHERE;
+    };
+    auto fetch_in = [&](int b, int x0, int y) __attribute__((always_inline)) {   // input rows y and y + 1
+        const __amdgpu_buffer_rsrc_t base =
+            uniform_base(src + (((int64_t)b * Hs + (y >> sh)) * Ws + (x0 >> sh) - 1) * scs);
+        const uint32_t step = (uint32_t)(2 * (((y + 1) >> sh) - (y >> sh)) * Ws * scs);   // to the second row
+        const bool ok0 = y >= 0 && y < H, ok1 = y + 1 >= 0 && y + 1 < H;
+#pragma unroll
+        for (int q = 0; q < 3; q++) {
+            const bool second = t + 256 * q >= 4 * WG_IW;
+            uint32_t o = oin[q] + (second ? step : 0u);   // (NOWHERE stays beyond the range)
+            if (!(second ? ok1 : ok0)) o = NOWHERE;
+            vin[q] = load16(base, o);
         }
     };
     auto store_in = [&](int y) __attribute__((always_inline)) {
@@ -400,12 +447,8 @@ __global__ void __launch_bounds__(256, 3) conv3x3_wgrad_lds(const uint16_t* __re
     };
     auto fetch_g = [&](int b, int x0, int y, int nr) __attribute__((always_inline)) {   // gradient rows y and y + 1
 #pragma unroll
-        for (int r = 0; r < 2; r++) {
-            const int xx = x0 + (t >> 2);
-            const bool ok = r < nr && xx < Wd;   // (a second row outside of the run counts as zero)
-            const size_t o = ok ? (((size_t)b * H + y + r) * Wd + xx) * N + n0 + (t & 3) * 8 : 0;
-            vg[r] = sel4(ok, *reinterpret_cast<const uint4*>(g + o));
-        }
+        for (int r = 0; r < 2; r++)   // (a second row outside of the run counts as zero)
+            vg[r] = load16(uniform_base(g + (((int64_t)b * H + y + r) * Wd + x0) * N + n0), r < nr ? og : NOWHERE);
     };
     auto store_g = [&](int half) __attribute__((always_inline)) {
 #pragma unroll
@@ -467,6 +510,7 @@ __global__ void __launch_bounds__(256, 3) conv3x3_wgrad_lds(const uint16_t* __re
         auto rows = [&](int q) { return c + q + 1 < c_end && y + q + 1 < H ? 2 : 1; };
         if (fresh) {
             __syncthreads();   // the previous band's fragments are read
+            band_offsets(x0);
             fetch_in(b, x0, y - 1);
             fetch_g(b, x0, y, rows(0));
             store_in(y - 1);
