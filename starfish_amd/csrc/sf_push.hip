@@ -2151,9 +2151,9 @@ int add_particles_device(sf_ctx* ctx, Species* sp, int64_t n, const double* x, c
     const MeshP& m = ctx->mp;
     const double xd0 = m.x0[0] + (m.ni - 1) * m.dh[0], xd1 = m.x0[1] + (m.nj - 1) * m.dh[1];
     // A batch of up to STAGE_MAX (a source's, step by step) is written to the context's pinned columns,
-    // which the kernel reads over the link: at 81 x 41 a step's sources take 61 us with
-    // their sampling instead of 84 with device memory allocated, filled from pageable memory and freed.  Larger ones (a load) are
-    // copied.
+    // which the kernel reads over the link: at 81 x 41 a step's sources take 61 us with their sampling,
+    // instead of 84 with device memory allocated, filled from pageable memory and freed.  Larger ones (a
+    // load) are copied.
     const bool staged = n <= STAGE_MAX;
     if (staged && !ctx->stage)
         SF_HIP(ctx, hipHostMalloc((void**)&ctx->stage, (size_t)STAGE_MAX * (5 * sizeof(double) + sizeof(int32_t))));
