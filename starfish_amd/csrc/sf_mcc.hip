@@ -244,6 +244,7 @@ struct sf_mcc {
     unsigned long long* d_count = nullptr;
     double* d_S = nullptr;
     unsigned long long* d_ncol = nullptr;
+    unsigned long long* h_ncol = nullptr;   // pinned: the pass's count without a staged copy
     unsigned int* d_bound = nullptr;     // [4] bounds of the target's density and velocity (mcc_target_bounds)
     bool have_target = false;
     int num_samples = 0;
@@ -293,6 +294,7 @@ int sf_mcc_create(sf_ctx* ctx, const sf_mcc_desc* desc, sf_mcc** out) {
     if (e == hipSuccess) e = hipMalloc((void**)&c->d_count, nn * sizeof(unsigned long long));
     if (e == hipSuccess) e = hipMalloc((void**)&c->d_S, nn * sizeof(double));
     if (e == hipSuccess) e = hipMalloc((void**)&c->d_ncol, sizeof(unsigned long long));
+    if (e == hipSuccess) e = hipHostMalloc((void**)&c->h_ncol, sizeof(unsigned long long));
     if (e == hipSuccess) e = hipMalloc((void**)&c->d_bound, 4 * sizeof(unsigned int));
     if (e == hipSuccess) e = hipMemset(c->d_target, 0, 5 * nn * sizeof(double));
     if (e == hipSuccess) e = hipMemset(c->d_count, 0, nn * sizeof(unsigned long long));
@@ -302,6 +304,7 @@ int sf_mcc_create(sf_ctx* ctx, const sf_mcc_desc* desc, sf_mcc** out) {
         hipFree(c->d_count);
         hipFree(c->d_S);
         hipFree(c->d_ncol);
+        hipHostFree(c->h_ncol);
         hipFree(c->d_bound);
         delete c;
         release_stream(ctx, desc->seed, stream_tag);
@@ -319,6 +322,7 @@ int sf_mcc_destroy(sf_mcc* c) {
     hipFree(c->d_count);
     hipFree(c->d_S);
     hipFree(c->d_ncol);
+    hipHostFree(c->h_ncol);
     hipFree(c->d_bound);
     release_stream(c->ctx, c->desc.seed, c->stream_tag);
     delete c;
@@ -379,10 +383,9 @@ int sf_mcc_perform(sf_mcc* c, int it, double time, int64_t* collisions) {
                            (const unsigned int*)c->d_bound, c->d_count, c->d_S, c->d_ncol);
         SF_HIP(ctx, hipGetLastError());
     }
-    unsigned long long n = 0;
-    SF_HIP(ctx, hipMemcpyAsync(&n, c->d_ncol, sizeof(n), hipMemcpyDeviceToHost, ctx->stream));
+    SF_HIP(ctx, hipMemcpyAsync(c->h_ncol, c->d_ncol, sizeof(unsigned long long), hipMemcpyDeviceToHost, ctx->stream));
     SF_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    if (collisions) *collisions = (int64_t)n;
+    if (collisions) *collisions = (int64_t)*c->h_ncol;
     return SF_OK;
 }
 
