@@ -879,9 +879,9 @@ __global__ void __launch_bounds__(PUSH_THREADS, 4) push_tile_fast(FastC fc, cons
                     sp0 += qbits(1.0, (double)vxn * fc.kst);
                     sp1 += qbits(1.0, (double)vyn * fc.kst);
                     sp2 += qbits(1.0, (double)vzn * fc.kst);
-                    if (F32) {
+                    if (!longer) {
                         se += qbits(1.0, (double)sqrtf(vxn * vxn + vyn * vyn + vzn * vzn) * fc.kst);
-                    } else {
+                    } else {   // (an FP64 move's speed is FP64 as well, as in stat_add)
                         const double a0 = vxn, a1 = vyn, a2 = vzn;
                         se += qbits(1.0, sqrt(a0 * a0 + a1 * a1 + a2 * a2) * fc.kst);
                     }

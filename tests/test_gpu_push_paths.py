@@ -72,3 +72,31 @@ def test_fast_push_matches_the_general_kernel(domain, b, n, ni, nj):
     for k in f0:
         assert np.abs(f0[k] - f1[k]).max() <= 1e-5 * max(np.abs(f0[k]).max(), 1e-300) * (20 if k == "t" else 1), k
     assert np.allclose(t0, t1, rtol=1e-6)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("v", [(12345.678, 3210.987, 777.77), (-10001.3, 17003.1, -2.5), (19000.7, -19000.7, 5000.9)])
+def test_speed_sum_of_long_moves_is_double_precision(v):
+    """The mover's speed sum of particles that move one to two cells a step, whose move the tile kernel
+    evaluates in FP64: their speed is FP64 too, as in the reference loop.  Every particle has the same
+    FP32 velocity, so a rounding of its speed to FP32 would not average out.  Bound: a contribution is
+    rounded to a fixed-point quantum of at most 2 vmax 2^-40, half of that off, next to FP64's own."""
+    from starfish_amd.plugin import Simulation
+    vmax, n = 4e4, 3000
+    mesh = D.MeshSpec("XY", 131, 70, (0.0, 0.0), (1e-3, 1e-3), {f: ("SYMMETRY", 0.0) for f in D.FACES})
+    mat = D.MaterialSpec("O+", "kinetic_hip", 16.0, 1.0, 1e4, 0.0)
+    sim = Simulation(D.Deck(mesh, materials=[mat], solver=None, num_it=1, dt=1e-7, seed=1), capacity=n, vmax=vmax)
+    try:
+        rng = np.random.default_rng(3)
+        v = np.array(v, np.float32).astype(np.float64)
+        x, y = 1e-3 * rng.uniform(40, 90, n), 1e-3 * rng.uniform(20, 50, n)
+        sim.materials[0].add_particles(x, y, *[np.full(n, c) for c in v], rewind=False)
+        for _ in range(3):   # the first push is of an unsorted population, by the reference loop
+            sim.materials[0].update()
+            s = sim.materials[0].stats()
+            speed = np.sqrt((v * v).sum())
+            err = abs(s[4] / s[0] / speed - 1)
+            print("speed sum off by %.1e" % err, flush=True)
+            assert err <= vmax / speed * 2.0 ** -40 + 1e-14
+    finally:
+        sim.close()
