@@ -614,6 +614,7 @@ static_assert(MG_W * MG_H == 4 * MG_NT, "one thread per 2 x 2 aggregate");
 // The first linear solve of a cold solve shows it too (56 iterations at 1e-3 on the 1024 x 512 cylinder
 // deck, 184 on the RZ mesh; 13 at 256 x 128, where the tiles stay the better choice: 2.4 ms).
 constexpr int MG_SWITCH = 16;
+constexpr int MG_LOOSE_STEPS = 32;       // Newton steps of a solve that may use ETA_MG
 constexpr int64_t MG_MIN_NODES = 1024;   // below, a few tiles are the whole mesh
 
 struct MgLevel {
@@ -1810,6 +1811,11 @@ int poisson_solve(sf_ctx* ctx, sf_solve_info* info) {
         return fin.done;
     };
     const double eta_warm = P->wide_tiles ? ETA_WARM : ETA_WARM_LARGE;
+    // ETA_MG costs a cold solve two to four more Newton steps.  A solve that may stop on its step norm
+    // would stop that much further from its solution (RZ 1024 x 512, nl_tol 1e-6: 3.8e-4 V instead of
+    // 1.2e-4), and one whose steps are few would run out of them (nl_max_it 12 there), so the term holds
+    // where only the residual stops the solve, and for the first half of an ample number of steps.
+    const bool loose_ok = !(nl_tol > 0) && nl_max >= MG_LOOSE_STEPS;
     int rc = 0;
     // the last solve converged and this one starts from its potential: go straight to the device
     // loop (it hands a cold start back untouched)
@@ -1869,7 +1875,6 @@ int poisson_solve(sf_ctx* ctx, sf_solve_info* info) {
             eta = rel < 0.5 ? eta_warm : ETA_COLD;
             eta_chosen = true;
             warm = rel < 0.5;
-            if (mg) eta = ETA_MG;
         }
         if (it == 0 && rel < 0.5 && device_ok && !mg) {
             const int code = device_newton(eta);
@@ -1877,14 +1882,14 @@ int poisson_solve(sf_ctx* ctx, sf_solve_info* info) {
             if (code != NK_COLD && code != NK_SLOW) break;
             if (code == NK_SLOW) {
                 mg = true;
-                eta = ETA_MG;
                 it = newton - 1;
                 continue;   // the residual of the updated x
             }
         }
         newton++;
         // inexact Newton: solve J y = r to max(eta*||r||, 0.5*tol*ref) with FP32 PCG + FP64 refinement
-        double lin_target = std::max(D.linear ? 0.5 * rel_tol * ref : eta * rnorm, 0.5 * rel_tol * ref);
+        const double eta_it = mg && loose_ok && 2 * it < nl_max ? ETA_MG : eta;
+        double lin_target = std::max(D.linear ? 0.5 * rel_tol * ref : eta_it * rnorm, 0.5 * rel_tol * ref);
         int refine = 0;
         bool stepped = false;   // the update and the next residual ran behind the linear solve
         while (true) {
@@ -1978,7 +1983,6 @@ int poisson_solve(sf_ctx* ctx, sf_solve_info* info) {
                     // the same linear solve from its current residual and correction, conjugate
                     // directions started anew
                     mg = true;
-                    if (!D.linear) eta = ETA_MG;   // of the Newton steps after this one
                     before = k;
                     k = 0;
                     batch = 4;

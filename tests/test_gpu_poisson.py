@@ -305,3 +305,77 @@ def test_multigrid_solves_a_thin_plasma(ni, nj, ratio):
             assert info.pcg_iterations <= 8 * info.newton_iterations
     finally:
         sim.close()
+
+
+def _thin_rz_deck(ni=128, nj=100):
+    """A plasma with a Debye length of a quarter of the mesh and -200 V on one end: a cold solve takes a
+    dozen Newton steps and goes over to the multigrid in the first."""
+    mesh = D.MeshSpec("RZ", ni, nj, (0.0, 0.0), (1e-4, 1e-4),
+                      {"LEFT": ("SYMMETRY", 0.0), "BOTTOM": ("DIRICHLET", 0.0), "TOP": ("DIRICHLET", -200.0)})
+    y, x = np.mgrid[0:nj, 0:ni]
+    rho = QE * 1e12 * (1 + 0.4 * np.cos(6.0 * x / ni + 1) * np.cos(5.0 * y / nj)).ravel()
+    deck = D.Deck(mesh, materials=[D.MaterialSpec("Xe+", "kinetic_hip", 131.0, 1.0, 1e4, 0.0)],
+                  solver=D.SolverSpec("poisson_hip", "PCG", False, 1e12, 2.0, 0.0), num_it=1, dt=1e-8, seed=1)
+    return deck, rho
+
+
+def _cold_solve(deck, rho):
+    import ctypes as C
+    from starfish_amd import _lib
+    from starfish_amd.plugin import Simulation, _dp
+    sim = Simulation(deck, capacity=16)
+    try:
+        sim.ctx.call("sf_rho_set", _dp(rho))
+        info = _lib.SolveInfo()
+        return sim.ctx.call("sf_poisson_solve", None, C.byref(info)), info
+    finally:
+        sim.close()
+
+
+@pytest.mark.gpu
+def test_multigrid_keeps_within_few_newton_steps():
+    """A solve whose nl_max_it leaves one step more than Newton's method with linear solves to 1e-3 of the
+    residual and the same step limit takes converges: the looser term of an ample nl_max_it is not used
+    there.  The steps are counted here with a direct solver and 0.999 of its solution, whose linear
+    residual is 1e-3 of the right-hand side."""
+    deck, rho = _thin_rz_deck()
+    geo, st = geometry(deck)
+    A = oracle_for(deck, geo, st).operator(0).tocsr()
+    ni, nj, kTe = deck.mesh.ni, deck.mesh.nj, deck.solver.Te0
+    I, J = np.arange(ni * nj) % ni, np.arange(ni * nj) // ni
+    fixed = (J == 0) | (J == nj - 1)
+    face = ((I == 0) | (I == ni - 1)) & ~fixed
+    x, norm = np.where(J == nj - 1, -200.0, 0.0), []
+    for steps in range(40):
+        bx = np.where(fixed | face, 0.0, QE / EPS0 * 1e12 * np.exp(x / kTe))
+        F = A @ x - np.where(fixed, np.where(J == nj - 1, -200.0, 0.0), np.where(face, 0.0, bx - rho / EPS0))
+        norm.append(np.linalg.norm(F[~fixed] * np.maximum(I[~fixed], 0.25)))   # rows weighted with their volume
+        if norm[-1] <= 1e-8 * norm[0]:
+            break
+        y = -0.999 * spla.spsolve((A - sps.diags(bx / kTe)).tocsc(), F)
+        x = x + np.where(y > kTe, kTe * (1 + np.log(np.maximum(y, kTe) / kTe)), np.maximum(y, -10 * kTe))
+    deck.solver.nl_max_it = steps + 1
+    rc, info = _cold_solve(deck, rho)
+    print("reference %d steps, device %d, pcg %d, rel %.1e" % (steps, info.newton_iterations, info.pcg_iterations,
+                                                                  info.rel_residual), flush=True)
+    assert 8 <= steps <= 16
+    assert rc == 0 and info.rel_residual <= 1e-8
+
+
+@pytest.mark.gpu
+def test_multigrid_under_the_step_norm_stop():
+    """A cold solve that nl_tol stops has solved its last step as tightly as the tile path does, to 1e-3
+    of the residual.  The residual after a step y is the linear solve's plus the second-order term
+    W b(x) y^2 / (2 kTe^2), at most max|y| / (2 kTe) of J y; the stop bounds max|y| <= nl_tol N.  So from
+    the step before last to the last the residual falls to 1e-3 + nl_tol N / (2 kTe) of it, next to the
+    half of rel_tol at which a linear solve ends anyway."""
+    deck, rho = _thin_rz_deck()
+    deck.solver.nl_tol, deck.solver.nl_tol_set = 1e-5, True
+    rc, last = _cold_solve(deck, rho)
+    assert rc == 0
+    deck.solver.nl_max_it = last.newton_iterations - 1
+    rc, before = _cold_solve(deck, rho)
+    print("rel %.2e after %d steps, %.2e after %d" % (before.rel_residual, before.newton_iterations, last.rel_residual,
+                                                      last.newton_iterations), flush=True)
+    assert rc == 1 and before.newton_iterations == last.newton_iterations - 1
+    assert last.rel_residual <= (1e-3 + 1e-5 * len(rho) / 4.0) * before.rel_residual + 0.5e-8
