@@ -613,7 +613,10 @@ static_assert(MG_W * MG_H == 4 * MG_NT, "one thread per 2 x 2 aggregate");
 // needs 3 to 6: past 16 the switch pays however long the linear solve would have been.
 // The first linear solve of a cold solve shows it too (56 iterations at 1e-3 on the 1024 x 512 cylinder
 // deck, 184 on the RZ mesh; 13 at 256 x 128, where the tiles stay the better choice: 2.4 ms).
-constexpr int MG_SWITCH = 16;
+// The host's loop (cold and linear solves) looks after MG_SWITCH_HOST: the tiles' cheap iterations still
+// gain there (a switch after 17 made the cold solve 0.2 ms longer), and the count is the same whatever
+// batches the solves before have left.
+constexpr int MG_SWITCH = 16, MG_SWITCH_HOST = 24;
 constexpr int MG_LOOSE_STEPS = 32;       // Newton steps of a solve that may use ETA_MG
 constexpr int64_t MG_MIN_NODES = 1024;   // below, a few tiles are the whole mesh
 
@@ -1822,11 +1825,13 @@ int poisson_solve(sf_ctx* ctx, sf_solve_info* info) {
     bool device_done = false;
     // A solve goes on with the multigrid preconditioner once a linear solve has taken MG_SWITCH
     // iterations; the next warm solve then starts with it, until it needs no more than one iteration
-    // per Newton step.
-    bool mg = P->mg_hint && P->warm_hint;
+    // per Newton step.  Whether a solve is warm shows in its first residual: a cold one takes the same
+    // path whatever was solved before.
+    const bool hinted = P->mg_hint && P->warm_hint;
+    bool mg = false;
     int mg_its = 0, mg_steps = 0;
     bool warm = true;
-    if (device_ok && P->warm_hint && !mg) {
+    if (device_ok && P->warm_hint && !hinted) {
         const int code = device_newton(eta_warm);
         if (code < 0) return code;
         device_done = code != NK_COLD && code != NK_SLOW;
@@ -1875,6 +1880,7 @@ int poisson_solve(sf_ctx* ctx, sf_solve_info* info) {
             eta = rel < 0.5 ? eta_warm : ETA_COLD;
             eta_chosen = true;
             warm = rel < 0.5;
+            if (hinted && warm) mg = true;
         }
         if (it == 0 && rel < 0.5 && device_ok && !mg) {
             const int code = device_newton(eta);
@@ -1931,7 +1937,9 @@ int poisson_solve(sf_ctx* ctx, sf_solve_info* info) {
             int before = 0;   // tile-preconditioned iterations before a switch to the multigrid
             bool first_batch = true, done_in_first = false;
             while (true) {
-                const int nb = std::min(batch, max_it - before - k);
+                int nb = std::min(batch, max_it - before - k);
+                // (the host looks there, whatever batches the last solve left)
+                if (!mg && P->nlev > 1 && k < MG_SWITCH_HOST) nb = std::min(nb, MG_SWITCH_HOST - k);
                 for (int b = 0; b < nb; b++, k++) {
                     double* cur = (k & 1) ? pz1 : pz0;
                     double* nxt = (k & 1) ? pz0 : pz1;
@@ -1979,7 +1987,7 @@ int poisson_solve(sf_ctx* ctx, sf_solve_info* info) {
                 if (before + k >= max_it) { its = k; break; }
                 batch = std::min(2 * batch, mg ? 8 : 64);
                 first_batch = false;
-                if (!mg && P->nlev > 1 && k >= MG_SWITCH) {
+                if (!mg && P->nlev > 1 && k >= MG_SWITCH_HOST) {
                     // the same linear solve from its current residual and correction, conjugate
                     // directions started anew
                     mg = true;
@@ -2033,7 +2041,7 @@ int poisson_solve(sf_ctx* ctx, sf_solve_info* info) {
     }
     }   // !device_done
     P->warm_hint = converged;
-    if (mg && warm) P->mg_hint = mg_its > mg_steps;
+    if (mg_steps > 0 && warm) P->mg_hint = mg_its > mg_steps;   // (a solve without a step tells nothing)
     if (!device_done) {   // (the device loop expanded phi and recorded its end with its last batch)
         hipLaunchKernelGGL(expand_phi, dim3(ge), dim3(256), 0, st, nn, (const int32_t*)P->src,
                            (const double*)P->fixval, (const double*)P->x, ctx->d_phi, (const NkState*)nullptr,

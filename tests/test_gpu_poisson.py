@@ -379,3 +379,40 @@ def test_multigrid_under_the_step_norm_stop():
                                                       last.newton_iterations), flush=True)
     assert rc == 1 and before.newton_iterations == last.newton_iterations - 1
     assert last.rel_residual <= (1e-3 + 1e-5 * len(rho) / 4.0) * before.rel_residual + 0.5e-8
+
+
+@pytest.mark.gpu
+def test_solves_do_not_depend_on_what_was_solved_before():
+    """A cold solve in a context that has solved warm with the multigrid repeats the fresh context's, bit
+    for bit and in its counts; a solve that is converged at its first residual does not send the next warm
+    one back to the tiles, whose 16 iterations it would discard."""
+    import ctypes as C
+    from starfish_amd import _lib
+    from starfish_amd.plugin import Simulation, _dp
+    deck, rho = _thin_rz_deck(301, 157)
+    ni, nj = deck.mesh.ni, deck.mesh.nj
+    y, x = np.mgrid[0:nj, 0:ni]
+    rhos = [rho * (1 + 0.03 * np.cos(4.0 * x / ni + q) * np.sin(7.0 * y / nj)).ravel() for q in range(3)]
+    sim = Simulation(deck, capacity=16)
+
+    def solve(r, start=None):
+        info = _lib.SolveInfo()
+        sim.ctx.call("sf_rho_set", _dp(r))
+        if start is not None:
+            sim.ctx.call("sf_phi_set", _dp(start))
+        assert sim.ctx.call("sf_poisson_solve", None, C.byref(info)) == 0
+        print("newton", info.newton_iterations, "pcg", info.pcg_iterations, flush=True)
+        return info.newton_iterations, info.pcg_iterations
+
+    try:
+        zero = np.zeros(ni * nj)
+        first, phi = solve(rho, zero), sim.phi()
+        for r in rhos[:2]:
+            solve(r)
+        assert solve(rhos[1]) == (0, 0)
+        newton, pcg = solve(rhos[2])
+        assert 0 < pcg <= 8 * newton < 16 + newton
+        assert solve(rho, zero) == first
+        assert np.array_equal(sim.phi(), phi)
+    finally:
+        sim.close()
