@@ -702,7 +702,7 @@ int sf_mesh_segment_boundaries(sf_ctx* ctx, int nseg, const int* seg_bnd, int nb
         dfree(sp->bnd_hits);
         if (nbnd > 0) {
             TRY(dalloc(ctx, &sp->bnd_hits, (size_t)nbnd));
-            SF_HIP(ctx, hipMemset(sp->bnd_hits, 0, nbnd * sizeof(unsigned long long)));
+            SF_HIP(ctx, hipMemsetAsync(sp->bnd_hits, 0, nbnd * sizeof(unsigned long long), ctx->stream));
         }
     }
     return SF_OK;

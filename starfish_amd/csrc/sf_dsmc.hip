@@ -454,9 +454,9 @@ int sf_dsmc_create(sf_ctx* ctx, const sf_dsmc_desc* desc, sf_dsmc** out) {
     if (e == hipSuccess) e = hipMalloc((void**)&d->d_ncol, 8);
     if (e == hipSuccess) e = hipMalloc((void**)&d->d_overflow, 4);
     if (e == hipSuccess) e = hipMemcpy(d->d_scm, scm.data(), nc * 8, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemset(d->d_rem, 0, nc * 8);
-    if (e == hipSuccess) e = hipMemset(d->d_count, 0, nn * 8);
-    if (e == hipSuccess) e = hipMemset(d->d_real, 0, nn * 8);
+    if (e == hipSuccess) e = hipMemsetAsync(d->d_rem, 0, nc * 8, ctx->stream);
+    if (e == hipSuccess) e = hipMemsetAsync(d->d_count, 0, nn * 8, ctx->stream);
+    if (e == hipSuccess) e = hipMemsetAsync(d->d_real, 0, nn * 8, ctx->stream);
     if (e != hipSuccess) {
         hipFree(d->d_scm);
         hipFree(d->d_rem);

@@ -296,9 +296,9 @@ int sf_mcc_create(sf_ctx* ctx, const sf_mcc_desc* desc, sf_mcc** out) {
     if (e == hipSuccess) e = hipMalloc((void**)&c->d_ncol, sizeof(unsigned long long));
     if (e == hipSuccess) e = hipHostMalloc((void**)&c->h_ncol, sizeof(unsigned long long));
     if (e == hipSuccess) e = hipMalloc((void**)&c->d_bound, 4 * sizeof(unsigned int));
-    if (e == hipSuccess) e = hipMemset(c->d_target, 0, 5 * nn * sizeof(double));
-    if (e == hipSuccess) e = hipMemset(c->d_count, 0, nn * sizeof(unsigned long long));
-    if (e == hipSuccess) e = hipMemset(c->d_S, 0, nn * sizeof(double));
+    if (e == hipSuccess) e = hipMemsetAsync(c->d_target, 0, 5 * nn * sizeof(double), ctx->stream);
+    if (e == hipSuccess) e = hipMemsetAsync(c->d_count, 0, nn * sizeof(unsigned long long), ctx->stream);
+    if (e == hipSuccess) e = hipMemsetAsync(c->d_S, 0, nn * sizeof(double), ctx->stream);
     if (e != hipSuccess) {
         hipFree(c->d_target);
         hipFree(c->d_count);
@@ -337,10 +337,12 @@ int sf_mcc_set_target(sf_mcc* c, const double* den, const double* u, const doubl
     SF_HIP(ctx, hipSetDevice(ctx->device));
     const size_t nn = (size_t)ctx->mp.ni * ctx->mp.nj;
     SF_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    // (the copies wait for the device; the clears follow on the context's stream, which the bounds and the
+    // next pass run on: a clear on the null stream would not be ordered before them)
     const double* src[5] = {den, u, v, w, temp};
     for (int k = 0; k < 5; k++) {
         if (src[k]) SF_HIP(ctx, hipMemcpy(c->d_target + k * nn, src[k], nn * sizeof(double), hipMemcpyHostToDevice));
-        else SF_HIP(ctx, hipMemset(c->d_target + k * nn, 0, nn * sizeof(double)));
+        else SF_HIP(ctx, hipMemsetAsync(c->d_target + k * nn, 0, nn * sizeof(double), ctx->stream));
     }
     SF_HIP(ctx, hipMemsetAsync(c->d_bound, 0, 4 * sizeof(unsigned int), ctx->stream));
     hipLaunchKernelGGL(mcc_target_bounds, dim3(grid_n((int64_t)nn, 128)), dim3(256), 0, ctx->stream, (int64_t)nn,

@@ -167,3 +167,35 @@ def test_mcc_queue_edges_match_oracle(n, scale):
         if mcc is not None:
             mcc.close()
         sim.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("given", [(), ("u",), ("u", "v"), ("temp",)])
+def test_fields_left_out_of_a_new_target_are_zero_in_the_next_pass(given):
+    """A target set after another one, with trailing fields left out: the pass right behind it sees zeros
+    there and nothing of the target before.  At this density every ion collides, and charge exchange
+    with a gas at 0 K gives it exactly the gas's velocity, one of the given fields (a constant, which the
+    gather returns within its own rounding, 4 x 2^-53, far below the FP32 of the stored velocity)."""
+    from starfish_amd.interactions import MccHip
+    from starfish_amd.plugin import Simulation
+    mesh = D.MeshSpec("XY", 1025, 769, (0.0, 0.0), (1e-3, 1e-3), {})
+    deck = D.Deck(mesh, materials=[D.MaterialSpec("Xe+", "kinetic_hip", 131.0, 1.0, 1e7, 0.0)], solver=None, num_it=1,
+                  dt=1e-6, seed=0)
+    sim = Simulation(deck, capacity=4096, track_ids=True)
+    mcc = None
+    try:
+        mat = sim.materials[0]
+        mat.preload(4000, (300.0, 200.0, 100.0), 1000.0, seed=2)
+        mcc = MccHip(sim, mat, "CEX", 5e-19, 131.0, seed=5)
+        mcc.set_target(1e26, u=5000.0, v=6000.0, w=7000.0, temp=1e6)
+        assert mcc.perform(1, 0.0) == 4000
+        value = {"u": 10.0, "v": 20.0, "temp": 0.0}
+        mcc.set_target(1e26, **{k: value[k] for k in given})
+        assert mcc.perform(2, 1e-6) == 4000
+        p = mat.particles()
+        for k in ("u", "v", "w"):
+            assert np.all(p[k] == (value[k] if k in given else 0.0)), k
+    finally:
+        if mcc is not None:
+            mcc.close()
+        sim.close()
