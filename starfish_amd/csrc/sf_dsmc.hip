@@ -55,6 +55,12 @@ __device__ int dsmc_count(const MeshP& m, const PState& s, int a, int b, bool ed
 struct DsmcCell {
     int nsel, n1, n2;
 };
+// What a pass counts, zero before it: one clear and one readback (into pinned memory) for all three.
+struct DsmcStatus {
+    unsigned long long ncol;   // collisions
+    int overflow;              // most particles of a cell that was refused (0: none)
+    int nbig;                  // cells in the list that dsmc_order_big orders
+};
 
 // Slots of the binned particles of [a, b), ordered by id, into order[a ..), for ranges of at most
 // 64 E particles: a bitonic sort of (id << 32 | slot) in registers.  Element i of the list is
@@ -161,7 +167,7 @@ __device__ void order_in_lds(const MeshP& m, const PState& s, int a, int b, int3
 // Pair count and particle order of every cell, one wave per cell.  The sort is what bounds it
 // (about 45 compare-exchange steps for the 380 particles of a cell of the 512 x 256 gas); it
 // stays in registers, so no LDS limits the waves in flight.  Cells with a range longer than
-// DSMC_SMALL go to the list big (big[0] counts it), whose order dsmc_order_big makes.
+// DSMC_SMALL go to the list big (status->nbig counts it), whose order dsmc_order_big makes.
 // 5e7 particles in 512 x 256 cells, at least one candidate pair in each: a pass of a step (order
 // and collisions) takes 0.52 ms here, 0.02 in dsmc_order_big and 0.30 in dsmc_collide; it took 4.8 ms
 // as one kernel with a bitonic sort in LDS and the pair loop on one lane of the cell's wave.
@@ -170,7 +176,7 @@ __global__ void __launch_bounds__(256) dsmc_order(MeshP m, PState sa, const int3
                                                   const double* __restrict__ sig_cr_max, double* __restrict__ rem,
                                                   int32_t* __restrict__ order_a, int32_t* __restrict__ order_b,
                                                   DsmcCell* __restrict__ cells, int* __restrict__ big,
-                                                  int* __restrict__ overflow) {
+                                                  DsmcStatus* __restrict__ status) {
     const int lane = threadIdx.x & 63;
     const int c = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (c >= m.nci * m.ncj) return;
@@ -210,12 +216,12 @@ __global__ void __launch_bounds__(256) dsmc_order(MeshP m, PState sa, const int3
     const bool go = pairs && nsel != 0 && !over;
     if (lane == 0) {
         if (pairs && !over) rem[c] = new_rem;
-        if (over) atomicMax(overflow, (int)fmax(np1, np2));
+        if (over) atomicMax(&status->overflow, (int)fmax(np1, np2));
         cells[c] = DsmcCell{go ? nsel : 0, (int)np1, (int)np2};
     }
     if (!go) return;
     if (a1 - a0 > DSMC_SMALL || b1 - b0 > DSMC_SMALL) {
-        if (lane == 0) big[1 + atomicAdd(&big[0], 1)] = c;
+        if (lane == 0) big[atomicAdd(&status->nbig, 1)] = c;
         return;
     }
     order_small(m, sa, a0, a1, order_a);
@@ -227,12 +233,13 @@ __global__ void __launch_bounds__(256) dsmc_order(MeshP m, PState sa, const int3
 __global__ void __launch_bounds__(256) dsmc_order_big(MeshP m, PState sa, const int32_t* __restrict__ off_a, PState sb,
                                                       const int32_t* __restrict__ off_b, int same,
                                                       int32_t* __restrict__ order_a, int32_t* __restrict__ order_b,
-                                                      const int* __restrict__ big) {
+                                                      const int* __restrict__ big,
+                                                      const DsmcStatus* __restrict__ status) {
     __shared__ unsigned long long key[DSMC_MAXP];
     __shared__ int count;
-    const int nbig = big[0];
+    const int nbig = status->nbig;
     for (int q = blockIdx.x; q < nbig; q += gridDim.x) {
-        const int c = big[1 + q];
+        const int c = big[q];
         order_in_lds(m, sa, off_a[c], off_a[c + 1], order_a, key, &count);
         if (!same) order_in_lds(m, sb, off_b[c], off_b[c + 1], order_b, key, &count);
     }
@@ -264,7 +271,7 @@ __global__ void __launch_bounds__(64) dsmc_collide(MeshP m, PState sa, const int
                                                    const int32_t* __restrict__ order_b,
                                                    const DsmcCell* __restrict__ cells, double* __restrict__ sig_cr_max,
                                                    double* __restrict__ count_sum, double* __restrict__ real_sum,
-                                                   unsigned long long* __restrict__ ncol) {
+                                                   DsmcStatus* __restrict__ status) {
     const int c = blockIdx.x * 64 + threadIdx.x;
     double sums0 = 0, sums1 = 0;
     if (c < m.nci * m.ncj && cells[c].nsel > 0) {
@@ -344,7 +351,7 @@ __global__ void __launch_bounds__(64) dsmc_collide(MeshP m, PState sa, const int
         real_sum[u] += sums1;
     }
     for (int o = 32; o > 0; o >>= 1) sums0 += __shfl_xor(sums0, o);
-    if (threadIdx.x == 0 && sums0 > 0) atomicAdd(ncol, (unsigned long long)sums0);
+    if (threadIdx.x == 0 && sums0 > 0) atomicAdd(&status->ncol, (unsigned long long)sums0);
 }
 
 __global__ void dsmc_fields_kernel(int64_t nn, int which, const double* __restrict__ count_sum,
@@ -390,9 +397,9 @@ struct sf_dsmc {
     double* d_count = nullptr;    // [nn] col-count-sum
     double* d_real = nullptr;     // [nn] col-real-sum
     DsmcCell* d_cells = nullptr;  // [ncells] pair and particle counts of the running pass
-    int* d_big = nullptr;         // [1 + ncells] count and list of the cells that dsmc_order_big orders
-    unsigned long long* d_ncol = nullptr;
-    int* d_overflow = nullptr;
+    int* d_big = nullptr;         // [ncells] list of the cells that dsmc_order_big orders
+    DsmcStatus* d_status = nullptr;
+    DsmcStatus* h_status = nullptr;   // pinned
     int num_samples = 0;
 };
 
@@ -450,9 +457,9 @@ int sf_dsmc_create(sf_ctx* ctx, const sf_dsmc_desc* desc, sf_dsmc** out) {
     if (e == hipSuccess) e = hipMalloc((void**)&d->d_count, nn * 8);
     if (e == hipSuccess) e = hipMalloc((void**)&d->d_real, nn * 8);
     if (e == hipSuccess) e = hipMalloc((void**)&d->d_cells, nc * sizeof(DsmcCell));
-    if (e == hipSuccess) e = hipMalloc((void**)&d->d_big, (nc + 1) * sizeof(int));
-    if (e == hipSuccess) e = hipMalloc((void**)&d->d_ncol, 8);
-    if (e == hipSuccess) e = hipMalloc((void**)&d->d_overflow, 4);
+    if (e == hipSuccess) e = hipMalloc((void**)&d->d_big, nc * sizeof(int));
+    if (e == hipSuccess) e = hipMalloc((void**)&d->d_status, sizeof(DsmcStatus));
+    if (e == hipSuccess) e = hipHostMalloc((void**)&d->h_status, sizeof(DsmcStatus));
     if (e == hipSuccess) e = hipMemcpy(d->d_scm, scm.data(), nc * 8, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemsetAsync(d->d_rem, 0, nc * 8, ctx->stream);
     if (e == hipSuccess) e = hipMemsetAsync(d->d_count, 0, nn * 8, ctx->stream);
@@ -464,8 +471,8 @@ int sf_dsmc_create(sf_ctx* ctx, const sf_dsmc_desc* desc, sf_dsmc** out) {
         hipFree(d->d_real);
         hipFree(d->d_cells);
         hipFree(d->d_big);
-        hipFree(d->d_ncol);
-        hipFree(d->d_overflow);
+        hipFree(d->d_status);
+        hipHostFree(d->h_status);
         delete d;
         release_stream(ctx, desc->seed, pp.tag);
         return sf_fail(ctx, SF_ERR_HIP, "sf_dsmc_create: %s", hipGetErrorString(e));
@@ -484,8 +491,8 @@ int sf_dsmc_destroy(sf_dsmc* d) {
     hipFree(d->d_real);
     hipFree(d->d_cells);
     hipFree(d->d_big);
-    hipFree(d->d_ncol);
-    hipFree(d->d_overflow);
+    hipFree(d->d_status);
+    hipHostFree(d->h_status);
     release_stream(d->ctx, d->desc.seed, d->pp.tag);
     delete d;
     return SF_OK;
@@ -510,27 +517,23 @@ int sf_dsmc_perform(sf_dsmc* d, int it, int64_t* collisions) {
     DsmcParams pp = d->pp;
     pp.delta_t = d->desc.frequency * ctx->dt;
     pp.step = (uint32_t)it;
-    SF_HIP(ctx, hipMemsetAsync(d->d_ncol, 0, 8, ctx->stream));
-    SF_HIP(ctx, hipMemsetAsync(d->d_overflow, 0, 4, ctx->stream));
-    SF_HIP(ctx, hipMemsetAsync(d->d_big, 0, 4, ctx->stream));
+    SF_HIP(ctx, hipMemsetAsync(d->d_status, 0, sizeof(DsmcStatus), ctx->stream));
     const int ncells = ctx->mp.nci * ctx->mp.ncj;
     // the species' key arrays hold nothing between pushes: the passes keep the cells' orders there
     const PState sa = A->buf[A->cur], sb = B->buf[B->cur];
     const int32_t *oa = A->offsets, *ob = B->offsets;
     hipLaunchKernelGGL(dsmc_order, dim3((ncells + 3) / 4), dim3(256), 0, ctx->stream, ctx->mp, sa, oa, sb, ob, pp,
-                       (const double*)d->d_scm, d->d_rem, A->key, B->key, d->d_cells, d->d_big, d->d_overflow);
+                       (const double*)d->d_scm, d->d_rem, A->key, B->key, d->d_cells, d->d_big, d->d_status);
     hipLaunchKernelGGL(dsmc_order_big, dim3(std::min(ncells, 1024)), dim3(256), 0, ctx->stream, ctx->mp, sa, oa, sb, ob,
-                       pp.same, A->key, B->key, (const int*)d->d_big);
+                       pp.same, A->key, B->key, (const int*)d->d_big, (const DsmcStatus*)d->d_status);
     hipLaunchKernelGGL(dsmc_collide, dim3((ncells + 63) / 64), dim3(64), 0, ctx->stream, ctx->mp, sa, oa, sb, ob, pp,
                        (const int32_t*)A->key, (const int32_t*)B->key, (const DsmcCell*)d->d_cells, d->d_scm,
-                       d->d_count, d->d_real, d->d_ncol);
+                       d->d_count, d->d_real, d->d_status);
     SF_HIP(ctx, hipGetLastError());
-    unsigned long long n = 0;
-    int over = 0;
-    SF_HIP(ctx, hipMemcpyAsync(&n, d->d_ncol, 8, hipMemcpyDeviceToHost, ctx->stream));
-    SF_HIP(ctx, hipMemcpyAsync(&over, d->d_overflow, 4, hipMemcpyDeviceToHost, ctx->stream));
+    SF_HIP(ctx, hipMemcpyAsync(d->h_status, d->d_status, sizeof(DsmcStatus), hipMemcpyDeviceToHost, ctx->stream));
     SF_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    if (collisions) *collisions = (int64_t)n;
+    const int over = d->h_status->overflow;
+    if (collisions) *collisions = (int64_t)d->h_status->ncol;
     if (over > 0)
         return sf_fail(ctx, SF_ERR_UNSUPPORTED, "sf_dsmc_perform: a cell holds %d particles of one species (limit %d);"
                        " its collisions were skipped", over, DSMC_MAXP);
