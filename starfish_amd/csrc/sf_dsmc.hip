@@ -263,18 +263,23 @@ struct PairedRng {
 
 // The collision loop of every cell, one LANE per cell.  A cell's pairs are sequential (a particle
 // drawn twice must see its first collision's velocity, and a pair's draws follow the last one's),
-// but the cells are independent: 64 of them share a wave's instruction stream, where a loop on one
-// lane of a wave per cell spent the same instructions (Philox, pow, sin, cos) on one cell.
+// but the cells are independent: those of a wave share its instruction stream, where a loop on one
+// lane of a wave per cell spent the same instructions (Philox, pow, sin, cos) on one cell.  Only where
+// all cells together are a few waves do lanes wait more for each other's collisions than they share:
+// a wave takes 2^cell_shift cells, 64 unless that leaves fewer than DSMC_WAVES waves.  A pass with
+// many pairs a cell: 4 cells of 1500 particles 1.84 ms (64 cells a wave 2.11), 100 of 400 0.63 (0.78);
+// but 3200 of 400 0.93 ms with 64 cells a wave, 1.05 with 32, 1.28 with 8 and 1.68 with 2.
+constexpr int DSMC_WAVES = 32;
 __global__ void __launch_bounds__(64) dsmc_collide(MeshP m, PState sa, const int32_t* __restrict__ off_a, PState sb,
-                                                   const int32_t* __restrict__ off_b, DsmcParams pp,
+                                                   const int32_t* __restrict__ off_b, DsmcParams pp, int cell_shift,
                                                    const int32_t* __restrict__ order_a,
                                                    const int32_t* __restrict__ order_b,
                                                    const DsmcCell* __restrict__ cells, double* __restrict__ sig_cr_max,
                                                    double* __restrict__ count_sum, double* __restrict__ real_sum,
                                                    DsmcStatus* __restrict__ status) {
-    const int c = blockIdx.x * 64 + threadIdx.x;
+    const int c = (blockIdx.x << cell_shift) + threadIdx.x;
     double sums0 = 0, sums1 = 0;
-    if (c < m.nci * m.ncj && cells[c].nsel > 0) {
+    if ((int)threadIdx.x < (1 << cell_shift) && c < m.nci * m.ncj && cells[c].nsel > 0) {
         const DsmcCell cell = cells[c];
         const int ci = c % m.nci, cj = c / m.nci;
         const double np1 = cell.n1, np2 = cell.n2, scm0 = sig_cr_max[c];
@@ -526,9 +531,11 @@ int sf_dsmc_perform(sf_dsmc* d, int it, int64_t* collisions) {
                        (const double*)d->d_scm, d->d_rem, A->key, B->key, d->d_cells, d->d_big, d->d_status);
     hipLaunchKernelGGL(dsmc_order_big, dim3(std::min(ncells, 1024)), dim3(256), 0, ctx->stream, ctx->mp, sa, oa, sb, ob,
                        pp.same, A->key, B->key, (const int*)d->d_big, (const DsmcStatus*)d->d_status);
-    hipLaunchKernelGGL(dsmc_collide, dim3((ncells + 63) / 64), dim3(64), 0, ctx->stream, ctx->mp, sa, oa, sb, ob, pp,
-                       (const int32_t*)A->key, (const int32_t*)B->key, (const DsmcCell*)d->d_cells, d->d_scm,
-                       d->d_count, d->d_real, d->d_status);
+    int shift = 6;
+    while (shift > 0 && (ncells >> shift) < DSMC_WAVES) shift--;
+    hipLaunchKernelGGL(dsmc_collide, dim3((ncells + (1 << shift) - 1) >> shift), dim3(64), 0, ctx->stream, ctx->mp, sa, oa,
+                       sb, ob, pp, shift, (const int32_t*)A->key, (const int32_t*)B->key, (const DsmcCell*)d->d_cells,
+                       d->d_scm, d->d_count, d->d_real, d->d_status);
     SF_HIP(ctx, hipGetLastError());
     SF_HIP(ctx, hipMemcpyAsync(d->h_status, d->d_status, sizeof(DsmcStatus), hipMemcpyDeviceToHost, ctx->stream));
     SF_HIP(ctx, hipStreamSynchronize(ctx->stream));

@@ -202,3 +202,48 @@ def test_cell_orders_at_their_size_limits(two):
         if dsmc is not None:
             dsmc.close()
         sim.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ni,nj", [(2, 3), (5, 9), (9, 9), (17, 5), (33, 33), (46, 46), (65, 64)])
+def test_cells_of_a_wave_match_oracle(ni, nj):
+    """2, 32, 64, 64, 1024, 2025 and 4032 cells, which the collision loop takes 1 to 64 to a wave (whole
+    and partial waves): two passes of a gas of about 30 particles a cell collide as the oracle does, cell
+    for cell."""
+    from starfish_amd.interactions import DsmcHip
+    from starfish_amd.plugin import Simulation
+    mesh = D.MeshSpec("XY", ni, nj, (0.0, 0.0), (1e-4, 1e-4), {f: ("SYMMETRY", 0.0) for f in D.FACES})
+    ncell = (ni - 1) * (nj - 1)
+    n = 30 * ncell
+    deck = D.Deck(mesh, materials=[D.MaterialSpec("N2", "kinetic_hip", 28.0, 0.0, 1e22 * ncell * 1e-8 / n, 0.0)],
+                  solver=None, num_it=1, dt=2e-7, seed=0)
+    geo, _ = geometry(deck)
+    o = oracle_for(deck, geo)
+    rng = np.random.default_rng(ncell)
+    lc = (rng.random((n, 2)) * [ni - 1, nj - 1] * 0.9999).astype(np.float32).astype(np.float64)
+    v = (rng.normal(size=(n, 3)) * 400.0).astype(np.float32).astype(np.float64)
+    x, y = lc[:, 0] * 1e-4, lc[:, 1] * 1e-4
+    ids = np.arange(n, dtype=np.int32)
+    sim = Simulation(deck, capacity=n + 16, track_ids=True)
+    dsmc = None
+    try:
+        mat = sim.materials[0]
+        mat.add_particles(x, y, v[:, 0], v[:, 1], v[:, 2], ids=ids, rewind=False)
+        o.load_particles(0, np.stack([x, y, np.zeros(n)], 1), v, ids=ids, rewind=False)
+        dsmc = DsmcHip(sim, mat, mat, sig_cr_max=2e-16, seed=9, tag=2, **N2)
+        st = {"sig_cr_max": np.full(ncell, 2e-16), "rem": np.zeros(ncell)}
+        acc = {"count_sum": np.zeros(sim.nn), "real_sum": np.zeros(sim.nn)}
+        pair = {"sigma_type": 1, "diam": N2["diam"], "ref_temp": N2["ref_temp"],
+                "visc_temp_index": N2["visc_temp_index"], "vss_alpha": (1.0, 1.0)}
+        total = 0
+        for it in (1, 2):
+            ng = dsmc.perform(it)
+            assert ng == o.dsmc_perform(0, 0, pair, 9, 2, it, 1, st, acc)
+            assert np.array_equal(dsmc.field("col-count-sum"), acc["count_sum"])
+            o.round_state_fp32(0)
+            total += ng
+        assert total > 0.1 * ncell
+    finally:
+        if dsmc is not None:
+            dsmc.close()
+        sim.close()
