@@ -113,25 +113,65 @@ __device__ __forceinline__ unsigned int mcc_particle(const MeshP& m, const PStat
 
 // Largest target density and largest |u|, |v|, |w| over the nodes, rounded up to FP32, as the bit
 // patterns of non-negative floats (which order like the numbers).  A value that is not finite gives
-// infinity.  bound[0..4) is zero before the launch.
-__global__ void __launch_bounds__(256) mcc_target_bounds(int64_t nn, MccTarget tg, unsigned int* __restrict__ bound) {
+// infinity.  Each workgroup leaves its maxima, the last one combines them and leaves the counter at zero
+// for the next target (zero at first), so a target costs one launch.  Few workgroups with four nodes a
+// thread in flight: a thousand would wait for their atomics on that counter (1024 x 512 nodes: 45 us
+// with 1024 of them, 10 with these).
+constexpr int MCC_BOUND_BLOCKS = 256;
+constexpr int64_t MCC_BOUND_MIN = 1 << 19;   // particles (beyond the nodes) for which one pass pays for the bound
+struct MccBound {
+    unsigned int bound[4], done;
+    float part[MCC_BOUND_BLOCKS][4];
+};
+__global__ void __launch_bounds__(256) mcc_target_bounds(int64_t nn, MccTarget tg, MccBound* __restrict__ out) {
+    __shared__ float red[4][4];
+    __shared__ bool last;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     float b[4] = {0.f, 0.f, 0.f, 0.f};
     auto up = [](double x) {   // FP32 at least x
         const float f = (float)(x * (1.0 + 1e-6));
         return f <= 3e38f ? f : __int_as_float(0x7F800000);   // NaN and overflow: infinity
     };
-    for (int64_t u = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; u < nn; u += (int64_t)gridDim.x * blockDim.x) {
-        const double d = tg.den[u];
-        b[0] = fmaxf(b[0], up(d < 0 ? 0.0 : d));
-        b[1] = fmaxf(b[1], up(fabs(tg.u[u])));
-        b[2] = fmaxf(b[2], up(fabs(tg.v[u])));
-        b[3] = fmaxf(b[3], up(fabs(tg.w[u])));
-    }
+    auto wave_max = [&]() {   // of b, each wave's into red
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-        for (int o = 32; o > 0; o >>= 1) b[k] = fmaxf(b[k], __shfl_xor(b[k], o));
-        if ((threadIdx.x & 63) == 0) atomicMax(&bound[k], __float_as_uint(b[k]));
+        for (int k = 0; k < 4; k++) {
+            for (int o = 32; o > 0; o >>= 1) b[k] = fmaxf(b[k], __shfl_xor(b[k], o));
+            if (lane == 0) red[k][wave] = b[k];
+        }
+        __syncthreads();
+    };
+    const int64_t stride = (int64_t)gridDim.x * 256;
+    for (int64_t u0 = blockIdx.x * (int64_t)256 + t; u0 < nn; u0 += 4 * stride) {
+        double f[4][4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int64_t u = u0 + q * stride < nn ? u0 + q * stride : u0;
+            f[q][0] = tg.den[u];
+            f[q][1] = tg.u[u];
+            f[q][2] = tg.v[u];
+            f[q][3] = tg.w[u];
+        }
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            b[0] = fmaxf(b[0], up(f[q][0] < 0 ? 0.0 : f[q][0]));
+#pragma unroll
+            for (int k = 1; k < 4; k++) b[k] = fmaxf(b[k], up(fabs(f[q][k])));
+        }
     }
+    wave_max();
+    if (t < 4) out->part[blockIdx.x][t] = fmaxf(fmaxf(red[t][0], red[t][1]), fmaxf(red[t][2], red[t][3]));
+    __threadfence();
+    __syncthreads();
+    if (t == 0) last = atomicAdd(&out->done, 1u) == gridDim.x - 1;
+    __syncthreads();
+    if (!last) return;
+    __threadfence();   // the other workgroups' parts
+    static_assert(MCC_BOUND_BLOCKS == 256, "one part a thread");
+#pragma unroll
+    for (int k = 0; k < 4; k++) b[k] = t < (int)gridDim.x ? out->part[t][k] : 0.f;
+    wave_max();
+    if (t < 4) out->bound[t] = __float_as_uint(fmaxf(fmaxf(red[t][0], red[t][1]), fmaxf(red[t][2], red[t][3])));
+    if (t == 0) out->done = 0;
 }
 
 // Few particles collide in a pass (1e-5 to 1e-2 of them), and most are ruled out without the
@@ -147,13 +187,15 @@ __global__ void __launch_bounds__(256) mcc_target_bounds(int64_t nn, MccTarget t
 // 5.9 -> 4.7 ms; without the queue the collisions ran on a few lanes of each wave.)
 constexpr int MCC_CHUNK = 1024;            // slots a workgroup tests at a time, 4 a thread
 __global__ void __launch_bounds__(256) mcc_kernel(MeshP m, PState s, int64_t np, MccTarget tg, MccParams pp,
-                                                  const unsigned int* __restrict__ bound,
+                                                  const MccBound* __restrict__ bounds, int bounded,
                                                   unsigned long long* __restrict__ count, double* __restrict__ S,
                                                   unsigned long long* __restrict__ ncol) {
     __shared__ int64_t queue[MCC_CHUNK + 256];
     __shared__ int nq;
     const int t = threadIdx.x, lane = t & 63;
-    const float kx = (float)(pp.sigma * pp.dt * 1.0001 * (double)__uint_as_float(bound[0]));
+    const unsigned int* const bound = bounds->bound;
+    const float inf = __int_as_float(0x7F800000);   // (rules out no particle)
+    const float kx = bounded ? (float)(pp.sigma * pp.dt * 1.0001 * (double)__uint_as_float(bound[0])) : inf;
     const float tu = __uint_as_float(bound[1]), tv = __uint_as_float(bound[2]), tw = __uint_as_float(bound[3]);
     unsigned int ncol_local = 0;   // added to ncol once per wave
     if (t == 0) nq = 0;
@@ -245,8 +287,10 @@ struct sf_mcc {
     double* d_S = nullptr;
     unsigned long long* d_ncol = nullptr;
     unsigned long long* h_ncol = nullptr;   // pinned: the pass's count without a staged copy
-    unsigned int* d_bound = nullptr;     // [4] bounds of the target's density and velocity (mcc_target_bounds)
+    MccBound* d_bound = nullptr;         // bounds of the target's density and velocity (mcc_target_bounds)
     bool have_target = false;
+    bool bounded = false;                // d_bound is the present target's
+    int target_passes = 0;               // passes over the present target
     int num_samples = 0;
     double time_start = 0, time_last = 0;
     uint32_t stream_tag = 0;             // module-tagged counter word of the Philox streams
@@ -261,6 +305,23 @@ static int grid_n(int64_t n, int max_blocks) {
     if (b < 1) b = 1;
     return (int)(b < max_blocks ? b : max_blocks);
 }
+
+// The bound of a target takes about 6 us and 8 ps a node, and saves 13 ps a particle and pass: it is made
+// with the target where one pass pays for it, else at its second pass.  (A host that sets the target of
+// few particles before every pass had paid 10 to 20 us a pass for it.)
+static bool bound_pays(const sf_mcc* c) {
+    return c->ctx->species[c->desc.source_species]->np > MCC_BOUND_MIN + (int64_t)c->ctx->mp.ni * c->ctx->mp.nj;
+}
+static int make_bound(sf_mcc* c) {
+    sf_ctx* ctx = c->ctx;
+    const int64_t nn = (int64_t)ctx->mp.ni * ctx->mp.nj;
+    hipLaunchKernelGGL(mcc_target_bounds, dim3(grid_n(nn, MCC_BOUND_BLOCKS)), dim3(256), 0, ctx->stream, nn,
+                       mcc_target(c, (size_t)nn), c->d_bound);
+    SF_HIP(ctx, hipGetLastError());
+    c->bounded = true;
+    return SF_OK;
+}
+
 
 extern "C" {
 
@@ -295,7 +356,8 @@ int sf_mcc_create(sf_ctx* ctx, const sf_mcc_desc* desc, sf_mcc** out) {
     if (e == hipSuccess) e = hipMalloc((void**)&c->d_S, nn * sizeof(double));
     if (e == hipSuccess) e = hipMalloc((void**)&c->d_ncol, sizeof(unsigned long long));
     if (e == hipSuccess) e = hipHostMalloc((void**)&c->h_ncol, sizeof(unsigned long long));
-    if (e == hipSuccess) e = hipMalloc((void**)&c->d_bound, 4 * sizeof(unsigned int));
+    if (e == hipSuccess) e = hipMalloc((void**)&c->d_bound, sizeof(MccBound));
+    if (e == hipSuccess) e = hipMemsetAsync(c->d_bound, 0, sizeof(MccBound), ctx->stream);
     if (e == hipSuccess) e = hipMemsetAsync(c->d_target, 0, 5 * nn * sizeof(double), ctx->stream);
     if (e == hipSuccess) e = hipMemsetAsync(c->d_count, 0, nn * sizeof(unsigned long long), ctx->stream);
     if (e == hipSuccess) e = hipMemsetAsync(c->d_S, 0, nn * sizeof(double), ctx->stream);
@@ -339,17 +401,15 @@ int sf_mcc_set_target(sf_mcc* c, const double* den, const double* u, const doubl
     SF_HIP(ctx, hipStreamSynchronize(ctx->stream));
     // (the copies wait for the device; the clears follow on the context's stream, which the bounds and the
     // next pass run on: a clear on the null stream would not be ordered before them)
+    c->bounded = false;
+    c->target_passes = 0;
     const double* src[5] = {den, u, v, w, temp};
     for (int k = 0; k < 5; k++) {
         if (src[k]) SF_HIP(ctx, hipMemcpy(c->d_target + k * nn, src[k], nn * sizeof(double), hipMemcpyHostToDevice));
         else SF_HIP(ctx, hipMemsetAsync(c->d_target + k * nn, 0, nn * sizeof(double), ctx->stream));
     }
-    SF_HIP(ctx, hipMemsetAsync(c->d_bound, 0, 4 * sizeof(unsigned int), ctx->stream));
-    hipLaunchKernelGGL(mcc_target_bounds, dim3(grid_n((int64_t)nn, 128)), dim3(256), 0, ctx->stream, (int64_t)nn,
-                       mcc_target(c, nn), c->d_bound);
-    SF_HIP(ctx, hipGetLastError());
     c->have_target = true;
-    return SF_OK;
+    return bound_pays(c) ? make_bound(c) : SF_OK;
 }
 
 int sf_mcc_perform(sf_mcc* c, int it, double time, int64_t* collisions) {
@@ -380,9 +440,14 @@ int sf_mcc_perform(sf_mcc* c, int it, double time, int64_t* collisions) {
     pp.tag = c->stream_tag;
     SF_HIP(ctx, hipMemsetAsync(c->d_ncol, 0, sizeof(unsigned long long), ctx->stream));
     if (sp->np > 0) {
+        if (!c->bounded && (c->target_passes > 0 || bound_pays(c))) {   // (the particles may have come later)
+            const int rc = make_bound(c);
+            if (rc) return rc;
+        }
+        c->target_passes++;
         hipLaunchKernelGGL(mcc_kernel, dim3((unsigned)std::min<int64_t>((sp->np + MCC_CHUNK - 1) / MCC_CHUNK, 2048)),
                            dim3(256), 0, ctx->stream, ctx->mp, sp->buf[sp->cur], sp->np, tg, pp,
-                           (const unsigned int*)c->d_bound, c->d_count, c->d_S, c->d_ncol);
+                           (const MccBound*)c->d_bound, (int)c->bounded, c->d_count, c->d_S, c->d_ncol);
         SF_HIP(ctx, hipGetLastError());
     }
     SF_HIP(ctx, hipMemcpyAsync(c->h_ncol, c->d_ncol, sizeof(unsigned long long), hipMemcpyDeviceToHost, ctx->stream));

@@ -199,3 +199,60 @@ def test_fields_left_out_of_a_new_target_are_zero_in_the_next_pass(given):
         if mcc is not None:
             mcc.close()
         sim.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bad", ["negative", "nan_density", "inf_velocity", "nan_velocity"])
+def test_mcc_target_values_outside_the_ordinary(bad):
+    """Target fields that the bound has to let through: densities of either sign (no collision where the
+    gathered one is not positive), and one node that is not finite, around which the test for every
+    particle decides (1 - exp(-NaN) < draw is false there, so a NaN collides).  6e5 particles, enough for
+    the bound, against the oracle: the same particles collide in a pass over the new and the kept target,
+    and the others keep their velocity bit for bit."""
+    from starfish_amd.interactions import MccHip
+    from starfish_amd.plugin import Simulation
+    deck = _deck("XY")
+    m = deck.mesh
+    geo, _ = geometry(deck)
+    o = oracle_for(deck, geo)
+    rng = np.random.default_rng(8)
+    n = 600_000
+    lc = np.stack([rng.uniform(0, m.ni - 1, n), rng.uniform(0, m.nj - 1, n)], 1).astype(np.float32).astype(np.float64)
+    v = (rng.normal(size=(n, 3)) * 800.0).astype(np.float32).astype(np.float64)
+    x, y = m.x0[0] + lc[:, 0] * m.dh[0], m.x0[1] + lc[:, 1] * m.dh[1]
+    ids = np.arange(n, dtype=np.int32)
+    o.load_particles(0, np.stack([x, y, np.zeros(n)], 1), v, ids=ids, rewind=False)
+    tgt = _target(m)
+    tgt["den"] = tgt["den"] * 1e-2
+    node = 20 * m.ni + 40
+    if bad == "negative":
+        tgt["den"] = np.where(np.arange(tgt["den"].size) % 7 < 3, -1e20, tgt["den"])
+    elif bad == "nan_density":
+        tgt["den"][node] = np.nan
+    else:
+        tgt["u"] = tgt["u"].copy()
+        tgt["u"][node] = np.inf if bad == "inf_velocity" else np.nan
+    acc = {k: np.zeros(m.ni * m.nj) for k in ("count_sum", "real_sum", "S")}
+    sim = Simulation(deck, capacity=n + 16, track_ids=True)
+    mcc = None
+    try:
+        mat = sim.materials[0]
+        mat.add_particles(x, y, v[:, 0], v[:, 1], v[:, 2], ids=ids, rewind=False)
+        mcc = MccHip(sim, mat, "CEX", 5e-19, 131.0, seed=31, tag=4)
+        mcc.set_target(tgt["den"], tgt["u"], tgt["v"], tgt["w"], tgt["T"])
+        for it in (1, 2):
+            ng = mcc.perform(it, it * deck.dt)
+            no = o.mcc_perform(0, tgt, 131.0 * AMU, 5e-19, 0, -1.0, 31, 4, it, 1, acc)
+            print(bad, "collisions", ng, no, flush=True)
+            assert ng == no > 100
+            assert np.array_equal(mcc.field("col-count-sum"), acc["count_sum"])
+        p, q = mat.particles(ids=True), o.particles(0)
+        gi, oi = np.argsort(p["id"]), np.argsort(q["id"])
+        vg, vo = np.stack([p["u"], p["v"], p["w"]], 1)[gi], q["vel"][oi]
+        same = np.all(vo == v, axis=1)
+        assert same.sum() > n // 2 and np.array_equal(vg[same], v[same])
+        assert np.array_equal(np.isfinite(vg), np.isfinite(vo))
+    finally:
+        if mcc is not None:
+            mcc.close()
+        sim.close()
