@@ -185,12 +185,18 @@ __global__ void __launch_bounds__(256) mcc_target_bounds(int64_t nn, MccTarget t
 // waves.  4e7 particles: 0.70 ms with the full test for every particle, 0.164 ms so: 4.9 TB/s
 // of the 20 B.  (2e7 particles of which 2e-3, 2e-2 and 0.9 pass the bound: 1.43 -> 0.14, 3.2 -> 0.28 and
 // 5.9 -> 4.7 ms; without the queue the collisions ran on a few lanes of each wave.)
-constexpr int MCC_CHUNK = 1024;            // slots a workgroup tests at a time, 4 a thread
+// A workgroup tests SLOTS slots a thread at a time, 4 in 16-byte loads.  A population of at most a workgroup
+// of 256 for every CU takes 1: the colliding particles of 1024 slots would take their workgroup four
+// rounds while most CUs have none (1e4 particles that all collide: 42.0 us with 4, 26.6 with 1; 6.5e4 50
+// and 41; 2e5, on more workgroups than CUs, 67 and 102).
+template <int SLOTS>
 __global__ void __launch_bounds__(256) mcc_kernel(MeshP m, PState s, int64_t np, MccTarget tg, MccParams pp,
                                                   const MccBound* __restrict__ bounds, int bounded,
                                                   unsigned long long* __restrict__ count, double* __restrict__ S,
                                                   unsigned long long* __restrict__ ncol) {
-    __shared__ int64_t queue[MCC_CHUNK + 256];
+    static_assert(SLOTS == 1 || SLOTS == 4, "slots of a thread");
+    constexpr int CHUNK_SLOTS = 256 * SLOTS;
+    __shared__ int64_t queue[CHUNK_SLOTS + 256];
     __shared__ int nq;
     const int t = threadIdx.x, lane = t & 63;
     const unsigned int* const bound = bounds->bound;
@@ -200,12 +206,20 @@ __global__ void __launch_bounds__(256) mcc_kernel(MeshP m, PState s, int64_t np,
     unsigned int ncol_local = 0;   // added to ncol once per wave
     if (t == 0) nq = 0;
     __syncthreads();
-    for (int64_t c0 = (int64_t)blockIdx.x * MCC_CHUNK; c0 < np; c0 += (int64_t)gridDim.x * MCC_CHUNK) {
-        // a chunk starts on a multiple of 1024 slots, so a thread's 4 slots are 16-byte aligned
-        const int64_t p0 = c0 + 4 * t;
+    for (int64_t c0 = (int64_t)blockIdx.x * CHUNK_SLOTS; c0 < np; c0 += (int64_t)gridDim.x * CHUNK_SLOTS) {
+        // a chunk starts on a multiple of 1024 slots where a thread has 4, so those are 16-byte aligned
+        const int64_t p0 = c0 + SLOTS * t;
         int4 c = make_int4(-1, -1, -1, -1), id = make_int4(0, 0, 0, 0);
         float4 vx = make_float4(0.f, 0.f, 0.f, 0.f), vy = vx, vz = vx;
-        if (p0 + 3 < np) {
+        if (SLOTS == 1) {
+            if (p0 < np) {
+                c.x = s.cell[p0];
+                id.x = s.id[p0];
+                vx.x = s.vx[p0];
+                vy.x = s.vy[p0];
+                vz.x = s.vz[p0];
+            }
+        } else if (p0 + 3 < np) {
             c = *reinterpret_cast<const int4*>(s.cell + p0);
             id = *reinterpret_cast<const int4*>(s.id + p0);
             vx = *reinterpret_cast<const float4*>(s.vx + p0);
@@ -234,12 +248,14 @@ __global__ void __launch_bounds__(256) mcc_kernel(MeshP m, PState s, int64_t np,
             }
         };
         test(0, c.x, id.x, vx.x, vy.x, vz.x);
-        test(1, c.y, id.y, vx.y, vy.y, vz.y);
-        test(2, c.z, id.z, vx.z, vy.z, vz.z);
-        test(3, c.w, id.w, vx.w, vy.w, vz.w);
+        if (SLOTS > 1) {
+            test(1, c.y, id.y, vx.y, vy.y, vz.y);
+            test(2, c.z, id.z, vx.z, vy.z, vz.z);
+            test(3, c.w, id.w, vx.w, vy.w, vz.w);
+        }
         __syncthreads();
         // whole groups of 256 now, the rest with the next chunk's (or at the end)
-        const bool last = c0 + (int64_t)gridDim.x * MCC_CHUNK >= np;
+        const bool last = c0 + (int64_t)gridDim.x * CHUNK_SLOTS >= np;
         const int n = nq;
         __syncthreads();   // every thread has n before the next chunk adds to nq
         if (n >= 256 || last) {
@@ -445,9 +461,13 @@ int sf_mcc_perform(sf_mcc* c, int it, double time, int64_t* collisions) {
             if (rc) return rc;
         }
         c->target_passes++;
-        hipLaunchKernelGGL(mcc_kernel, dim3((unsigned)std::min<int64_t>((sp->np + MCC_CHUNK - 1) / MCC_CHUNK, 2048)),
-                           dim3(256), 0, ctx->stream, ctx->mp, sp->buf[sp->cur], sp->np, tg, pp,
-                           (const MccBound*)c->d_bound, (int)c->bounded, c->d_count, c->d_S, c->d_ncol);
+        auto pass = [&](auto kernel, int chunk) {
+            hipLaunchKernelGGL(kernel, dim3((unsigned)std::min<int64_t>((sp->np + chunk - 1) / chunk, 2048)), dim3(256), 0,
+                               ctx->stream, ctx->mp, sp->buf[sp->cur], sp->np, tg, pp, (const MccBound*)c->d_bound,
+                               (int)c->bounded, c->d_count, c->d_S, c->d_ncol);
+        };
+        if (sp->np <= 256 * (int64_t)ctx->ncu) pass(mcc_kernel<1>, 256);
+        else pass(mcc_kernel<4>, 1024);
         SF_HIP(ctx, hipGetLastError());
     }
     SF_HIP(ctx, hipMemcpyAsync(c->h_ncol, c->d_ncol, sizeof(unsigned long long), hipMemcpyDeviceToHost, ctx->stream));

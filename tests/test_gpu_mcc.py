@@ -202,6 +202,48 @@ def test_fields_left_out_of_a_new_target_are_zero_in_the_next_pass(given):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [65, 255, 257, 65535, 65537])
+@pytest.mark.parametrize("scale", [1e-2, 100.0])
+def test_mcc_passes_over_new_and_kept_targets_match_oracle(n, scale):
+    """Populations on both sides of one workgroup a CU (1 or 4 slots a thread), with partial waves and
+    workgroups, at densities where few and where all particles collide: a pass over a new target (no
+    bound is made for so few), two over the kept one (with the bound), and one after another target has
+    been set, all collide the oracle's particles."""
+    from starfish_amd.interactions import MccHip
+    from starfish_amd.plugin import Simulation
+    deck = _deck("RZ")
+    m = deck.mesh
+    geo, _ = geometry(deck)
+    o = oracle_for(deck, geo)
+    rng = np.random.default_rng(n)
+    lc = np.stack([rng.uniform(0, m.ni - 1, n), rng.uniform(0, m.nj - 1, n)], 1).astype(np.float32).astype(np.float64)
+    v = (rng.normal(size=(n, 3)) * 800.0 + [300.0, 0, 0]).astype(np.float32).astype(np.float64)
+    x, y = m.x0[0] + lc[:, 0] * m.dh[0], m.x0[1] + lc[:, 1] * m.dh[1]
+    ids = rng.permutation(n).astype(np.int32)
+    o.load_particles(0, np.stack([x, y, np.zeros(n)], 1), v, ids=ids, rewind=False)
+    acc = {k: np.zeros(m.ni * m.nj) for k in ("count_sum", "real_sum", "S")}
+    sim = Simulation(deck, capacity=n + 16, track_ids=True)
+    mcc = None
+    try:
+        mat = sim.materials[0]
+        mat.add_particles(x, y, v[:, 0], v[:, 1], v[:, 2], ids=ids, rewind=False)
+        mcc = MccHip(sim, mat, "CEX", 5e-19, 131.0, seed=21, tag=4)
+        for it, factor in enumerate((scale, None, None, 3 * scale), 1):
+            if factor is not None:
+                tgt = _target(m)
+                tgt["den"] = tgt["den"] * factor
+                tgt["u"] = tgt["u"] * it
+                mcc.set_target(tgt["den"], tgt["u"], tgt["v"], tgt["w"], tgt["T"])
+            assert mcc.perform(it, it * deck.dt) == o.mcc_perform(0, tgt, 131.0 * AMU, 5e-19, 0, -1.0, 21, 4, it, 1, acc)
+            assert np.array_equal(mcc.field("col-count-sum"), acc["count_sum"])
+            o.round_state_fp32(0)
+    finally:
+        if mcc is not None:
+            mcc.close()
+        sim.close()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("bad", ["negative", "nan_density", "inf_velocity", "nan_velocity"])
 def test_mcc_target_values_outside_the_ordinary(bad):
     """Target fields that the bound has to let through: densities of either sign (no collision where the
