@@ -87,6 +87,7 @@ struct PoissonState {
     int lev_ni[MG_MAXLEV] = {}, lev_nj[MG_MAXLEV] = {};
     int lev_si[MG_MAXLEV] = {}, lev_sj[MG_MAXLEV] = {};   // a level's node (i, j) is (i >> si, j >> sj) on the next
     int64_t lev_off[MG_MAXLEV + 1] = {};
+    float* mg_mem = nullptr;      // the block that holds them all
     float *mgE0 = nullptr, *mgN0 = nullptr, *mfix = nullptr, *res2 = nullptr;
     float *mgE = nullptr, *mgN = nullptr, *mgS = nullptr;   // links and their sum per node
     float *mgm = nullptr, *mgd = nullptr;                   // diagonal beyond the links, diagonal
@@ -169,8 +170,7 @@ void poisson_free(PoissonState* p) {
     if (!p) return;
     void* ptrs[] = {p->cls, p->W,  p->bfix, p->src, p->fixval, p->x,  p->r,       p->y,    p->rr,
                     p->D,   p->P,  p->d,    p->res, p->z,      p->p0, p->p1,      p->q,    p->partial,
-                    p->pz,  p->ppq, p->scal, p->istate, p->mgE0, p->mgN0, p->mfix, p->res2, p->mgE, p->mgN,
-                    p->mgS, p->mgm, p->mgd, p->mgr, p->mge};
+                    p->pz,  p->ppq, p->scal, p->istate, p->mg_mem};
     for (void* q : ptrs)
         if (q) hipFree(q);
     if (p->host_scal) hipHostFree(p->host_scal);
@@ -846,6 +846,56 @@ __global__ void __launch_bounds__(1024) mg_bottom(MgBottom B, const float* __res
     for (int u = t; u < B.ni[0] * B.nj[0]; u += 1024) e[u] = sx[u];
 }
 
+// Links of the finest level, from the classes and the stencil, and the part of its diagonal that fixed
+// neighbours add.
+__global__ void __launch_bounds__(256) mg_links0(MeshP m, const uint8_t* __restrict__ cls, float* __restrict__ E,
+                                                 float* __restrict__ N, float* __restrict__ mfix) {
+    for (int64_t u = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; u < (int64_t)m.ni * m.nj;
+         u += (int64_t)gridDim.x * blockDim.x) {
+        const uint8_t c = cls[u];
+        float e = 0.0f, n = 0.0f, fix = 0.0f;
+        if (c != CLS_NOT_FREE) {
+            const Stencil st = stencil(m, (int)(u % m.ni), (int)(u / m.ni));
+            const double cc[4] = {st.cE, st.cW, st.cN, st.cS};
+#pragma unroll
+            for (int d = 0; d < 4; d++)
+                if (nbc(c, d) == NB_FIXED) fix += (float)cc[d];
+            if (nbc(c, 0) == NB_FREE) e = (float)st.cE;
+            if (nbc(c, 2) == NB_FREE) n = (float)st.cN;
+        }
+        E[u] = e;
+        N[u] = n;
+        mfix[u] = fix;
+    }
+}
+
+// Links of a level (nI x nJ) and their sum per node from those of the finer one (ni x nj): the links that
+// cross into another aggregate, halved along a halved direction.
+__global__ void __launch_bounds__(256) mg_links_one(int ni, int nj, int si, int sj, int nI, int nJ,
+                                                    const float* __restrict__ fE, const float* __restrict__ fN,
+                                                    float* __restrict__ E, float* __restrict__ N,
+                                                    float* __restrict__ S) {
+    auto link = [&](int I, int J, bool east) {
+        const int i1 = min((I + 1) << si, ni), j1 = min((J + 1) << sj, nj);
+        float v = 0.0f;
+        for (int j = J << sj; j < j1; j++)
+            for (int i = I << si; i < i1; i++) {
+                const size_t u = (size_t)j * ni + i;
+                if (east && (!si || (i & 1))) v += (si ? 0.5f : 1.0f) * fE[u];
+                if (!east && (!sj || (j & 1))) v += (sj ? 0.5f : 1.0f) * fN[u];
+            }
+        return v;
+    };
+    for (int64_t U = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; U < (int64_t)nI * nJ;
+         U += (int64_t)gridDim.x * blockDim.x) {
+        const int I = (int)(U % nI), J = (int)(U / nI);
+        const float e = link(I, J, true), n = link(I, J, false);
+        E[U] = e;
+        N[U] = n;
+        S[U] = e + n + (I > 0 ? link(I - 1, J, true) : 0.0f) + (J > 0 ? link(I, J - 1, false) : 0.0f);
+    }
+}
+
 // Diagonal of one level that halves one direction only.
 __global__ void __launch_bounds__(256) mg_mass_one(int ni, int nj, int si, int sj, int nI, int nJ, int64_t off,
                                                    const double* __restrict__ P, const float* __restrict__ mfix,
@@ -1415,52 +1465,22 @@ static void mg_levels(PoissonState* P, int ni, int nj, double ratio) {   // rati
     while (P->lev_off[n] - P->lev_off[P->lev_bottom] > MG_BOTTOM || P->lev_ni[P->lev_bottom] > MG_PAD) P->lev_bottom++;
 }
 
-// The links of every level and the constant part of the finest diagonal beyond its links.
-static int mg_setup(sf_ctx* ctx, PoissonState* P, const std::vector<uint8_t>& cls) {
+// The links of every level and the constant part of the finest diagonal beyond its links: one launch a
+// level, queued (built on the host and copied, three arrays a level, they took 0.3 ms of a set-up at
+// 81 x 41 nodes and 10 ms at 2048 x 1024).
+static int mg_setup(sf_ctx* ctx, PoissonState* P) {
     const MeshP& m = ctx->mp;
-    const size_t nn = (size_t)m.ni * m.nj;
-    std::vector<float> E(nn, 0.f), N(nn, 0.f), mfix(nn, 0.f);
-    for (int j = 0; j < m.nj; j++)
-        for (int i = 0; i < m.ni; i++) {
-            const size_t u = (size_t)j * m.ni + i;
-            const uint8_t c = cls[u];
-            if (c == CLS_NOT_FREE) continue;
-            const Stencil st = stencil(m, i, j);
-            const double cc[4] = {st.cE, st.cW, st.cN, st.cS};
-            for (int d = 0; d < 4; d++)
-                if (((c >> (2 * d)) & 3) == NB_FIXED) mfix[u] += (float)cc[d];
-            if ((c & 3) == NB_FREE) E[u] = (float)st.cE;
-            if (((c >> 4) & 3) == NB_FREE) N[u] = (float)st.cN;
-        }
-    SF_HIP(ctx, hipMemcpy(P->mgE0, E.data(), nn * 4, hipMemcpyHostToDevice));
-    SF_HIP(ctx, hipMemcpy(P->mgN0, N.data(), nn * 4, hipMemcpyHostToDevice));
-    SF_HIP(ctx, hipMemcpy(P->mfix, mfix.data(), nn * 4, hipMemcpyHostToDevice));
-    std::vector<float> cE, cN, cS;
+    hipStream_t st = ctx->stream;
+    hipLaunchKernelGGL(mg_links0, dim3(grid_elem((int64_t)m.ni * m.nj)), dim3(256), 0, st, m, (const uint8_t*)P->cls,
+                       P->mgE0, P->mgN0, P->mfix);
     for (int l = 1; l < P->nlev; l++) {
-        const int ni = P->lev_ni[l - 1], nj = P->lev_nj[l - 1], nI = P->lev_ni[l], nJ = P->lev_nj[l];
-        const int si = P->lev_si[l - 1], sj = P->lev_sj[l - 1];
-        const float fx = si ? 0.5f : 1.0f, fy = sj ? 0.5f : 1.0f;
-        cE.assign((size_t)nI * nJ, 0.f);
-        cN.assign((size_t)nI * nJ, 0.f);
-        cS.assign((size_t)nI * nJ, 0.f);
-        for (int j = 0; j < nj; j++)
-            for (int i = 0; i < ni; i++) {
-                const size_t u = (size_t)j * ni + i, U = (size_t)(j >> sj) * nI + (i >> si);
-                if (!si || (i & 1)) cE[U] += fx * E[u];   // the links that cross into another aggregate
-                if (!sj || (j & 1)) cN[U] += fy * N[u];
-            }
-        for (int J = 0; J < nJ; J++)
-            for (int I = 0; I < nI; I++) {
-                const size_t U = (size_t)J * nI + I;
-                cS[U] = cE[U] + cN[U] + (I > 0 ? cE[U - 1] : 0.f) + (J > 0 ? cN[U - nI] : 0.f);
-            }
-        const size_t bytes = cE.size() * 4;
-        SF_HIP(ctx, hipMemcpy(P->mgE + P->lev_off[l], cE.data(), bytes, hipMemcpyHostToDevice));
-        SF_HIP(ctx, hipMemcpy(P->mgN + P->lev_off[l], cN.data(), bytes, hipMemcpyHostToDevice));
-        SF_HIP(ctx, hipMemcpy(P->mgS + P->lev_off[l], cS.data(), bytes, hipMemcpyHostToDevice));
-        E.swap(cE);
-        N.swap(cN);
+        const int64_t f = P->lev_off[l - 1], o = P->lev_off[l];
+        hipLaunchKernelGGL(mg_links_one, dim3(grid_elem((int64_t)P->lev_ni[l] * P->lev_nj[l])), dim3(256), 0, st,
+                           P->lev_ni[l - 1], P->lev_nj[l - 1], P->lev_si[l - 1], P->lev_sj[l - 1], P->lev_ni[l],
+                           P->lev_nj[l], (const float*)(l == 1 ? P->mgE0 : P->mgE + f),
+                           (const float*)(l == 1 ? P->mgN0 : P->mgN + f), P->mgE + o, P->mgN + o, P->mgS + o);
     }
+    SF_HIP(ctx, hipGetLastError());
     return SF_OK;
 }
 
@@ -1652,11 +1672,14 @@ int poisson_setup(sf_ctx* ctx, const sf_poisson_desc* dsc) {
         if (!e) e = A((void**)&P->pz, (size_t)4 * nb_pz * 8);
         if (!e && (int64_t)nn >= MG_MIN_NODES) {
             mg_levels(P, ni, nj, m.dh[0] / m.dh[1]);
-            const size_t nc = (size_t)P->lev_off[P->nlev];
-            for (float** f : {&P->mgE0, &P->mgN0, &P->mfix, &P->res2})
-                if (!e) e = A((void**)f, nn * 4);
-            for (float** f : {&P->mgE, &P->mgN, &P->mgS, &P->mgm, &P->mgd, &P->mgr, &P->mge})
-                if (!e) e = A((void**)f, nc * 4);
+            auto pad = [](size_t n) { return (n + 63) / 64 * 64; };
+            const size_t nf = pad(nn), nc = pad((size_t)P->lev_off[P->nlev]);
+            e = A((void**)&P->mg_mem, (4 * nf + 7 * nc) * 4);
+            float* at = P->mg_mem;
+            if (!e)
+                for (float** f : {&P->mgE0, &P->mgN0, &P->mfix, &P->res2}) *f = at, at += nf;
+            if (!e)
+                for (float** f : {&P->mgE, &P->mgN, &P->mgS, &P->mgm, &P->mgd, &P->mgr, &P->mge}) *f = at, at += nc;
         }
         if (!e) e = A((void**)&P->ppq, (size_t)P->nblk_tile * 8);
         if (!e) e = A((void**)&P->scal, S_NSCAL * 8 * 2);
@@ -1668,7 +1691,11 @@ int poisson_setup(sf_ctx* ctx, const sf_poisson_desc* dsc) {
         if (!e) e = hipHostMalloc((void**)&P->host_nk, sizeof(NkState));
         if (!e) e = hipEventCreate(&P->e0);
         if (!e) e = hipEventCreate(&P->e1);
-        if (e) return sf_fail(ctx, SF_ERR_OOM, "poisson allocation failed: %s", hipGetErrorString(e));
+        if (e) {
+            poisson_free(P);
+            ctx->poisson = nullptr;
+            return sf_fail(ctx, SF_ERR_OOM, "poisson allocation failed: %s", hipGetErrorString(e));
+        }
         hipMemset(P->istate, 0, 16);
         hipMemset(P->nk, 0, NK_RING * sizeof(NkState));
         hipMemset(P->nkc, 0, NK_RING * 2 * sizeof(double));
@@ -1694,7 +1721,7 @@ int poisson_setup(sf_ctx* ctx, const sf_poisson_desc* dsc) {
     SF_HIP(ctx, hipMemcpy(P->src, src.data(), nn * 4, hipMemcpyHostToDevice));
     SF_HIP(ctx, hipMemcpy(P->fixval, fixval.data(), nn * 8, hipMemcpyHostToDevice));
     if (P->nlev > 1) {
-        rc = mg_setup(ctx, P, cls);
+        rc = mg_setup(ctx, P);
         if (rc) return rc;
     }
     P->mg_hint = false;
