@@ -100,3 +100,67 @@ def test_speed_sum_of_long_moves_is_double_precision(v):
             assert err <= vmax / speed * 2.0 ** -40 + 1e-14
     finally:
         sim.close()
+
+
+def _push_scene(domain, b, x0, faces, reverse, general):
+    """Six steps of 20000 ions, a fifth of them one to two cells fast, around an object on 131 x 70 nodes;
+    fifty more join after the third."""
+    from starfish_amd.plugin import Simulation
+    ni, nj, n = 131, 70, 20000
+    mesh = D.MeshSpec(domain, ni, nj, x0, (1e-3, 7e-4), faces)
+    Lx, Ly = (ni - 1) * 1e-3, (nj - 1) * 7e-4
+    bnd = [D.BoundarySpec("c", "DIRICHLET", -100.0, D.circle_path(0.2 * Ly, 24, x0[0] + 0.5 * Lx, x0[1] + 0.5 * Ly), reverse,
+                          "SS")]
+    deck = D.Deck(mesh, boundaries=bnd, materials=[D.MaterialSpec("O+", "kinetic_hip", 16.0, 1.0, 1e4, 0.0)], solver=None,
+                  num_it=1, dt=1e-7, seed=1)
+    rng = np.random.default_rng(11)
+    lc = rng.random((n, 2)) * [ni - 1, nj - 1]
+    lc = lc[np.hypot((lc[:, 0] - 65) * 1e-3, (lc[:, 1] - 34.5) * 7e-4) > 0.22 * Ly]
+    v = rng.normal(size=(len(lc), 3)) * 2000.0
+    v[::5] = rng.choice([-1, 1], (len(v[::5]), 3)) * rng.uniform(8000, 14000, (len(v[::5]), 3))
+    v = v.astype(np.float32).astype(np.float64)
+    if general:
+        os.environ["SF_NO_FAST_PUSH"] = "1"
+    try:
+        sim = Simulation(deck, capacity=n + 64, track_ids=True, vmax=4e4)
+    finally:
+        os.environ.pop("SF_NO_FAST_PUSH", None)
+    try:
+        y, x = np.mgrid[0:nj, 0:ni]
+        sim.set_efield((3000 * np.cos(x / 9.0 + y / 5.0)).ravel(), (3000 * np.sin(x / 7.0 - y / 4.0)).ravel())
+        if b:
+            sim.set_bfield(np.where(x > ni // 2, 0.3, 0.0).ravel(), np.where(x > ni // 2, -0.2, 0.0).ravel())
+        mat = sim.materials[0]
+        add = lambda s: mat.add_particles(x0[0] + lc[s, 0] * 1e-3, x0[1] + lc[s, 1] * 7e-4, v[s, 0], v[s, 1], v[s, 2])  # noqa: E731
+        add(slice(50, None))
+        for k in range(6):
+            mat.update()
+            if k == 2:
+                add(slice(0, 50))
+        p = mat.particles(ids=True)
+        o = np.argsort(p["id"])
+        return {k: p[k][o] for k in ("id", "lc0", "lc1", "u", "v", "w")}, {f: mat.field(f) for f in ("nd", "u", "mpc-sum")}
+    finally:
+        sim.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("b", [False, True])
+@pytest.mark.parametrize("faces", ["OPEN", "PERIODIC"])
+@pytest.mark.parametrize("domain,x0,reverse", [("RZ", (0.02, -0.03), False), ("RZ", (5.0, 7.0), True),
+                                               ("ZR", (-0.03, 0.013), False), ("ZR", (1.0, 0.4), True),
+                                               ("XY", (-0.15, 0.3), False)])
+def test_fast_push_away_from_the_axis_and_around_objects(domain, x0, reverse, faces, b):
+    """The radial weights and the rotation of the tile kernel at an origin off the axis, near an object and
+    with faces that absorb or wrap, against the general kernel: the same ions survive, with the bounds of
+    the test above (state within two FP32 roundings a step, in XY without B within the parity tests')."""
+    bc = {f: (faces, 0.0) for f in D.FACES} if faces == "PERIODIC" else {}
+    s0, f0 = _push_scene(domain, b, x0, bc, reverse, True)
+    s1, f1 = _push_scene(domain, b, x0, bc, reverse, False)
+    assert len(s0["id"]) > 5000 and np.array_equal(s0["id"], s1["id"])
+    f32 = domain == "XY" and not b
+    for k, scale in (("lc0", 131), ("lc1", 70), ("u", None), ("v", None), ("w", None)):
+        scale = scale or np.abs(s0[k]).max()
+        assert np.abs(s0[k] - s1[k]).max() <= (1e-5 if f32 else 12 * 2.0 ** -23) * scale, k
+    for k in f0:
+        assert np.abs(f0[k] - f1[k]).max() <= 1e-5 * max(np.abs(f0[k]).max(), 1e-300), k
