@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "sf_internal.h"
+#include "sf_normal.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -53,26 +54,9 @@ __device__ __forceinline__ uint2 pack_bf16x4(const float4 e) {
     return make_uint2(pack_bf16x2(e.x, e.y), pack_bf16x2(e.z, e.w));
 }
 
-__device__ __forceinline__ bf16x8 load8(const uint16_t* p) {
-    uint4 v = *reinterpret_cast<const uint4*>(p);
-    bf16x8 r;
-    memcpy(&r, &v, 16);
-    return r;
-}
 __device__ __forceinline__ uint32_t bf_at(const uint4& v, int c) {
     const uint32_t w = c < 2 ? v.x : (c < 4 ? v.y : (c < 6 ? v.z : v.w));
     return (c & 1) ? (w >> 16) : (w & 0xFFFFu);
-}
-// u where ok, else zero: a select on the values (a select between the addresses of two locals
-// would keep them in scratch memory)
-__device__ __forceinline__ uint4 sel4(bool ok, const uint4 u) {
-    return make_uint4(ok ? u.x : 0u, ok ? u.y : 0u, ok ? u.z : 0u, ok ? u.w : 0u);
-}
-__device__ __forceinline__ bf16x8 zero8() {
-    uint4 v = make_uint4(0, 0, 0, 0);
-    bf16x8 r;
-    memcpy(&r, &v, 16);
-    return r;
 }
 
 // ------------------------------------------------------------------------------------------
@@ -797,30 +781,6 @@ static int cnn_alloc(sf_cnn* c, T** p, size_t n) {
 
 // real input channels and output channels of the layers c1a, c1b, c2a, c2b, c3a, c3b, c4a, c4b, c5a, c5b
 enum { C1A, C1B, C2A, C2B, C3A, C3B, C4A, C4B, C5A, C5B };
-// Normal deviates by Marsaglia's polar method, the sequence of std::normal_distribution<double> on this
-// generator (compared over 2e7 draws), without the long double logarithms that each of its draws can
-// cost: a network's 480 000 take 7 ms instead of 20 to 35.
-struct PolarNormal {
-    double sigma, kept = 0.0;
-    bool have = false;
-    static double unit(std::mt19937_64& r) {
-        const double u = (double)r() * 0x1p-64;
-        return u < 1.0 ? u : 1.0 - 0x1p-53;
-    }
-    double operator()(std::mt19937_64& r) {
-        have = !have;
-        if (!have) return kept * sigma;
-        double x, y, s;
-        do {
-            x = 2.0 * unit(r) - 1.0;
-            y = 2.0 * unit(r) - 1.0;
-            s = x * x + y * y;
-        } while (s > 1.0 || s == 0.0);
-        const double f = std::sqrt(-2.0 * std::log(s) / s);
-        kept = x * f;
-        return y * f * sigma;
-    }
-};
 static int conv_init(sf_cnn* c, ConvL& L, std::mt19937_64& rng) {
     const size_t nw = L.nw();
     if (cnn_alloc(c, &L.wf, nw) || cnn_alloc(c, &L.wt, nw)) return SF_ERR_OOM;
