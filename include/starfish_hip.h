@@ -326,13 +326,13 @@ int sf_source_added(sf_ctx* ctx, int source, int64_t* count);
  * ------------------------------------------------------------------------------------------ */
 int sf_last_timings(sf_ctx* ctx, double* out4);
 /* Split of out4[0]: out3[0] the tiled kernel over the cell-sorted particles, out3[1] the kernel
- * over the particles appended since the last sort (injected ones) where it runs by itself (otherwise
- * the slow-list kernel pushes them beside its own), out3[2] how many slots are appended ones. */
+ * over the particles appended since the last sort (injected ones) where it runs by itself (exactly 0
+ * otherwise: the slow-list kernel pushes them beside its own), out3[2] how many slots are appended ones. */
 int sf_last_push_timings(sf_ctx* ctx, double* out3);
 /* The tile kernel pushes every particle whose cell is away from segments and mesh faces and that moves
  * less than two cells, and leaves the others to slow lists that a second kernel pushes with the full
- * reference loop: out2[0] that kernel's ms (with sf_set_timing), out2[1] how many particles the last push
- * left to it.  The environment variable SF_NO_FAST_PUSH (at context creation) makes every step
+ * reference loop: out2[0] that kernel's ms (with sf_set_timing; the appended particles' with them), out2[1]
+ * how many particles the last push left to it.  The environment variable SF_NO_FAST_PUSH (at context creation) makes every step
  * run the full loop in the general tile kernel. */
 int sf_last_push_queue(sf_ctx* ctx, double* out2);
 int sf_set_timing(sf_ctx* ctx, int enabled);

@@ -976,8 +976,9 @@ __global__ void __launch_bounds__(PUSH_THREADS, 4) push_tile_fast(FastC fc, cons
     stat_flush(st, stats);
 }
 
-// The particles push_tile_fast left to the reference loop (cells next to segments or mesh
-// faces, moves of 0.99 cell or more, deviations beyond the fast quantisation range): the full
+// The particles push_tile_fast left to the reference loop (cells next to segments or mesh faces, moves of
+// 0.99 cells or more from a cell of flag 1 and of 1.99 or more from one of flag 0, particles that drifted
+// out of the tile's window, deviations beyond the fast quantisation range): the full
 // FP64 push with ProcessBoundary and the deposit into the tile's LDS window (raw patterns and
 // histogram as in the fast kernel), into global memory for particles that land outside it, or
 // with the exact quantisation past the fast range.  The work is a list of items (tile, index of the
@@ -2033,7 +2034,7 @@ int push_deposit(sf_ctx* ctx, Species* sp) {
         hipEventElapsedTime(&t0, ctx->ev[0], ctx->ev[5]);
         hipEventElapsedTime(&t1, ctx->ev[0], ctx->ev[6]);
         ctx->last_push_ms[0] = t0;
-        ctx->last_push_ms[1] = a - t1;
+        ctx->last_push_ms[1] = merged ? 0.0 : a - t1;   // (pushed beside the slow list)
         ctx->last_push_ms[2] = (double)(np_before - nsorted_before);
         ctx->last_queue[0] = t1 - t0;
         hipEventElapsedTime(&b, ctx->ev[1], ctx->ev[2]);

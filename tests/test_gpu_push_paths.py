@@ -164,3 +164,38 @@ def test_fast_push_away_from_the_axis_and_around_objects(domain, x0, reverse, fa
         assert np.abs(s0[k] - s1[k]).max() <= (1e-5 if f32 else 12 * 2.0 ** -23) * scale, k
     for k in f0:
         assert np.abs(f0[k] - f1[k]).max() <= 1e-5 * max(np.abs(f0[k]).max(), 1e-300), k
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("general", [False, True])
+def test_timings_name_the_kernel_that_pushed_appended_particles(general):
+    """sf_last_push_timings: particles appended since the last sort are pushed in the slow-list kernel's
+    launch, so their own interval is exactly zero; with the general tile kernel they have a kernel of
+    their own, with a time.  The slots are counted either way."""
+    import ctypes as C
+    from starfish_amd.plugin import Simulation
+    mesh = D.MeshSpec("XY", 131, 70, (0.0, 0.0), (1e-3, 1e-3), {f: ("SYMMETRY", 0.0) for f in D.FACES})
+    mat = D.MaterialSpec("O+", "kinetic_hip", 16.0, 1.0, 1e4, 0.0)
+    if general:
+        os.environ["SF_NO_FAST_PUSH"] = "1"
+    try:
+        sim = Simulation(D.Deck(mesh, materials=[mat], solver=None, num_it=1, dt=1e-8, seed=1), capacity=30000, vmax=4e4)
+    finally:
+        os.environ.pop("SF_NO_FAST_PUSH", None)
+    try:
+        sim.ctx.call("sf_set_timing", 1)
+        m = sim.materials[0]
+        m.preload(20000, (100.0, 0.0, 0.0), 300.0, seed=1)
+        m.update()
+        one = np.full(300, 1000.0)
+        m.add_particles(np.full(300, 0.05), np.full(300, 0.03), one, one, one)
+        m.update()
+        split, queue = np.zeros(3), np.zeros(2)
+        dp = C.POINTER(C.c_double)
+        sim.ctx.call("sf_last_push_timings", split.ctypes.data_as(dp))
+        sim.ctx.call("sf_last_push_queue", queue.ctypes.data_as(dp))
+        print(split, queue, flush=True)
+        assert split[2] == 300 and split[0] > 0
+        assert split[1] > 0 if general else split[1] == 0 and queue[0] > 0
+    finally:
+        sim.close()
