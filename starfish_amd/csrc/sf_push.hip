@@ -788,6 +788,7 @@ __global__ void __launch_bounds__(PUSH_THREADS, 4) push_tile_fast(FastC fc, cons
                 const float2 e00 = L.ef[l], e10 = L.ef[l + 1], e01 = L.ef[l + TILE_NW], e11 = L.ef[l + TILE_NW + 1];
                 int nci = ci, ncj = cj;
                 bool longer = !F32;
+                double speed = 0.0;   // in the precision of the move
                 if (F32) {
                     const float gx = 1.0f - cur.fx, gy = 1.0f - cur.fy;
                     const float ex = gy * (gx * e00.x + cur.fx * e10.x) + cur.fy * (gx * e01.x + cur.fx * e11.x);
@@ -809,6 +810,7 @@ __global__ void __launch_bounds__(PUSH_THREADS, 4) push_tile_fast(FastC fc, cons
                     fyn = yn - fly;
                     nci += (int)flx;
                     ncj += (int)fly;
+                    speed = (double)sqrtf(vxn * vxn + vyn * vyn + vzn * vzn);
                 }
                 if (longer) {
                     // push_particle's single sub-move in its order of operations; a cell without the
@@ -864,6 +866,8 @@ __global__ void __launch_bounds__(PUSH_THREADS, 4) push_tile_fast(FastC fc, cons
                     vxn = (float)v0;
                     vyn = (float)v1;
                     vzn = (float)v2;
+                    const double a0 = vxn, a1 = vyn, a2 = vzn;
+                    speed = sqrt(a0 * a0 + a1 * a1 + a2 * a2);
                 }
                 // x' - floor(x') can round up to 1 for x' just below an integer: that position is
                 // offset 0 of the next cell (the stored cell is floor(lc))
@@ -879,12 +883,7 @@ __global__ void __launch_bounds__(PUSH_THREADS, 4) push_tile_fast(FastC fc, cons
                     sp0 += qbits(1.0, (double)vxn * fc.kst);
                     sp1 += qbits(1.0, (double)vyn * fc.kst);
                     sp2 += qbits(1.0, (double)vzn * fc.kst);
-                    if (!longer) {
-                        se += qbits(1.0, (double)sqrtf(vxn * vxn + vyn * vyn + vzn * vzn) * fc.kst);
-                    } else {   // (an FP64 move's speed is FP64 as well, as in stat_add)
-                        const double a0 = vxn, a1 = vyn, a2 = vzn;
-                        se += qbits(1.0, sqrt(a0 * a0 + a1 * a1 + a2 * a2) * fc.kst);
-                    }
+                    se += qbits(1.0, speed * fc.kst);
                     dmax = fmax(dmax, dev);
                     // deposit of the 7 channels from the stored FP32 state (Field2D.scatter), with
                     // Ruyten's radial weight in RZ and ZR
