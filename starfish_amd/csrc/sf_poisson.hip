@@ -613,9 +613,10 @@ static_assert(MG_W * MG_H == 4 * MG_NT, "one thread per 2 x 2 aggregate");
 // needs 3 to 6: past 16 the switch pays however long the linear solve would have been.
 // The first linear solve of a cold solve shows it too (56 iterations at 1e-3 on the 1024 x 512 cylinder
 // deck, 184 on the RZ mesh; 13 at 256 x 128, where the tiles stay the better choice: 2.4 ms).
-// The host's loop (cold and linear solves) looks after MG_SWITCH_HOST: the tiles' cheap iterations still
-// gain there (a switch after 17 made the cold solve 0.2 ms longer), and the count is the same whatever
-// batches the solves before have left.
+// The host's loop looks after exactly that many in a linear solve and after MG_SWITCH_HOST in a Newton
+// step of a cold one, whose tighter steps the tiles' cheap iterations still help (a switch after 17 made
+// the 1024 x 512 RZ solve 0.2 ms longer; in linear solves 16 instead of 24 take 0.1 ms off): a fixed
+// count, whatever batches the solves before have left.
 constexpr int MG_SWITCH = 16, MG_SWITCH_HOST = 24;
 constexpr int MG_LOOSE_STEPS = 32;       // Newton steps of a solve that may use ETA_MG
 constexpr int64_t MG_MIN_NODES = 1024;   // below, a few tiles are the whole mesh
@@ -1846,6 +1847,7 @@ int poisson_solve(sf_ctx* ctx, sf_solve_info* info) {
     // 1.2e-4), and one whose steps are few would run out of them (nl_max_it 12 there), so the term holds
     // where only the residual stops the solve, and for the first half of an ample number of steps.
     const bool loose_ok = !(nl_tol > 0) && nl_max >= MG_LOOSE_STEPS;
+    const int host_switch = D.linear ? MG_SWITCH : MG_SWITCH_HOST;
     int rc = 0;
     // the last solve converged and this one starts from its potential: go straight to the device
     // loop (it hands a cold start back untouched)
@@ -1965,8 +1967,9 @@ int poisson_solve(sf_ctx* ctx, sf_solve_info* info) {
             bool first_batch = true, done_in_first = false;
             while (true) {
                 int nb = std::min(batch, max_it - before - k);
-                // (the host looks there, whatever batches the last solve left)
-                if (!mg && P->nlev > 1 && k < MG_SWITCH_HOST) nb = std::min(nb, MG_SWITCH_HOST - k);
+                // (the host looks there, whatever batches the last solve left, and not shortly before)
+                if (!mg && P->nlev > 1 && k < host_switch && k + nb > host_switch - 8)
+                    nb = std::min(host_switch - k, max_it - before - k);
                 for (int b = 0; b < nb; b++, k++) {
                     double* cur = (k & 1) ? pz1 : pz0;
                     double* nxt = (k & 1) ? pz0 : pz1;
@@ -2014,7 +2017,7 @@ int poisson_solve(sf_ctx* ctx, sf_solve_info* info) {
                 if (before + k >= max_it) { its = k; break; }
                 batch = std::min(2 * batch, mg ? 8 : 64);
                 first_batch = false;
-                if (!mg && P->nlev > 1 && k >= MG_SWITCH_HOST) {
+                if (!mg && P->nlev > 1 && k >= host_switch) {
                     // the same linear solve from its current residual and correction, conjugate
                     // directions started anew
                     mg = true;
