@@ -32,13 +32,12 @@ constexpr int NK_RING = 8;
 // Forcing terms of the inexact Newton steps: a linear solve stops at eta times its starting
 // residual.  ETA_COLD for a solve that starts far from its solution (first residual at least half
 // the reference residual, as from phi = 0), ETA_WARM for one started from the previous step's phi.
-// Measured on the 1024x512 cylinder deck: warm solves take 0.82, 0.76, 0.74, 0.70, 0.67 and
-// 0.68 ms at eta = 1e-3, 3e-3, 1e-2, 3e-2, 5e-2 and 1e-1 (fewer PCG iterations, a few more Newton
-// updates); a cold solve with 1e-2 takes 117 instead of 70 ms.  On meshes too large for one
-// wide PCG tile per CU (narrow tiles, choose_tile_shape) a PCG iteration costs more and the
-// linear solves converge more slowly, and looser inner solves pay: on the 2048 x 1024 RZ deck warm
-// solves take 18.1, 17.6, 16.2 and 19.0 ms at eta = 2e-2, 5e-2, 1e-1 and 2e-1 (the 1024 x 512
-// deck: 0.63 ms at 5e-2, 0.66 at 1e-1, 0.70 at 2e-1).
+// ETA_WARM_LARGE for warm solves on meshes too large for one wide PCG tile per CU (choose_tile_shape).
+// Only solves that the tiles finish in MG_SWITCH iterations a step are left to the last two, and those
+// do not depend on the term where one iteration a step reaches any of them (cylinder deck, 1024 x 512:
+// 0.25 ms at 1e-2 to 1e-1).  On 2048 x 1024 and 1500 x 1200 a Newton step costs more than an iteration:
+// 0.78 and 0.82 ms at 2e-2, 0.76 and 0.93 at 5e-2, 0.90 and 0.97 at 1e-1, 0.89 and 1.04 at 2e-1.  (1e-1
+// was chosen when such meshes' warm solves took hundreds of iterations, which now go to the multigrid.)
 // With the multigrid preconditioner an iteration gains about a digit and a loose inner solve costs
 // little: cold solves of the 1024 x 512 RZ mesh take 9.8, 7.8, 6.7, 7.0 and 6.2 ms at eta = 1e-3, 1e-2,
 // 5e-2, 1e-1 and 2e-1, warm ones of 2048 x 1024 2.2, 2.3 and 2.1 ms at the last three and of 600 x 400
@@ -340,8 +339,8 @@ struct TileShape {
 };
 // 128 x 16 tiles of 1024 threads: the stronger block preconditioner, for meshes whose tiles fit in
 // one workgroup per CU.  64 x 16 tiles of 512 threads on larger meshes, where several workgroups
-// per CU hide each other's barriers (choose_tile_shape); there nk_step_b is held to 64 registers so
-// that four of them fit a CU (69 registers allow three).
+// per CU hide each other's barriers (choose_tile_shape); there nk_step_b is held to 64 registers (it
+// takes 60) so that four of them fit a CU; with the 82 that the wide one takes two would.
 using TileWide = TileShape<128, 16, 1024, 4>;
 using TileNarrow = TileShape<64, 16, 512, 8>;
 
@@ -612,7 +611,7 @@ static_assert(MG_W * MG_H == 4 * MG_NT, "one thread per 2 x 2 aggregate");
 // multigrid.  At 1024 x 512 an iteration costs 20 us with the tiles and 70 us with the multigrid, which
 // needs 3 to 6: past 16 the switch pays however long the linear solve would have been.
 // The first linear solve of a cold solve shows it too (56 iterations at 1e-3 on the 1024 x 512 cylinder
-// deck, 184 on the RZ mesh; 13 at 256 x 128, where the tiles stay the better choice: 2.4 ms).
+// deck, 184 on the RZ mesh, 13 at 256 x 128).
 // The host's loop looks after exactly that many in a linear solve and after MG_SWITCH_HOST in a Newton
 // step of a cold one, whose tighter steps the tiles' cheap iterations still help (a switch after 17 made
 // the 1024 x 512 RZ solve 0.2 ms longer; in linear solves 16 instead of 24 take 0.1 ms off): a fixed
@@ -1282,11 +1281,12 @@ __global__ void __launch_bounds__(TS::NT, TS::MINW) nk_step_b(MeshP m, const uin
 
 template <class TS>
 static int tile_count(int ni, int nj) { return ((ni + TS::W - 1) / TS::W) * ((nj + TS::H - 1) / TS::H); }
-// Wide tiles while the mesh needs at most one of their workgroups per CU.  nk_step_b's 69 registers
+// Wide tiles while the mesh needs at most one of their workgroups per CU.  nk_step_b's 82 registers
 // leave room for one 16-wave workgroup per CU, so more wide tiles than CUs run in rounds with no
-// second workgroup to overlap a round's barriers and tail.  Measured warm solves: 1024 x 512 (256
-// wide tiles) 0.62 ms with wide tiles, 0.65 with narrow ones; 2048 x 1024 (1024 wide tiles) 21.9 ms
-// with wide tiles, 17.6 with narrow ones held to 64 registers (17.9 with wide ones held to 64).
+// second workgroup to overlap a round's barriers and tail.  Measured warm solves that end on the tiles,
+// wide and narrow: 1024 x 512 (256 wide tiles) 0.250 and 0.247 ms with one iteration a step; 1500 x 1200
+// (900) 1.10 and 0.97 ms, 2048 x 1024 (1024) 1.76 and 1.55 ms with three, 0.86 and 0.90 with one; solves
+// that go on to the multigrid after 16 3.4 and 2.9 ms.
 static bool choose_tile_shape(int ni, int nj) {
     int dev = 0, ncu = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
@@ -1809,8 +1809,8 @@ int poisson_solve(sf_ctx* ctx, sf_solve_info* info) {
                 step_b(i, 0);
             }
             SF_HIP(ctx, hipGetLastError());
-            // the state, the scalars, and phi from x, queued before the host reads the state: when the batch ended the solve the
-            // potential is already written (otherwise the next batch's expansion overwrites it)
+            // the state, the scalars, and phi from x, queued before the host reads the state: when the batch
+            // ended the solve the potential is already written (otherwise the next batch's expansion overwrites it)
             hipLaunchKernelGGL(expand_phi, dim3(ge), dim3(256), 0, st, nn, (const int32_t*)P->src,
                                (const double*)P->fixval, (const double*)P->x, ctx->d_phi,
                                (const NkState*)(P->nk + (i - 1) % NK_RING), P->host_nk, (const double*)P->scal,
