@@ -118,7 +118,7 @@ __device__ __forceinline__ unsigned int mcc_particle(const MeshP& m, const PStat
 // thread in flight: a thousand would wait for their atomics on that counter (1024 x 512 nodes: 45 us
 // with 1024 of them, 10 with these).
 constexpr int MCC_BOUND_BLOCKS = 256;
-constexpr int64_t MCC_BOUND_MIN = 1 << 19;   // particles (beyond the nodes) for which one pass pays for the bound
+constexpr int64_t MCC_BOUND_MIN = 1 << 18;   // particles (beyond a quarter of the nodes) for which a pass pays for the bound
 struct MccBound {
     unsigned int bound[4], done;
     float part[MCC_BOUND_BLOCKS][4];
@@ -188,7 +188,8 @@ __global__ void __launch_bounds__(256) mcc_target_bounds(int64_t nn, MccTarget t
 // A workgroup tests SLOTS slots a thread at a time, 4 in 16-byte loads.  A population of at most a workgroup
 // of 256 for every CU takes 1: the colliding particles of 1024 slots would take their workgroup four
 // rounds while most CUs have none (1e4 particles that all collide: 42.0 us with 4, 26.6 with 1; 6.5e4 50
-// and 41; 2e5, on more workgroups than CUs, 67 and 102).
+// and 41; 2e5, on more workgroups than CUs, 67 and 102).  So does a pass without a bound, which tests all
+// of them (1024 x 512 nodes, 7e4 and 2.7e5 particles: 29 and 33 us, 42 with 4).
 template <int SLOTS>
 __global__ void __launch_bounds__(256) mcc_kernel(MeshP m, PState s, int64_t np, MccTarget tg, MccParams pp,
                                                   const MccBound* __restrict__ bounds, int bounded,
@@ -322,11 +323,13 @@ static int grid_n(int64_t n, int max_blocks) {
     return (int)(b < max_blocks ? b : max_blocks);
 }
 
-// The bound of a target takes about 6 us and 8 ps a node, and saves 13 ps a particle and pass: it is made
-// with the target where one pass pays for it, else at its second pass.  (A host that sets the target of
-// few particles before every pass had paid 10 to 20 us a pass for it.)
+// The bound of a target takes 6 to 10 us on a mesh up to 1024 x 512 and saves 13 ps a particle and pass: it
+// is made with the target where a pass about pays for it, else at the target's second pass.  A host that
+// sets the target before every pass waits for both (301 x 157 nodes, 7e4 and 2.7e5 particles: 137 and
+// 140 us without the bound, 153 with); one that keeps it loses 1 to 4 us of the first pass.
 static bool bound_pays(const sf_mcc* c) {
-    return c->ctx->species[c->desc.source_species]->np > MCC_BOUND_MIN + (int64_t)c->ctx->mp.ni * c->ctx->mp.nj;
+    return c->ctx->species[c->desc.source_species]->np >
+           MCC_BOUND_MIN + (int64_t)c->ctx->mp.ni * c->ctx->mp.nj / 4;
 }
 static int make_bound(sf_mcc* c) {
     sf_ctx* ctx = c->ctx;
@@ -466,7 +469,7 @@ int sf_mcc_perform(sf_mcc* c, int it, double time, int64_t* collisions) {
                                ctx->stream, ctx->mp, sp->buf[sp->cur], sp->np, tg, pp, (const MccBound*)c->d_bound,
                                (int)c->bounded, c->d_count, c->d_S, c->d_ncol);
         };
-        if (sp->np <= 256 * (int64_t)ctx->ncu) pass(mcc_kernel<1>, 256);
+        if (!c->bounded || sp->np <= 256 * (int64_t)ctx->ncu) pass(mcc_kernel<1>, 256);
         else pass(mcc_kernel<4>, 1024);
         SF_HIP(ctx, hipGetLastError());
     }
