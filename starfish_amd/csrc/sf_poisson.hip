@@ -598,9 +598,9 @@ __global__ void __launch_bounds__(TS::NT) pcg_update(MeshP m, const uint8_t* __r
 // block computes the two rings of halo values it needs itself, which makes each level two kernels
 // without any exchange; the levels of at most MG_BOTTOM nodes in all run in one workgroup in LDS.
 // Measured: warm solves of the 2048 x 1024 RZ mesh 30.4 -> 2.2 ms (554 -> 8 iterations), the cold one of
-// 1024 x 512 57.6 -> 7.6 ms (2206 -> 69).  An iteration at 2048 x 1024 takes about 125 us: 18 + 34 + 23 in
-// the three kernels on the fine level (21 + 36 + 21 B a node), 5 in each of the two kernels of the
-// four middle levels, 14 in the bottom kernel, the rest between launches.
+// 1024 x 512 57.6 -> 7.6 ms (2206 -> 70).  An iteration at 2048 x 1024 takes about 125 us: 28 + 34 + 22 in
+// the three kernels on the fine level (21 + 36 + 21 B a node), 6 in each of the two kernels of the
+// four middle levels, 16 in the bottom kernel, the rest between launches.
 // ------------------------------------------------------------------------------------------
 constexpr int MG_W = 64, MG_H = 16, MG_NT = 256;      // nodes of a block's tile, threads
 constexpr int MG_LW = MG_W + 4, MG_LH = MG_H + 4;     // with two rings of halo
