@@ -258,6 +258,8 @@ def learned_guess(sim, deck, args, rho0):
                "all_converged": all(r[k][4] == 0 for r in rows for k in r) and cold["zero"]["converged"]
                and cold["learned"]["converged"]}
         out["iteration_ratio_plain_over_learned"] = out["plain"]["pcg_iterations"] / max(1.0, out["learned"]["pcg_iterations"])
+        # (iterations count the tiles' and the V-cycle's alike, which cost 20 and 70 us: times decide)
+        out["time_ratio_plain_over_learned"] = out["plain"]["ms"] / max(1e-9, out["learned"]["ms"])
         out["network_throughput"] = cnn_throughput(sim.ctx, m.ni, m.nj)
         return out, net
     except Exception:

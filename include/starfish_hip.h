@@ -240,8 +240,9 @@ int sf_species_boundary_hits(sf_ctx* ctx, int species, int nbnd, int64_t* counts
  * (core/solver/SolverModule.java:71-86).  The operator is the reference's finite-volume
  * assembly (Solver.initCoefficients, core/solver/Solver.java:204-256, 451-726) applied
  * matrix-free; Dirichlet and one-sided Neumann rows are eliminated into an equivalent
- * symmetric system solved with Jacobi-PCG in FP32 and FP64 residual refinement inside the
- * FP64 Newton iteration on the Boltzmann term (Solver.solveNonLinearNR, Solver.java:293-387).
+ * symmetric system solved with PCG in FP32 (tile or multigrid preconditioner) and FP64
+ * residual refinement inside the FP64 Newton iteration on the Boltzmann term
+ * (Solver.solveNonLinearNR, Solver.java:293-387).
  * ------------------------------------------------------------------------------------------ */
 typedef struct {
     int linear;          /* PoissonSolver "linear" */

@@ -1,10 +1,10 @@
 // DSMC collisions on the device (collisions/DSMC.java:167-430): Bird's no-time-counter scheme
 // per cell after the counting sort, with Boyd's weighting for two species, a constant or VHS
 // (SigmaPlus.SigmaBird463) cross-section and the elastic VHS/VSS scattering of ModelElastic.
-// A cell's particle list is the cell range of the sorted species, ordered by particle id (one wave
-// per cell, dsmc_order), so that the pair choice (an index into that list) and the cell's Philox
+// A cell's particle list is the cell range of the sorted species, ordered by particle id
+// (dsmc_order), so that the pair choice (an index into that list) and the cell's Philox
 // stream give the same collisions on every run.  The pairs of a cell are processed in sequence, as
-// in the reference, by one lane; a wave runs 64 cells (dsmc_collide).
+// in the reference, by one lane; a wave runs up to 64 cells (dsmc_collide).
 #include <algorithm>
 #include <cmath>
 #include <vector>
